@@ -13,10 +13,14 @@
 // an 8 x 8 block of a 128 x 128 tile, split as rows {4ty..4ty+3} and
 // {64+4ty..64+4ty+3} (same for columns) so that every ds_read_b128 of a
 // wave covers 256 contiguous bytes.  K advances in chunks of 16 staged
-// through LDS in k-major layout, double-buffered.  k_scores_store is held to
-// 168 VGPRs so that 3 workgroups share a CU: gfx950 issues independent FP32
-// VALU work fastest with several waves per SIMD ready (9% over 2 per SIMD).
-// A fourth does not fit without spilling the tile.
+// through LDS in k-major layout, double-buffered.  The bound is VALU issue,
+// 128 instructions per thread and k-step: one wave issues at most one every
+// 4.9 cycles, two or more ready waves one per 2.16 cycles and SIMD (a probe of
+// independent v_mul / v_add).  Three waves per SIMD (156 VGPRs) cover each
+// other's LDS reads and barriers; the tile's loads carry no bounds branches
+// and few address registers, which a fourth wave (128 VGPRs) still spills.
+// 40,000 x 50,000 x 150: 13.6 -> 11.3 ms, 26.4e12 products/s, 2.28 cycles per
+// instruction at the 1.97 GHz the card holds under this load.
 #include "rkr_internal.hpp"
 
 namespace rkr {
@@ -25,29 +29,43 @@ namespace {
 constexpr int BM = 128, BN = 128, KC = 16, NT = 256;
 constexpr int LDS_PAD = 4;  // k-major rows of BM + pad floats
 
-struct TileSmem {
+// 16-byte aligned rows, so a thread's four values are one ds_read_b128.
+struct alignas(16) TileSmem {
     float a[2][KC][BM + LDS_PAD];
     float b[2][KC][BN + LDS_PAD];
 };
 
-// Loads rows [r0, r0+128) x k-chunk [k0, k0+16) of a row-major matrix
-// (leading dimension ld, a multiple of 4) into two float4 registers.
-// Rows past n_rows and columns at or past ld load as zero.
-__device__ __forceinline__ void load_chunk(const float *__restrict__ X, const int32_t *__restrict__ rows,
-                                           int64_t r0, int64_t n_rows, int32_t ld, int32_t k0, float4 (&reg)[2]) {
-    const int t = threadIdx.x;
-    const int kq = (t & 3) * 4;
+// One thread's share of the staging of a 128-row operand: rows t / 4 and
+// t / 4 + 64, the four k's at 4 (t % 4) of every chunk.  Rows past n_rows read
+// the last row (their outputs are never stored or counted) and columns past
+// ld the row's last four (never computed: ld >= K).
+// GATHER: row r of the operand is row rows[r] of X.
+template <bool GATHER>
+struct ChunkLoader {
+    const float *base;  // the tile's first row (X itself when gathered)
+    const float *p[GATHER ? 2 : 1];
+    uint32_t off[GATHER ? 1 : 2];
+    int32_t ld;
+    __device__ __forceinline__ ChunkLoader(const float *__restrict__ X, const int32_t *__restrict__ rows, int64_t r0,
+                                           int64_t n_rows, int32_t ld_)
+        : base(X + (GATHER ? 0 : r0 * ld_)), ld(ld_) {
+        const int last = (int)min((int64_t)(BM - 1), n_rows - 1 - r0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int64_t r = r0 + (t >> 2) + h * 64;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (r < n_rows && k0 + kq < ld) {
-            const int64_t src = rows ? (int64_t)rows[r] : r;
-            v = *reinterpret_cast<const float4 *>(X + src * (int64_t)ld + k0 + kq);
+        for (int h = 0; h < 2; ++h) {
+            const int r = min((int)(threadIdx.x >> 2) + h * 64, last);
+            if constexpr (GATHER) p[h] = X + (int64_t)rows[r0 + r] * ld;
+            else off[h] = (uint32_t)r * (uint32_t)ld;
         }
-        reg[h] = v;
     }
-}
+    __device__ __forceinline__ void load(int32_t k0, float4 (&reg)[2]) const {
+        const uint32_t k = (uint32_t)min(k0 + (int32_t)(threadIdx.x & 3) * 4, ld - 4);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (GATHER) reg[h] = *reinterpret_cast<const float4 *>(p[h] + k);
+            else reg[h] = *reinterpret_cast<const float4 *>(base + (off[h] + k));
+        }
+    }
+};
 
 __device__ __forceinline__ void store_chunk(float (*dst)[BM + LDS_PAD], const float4 (&reg)[2]) {
     const int t = threadIdx.x;
@@ -62,7 +80,30 @@ __device__ __forceinline__ void store_chunk(float (*dst)[BM + LDS_PAD], const fl
     }
 }
 
+// A thread's operands of one k-step.
+struct StepFrag {
+    float4 a0, a1, b0, b1;
+    __device__ __forceinline__ void read(const float *__restrict__ pa, const float *__restrict__ pb) {
+        a0 = *reinterpret_cast<const float4 *>(pa);
+        a1 = *reinterpret_cast<const float4 *>(pa + 64);
+        b0 = *reinterpret_cast<const float4 *>(pb);
+        b1 = *reinterpret_cast<const float4 *>(pb + 64);
+    }
+    __device__ __forceinline__ void add_to(float (&acc)[8][8]) const {
+        const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        const float bv[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float p = av[i] * bv[j];
+                acc[i][j] = acc[i][j] + p;
+            }
+    }
+};
+
 // acc[i][j] = score(A row i of the tile, B row j of the tile) over k < K.
+template <bool GATHER>
 __device__ __forceinline__ void tile_scores(TileSmem &sm, const float *__restrict__ A,
                                             const int32_t *__restrict__ a_rows, int64_t m0, int64_t M,
                                             int32_t lda, const float *__restrict__ B, int64_t n0, int64_t N,
@@ -73,35 +114,33 @@ __device__ __forceinline__ void tile_scores(TileSmem &sm, const float *__restric
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[i][j] = 0.0f;
 
+    const ChunkLoader<GATHER> la(A, a_rows, m0, M, lda);
+    const ChunkLoader<false> lb(B, nullptr, n0, N, ldb);
     float4 ra[2], rb[2];
     const int nchunk = (K + KC - 1) / KC;
-    load_chunk(A, a_rows, m0, M, lda, 0, ra);
-    load_chunk(B, nullptr, n0, N, ldb, 0, rb);
+    la.load(0, ra);
+    lb.load(0, rb);
     store_chunk(sm.a[0], ra);
     store_chunk(sm.b[0], rb);
     __syncthreads();
     for (int c = 0; c < nchunk; ++c) {
         const int buf = c & 1;
         const int k0 = c * KC;
-        if (c + 1 < nchunk) {
-            load_chunk(A, a_rows, m0, M, lda, k0 + KC, ra);
-            load_chunk(B, nullptr, n0, N, ldb, k0 + KC, rb);
-        }
+        // the next chunk's loads are in flight while this one is computed (the
+        // last chunk's are its own again, unused)
+        la.load(min(k0 + KC, (nchunk - 1) * KC), ra);
+        lb.load(min(k0 + KC, (nchunk - 1) * KC), rb);
+        const float *pa = &sm.a[buf][0][ty * 4], *pb = &sm.b[buf][0][tx * 4];
+        constexpr int ROW = BM + LDS_PAD;
+        static_assert(BM == BN, "one row stride for both operands");
         const int kend = min(KC, K - k0);
+#pragma unroll 4
         for (int kk = 0; kk < kend; ++kk) {
-            const float4 a0 = *reinterpret_cast<const float4 *>(&sm.a[buf][kk][ty * 4]);
-            const float4 a1 = *reinterpret_cast<const float4 *>(&sm.a[buf][kk][64 + ty * 4]);
-            const float4 b0 = *reinterpret_cast<const float4 *>(&sm.b[buf][kk][tx * 4]);
-            const float4 b1 = *reinterpret_cast<const float4 *>(&sm.b[buf][kk][64 + tx * 4]);
-            const float av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-            const float bv[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float p = av[i] * bv[j];
-                    acc[i][j] = acc[i][j] + p;
-                }
+            StepFrag f;
+            f.read(pa, pb);
+            f.add_to(acc);
+            pa += ROW;
+            pb += ROW;
         }
         if (c + 1 < nchunk) {
             store_chunk(sm.a[buf ^ 1], ra);
@@ -114,26 +153,57 @@ __device__ __forceinline__ void tile_scores(TileSmem &sm, const float *__restric
 __device__ __forceinline__ int tile_row(int i) { return (i < 4) ? ((threadIdx.x >> 4) * 4 + i) : (64 + (threadIdx.x >> 4) * 4 + i - 4); }
 __device__ __forceinline__ int tile_col(int j) { return (j < 4) ? ((threadIdx.x & 15) * 4 + j) : (64 + (threadIdx.x & 15) * 4 + j - 4); }
 
-__global__ void __launch_bounds__(NT, 3) k_scores_store(const float *__restrict__ A, const int32_t *__restrict__ a_rows,
-                                                     int64_t M, int32_t lda, const float *__restrict__ B, int64_t N,
+// Workgroups go to the 8 XCDs in turn, each with its own L2: block p takes
+// logical tile (p % 8) * per + p / 8, so an XCD runs one contiguous eighth of
+// the tiles, and logical tiles walk the columns of a band of kBand tile rows,
+// the band's rows first, so the tiles an XCD runs at one time share their A
+// rows and a few B column blocks.
+constexpr int64_t kBand = 8;
+
+__device__ __forceinline__ bool tile_of_block(int64_t n_tiles_m, int64_t n_tiles_n, int64_t &tm, int64_t &tn) {
+    const int64_t n_tiles = n_tiles_m * n_tiles_n, per = (n_tiles + 7) / 8;
+    const int64_t t = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (t >= n_tiles || (int64_t)(blockIdx.x >> 3) >= per) return false;
+    const int64_t band = t / (kBand * n_tiles_n), in = t - band * (kBand * n_tiles_n);
+    const int64_t rows = min(kBand, n_tiles_m - band * kBand);
+    tm = band * kBand + in % rows;
+    tn = in / rows;
+    return true;
+}
+
+// ROW_M: C[m * ldc + n], else C[n * ldc + m].  vec: rows of C start 16-byte
+// aligned, so four neighbouring outputs are one store.
+template <bool ROW_M>
+__global__ void __launch_bounds__(NT, 3) k_scores_store(const float *__restrict__ A, int64_t M, int32_t lda,
+                                                     const float *__restrict__ B, int64_t N,
                                                      int32_t ldb, int32_t K, float *__restrict__ C, int64_t ldc,
-                                                     int c_row_major_m, int64_t n_tiles_n) {
+                                                     int vec, int64_t n_tiles_m, int64_t n_tiles_n) {
     __shared__ TileSmem sm;
-    const int64_t tile = blockIdx.x;
-    const int64_t tm = tile / n_tiles_n, tn = tile % n_tiles_n;
+    int64_t tm, tn;
+    if (!tile_of_block(n_tiles_m, n_tiles_n, tm, tn)) return;
     const int64_t m0 = tm * BM, n0 = tn * BN;
     float acc[8][8];
-    tile_scores(sm, A, a_rows, m0, M, lda, B, n0, N, ldb, K, acc);
+    tile_scores<false>(sm, A, nullptr, m0, M, lda, B, n0, N, ldb, K, acc);
+    // outer index o runs over C's rows, inner over the contiguous direction
+    const int64_t o0 = ROW_M ? m0 : n0, i0 = ROW_M ? n0 : m0, n_o = ROW_M ? M : N, n_i = ROW_M ? N : M;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int64_t m = m0 + tile_row(i);
-        if (m >= M) continue;
+    for (int o = 0; o < 8; ++o) {
+        const int64_t r = o0 + (ROW_M ? tile_row(o) : tile_col(o));
+        if (r >= n_o) continue;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int64_t n = n0 + tile_col(j);
-            if (n >= N) continue;
-            if (c_row_major_m) C[m * ldc + n] = acc[i][j];
-            else C[n * ldc + m] = acc[i][j];
+        for (int h = 0; h < 2; ++h) {
+            const int64_t q = i0 + (ROW_M ? tile_col(4 * h) : tile_row(4 * h));
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = ROW_M ? acc[o][4 * h + j] : acc[4 * h + j][o];
+            float *dst = C + r * ldc + q;
+            if (vec && q + 3 < n_i) {
+                *reinterpret_cast<float4 *>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (q + j < n_i) dst[j] = v[j];
+            }
         }
     }
 }
@@ -141,9 +211,9 @@ __global__ void __launch_bounds__(NT, 3) k_scores_store(const float *__restrict_
 // Persistent refinement count.  Work unit = (block of 128 refine rows,
 // group of kGroup item tiles).  Each unit adds, for every row r of its
 // block, #{items p in the group : score(user(r), p) > thr(r)} to cnt[r].
-constexpr int kGroup = 8;
+constexpr int kGroup = 8;  // a thread counts at most 8 per tile and row: 8 * kGroup < 256
 
-__global__ void __launch_bounds__(NT) k_refine_count(const float *__restrict__ users, const float *__restrict__ items,
+__global__ void __launch_bounds__(NT, 3) k_refine_count(const float *__restrict__ users, const float *__restrict__ items,
                                                      int64_t n_item, int32_t ld, int32_t K,
                                                      const int32_t *__restrict__ rows_user,
                                                      const float *__restrict__ rows_thr,
@@ -151,6 +221,7 @@ __global__ void __launch_bounds__(NT) k_refine_count(const float *__restrict__ u
                                                      int32_t *__restrict__ cnt) {
     __shared__ TileSmem sm;
     __shared__ int32_t red[BM];
+    __shared__ float s_thr[BM];
     const int64_t n_rows = min((int64_t)*n_rows_dev, max_rows);
     const int64_t n_rb = (n_rows + BM - 1) / BM;
     const int64_t n_it = (n_item + BN - 1) / BN;
@@ -159,31 +230,35 @@ __global__ void __launch_bounds__(NT) k_refine_count(const float *__restrict__ u
     for (int64_t unit = blockIdx.x; unit < n_units; unit += gridDim.x) {
         const int64_t rb = unit / n_grp, g = unit % n_grp;
         const int64_t m0 = rb * BM;
-        float thr[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int64_t m = m0 + tile_row(i);
-            thr[i] = m < n_rows ? rows_thr[m] : 0.0f;
+        if (threadIdx.x < BM) {
+            const int64_t m = m0 + threadIdx.x;
+            s_thr[threadIdx.x] = m < n_rows ? rows_thr[m] : 0.0f;  // read after tile_scores' barriers
+            red[threadIdx.x] = 0;
         }
-        int32_t c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        // the thread's eight row counts, a byte each (at most 8 per tile, 64
+        // per unit): registers are short beside the tile
+        uint32_t c[2] = {0u, 0u};
         const int64_t t_end = min((g + 1) * kGroup, n_it);
         for (int64_t it = g * kGroup; it < t_end; ++it) {
             const int64_t n0 = it * BN;
             float acc[8][8];
-            tile_scores(sm, users, rows_user, m0, n_rows, ld, items, n0, n_item, ld, K, acc);
+            tile_scores<true>(sm, users, rows_user, m0, n_rows, ld, items, n0, n_item, ld, K, acc);
+            const int n_in = (int)min((int64_t)BN, n_item - n0);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const bool in = n0 + tile_col(j) < n_item;
+            for (int i = 0; i < 8; ++i) {
+                const float thr = s_thr[tile_row(i)];
+                uint32_t v = 0;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) c[i] += (in && acc[i][j] > thr[i]) ? 1 : 0;
+                for (int j = 0; j < 8; ++j) v += (tile_col(j) < n_in && acc[i][j] > thr) ? 1u : 0u;
+                c[i >> 2] += v << (8 * (i & 3));
             }
         }
         // reduce over the 16 threads that share each row
-        if (threadIdx.x < BM) red[threadIdx.x] = 0;
-        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (c[i]) atomicAdd(&red[tile_row(i)], c[i]);
+        for (int i = 0; i < 8; ++i) {
+            const int32_t v = (int32_t)((c[i >> 2] >> (8 * (i & 3))) & 0xFFu);
+            if (v) atomicAdd(&red[tile_row(i)], v);
+        }
         __syncthreads();
         if (threadIdx.x < BM) {
             const int64_t m = m0 + threadIdx.x;
@@ -242,13 +317,17 @@ __global__ void k_make_panels(const float *__restrict__ users, int64_t n_user, i
 
 }  // namespace
 
-hipError_t launch_scores_store(hipStream_t s, const float *A, const int32_t *a_rows, int64_t M, int32_t lda,
+hipError_t launch_scores_store(hipStream_t s, const float *A, int64_t M, int32_t lda,
                                const float *B, int64_t N, int32_t ldb, int32_t K, float *C, int64_t ldc,
                                bool c_row_major_m) {
     if (M <= 0 || N <= 0) return hipSuccess;
     const int64_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-    hipLaunchKernelGGL(k_scores_store, dim3((unsigned)(tm * tn)), dim3(NT), 0, s, A, a_rows, M, lda, B, N, ldb, K,
-                       C, ldc, c_row_major_m ? 1 : 0, tn);
+    const dim3 grid((unsigned)((tm * tn + 7) / 8 * 8));
+    const int vec = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0 ? 1 : 0;
+    if (c_row_major_m)
+        hipLaunchKernelGGL(k_scores_store<true>, grid, dim3(NT), 0, s, A, M, lda, B, N, ldb, K, C, ldc, vec, tm, tn);
+    else
+        hipLaunchKernelGGL(k_scores_store<false>, grid, dim3(NT), 0, s, A, M, lda, B, N, ldb, K, C, ldc, vec, tm, tn);
     return hipGetLastError();
 }
 
@@ -261,7 +340,7 @@ hipError_t launch_refine_count(hipStream_t s, const float *users, const float *i
     (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
     const int64_t n_it = (n_item + BN - 1) / BN;
     const int64_t max_units = ((max_rows + BM - 1) / BM) * ((n_it + kGroup - 1) / kGroup);
-    const int64_t grid = std::min<int64_t>(max_units, (int64_t)n_cu * 4);
+    const int64_t grid = std::min<int64_t>(max_units, (int64_t)n_cu * 3);  // three workgroups fit a CU
     hipLaunchKernelGGL(k_refine_count, dim3((unsigned)grid), dim3(NT), 0, s, users, items, n_item, ld, K, rows_user,
                        rows_thr, n_rows_dev, max_rows, cnt);
     return hipGetLastError();

@@ -80,7 +80,7 @@ extern "C" int rkr_sorted_scores_noalloc(rkr_ctx *c, int64_t user_begin, int64_t
     for (int64_t b0 = 0; b0 < n_rows; b0 += cap_rows) {
         const int64_t m = std::min<int64_t>(cap_rows, n_rows - b0);
         float *rows = out_dev + b0 * I;
-        RKR_HIP(c, launch_scores_store(c->stream, c->users + (user_begin + b0) * c->ld, nullptr, m, c->ld, c->items,
+        RKR_HIP(c, launch_scores_store(c->stream, c->users + (user_begin + b0) * c->ld, m, c->ld, c->items,
                                        I, c->ld, c->dim, rows, I, true));
         RKR_HIP(c, launch_sort_rows(c->stream, rows, I, m, I, rows, tmp, I, c->n_cu));
     }

@@ -739,7 +739,7 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
     RKR_HIP(c, hipEventRecord(c->ev[0], c->stream));
     for (int64_t u0 = 0; u0 < c->n_user; u0 += nb) {
         const int64_t n = std::min<int64_t>(nb, c->n_user - u0);
-        RKR_HIP(c, launch_scores_store(c->stream, c->users + u0 * c->ld, nullptr, n, c->ld, c->items, c->n_item, c->ld,
+        RKR_HIP(c, launch_scores_store(c->stream, c->users + u0 * c->ld, n, c->ld, c->items, c->n_item, c->ld,
                                        c->dim, scores, c->n_item, true));
         if (c->qtable) {
             RKR_HIP(c, launch_select_rows(c->stream, scores, n, c->n_item, c->qranks, c->n_qs,
@@ -924,7 +924,7 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
     for (int64_t b0 = 0; b0 < n; b0 += nb) {
         const int64_t m = std::min<int64_t>(nb, n - b0);
         RKR_HIP(c, hipEventRecord(c->ev[0], c->stream));
-        RKR_HIP(c, launch_scores_store(c->stream, c->users + (u0 + b0) * c->ld, nullptr, m, c->ld, c->items, I, c->ld,
+        RKR_HIP(c, launch_scores_store(c->stream, c->users + (u0 + b0) * c->ld, m, c->ld, c->items, I, c->ld,
                                        c->dim, blk, I, true));
         RKR_HIP(c, hipEventRecord(c->ev[1], c->stream));
         RKR_HIP(c, launch_sort_rows(c->stream, blk, I, m, I, blk, tmp, I, c->n_cu));
@@ -1054,7 +1054,7 @@ int rkr_query_rank_distribution(rkr_ctx *c, const int32_t *item_ids, int32_t n_s
             if (r2) return r2;
         }
         RKR_HIP(c, hipEventRecord(c->ev[3], c->stream));
-        RKR_HIP(c, launch_scores_store(c->stream, c->users + u * c->ld, nullptr, m, c->ld, smat.as<float>(), ns, c->ld,
+        RKR_HIP(c, launch_scores_store(c->stream, c->users + u * c->ld, m, c->ld, smat.as<float>(), ns, c->ld,
                                        c->dim, qbuf.as<float>(), ns, true));
         RKR_HIP(c, launch_rank_hist(c->stream, rows, I, m, I, qbuf.as<float>(), ns, (int32_t)ns, h));
         RKR_HIP(c, hipEventRecord(c->ev[4], c->stream));
@@ -1684,10 +1684,10 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // they keep, and the k-th bound again (the exact path's from here)
             float *qrot = reinterpret_cast<float *>(sl.q_split.p);
             float *qn = qrot + (size_t)nqb * dv.qsrp_ldr;
-            RKR_HIP(c, launch_scores_store(sl.stream, q_in, nullptr, nq, ld, dv.qsrp_rot, d, ld, d, qrot,
+            RKR_HIP(c, launch_scores_store(sl.stream, q_in, nq, ld, dv.qsrp_rot, d, ld, d, qrot,
                                            dv.qsrp_ldr, true));
             RKR_HIP(c, launch_qsrp_qnorms(sl.stream, qrot, dv.qsrp_ldr, q_in, ld, d, dv.qsrp_cd, nq, qn));
-            RKR_HIP(c, launch_scores_store(sl.stream, dv.qsrp_users, nullptr, U, dv.qsrp_ldr, qrot, nq, dv.qsrp_ldr,
+            RKR_HIP(c, launch_scores_store(sl.stream, dv.qsrp_users, U, dv.qsrp_ldr, qrot, nq, dv.qsrp_ldr,
                                            dv.qsrp_cd, qip, U, false));
             RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
             // eps widens the interval as the exact path widens its search; the
@@ -1703,7 +1703,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // <u, q> for every (query, user): qip[b * U + u]
             if (nq <= 16 && (size_t)nq * d * sizeof(float) <= 65536)
                 RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip));
-            else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, nullptr, U, ld, q_in, nq, ld, d, qip, U, false));
+            else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false));
             RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
             if (upd)
                 RKR_HIP(c, launch_bounds_upd(sl.stream, qip, T, U, S, R, dv.n_item_base, eps, dv.side_ins,

@@ -325,10 +325,9 @@ int dev_alloc_t(Ctx *c, T **p, size_t n, const char *what) {
     } while (0)
 
 // ---- kernel launchers (k_gemm.hip) ----------------------------------------
-// C = A * B^T with the sequential FP32 score rule.  A rows are gathered
-// through a_rows when non-null.  Store epilogue: C[n * ldc_n + m] (query-major
-// when A = users, B = queries).
-hipError_t launch_scores_store(hipStream_t s, const float *A, const int32_t *a_rows, int64_t M, int32_t lda,
+// C = A * B^T with the sequential FP32 score rule.  Store epilogue:
+// C[n * ldc + m] (query-major when A = users, B = queries), or C[m * ldc + n].
+hipError_t launch_scores_store(hipStream_t s, const float *A, int64_t M, int32_t lda,
                                const float *B, int64_t N, int32_t ldb, int32_t K, float *C, int64_t ldc,
                                bool c_row_major_m);
 // Small-batch <u,q>: qip[b * n_user + u] for b < nq (nq <= 16), users in

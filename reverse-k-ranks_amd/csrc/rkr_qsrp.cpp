@@ -415,11 +415,11 @@ extern "C" int rkr_qsrp_screen(rkr_ctx *c, const float *queries, int32_t n_query
         (rc = bk.alloc(sizeof(uint32_t) * (size_t)n_query * U, "QSRP bounds")))
         return rc;
     RKR_HIP(c, hipMemcpyAsync(q.p, hq.data(), sizeof(float) * hq.size(), hipMemcpyHostToDevice, c->stream));
-    RKR_HIP(c, launch_scores_store(c->stream, q.as<float>(), nullptr, n_query, ld, c->qsrp_rot, d, ld, d,
+    RKR_HIP(c, launch_scores_store(c->stream, q.as<float>(), n_query, ld, c->qsrp_rot, d, ld, d,
                                    qrot.as<float>(), ldr, true));
     RKR_HIP(c, launch_qsrp_qnorms(c->stream, qrot.as<float>(), ldr, q.as<float>(), ld, d, c->qsrp_cd, n_query,
                                   qn.as<float>()));
-    RKR_HIP(c, launch_scores_store(c->stream, c->qsrp_users, nullptr, U, ldr, qrot.as<float>(), n_query, ldr,
+    RKR_HIP(c, launch_scores_store(c->stream, c->qsrp_users, U, ldr, qrot.as<float>(), n_query, ldr,
                                    c->qsrp_cd, left.as<float>(), U, false));
     const float absf = std::nextafter((float)((double)eps + (double)d * std::ldexp(1.0, -140)), INFINITY);
     RKR_HIP(c, launch_qsrp_bounds(c->stream, left.as<float>(), U, n_query, c->qsrp_par, qn.as<float>(), c->qsrp_gcd,

@@ -222,7 +222,7 @@ int update_side(Ctx *c, bool ins_side, const float *X, int64_t n, int sign) {
             return rc;
         }
         float *block = reinterpret_cast<float *>(c->upd_scratch.p);
-        RKR_HIP(c, launch_scores_store(c->stream, c->users, nullptr, U, c->ld, X + x0 * c->ld, m, c->ld, c->dim, block,
+        RKR_HIP(c, launch_scores_store(c->stream, c->users, U, c->ld, X + x0 * c->ld, m, c->ld, c->dim, block,
                                        m, true));
         RKR_HIP(c, launch_sort_rows_desc(c->stream, block, U, (int32_t)m, m));
         if (sign > 0)
@@ -502,7 +502,7 @@ int rkr_insert_users(rkr_ctx *c, const float *users, int64_t n) {
     float *block = reinterpret_cast<float *>(c->upd_scratch.p);
     for (int64_t u0 = 0; u0 < n; u0 += chunk) {
         const int64_t m = std::min<int64_t>(chunk, n - u0);
-        RKR_HIP(c, launch_scores_store(c->stream, c->users + (U0 + u0) * ld, nullptr, m, ld, c->items_base,
+        RKR_HIP(c, launch_scores_store(c->stream, c->users + (U0 + u0) * ld, m, ld, c->items_base,
                                        c->n_item_base, ld, c->dim, block, c->n_item_base, true));
         if (c->qtable) {  // query table rows, then their sampled columns
             const int32_t QS = c->n_qs;
@@ -522,7 +522,7 @@ int rkr_insert_users(rkr_ctx *c, const float *users, int64_t n) {
         const float *X = side == 0 ? c->items_ins : c->items_del;
         if (!ns) continue;
         float *rows = arr + U0 * lds;
-        RKR_HIP(c, launch_scores_store(c->stream, c->users + U0 * ld, nullptr, n, ld, X, ns, ld, c->dim, rows, lds, true));
+        RKR_HIP(c, launch_scores_store(c->stream, c->users + U0 * ld, n, ld, X, ns, ld, c->dim, rows, lds, true));
         RKR_HIP(c, launch_sort_rows_desc(c->stream, rows, n, ns, lds));
     }
     RKR_HIP(c, hipStreamSynchronize(c->stream));
