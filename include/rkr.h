@@ -201,7 +201,7 @@ int rkr_sorted_scores(rkr_ctx *ctx, int64_t user_begin, int64_t n_rows, float *o
  * enqueues work on the context's stream (rkr_sync waits for it).  The row
  * sort's scratch is a fixed 32 MiB device array per GPU, held until the
  * process ends: n_item may be at most 8,388,608 (RKR_ERR_INVALID above), and
- * rows run in chunks of 8,388,608 / n_item.  Every call on one GPU shares that
+ * at most 8,388,608 / n_item rows are sorted at a time.  Every call on one GPU shares that
  * array, so calls that overlap on one GPU (two contexts' streams at once)
  * race; calls on one context's stream follow each other and are safe. */
 int rkr_sorted_scores_noalloc(rkr_ctx *ctx, int64_t user_begin, int64_t n_rows, float *out_dev);

@@ -5,10 +5,10 @@
 // (src/include/score_computation/ComputeScoreTableBatch.hpp:83-89).  Only the values are kept, so the
 // order of equal values is irrelevant and the sort need not be stable.
 //
-// One 1024-thread workgroup per CU, taking rows in turn (rows that load 16 bytes at a time; others
-// take one workgroup each).  Rows of up to NMAX values are sorted in LDS (bucket path):
+// One 1024-thread workgroup per CU, taking rows in turn.  Rows of up to NMAX values are sorted in LDS
+// (bucket path):
 //   1. the row is in registers (coalesced loads, issued while the workgroup's previous row was
-//      ranked), and each wavefront's min and max of it were taken before that row's last barrier;
+//      sorted), and each wavefront's min and max of it were taken before that row's last barrier;
 //   2. a histogram over NBK value bins, descending, and its exclusive scan.  The bins are
 //      apportioned to NB1 linear coarse bins by the coarse bins' counts (a first histogram, of
 //      half the row), so bins are narrow where the row is dense and hold about n / NBK values
@@ -16,9 +16,12 @@
 //      arithmetic: fl(max - x) and fl(t * scale) are monotone in x, so bin order is value order;
 //   3. every value's order-preserving key is scattered into its bin's segment of an LDS buffer (any
 //      order inside a bin);
-//   4. each value's final position is its bin's start plus the keys of its bin above it (and the
-//      equal ones before it): threads walk the buffer in order, so the lanes of a wavefront read the
-//      same few bins and write within a few hundred bytes of the output row.
+//   4. each thread sorts its own 8 bins (2.4 keys each at 20k values) in registers, 8 keys at a time
+//      read from a bin's start, 16 for longer bins; bins over 16 are ranked by a wavefront each;
+//   5. the buffer, now sorted, is written out in whole cache lines.
+// LDS operations and barriers set the pace.  Ranking each value by counting over its bin read about
+// 14 LDS words per value, the bins' networks 3.3 and as many writes: 10,007 rows of 20,000 took 1263 us
+// (in 24 launches) and take 814 us, 1.97 TB/s of the 4.7 a large copy reaches.
 // A row longer than NMAX, or one with a bin over BIN_MAX values (heavy ties, extreme skew), takes
 // the merge path instead:
 //   1. tiles of TILE values are sorted in LDS by a bitonic network (a partial last tile is padded with
@@ -43,19 +46,18 @@ constexpr int NMAX = 28672;              // longest row of the bucket path (112 
 constexpr int EPT = NMAX / NT;           // values per thread
 constexpr uint32_t BIN_MAX = 192;        // largest bin the bucket path ranks by counting
 constexpr int NB1 = 1024;                // linear coarse bins that apportion the NBK bins
-constexpr int KPAD = 256;                // zero keys past the row's end, read by the rank step
-static_assert(KPAD >= (int)BIN_MAX + 3, "the rank step reads up to BIN_MAX + 2 keys past a bin's start");
+constexpr int KPAD = 16;                 // zero keys past the row's end, read by the bins' sort windows
 
-struct SortSmem {
+struct alignas(16) SortSmem {
     union {
         float tile[TILE];                // merge path
         struct {
             uint32_t key[NMAX + KPAD];   // the row's keys, bin by bin, then KPAD zero keys
-            uint32_t cnt[NBK];           // bin counts, then scatter cursors ending as bin ends
+            uint32_t cnt[NBK];           // bin counts, then scatter cursors, then the long bins' list
             uint32_t fseg[NB1];          // bins of coarse bin c: s0 | s1 << 16, bins s0 .. s1 - 1
             uint32_t coarse[NB1];        // coarse counts (zero between rows)
             float red_f[2 * NW];         // the row's min and max per wavefront, then the largest bin
-            uint32_t red_u[NW + 1];
+            uint32_t red_u[NW + 1];      // wavefront sums of the scans; [NW]: bins ranked by wavefronts
         } b;
     } u;
 };
@@ -84,6 +86,25 @@ __device__ __forceinline__ uint32_t sort_key(float f) {
 // The float of a key (NaN keys give one quiet NaN).
 __device__ __forceinline__ float key_value(uint32_t k) {
     return __uint_as_float(k ^ ((int32_t)k < 0 ? 0x80000000u : 0xFFFFFFFFu));
+}
+
+// Sorts z in descending order: Batcher's odd-even merge network (K. E. Batcher,
+// "Sorting networks and their applications", 1968), unrolled.
+template <int N>
+__device__ __forceinline__ void sort_desc(uint32_t (&z)[N]) {
+#pragma unroll
+    for (int p = 1; p < N; p *= 2)
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+            for (int j = k % p; j + k < N; j += 2 * k)
+#pragma unroll
+                for (int i = 0; i < k; ++i)
+                    if (i + j + k < N && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+                        const uint32_t a = z[i + j], b = z[i + j + k];
+                        z[i + j] = max(a, b);
+                        z[i + j + k] = min(a, b);
+                    }
 }
 
 // Sorts s[0..TILE) in descending order.  Stage (k, j) compares i with i + j for
@@ -204,7 +225,7 @@ __device__ __forceinline__ void row_partials(SortSmem &sm, const float (&v)[EPT]
 // min/max partials in red_f.  On entry red_f holds this row's partials and
 // coarse is zero.  y may be the row v came from.
 template <bool vec>
-__device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], int32_t n, float *y,
+__device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], int32_t n, float *y, bool out_vec,
                                                 const float *xn, int t) {
     const int lane = t & 63, w = t >> 6;
     const int ne = row_slots<vec>(n);
@@ -296,9 +317,13 @@ __device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], i
     uint32_t start = base + incl - run;
 #pragma unroll
     for (int k = 0; k < BPT; ++k) {
-        sm.u.b.cnt[t * BPT + k] = start;  // scatter cursor, ends as the bin's end
+        sm.u.b.cnt[t * BPT + k] = start;  // scatter cursor
         start += c[k];
     }
+    // the bins' lengths, a byte each (BIN_MAX < 256), for the sort of the bins
+    static_assert(BPT == 8 && BIN_MAX < 256, "eight byte lengths in two words");
+    const uint32_t len_lo = c[0] | c[1] << 8 | c[2] << 16 | c[3] << 24;
+    const uint32_t len_hi = c[4] | c[5] << 8 | c[6] << 16 | c[7] << 24;
     __syncthreads();
     // every slot is claimed before the first value is written
     uint32_t slot[EPT];
@@ -311,54 +336,83 @@ __device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], i
     for (int e = 0; e < EPT; ++e)
         if (e < ne && in_row<vec>(t, e, n)) sm.u.b.key[slot[e]] = sort_key(v[e]);
     if (t < KPAD) sm.u.b.key[n + t] = 0u;  // below every value's key
+    if (t == 0) sm.u.b.red_u[NW] = 0u;     // bins the wavefronts will rank
     __syncthreads();
     if constexpr (vec) load_row<vec>(t, v, xn, n);  // v's values are in LDS
-    // final positions, in buffer order (the lanes of a wavefront read the
-    // same few bins): the bin's start plus the number of the bin's keys that
-    // order before this one.  (key, position) pairs order by key, larger
-    // first, then by position, lower first, so equal values take consecutive
-    // places; one 64-bit compare of (key, ~position) does both.  Each value
-    // reads a window from its bin's start, as long as the longest bin of the
-    // thread's RB values rounded up to 4: the keys past its bin belong to later
-    // bins (smaller values, smaller keys) or to the zero padding, and never
-    // order before it, so the window needs no bounds.  The value goes straight
-    // to its place in the output row.  A thread takes RB values at a time, so
-    // their bin lookups and the window reads are in flight together.
-    constexpr int RB = 4;
-    for (int i0 = t; i0 < n; i0 += RB * NT) {
-        uint32_t kx[RB], b0[RB], b1[RB], r[RB], len = 0;
-        float x0[RB];
-        uint64_t me[RB];
+    // each thread sorts its BPT bins in place.  A window of 8 keys from a bin's
+    // start holds the bin's keys and, past it, keys of later bins (smaller
+    // values, smaller keys, whatever their owners have done with them so far)
+    // or the zero padding, so a register network over the whole window leaves
+    // the bin's keys sorted in front, with no bounds; the first s are written
+    // back.  Longer bins take 16 keys, the longest go to a list (cnt's words
+    // are free now) and are ranked by a wavefront each.
+    uint32_t pos = base + incl - run;
+#pragma unroll 1
+    for (int k = 0; k < BPT; ++k) {
+        const uint32_t s = (k < 4 ? len_lo : len_hi) >> (8 * (k & 3)) & 0xFFu;
+        uint32_t *bin_key = sm.u.b.key + pos;
+        if (__builtin_amdgcn_ballot_w64(s > 1) != 0) {
+            uint32_t z[8];
 #pragma unroll
-        for (int q = 0; q < RB; ++q) kx[q] = sm.u.b.key[min(i0 + q * NT, n - 1)];
+            for (int j = 0; j < 8; ++j) z[j] = bin_key[j];
+            sort_desc(z);
 #pragma unroll
-        for (int q = 0; q < RB; ++q) {
-            x0[q] = key_value(kx[q]);
-            const int b = sort_bin(sm.u.b.fseg, x0[q], mx, scale);
-            b0[q] = b ? sm.u.b.cnt[b - 1] : 0u;
-            b1[q] = sm.u.b.cnt[b];
+            for (int j = 0; j < 8; ++j)
+                if (j < (int)s && s <= 8) bin_key[j] = z[j];
         }
+        if (__builtin_amdgcn_ballot_w64(s > 8) != 0) {
+            if (s > 16) {
+                sm.u.b.cnt[atomicAdd(&sm.u.b.red_u[NW], 1u)] = pos | (s << 16);
+            } else if (s > 8) {
+                uint32_t z[16];
 #pragma unroll
-        for (int q = 0; q < RB; ++q) {
-            r[q] = 0;
-            len = max(len, b1[q] - b0[q]);
-            me[q] = ((uint64_t)kx[q] << 32) | (uint32_t)~(uint32_t)(i0 + q * NT);
+                for (int j = 0; j < 16; ++j) z[j] = bin_key[j];
+                sort_desc(z);
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (j < (int)s) bin_key[j] = z[j];
+            }
         }
-        for (uint32_t j = 0; j < len; j += 4) {
-            uint32_t z[RB][4];
+        pos += s;
+    }
+    __syncthreads();
+    const uint32_t n_long = sm.u.b.red_u[NW];
+    if (n_long) {  // uniform
+        constexpr int PL = (BIN_MAX + 63) / 64;  // keys per lane of the longest bin
+        for (uint32_t i = w; i < n_long; i += NW) {
+            const uint32_t e = sm.u.b.cnt[i];
+            const int s = (int)(e >> 16);
+            uint32_t *bin_key = sm.u.b.key + (e & 0xFFFFu);
+            uint32_t x[PL];
+            int r[PL];
 #pragma unroll
-            for (int q = 0; q < RB; ++q)
+            for (int j = 0; j < PL; ++j) {
+                x[j] = bin_key[min(lane + 64 * j, s - 1)];
+                r[j] = 0;
+            }
+            for (int m = 0; m < s; ++m) {
+                const uint32_t z = bin_key[m];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) z[q][k] = sm.u.b.key[b0[q] + j + k];
+                for (int j = 0; j < PL; ++j) r[j] += (z > x[j] || (z == x[j] && m < lane + 64 * j)) ? 1 : 0;
+            }
+            // the bin belongs to this wavefront alone, whose LDS operations
+            // are in order: every key has been read
 #pragma unroll
-            for (int q = 0; q < RB; ++q)
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    r[q] += (((uint64_t)z[q][k] << 32) | (uint32_t)~(b0[q] + j + k)) > me[q] ? 1u : 0u;
+            for (int j = 0; j < PL; ++j)
+                if (lane + 64 * j < s) bin_key[r[j]] = x[j];
         }
-#pragma unroll
-        for (int q = 0; q < RB; ++q)
-            if (i0 + q * NT < n) y[b0[q] + r[q]] = x0[q];
+        __syncthreads();
+    }
+    // the sorted row leaves in whole cache lines
+    if (out_vec) {
+        const uint4 *k4 = reinterpret_cast<const uint4 *>(sm.u.b.key);
+        float4 *y4 = reinterpret_cast<float4 *>(y);
+        for (int i = t; i < n / 4; i += NT) {
+            const uint4 q = k4[i];
+            y4[i] = make_float4(key_value(q.x), key_value(q.y), key_value(q.z), key_value(q.w));
+        }
+    } else {
+        for (int i = t; i < n; i += NT) y[i] = key_value(sm.u.b.key[i]);
     }
     // the largest-bin reads of red_f ended before the scatter's barrier
     if constexpr (vec) row_partials<vec>(sm, v, n, t);
@@ -412,18 +466,19 @@ __device__ void merge_sort_row(float *s, const float *x, int32_t n, float *out_r
     }
 }
 
-// vec (every row starts 16-byte aligned and n is a multiple of 4): persistent,
-// workgroup p sorts rows p, p + G, p + 2G, ... (G = gridDim.x, one workgroup
-// per CU), and on the bucket path the next row's loads are in flight while the
-// current row is ranked.  Otherwise one workgroup per row (G = n_rows).
+// Workgroup p sorts rows p, p + G, p + 2G, ... (G = gridDim.x); its merge
+// passes use scratch row p.  vec (every row starts 16-byte aligned and n is a
+// multiple of 4): on the bucket path the next row's loads are in flight while
+// the current row is sorted.
 template <bool vec>
 __global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_src, int64_t n_rows, int32_t n,
-                                                  float *out, float *tmp, int64_t ld) {
+                                                  float *out, float *tmp, int64_t ld, int out_vec) {
     __shared__ SortSmem sm;
     int64_t row = blockIdx.x;
+    float *tmp_row = tmp + (int64_t)blockIdx.x * ld;
     if (n > NMAX) {
         for (; row < n_rows; row += gridDim.x) {
-            merge_sort_row(sm.u.tile, src + row * ld_src, n, out + row * ld, tmp + row * ld);
+            merge_sort_row(sm.u.tile, src + row * ld_src, n, out + row * ld, tmp_row);
             __syncthreads();  // the tiles are free before the next row's first tile
         }
         return;
@@ -431,37 +486,37 @@ __global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_s
     float v[EPT];
     if (row >= n_rows) return;
     for (int i = threadIdx.x; i < NB1; i += NT) sm.u.b.coarse[i] = 0u;
-    if constexpr (!vec) {
-        const float *x = src + row * ld_src;
-        load_row<false>(threadIdx.x, v, x, n);
-        row_partials<false>(sm, v, n, threadIdx.x);
+    if constexpr (vec) {
+        load_row<vec>(threadIdx.x, v, src + row * ld_src, n);
+        row_partials<vec>(sm, v, n, threadIdx.x);
         __syncthreads();
-        if (bucket_sort_row<false>(sm, v, n, out + row * ld, nullptr, threadIdx.x)) return;
-        __syncthreads();  // the bucket path's LDS is done with before the tiles reuse it
-        merge_sort_row(sm.u.tile, x, n, out + row * ld, tmp + row * ld);
-        return;
     }
-    load_row<vec>(threadIdx.x, v, src + row * ld_src, n);
-    row_partials<vec>(sm, v, n, threadIdx.x);
-    __syncthreads();
     for (; row < n_rows; row += gridDim.x) {
-        // the next row's loads are issued unconditionally (so v is dead across
-        // the merge path); a workgroup's last row loads its own row again, which
-        // it has just read, and the values are not used.  n and the thread index
-        // pass through an empty asm statement each iteration, so the per-slot
-        // indexes and LDS addresses derived from them are computed where they
-        // are used instead of being hoisted out of the loop and held in
-        // registers (which spilled)
+        // n and the thread index pass through an empty asm statement each
+        // iteration, so the per-slot indexes and LDS addresses derived from
+        // them are computed where they are used instead of being hoisted out of
+        // the loop and held in registers (which spilled)
         int32_t nn = n;
         int t = threadIdx.x;
         asm volatile("" : "+s"(nn), "+v"(t));
+        const float *x = src + row * ld_src;
+        if constexpr (!vec) {
+            load_row<vec>(t, v, x, nn);
+            row_partials<vec>(sm, v, nn, t);
+            __syncthreads();
+        }
+        // the next row's loads are issued unconditionally (so v is dead across
+        // the merge path); a workgroup's last row loads its own row again, which
+        // it has just read, and the values are not used
         const int64_t next = row + gridDim.x;
         const float *xn = src + (next < n_rows ? next : row) * ld_src;
-        if (!bucket_sort_row<vec>(sm, v, nn, out + row * ld, xn, t)) {
+        if (!bucket_sort_row<vec>(sm, v, nn, out + row * ld, out_vec != 0, xn, t)) {
             __syncthreads();  // the bucket path's LDS is done with before the tiles reuse it
-            merge_sort_row(sm.u.tile, src + row * ld_src, n, out + row * ld, tmp + row * ld);
-            load_row<vec>(t, v, xn, nn);
-            row_partials<vec>(sm, v, nn, t);
+            merge_sort_row(sm.u.tile, x, n, out + row * ld, tmp_row);
+            if constexpr (vec) {
+                load_row<vec>(t, v, xn, nn);
+                row_partials<vec>(sm, v, nn, t);
+            }
         }
         __syncthreads();  // this row's LDS is done with, the next row's partials are visible
     }
@@ -470,15 +525,18 @@ __global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_s
 }  // namespace
 
 hipError_t launch_sort_rows(hipStream_t s, const float *src, int64_t ld_src, int64_t nb, int64_t n_item, float *out,
-                            float *tmp, int64_t ld, int grid_cap) {
+                            float *tmp, int64_t tmp_rows, int64_t ld, int n_cu) {
     if (nb <= 0 || n_item <= 0) return hipSuccess;
-    if (n_item > (int64_t)1 << 30 || ld < n_item || ld_src < n_item || grid_cap <= 0) return hipErrorInvalidValue;
+    if (n_item > (int64_t)1 << 30 || ld < n_item || ld_src < n_item || tmp_rows <= 0 || n_cu <= 0)
+        return hipErrorInvalidValue;
     const bool vec = (n_item & 3) == 0 && (ld_src & 3) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
-    const unsigned grid = (unsigned)(vec ? std::min<int64_t>(nb, grid_cap) : nb);
+    const int out_vec = (n_item & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 ? 1 : 0;
+    // one workgroup fits a CU, and each needs a scratch row of its own
+    const dim3 grid((unsigned)std::min<int64_t>({nb, (int64_t)n_cu, tmp_rows}));
     if (vec)
-        hipLaunchKernelGGL(k_sort_rows<true>, dim3(grid), dim3(NT), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, ld);
+        hipLaunchKernelGGL(k_sort_rows<true>, grid, dim3(NT), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, ld, out_vec);
     else
-        hipLaunchKernelGGL(k_sort_rows<false>, dim3(grid), dim3(NT), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, ld);
+        hipLaunchKernelGGL(k_sort_rows<false>, grid, dim3(NT), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, ld, out_vec);
     return hipGetLastError();
 }
 

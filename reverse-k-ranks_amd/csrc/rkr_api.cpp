@@ -918,7 +918,8 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
     if (nb <= 0) return set_err(c, RKR_ERR_NOMEM, std::string(what) + ": no memory for a score block");
     ScopedDev blk_buf{c}, tmp_buf{c};
     int rc = blk_buf.alloc((size_t)nb * row_bytes, "score block");
-    if (!rc) rc = tmp_buf.alloc((size_t)nb * row_bytes, "sort scratch");
+    const int64_t tmp_rows = std::min<int64_t>(nb, c->n_cu);  // one per workgroup of the row sort
+    if (!rc) rc = tmp_buf.alloc((size_t)tmp_rows * row_bytes, "sort scratch");
     if (rc) return rc;
     float *blk = blk_buf.as<float>(), *tmp = tmp_buf.as<float>();
     for (int64_t b0 = 0; b0 < n; b0 += nb) {
@@ -927,7 +928,7 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
         RKR_HIP(c, launch_scores_store(c->stream, c->users + (u0 + b0) * c->ld, m, c->ld, c->items, I, c->ld,
                                        c->dim, blk, I, true));
         RKR_HIP(c, hipEventRecord(c->ev[1], c->stream));
-        RKR_HIP(c, launch_sort_rows(c->stream, blk, I, m, I, blk, tmp, I, c->n_cu));
+        RKR_HIP(c, launch_sort_rows(c->stream, blk, I, m, I, blk, tmp, tmp_rows, I, c->n_cu));
         RKR_HIP(c, hipEventRecord(c->ev[2], c->stream));
         if ((rc = sink(blk, u0 + b0, m))) return rc;  // the sink synchronises the stream
         if (gemm_ms) *gemm_ms += ev_ms(c->ev, 0, 1);
