@@ -72,11 +72,14 @@ typedef struct rkr_ctx rkr_ctx;
                                    thread, so one part's host work between kernels
                                    overlaps the other's kernels; 1: one stream.
                                    Answers are unchanged.                        */
-#define RKR_OPT_COARSE 9        /* 1 (default): screened form, exact output: the
-                                   batch's <u,q> runs on BF16 matrix cores against
-                                   7 guard columns per user, and only the users
-                                   this cannot rule out are scored exactly and
-                                   searched; answers are unchanged.             */
+#define RKR_OPT_COARSE 9        /* 1 (default): exact output lists, per query, the
+                                   users whose score can reach a threshold column
+                                   of their table row, and only those are searched;
+                                   the screened form takes the scores for this from
+                                   BF16 matrix cores and scores the listed users
+                                   exactly, the plain form scores every user
+                                   exactly.  0: every user is scored and searched.
+                                   Answers are unchanged.                        */
 #define RKR_OPT_QSRP 11         /* 0 (default); 1: exact queries without pending
                                    updates screen users with the QSRP bounds that
                                    rkr_qsrp_build made (partial-dimension inner
@@ -114,9 +117,10 @@ typedef struct rkr_batch_timing {
     int64_t n_rechecked;
     int64_t n_screened;
     double max_screen_err;  /* screened form: max |screen - FP64| observed     */
-    int64_t n_listed;       /* coarse bounds: (query, user) pairs scored exactly */
-    int64_t n_fallback;     /* coarse bounds: queries that took the full path  */
-    int64_t n_coarse_refined; /* coarse bounds: queries given a second, finer pass */
+    int64_t n_listed;       /* RKR_OPT_COARSE: (query, user) pairs listed      */
+    int64_t n_fallback;     /* RKR_OPT_COARSE: queries that took the full path */
+    int64_t n_coarse_refined; /* RKR_OPT_COARSE: queries listed against a column
+                                 finer than the 7 guard columns                */
 } rkr_batch_timing;
 
 /* ---- context ------------------------------------------------------------ */

@@ -1,0 +1,984 @@
+// k_list.hip -- the bound stage of exact output: which users a query has to
+// look at, their exact scores, table buckets and the k-th bound.
+//
+// Every user keeps the values of up to 63 fine columns of its searched table
+// row (the guard row, G_0 >= G_1 >= ... at columns col_0 < col_1 < ...).  A
+// query is given one of them as its threshold t, and the users with
+//     s + e >= G_t      (s their score or its estimate, e its error bound)
+// are listed.  A user left out has G_t above its score, so its bucket
+// b_hi = #{T > score} is past col_t.  Only the listed users get an exact score
+// and a table search; when at least k of them have b_lo <= col_t, the k-th
+// smallest bound beta of all users is among theirs, beta <= col_t, and every
+// candidate (b_hi <= beta) is listed: beta, the candidates and the ranks are
+// those of a search over every user.  A query for which that fails is answered
+// by the full search instead, so t only decides how long the list is.
+//
+// t comes from a sample of the users, every stride-th (all of them for few
+// users, where the k-th bound is then exact): the smallest column that as many
+// sampled users reach for certain (s - e) as k users would need, plus a margin
+// of three standard deviations, since a threshold that is too tight costs a
+// full search and one that is too loose a longer list.
+//
+// Scores come either from the matrix cores (screened form: one BF16 product,
+// |s^ - s| <= e = ||u|| cs(q) + floor, see k_screen.hip) or from the exact
+// scores of the batch (plain form, e = eps of an installed table).
+#include "rkr_internal.hpp"
+
+namespace rkr {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// native vectors, not HIP's uint4 struct: a struct copy is a memcpy that keeps
+// staged values in scratch memory
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int NT = 256;
+constexpr int QST = 64;       // queries per LDS stage
+constexpr int KPAD_LDS = 8;   // bf16 pad per LDS row
+constexpr int GW = kGuardRow; // floats per guard row
+static_assert(kMaxFine < GW, "a position past every fine column is a bin of its own");
+
+union Frag {
+    bf16x8 v;
+    u32x4 q;
+};
+
+// #{f < 63 : row[f] > x} of a guard row (non-increasing, -inf past the fine
+// columns): a branchless binary search.
+__device__ __forceinline__ int guard_pos(const float *row, float x) {
+    int p = 0;
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) p += row[p + st - 1] > x ? st : 0;
+    return p;
+}
+
+// Guard rows of NU sampled users (users (r0 + i) * stride, i < NU, clamped to
+// the last) to LDS rows of stride GW + 1: an odd stride, so the lanes' searches
+// fall in different banks.  Every load is in flight before the first write.
+constexpr int GP = GW + 1;
+template <int NU>
+__device__ __forceinline__ void stage_guards(float *dst, const float *__restrict__ gvals, int64_t r0, int64_t n_s,
+                                             int64_t stride) {
+    constexpr int N = NU * GW / 4 / NT;
+    f32x4 v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int c = (int)threadIdx.x + k * NT;
+        v[k] = reinterpret_cast<const f32x4 *>(gvals)[min(r0 + c / (GW / 4), n_s - 1) * stride * (GW / 4) + c % (GW / 4)];
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int c = (int)threadIdx.x + k * NT;
+        float *d = dst + (c / (GW / 4)) * GP + c % (GW / 4) * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[j] = v[k][j];
+    }
+}
+
+// A float below x (finite): below(a - b) <= the exact a - b.
+__device__ __forceinline__ float below(float x) {
+    const int32_t i = __float_as_int(x);
+    return __int_as_float(x > 0.0f ? i - 1 : x < 0.0f ? i + 1 : (int32_t)0x80000001u);
+}
+
+// guard_pos with every eighth value of the row in registers: hd[j] = row[8 j + 7].
+// Three steps there, three in LDS.
+__device__ __forceinline__ int guard_pos_reg(const float (&hd)[7], const float *row, float x) {
+    const bool b2 = hd[3] > x;
+    const float h1 = __builtin_unpredictable(b2) ? hd[5] : hd[1];
+    const bool b1 = h1 > x;
+    const float ha = __builtin_unpredictable(b1) ? hd[6] : hd[4], hb = __builtin_unpredictable(b1) ? hd[2] : hd[0];
+    const bool b0 = (__builtin_unpredictable(b2) ? ha : hb) > x;
+    int p = (b2 ? 32 : 0) + (b1 ? 16 : 0) + (b0 ? 8 : 0);
+#pragma unroll
+    for (int st = 4; st > 0; st >>= 1) p += row[p + st - 1] > x ? st : 0;
+    return p;
+}
+
+// ---- sample ----------------------------------------------------------------
+// hist[b * 64 + p] += #{sampled users with p fine columns above s - e}, p <
+// n_fine.  A workgroup takes one stage of 64 queries (blockIdx.y) and every
+// gridDim.x-th block of 128 sampled users, so its counts leave LDS once.
+// Queries are the A operand, users the B operand: lane (lr, lq) of a 16 x 16
+// block owns user lr and queries 4 lq .. 4 lq + 3.
+template <int KS>
+__global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScreen P, int64_t n_s, int64_t stride,
+                                                         uint32_t *__restrict__ hist) {
+    constexpr int ROWQ = (KS * 32 + KPAD_LDS) / 8, KQ = KS * 4;
+    __shared__ u32x4 sA[QST * ROWQ];
+    __shared__ float sCs[QST];
+    __shared__ float sG[128 * GP];
+    __shared__ uint32_t sH[QST * GW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+    const int32_t q0 = (int32_t)blockIdx.y * QST;
+    u32x4 pre[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const int c = (int)threadIdx.x + k * NT;
+        pre[k] = reinterpret_cast<const u32x4 *>(P.q_hi)[(int64_t)min(q0 + c / KQ, P.nq - 1) * KQ + c % KQ];
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const int c = (int)threadIdx.x + k * NT;
+        sA[(c / KQ) * ROWQ + c % KQ] = pre[k];
+    }
+    if (threadIdx.x < QST) sCs[threadIdx.x] = P.q_cs[min(q0 + (int)threadIdx.x, P.nq - 1)];
+    for (int i = threadIdx.x; i < QST * GW; i += NT) sH[i] = 0u;
+    const int64_t n_rb = (n_s + 127) / 128;
+    for (int64_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x) {
+        __syncthreads();  // the previous block is done with sG
+        stage_guards<128>(sG, P.gvals, rb * 128, n_s, stride);
+        Frag uh[2][KS];
+        float ar[2];
+        bool live[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int64_t r = rb * 128 + wave * 32 + b * 16 + lr;
+            live[b] = r < n_s;
+            const int64_t u = min(r, n_s - 1) * stride;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) uh[b][ks].q = reinterpret_cast<const u32x4 *>(P.user_hi + u * P.Kp)[ks * 4 + lq];
+            ar[b] = P.C * P.user_norm[u];
+        }
+        __syncthreads();
+        float hd[2][7];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int j = 0; j < 7; ++j) hd[b][j] = sG[(wave * 32 + b * 16 + lr) * GP + 8 * j + 7];
+#pragma unroll 1
+        for (int g = 0; g < QST / 16 && q0 + g * 16 < P.nq; ++g) {
+            f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                Frag qh;
+                qh.q = sA[(g * 16 + lr) * ROWQ + ks * 4 + lq];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int ql = g * 16 + 4 * lq + i;
+                const float cs = sCs[ql];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const float e = __fmaf_rn(ar[b], cs, P.floor);
+                    const int p = guard_pos_reg(hd[b], &sG[(wave * 32 + b * 16 + lr) * GP], acc[b][i] - e);
+                    if (live[b] && p < P.n_fine) atomicAdd(&sH[ql * GW + p], 1u);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < QST * GW; i += NT)
+        if (sH[i] && q0 + i / GW < P.nq) atomicAdd(&hist[(int64_t)q0 * GW + i], sH[i]);
+}
+
+// The same counts from exact scores qip[b * n_user + u].
+__global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ qip, int64_t n_user, int32_t nq, float eps,
+                                                      const float *__restrict__ gvals, int32_t n_fine, int64_t n_s,
+                                                      int64_t stride, uint32_t *__restrict__ hist) {
+    constexpr int UB = 64, QB = 16;
+    __shared__ float sG[UB * GP];
+    __shared__ uint32_t sH[QB * GW];
+    const int32_t q0 = (int32_t)blockIdx.y * QB;
+    for (int i = threadIdx.x; i < QB * GW; i += NT) sH[i] = 0u;
+    const int64_t n_ub = (n_s + UB - 1) / UB;
+    for (int64_t ub = blockIdx.x; ub < n_ub; ub += gridDim.x) {
+        __syncthreads();
+        stage_guards<UB>(sG, gvals, ub * UB, n_s, stride);
+        __syncthreads();
+        const int ul = threadIdx.x & 63;
+        const int64_t r = ub * UB + ul;
+        if (r < n_s)
+            for (int ql = threadIdx.x >> 6; ql < QB && q0 + ql < nq; ql += NT / 64) {
+                const float s = qip[(int64_t)(q0 + ql) * n_user + r * stride];
+                const int p = guard_pos(&sG[ul * GP], eps > 0.0f ? __double2float_rd((double)s - (double)eps) : s);
+                if (p < n_fine) atomicAdd(&sH[ql * GW + p], 1u);
+            }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < QB * GW; i += NT)
+        if (sH[i] && q0 + i / GW < nq) atomicAdd(&hist[(int64_t)q0 * GW + i], sH[i]);
+}
+
+// ---- plan ------------------------------------------------------------------
+// One workgroup.  Each query's threshold column, the queries ordered by it
+// (slot -> query), and for every four neighbouring slots the largest of their
+// columns, which all four take (a larger column lists more users, never
+// fewer).  A query with no such column, with an estimated list over cap, or
+// past the point where the estimates fill half the list gets thr = -1 (the
+// full search answers it) and no slot.
+constexpr int PT = 1024;
+
+__global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ hist, int32_t nq, int32_t n_fine,
+                                                  int64_t stride, int64_t n_user, int64_t cap, int64_t list_cap,
+                                                  uint64_t coarse_mask, QueryInfo *__restrict__ qi,
+                                                  int32_t *__restrict__ order, int32_t *__restrict__ colg,
+                                                  ListCounters *__restrict__ ctr) {
+    __shared__ int32_t bin[GW], at[GW];
+    __shared__ int64_t load[GW];
+    __shared__ int32_t n_finer, n_slots;
+    for (int i = threadIdx.x; i < GW; i += PT) { bin[i] = 0; load[i] = 0; }
+    if (threadIdx.x == 0) n_finer = 0;
+    __syncthreads();
+    for (int32_t b = threadIdx.x; b < nq; b += PT) {
+        const uint4 *h4 = reinterpret_cast<const uint4 *>(hist + (int64_t)b * GW);
+        const int64_t k = qi[b].topk;
+        const double mean = (double)k / (double)stride;
+        const int64_t want = stride == 1 ? k : (int64_t)(mean + 3.0 * sqrt(mean) + 4.0) + 1;
+        int32_t t = -1;
+        int64_t cum = 0, n = 0;
+        for (int j = 0; j < GW / 4 && t < 0; ++j) {
+            const uint4 v = h4[j];
+            const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+            for (int c = 0; c < 4; ++c) {
+                cum += x[c];
+                if (t < 0 && 4 * j + c < n_fine && cum >= want) { t = 4 * j + c; n = cum; }
+            }
+        }
+        n = min(n * stride, n_user);
+        if (n > cap) t = -1;
+        qi[b].thr = t;
+        if (t >= 0) {
+            atomicAdd(&bin[t], 1);
+            atomicAdd(reinterpret_cast<unsigned long long *>(&load[t]), (unsigned long long)n);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // columns in order while their estimated lists fit
+        int32_t s = 0;
+        int64_t sum = 0;
+        for (int t = 0; t < GW; ++t) {
+            sum += load[t];
+            const bool fits = 2 * sum <= list_cap;
+            at[t] = fits ? s : -1;
+            if (fits) s += bin[t];
+        }
+        n_slots = s;
+    }
+    __syncthreads();
+    for (int32_t b = threadIdx.x; b < nq; b += PT) {
+        const int32_t t = qi[b].thr;
+        if (t < 0) continue;
+        if (at[t] < 0) { qi[b].thr = -1; continue; }
+        bin[t] = 0;
+    }
+    __syncthreads();
+    for (int32_t b = threadIdx.x; b < nq; b += PT) {
+        const int32_t t = qi[b].thr;
+        if (t < 0) continue;
+        order[at[t] + atomicAdd(&bin[t], 1)] = b;
+        if (!((coarse_mask >> t) & 1)) atomicAdd(&n_finer, 1);
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int32_t g = threadIdx.x; g < (n_slots + 3) / 4; g += PT) {
+        int32_t c = 0;
+        for (int j = 0; j < 4 && 4 * g + j < n_slots; ++j) c = max(c, qi[order[4 * g + j]].thr);
+        colg[g] = c;
+        for (int j = 0; j < 4 && 4 * g + j < n_slots; ++j) qi[order[4 * g + j]].thr = c;
+    }
+    if (threadIdx.x == 0) {
+        ctr->n_slots = n_slots;
+        ctr->n_finer = n_finer;
+    }
+}
+
+// ---- list ------------------------------------------------------------------
+// Zeroes the bucket histogram bins of the queries in slots blockIdx.x, +
+// gridDim.x, ... that the exact stage fills: buckets up to the threshold.
+__device__ __forceinline__ void zero_hist(const int32_t *__restrict__ order, int32_t n_slots, const QueryInfo *__restrict__ qi,
+                                          const FineCols &fc, int32_t S, uint32_t *__restrict__ ghist) {
+    for (int32_t s = blockIdx.x; s < n_slots; s += gridDim.x) {
+        const int32_t b = order[s];
+        uint32_t *g = ghist + (int64_t)b * 2 * (S + 1);
+        const int32_t n = fc.col[qi[b].thr] + 1;
+        for (int i = threadIdx.x; i < n; i += NT) { g[i] = 0u; g[S + 1 + i] = 0u; }
+    }
+}
+
+constexpr int QCAP = 512;    // listed pairs of a unit queued in LDS
+// slots per unit of k_list_screen: a unit's user rows are read once per slice,
+// and its workgroup runs long enough to hide them
+constexpr int kSlice = 512;
+
+struct ListQueue {
+    uint2 e[QCAP];
+    int32_t n, base;
+};
+
+// Appends each lane's pairs (bit 4 b + i of m: user u0 + 16 b, query slot_b[i])
+// to the queue, or, where it is full, to the list, with one atomic per
+// wavefront.  Called by whole wavefronts.
+__device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, const int32_t *slot_b,
+                                         int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b, int64_t cap,
+                                         int32_t *__restrict__ list_n) {
+    const int lane = threadIdx.x & 63;
+    const int32_t c = __popc(m);
+    int32_t x = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    const int32_t tot = __shfl(x, 63, 64);
+    int32_t base = 0;
+    if (lane == 0) base = atomicAdd(&sq.n, tot);
+    base = __shfl(base, 0, 64);
+    int32_t p = base + x - c;
+    // places at and past QCAP: the wavefront's share of the list
+    int32_t over = 0;
+    if (base + tot > QCAP) {
+        const int32_t first = max(base, QCAP);
+        if (lane == 0) over = atomicAdd(list_n, base + tot - first);
+        over = __shfl(over, 0, 64) - first;
+    }
+    while (m) {
+        const int t = __ffs(m) - 1;
+        m &= m - 1;
+        const int32_t u = u0 + (t >> 2) * 16, b = slot_b[t & 3];
+        if (p < QCAP) {
+            sq.e[p] = make_uint2((uint32_t)u, (uint32_t)b);
+        } else if ((int64_t)over + p < cap) {
+            cl_u[over + p] = u;
+            cl_b[over + p] = b;
+        }
+        ++p;
+    }
+}
+
+// The unit's queued pairs go to the list; every wave has passed a barrier
+// since the last push, and passes one before the next.
+__device__ __forceinline__ void list_flush(ListQueue &sq, int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b,
+                                           int64_t cap, int32_t *__restrict__ list_n) {
+    const int32_t n = min(sq.n, QCAP);
+    if (n > 0) {  // uniform
+        if (threadIdx.x == 0) sq.base = atomicAdd(list_n, n);
+        __syncthreads();
+        const int64_t base = sq.base;
+        for (int i = threadIdx.x; i < n; i += NT)
+            if (base + i < cap) { cl_u[base + i] = (int32_t)sq.e[i].x; cl_b[base + i] = (int32_t)sq.e[i].y; }
+        __syncthreads();
+        if (threadIdx.x == 0) sq.n = 0;
+    }
+}
+
+// Place of 16-byte piece j of staged query row r: rows are not padded (they
+// arrive by direct loads, 16 bytes per lane in lane order), so the pieces of a
+// row are permuted such that the 16 lanes that read piece j of 16 rows together
+// find them in different banks.
+template <int KS>
+__device__ __forceinline__ int swizzled(int r, int j) {
+    return KS % 4 == 0 ? j ^ (r & 15) : KS % 2 == 0 ? j ^ ((r >> 1) & 7) : j ^ ((r >> 2) & 3);
+}
+
+// 16 bytes per lane from global memory straight to LDS, lane l of the wavefront
+// to dst + 16 l (dst the same in every lane).
+__device__ __forceinline__ void load_to_lds(const void *src, void *dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                     (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+}
+
+// A wavefront's listed pairs, user in the unit | slot in the slice << 8, and
+// their number in a register of every lane.
+constexpr int WQ = 256;
+
+__device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int32_t base, int32_t u0, const int32_t *ord,
+                                           int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b, int64_t cap) {
+    for (int i = threadIdx.x & 63; i < n; i += 64)
+        if ((int64_t)base + i < cap) {
+            cl_u[base + i] = u0 + (int32_t)(q[i] & 0xFFu);
+            cl_b[base + i] = ord[q[i] >> 8];
+        }
+}
+
+// Lists from the matrix cores.  Unit = 64 NB users (each wave 16 NB, held in
+// VGPRs) x a slice of the slots, 64 queries at a time through LDS (two buffers:
+// the next stage's rows go straight to LDS while one is computed, one barrier
+// per stage); a block's thresholds are loaded while the previous one is
+// computed.  A pair costs one fused multiply-add and one compare beside its
+// share of the matrix products; listed pairs are queued per wavefront without
+// an atomic, and a unit takes its part of the list with one.  Bound: the
+// matrix cores' 16 cycles per 16x16x32 product and about 100 VALU instructions
+// per 16 queries x 16 NB users beside them.
+template <int KS, int NB>
+__global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen P, int64_t n_user,
+                                                                     const int32_t *__restrict__ order,
+                                                                     const int32_t *__restrict__ colg, FineCols fc,
+                                                                     int32_t S, const QueryInfo *__restrict__ qi,
+                                                                     uint32_t *__restrict__ ghist,
+                                                                     ListCounters *__restrict__ ctr,
+                                                                     int32_t *__restrict__ cl_u,
+                                                                     int32_t *__restrict__ cl_b, int64_t list_cap) {
+    constexpr int KQ = KS * 4, UB = 64 * NB;
+    static_assert(QST * KQ == KS * NT, "KS 16-byte pieces per thread and stage");
+    static_assert(UB <= 256 && kSlice % QST == 0, "a queued pair's user takes 8 bits");
+    // two variables, not one array: a read of one then does not wait for the
+    // loads into the other
+    __shared__ u32x4 sA0[QST * KQ], sA1[QST * KQ];
+    __shared__ f32x4 sCs[kSlice / 4];
+    __shared__ int32_t sCol[kSlice / 4 + QST / 4], sOrd[kSlice];
+    __shared__ uint32_t sQ[NT / 64][WQ];
+    __shared__ int32_t sN[NT / 64], sBase;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+    const int32_t n_slots = ctr->n_slots;
+    zero_hist(order, n_slots, qi, fc, S, ghist);
+    const int64_t n_rb = (n_user + UB - 1) / UB;
+    const int64_t n_sl = (n_slots + kSlice - 1) / kSlice, n_units = n_rb * n_sl;
+    for (int64_t unit = blockIdx.x; unit < n_units; unit += gridDim.x) {
+        const int64_t rb = unit / n_sl;
+        const int32_t s0 = (int32_t)(unit % n_sl) * kSlice, ns = min(n_slots - s0, kSlice);
+        // the slice's queries, scales and threshold columns (slots past it repeat its last)
+        for (int i = threadIdx.x; i < kSlice; i += NT) {
+            const int32_t q = order[s0 + min(i, ns - 1)];
+            sOrd[i] = q;
+            reinterpret_cast<float *>(sCs)[i] = P.q_cs[q];
+        }
+        for (int i = threadIdx.x; i < kSlice / 4 + QST / 4; i += NT) sCol[i] = colg[(s0 + min(4 * i, ns - 1)) / 4];
+        // the unit's rows: uniform base pointers and 32-bit offsets
+        const int last = (int)min((int64_t)(UB - 1), n_user - 1 - rb * UB);
+        const u32x4 *ubase = reinterpret_cast<const u32x4 *>(P.user_hi + rb * UB * P.Kp);
+        const float *gbase = P.gcols + rb * UB, *nbase = P.user_norm + rb * UB;
+        Frag uh[NB][KS];
+        float ar[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int ul = wave * 16 * NB + b * 16 + lr, uc = min(ul, last);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) uh[b][ks].q = ubase[uc * KQ + ks * 4 + lq];
+            // rows past the last user never reach a threshold
+            ar[b] = ul <= last ? P.C * nbase[uc] : -INFINITY;
+        }
+        int n_q = 0;  // queued pairs of the wavefront
+        auto load_stage = [&](u32x4 *dst, int32_t q) __attribute__((always_inline)) {  // slots s0 + q ..
+#pragma unroll
+            for (int k = 0; k < KS; ++k) {
+                const int c = (int)threadIdx.x + k * NT, r = c / KQ;
+                load_to_lds(reinterpret_cast<const u32x4 *>(P.q_hi) + ((uint32_t)sOrd[q + r] * KQ + swizzled<KS>(r, c % KQ)),
+                            dst + wave * 64 + k * NT);
+            }
+        };
+        auto load_thr = [&](int32_t col, float (&t)[NB]) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) t[b] = gbase[(int64_t)col * P.pitch + min(wave * 16 * NB + b * 16 + lr, last)];
+        };
+        __syncthreads();  // sOrd, sCs and sCol are complete
+        load_stage(sA0, 0);
+        int32_t cur = sCol[lq];  // the lane's threshold column
+        float raw[NB], thr[NB];
+        load_thr(cur, raw);
+        bool fresh = true;       // raw holds new thresholds (uniform)
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's rows are in LDS
+        __syncthreads();
+        auto stage = [&](const u32x4 *rows, u32x4 *ahead, int32_t q0) __attribute__((always_inline)) {
+            if (q0 + QST < ns) load_stage(ahead, q0 + QST);
+            const int n_g = min(QST / 16, (ns - q0 + 15) / 16);
+#pragma unroll 1
+            for (int g = 0; g < n_g; ++g) {
+                const int t4 = (q0 >> 2) + g * 4 + lq;  // the lane's four slots: s0 + 4 t4 ..
+                if (fresh) {
+                    // s^ + e >= G with the floor taken off G, rounded down (one
+                    // step below the rounded difference is below the difference)
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) thr[b] = below(raw[b] - P.floor);
+                }
+                const int32_t next = sCol[t4 + 4];
+                fresh = __builtin_amdgcn_ballot_w64(next != cur) != 0;
+                if (fresh) {
+                    cur = next;
+                    load_thr(cur, raw);
+                }
+                f32x4 acc[NB];
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    Frag qh;
+                    qh.q = rows[(g * 16 + lr) * KQ + swizzled<KS>(g * 16 + lr, ks * 4 + lq)];
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                }
+                // D[4 lq + i][lr]: slot s0 + 4 t4 + i, user b * 16 + lr of the wave
+                const f32x4 cs = sCs[t4];
+                bool any = false;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        acc[b][i] = __fmaf_rn(ar[b], cs[i], acc[b][i]);
+                        any |= acc[b][i] >= thr[b];
+                    }
+                if (__builtin_amdgcn_ballot_w64(any) != 0) {
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const bool hit = acc[b][i] >= thr[b] && 4 * t4 + i < ns;
+                            const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+                            if (m != 0) {
+                                if (n_q + 64 > WQ) {  // uniform: make room
+                                    int32_t base = 0;
+                                    if (lane == 0) base = atomicAdd(&ctr->n_list, n_q);
+                                    wave_flush(sQ[wave], n_q, __shfl(base, 0, 64), (int32_t)(rb * UB), sOrd, cl_u, cl_b,
+                                               list_cap);
+                                    n_q = 0;
+                                }
+                                const int at = n_q + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                                if (hit) sQ[wave][at] = (uint32_t)(wave * 16 * NB + b * 16 + lr) | (uint32_t)(4 * t4 + i) << 8;
+                                n_q += (int)__popcll(m);
+                            }
+                        }
+                }
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's rows of the next stage are in LDS
+            __syncthreads();
+        };
+        for (int32_t q0 = 0; q0 < ns; q0 += 2 * QST) {
+            stage(sA0, sA1, q0);
+            if (q0 + QST < ns) stage(sA1, sA0, q0 + QST);
+        }
+        // the unit's pairs: one place in the list for the four wavefronts
+        if (lane == 0) sN[wave] = n_q;
+        __syncthreads();
+        int32_t before = 0, tot = 0;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) {
+            before += w < wave ? sN[w] : 0;
+            tot += sN[w];
+        }
+        if (tot > 0) {  // uniform
+            if (threadIdx.x == 0) sBase = atomicAdd(&ctr->n_list, tot);
+            __syncthreads();
+            wave_flush(sQ[wave], n_q, sBase + before, (int32_t)(rb * UB), sOrd, cl_u, cl_b, list_cap);
+        }
+        __syncthreads();  // the next unit rewrites the slice, the queues and the stages
+    }
+}
+
+// Lists from exact scores: one thread per user and a slice of the slots
+// (blockIdx.y), four slots of one threshold column at a time; scores and
+// thresholds are read in whole lines per wavefront.
+constexpr int kScoreSlice = 64;
+
+__global__ void __launch_bounds__(NT) k_list_scores(const float *__restrict__ qip, int64_t n_user, float eps,
+                                                    const float *__restrict__ gcols, int64_t pitch,
+                                                    const int32_t *__restrict__ order, const int32_t *__restrict__ colg,
+                                                    FineCols fc, int32_t S, const QueryInfo *__restrict__ qi,
+                                                    uint32_t *__restrict__ ghist, ListCounters *__restrict__ ctr,
+                                                    int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b,
+                                                    int64_t list_cap) {
+    __shared__ ListQueue sq;
+    __shared__ int32_t sB[kScoreSlice], sCol[kScoreSlice / 4];
+    const int32_t n_slots = ctr->n_slots;
+    if (blockIdx.y == 0) zero_hist(order, n_slots, qi, fc, S, ghist);
+    const int32_t s0 = (int32_t)blockIdx.y * kScoreSlice, ns = min(n_slots - s0, kScoreSlice);
+    if (ns <= 0) return;
+    if (threadIdx.x == 0) sq.n = 0;
+    if (threadIdx.x < kScoreSlice) sB[threadIdx.x] = order[s0 + min((int)threadIdx.x, ns - 1)];
+    if (threadIdx.x < kScoreSlice / 4) sCol[threadIdx.x] = colg[(s0 + min(4 * (int)threadIdx.x, ns - 1)) / 4];
+    __syncthreads();
+    const int64_t u = (int64_t)blockIdx.x * NT + threadIdx.x, uc = min(u, n_user - 1);
+    for (int32_t s = 0; s < ns; s += 8) {
+        float x[8], thr[2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = qip[(int64_t)sB[s + j] * n_user + uc];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) thr[j] = gcols[(int64_t)sCol[s / 4 + j] * pitch + uc];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float v = x[4 * j + i], hi = eps > 0.0f ? __double2float_ru((double)v + (double)eps) : v;
+                m |= hi >= thr[j] && u < n_user && s + 4 * j + i < ns ? 1u << i : 0u;
+            }
+            if (__builtin_amdgcn_ballot_w64(m != 0) != 0)
+                list_put(sq, m, (int32_t)u, &sB[s + 4 * j], cl_u, cl_b, list_cap, &ctr->n_list);
+        }
+    }
+    __syncthreads();
+    list_flush(sq, cl_u, cl_b, list_cap, &ctr->n_list);
+}
+
+// ---- exact scores, buckets and the k-th bound of the listed pairs -----------
+
+// Workgroups are dispatched to the 8 XCDs in turn (block p on XCD p % 8), and
+// each XCD has its own L2.  Block p takes logical block (p % 8) * per + p / 8 of
+// the list, so each XCD takes one contiguous eighth of it: a unit's pairs (the
+// same users) share one L2.  -1 past the list.
+__device__ __forceinline__ int64_t xcd_block(int64_t n) {
+    const int64_t blocks = (n + NT - 1) / NT, per = (blocks + 7) / 8;
+    const int64_t p = blockIdx.x;
+    if (p >= per * 8) return -1;
+    const int64_t lb = (p % 8) * per + p / 8;
+    return lb < blocks ? lb : -1;
+}
+
+// #{row[j] > x} when it is known to lie in [lo, hi].
+__device__ __forceinline__ int32_t bucket_in(const float *__restrict__ row, int32_t lo, int32_t hi, float x) {
+    while (lo < hi) {
+        const int32_t mid = (lo + hi) >> 1;
+        if (row[mid] > x) lo = mid + 1; else hi = mid;
+    }
+    return lo;
+}
+
+// #{T > x} of a user: the guard row's search (two cache lines) leaves the few
+// columns between two fine columns.
+__device__ __forceinline__ int32_t bucket_of(const float *__restrict__ grow, const float *__restrict__ row,
+                                             const int32_t *col, int32_t n_fine, int32_t S, float x) {
+    const int f = guard_pos(grow, x);
+    return bucket_in(row, f > 0 ? col[f - 1] + 1 : 0, f < n_fine ? col[f] : S, x);
+}
+
+// The score rule's <u, q> of the 64 pairs of a wavefront, a pair per lane.  A
+// lane that reads its own two rows touches a cache line of its own with every
+// load, 64 lines per instruction; here the rows are read 64 bytes by four
+// neighbouring lanes, 16 rows per instruction, and pass through the
+// wavefront's LDS (rows of 16 terms and 4 floats of padding, so the 16-byte
+// reads spread over all banks), 16 terms ahead of the sum.
+constexpr int DC = 16, DP = DC + 4;
+
+__device__ __forceinline__ float wave_rule_dot(f32x4 *su, f32x4 *sv, const float *__restrict__ users,
+                                               const float *__restrict__ queries, int64_t u, int64_t b, int32_t ld,
+                                               int32_t dim) {
+    const int lane = threadIdx.x & 63, piece = lane & 3;
+    const float *ru[4], *rq[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // rows 16 j + lane / 4 of the wavefront
+        ru[j] = users + (int64_t)__shfl((int32_t)u, 16 * j + (lane >> 2), 64) * ld;
+        rq[j] = queries + (int64_t)__shfl((int32_t)b, 16 * j + (lane >> 2), 64) * ld;
+    }
+    f32x4 xu[4], xq[4];
+    auto load = [&](int32_t k0) {
+        const int32_t k = min(k0 + 4 * piece, ld - 4);  // past the row's end: unused
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            xu[j] = *reinterpret_cast<const f32x4 *>(ru[j] + k);
+            xq[j] = *reinterpret_cast<const f32x4 *>(rq[j] + k);
+        }
+    };
+    load(0);
+    float s = 0.0f;
+    for (int32_t k0 = 0; k0 < dim; k0 += DC) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            su[(16 * j + (lane >> 2)) * (DP / 4) + piece] = xu[j];
+            sv[(16 * j + (lane >> 2)) * (DP / 4) + piece] = xq[j];
+        }
+        if (k0 + DC < dim) load(k0 + DC);
+        // this wavefront's LDS only, whose operations are in order
+        __builtin_amdgcn_wave_barrier();
+        const int32_t n = min(DC, dim - k0);
+        f32x4 a[DC / 4], c[DC / 4];
+#pragma unroll
+        for (int j = 0; j < DC / 4; ++j) {
+            a[j] = su[lane * (DP / 4) + j];
+            c[j] = sv[lane * (DP / 4) + j];
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (n == DC) {
+#pragma unroll
+            for (int j = 0; j < DC; ++j) s = s + a[j / 4][j % 4] * c[j / 4][j % 4];
+        } else {
+#pragma unroll
+            for (int j = 0; j < DC; ++j)
+                if (j < n) s = s + a[j / 4][j % 4] * c[j / 4][j % 4];
+        }
+    }
+    return s;
+}
+
+// One lane per listed pair, grid-stride over the list's length on the device.
+// SCORES: the score is qip's; otherwise the score rule's <u,q> is computed here
+// and stored to qip for the top-k.
+template <bool SCORES>
+__global__ void __launch_bounds__(NT) k_list_exact(const float *__restrict__ users, const float *__restrict__ queries,
+                                                   int32_t ld, int32_t dim, const float *__restrict__ table, int32_t S,
+                                                   float eps, const float *__restrict__ gvals, FineCols fc,
+                                                   const ListCounters *__restrict__ ctr, int64_t list_cap,
+                                                   const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
+                                                   int64_t n_user, const QueryInfo *__restrict__ qi,
+                                                   uint32_t *__restrict__ bk_c, float *__restrict__ qip,
+                                                   uint32_t *__restrict__ ghist) {
+    __shared__ int32_t col[GW];
+    __shared__ f32x4 sd[SCORES ? 1 : NT / 64][2][SCORES ? 1 : 64 * DP / 4];
+    if (threadIdx.x < GW) col[threadIdx.x] = threadIdx.x < kMaxFine ? fc.col[threadIdx.x] : 0;
+    __syncthreads();
+    const int64_t n = min((int64_t)ctr->n_list, list_cap);
+    const int64_t per_round = (int64_t)gridDim.x * NT;
+    for (int64_t r0 = 0; r0 < n; r0 += per_round) {
+        const int64_t lb = xcd_block(min(n - r0, per_round));
+        const int64_t w0 = r0 + lb * NT + (threadIdx.x & ~63);  // the wavefront's first pair
+        if (lb < 0 || w0 >= n) continue;
+        const int64_t i = r0 + lb * NT + threadIdx.x, ic = min(i, n - 1);
+        const int64_t u = cl_u[ic], b = cl_b[ic];
+        float s;
+        if constexpr (SCORES) s = qip[b * n_user + u];
+        else s = wave_rule_dot(sd[threadIdx.x >> 6][0], sd[threadIdx.x >> 6][1], users, queries, u, b, ld, dim);
+        if (i >= n) continue;
+        if (!SCORES) qip[b * n_user + u] = s;
+        const float *row = table + u * (int64_t)S, *grow = gvals + u * GW;
+        int32_t lo, hi;
+        if (eps > 0.0f) {
+            lo = bucket_of(grow, row, col, fc.n, S, __double2float_rd((double)s - (double)eps));
+            hi = bucket_of(grow, row, col, fc.n, S, __double2float_ru((double)s + (double)eps));
+        } else {
+            lo = hi = bucket_of(grow, row, col, fc.n, S, s);
+        }
+        bk_c[i] = (uint32_t)lo | ((uint32_t)hi << 16);
+        // only buckets up to the threshold can hold the k-th bound or a candidate
+        const int32_t last = col[qi[b].thr];
+        uint32_t *g = ghist + b * 2 * (int64_t)(S + 1);
+        if (lo <= last) atomicAdd(&g[lo], 1u);
+        if (eps > 0.0f && hi <= last) atomicAdd(&g[S + 1 + hi], 1u);
+    }
+}
+
+// One workgroup per query: beta, the bucket of the k-th smallest b_lo, and the
+// candidates' count, from the histogram bins up to the threshold.  A query
+// with fewer than k buckets there (or a list that overflowed) gets thr = -1
+// and no candidates: the full search answers it.
+__global__ void __launch_bounds__(NT) k_list_kth(const uint32_t *__restrict__ ghist, int32_t S, int same, FineCols fc,
+                                                 int64_t list_cap, QueryInfo *__restrict__ qi,
+                                                 ListCounters *__restrict__ ctr) {
+    constexpr int NW = NT / 64;
+    __shared__ uint32_t red[NW];
+    __shared__ int32_t s_beta;
+    const int64_t b = blockIdx.x;
+    const QueryInfo q = qi[b];
+    const uint32_t *lo = ghist + b * 2 * (int64_t)(S + 1), *hi = same ? lo : lo + S + 1;
+    const int32_t n = q.thr >= 0 && (int64_t)ctr->n_list <= list_cap ? fc.col[q.thr] + 1 : 0;
+    const uint32_t k = (uint32_t)q.topk;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) s_beta = -1;
+    uint32_t before = 0, below = 0;  // totals of the bins already scanned
+    for (int32_t j0 = 0; j0 < n; j0 += NT) {
+        const int32_t j = j0 + (int)threadIdx.x;
+        const uint32_t v = j < n ? lo[j] : 0u, h = j < n ? hi[j] : 0u;
+        uint32_t x = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) red[w] = x;
+        __syncthreads();
+        uint32_t base = before, tot = 0;
+        for (int i = 0; i < NW; ++i) {
+            base += i < w ? red[i] : 0u;
+            tot += red[i];
+        }
+        if (base + x >= k && base + x - v < k) s_beta = j;
+        __syncthreads();
+        const int32_t beta = s_beta;
+        // candidates: buckets b_hi <= beta
+        uint32_t c = j < n && (beta < 0 || j <= beta) ? h : 0u;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+        if (lane == 0) red[w] = c;
+        __syncthreads();
+        for (int i = 0; i < NW; ++i) below += red[i];
+        __syncthreads();
+        if (beta >= 0) break;  // uniform
+        before += tot;
+    }
+    if (threadIdx.x == 0) {
+        const bool ok = s_beta >= 0;
+        QueryInfo r = q;
+        r.beta = s_beta;
+        r.gamma = s_beta;
+        r.thr = ok ? q.thr : -1;
+        r.n_cand = ok ? (int32_t)below : 0;
+        r.n_refine = r.fill = r.n_settled = 0;
+        r.cand_off = atomicAdd(&ctr->n_cand, r.n_cand);
+        qi[b] = r;
+    }
+}
+
+// One thread per listed pair: the candidates (b_hi <= beta) with their rank when
+// the bounds fix it, else ~(refine row).
+__global__ void __launch_bounds__(NT) k_list_final(const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
+                                                   const uint32_t *__restrict__ bk_c, const float *__restrict__ qip,
+                                                   const ListCounters *__restrict__ ctr, int64_t list_cap, int32_t S,
+                                                   const int32_t *__restrict__ ranks, int64_t n_item, int64_t n_user,
+                                                   QueryInfo *__restrict__ qi, int32_t *__restrict__ cand_user,
+                                                   int32_t *__restrict__ cand_rank, int32_t *__restrict__ refine_total,
+                                                   int32_t *__restrict__ refine_user, int32_t *__restrict__ refine_query,
+                                                   float *__restrict__ refine_thr, int32_t *__restrict__ cnt) {
+    const int64_t n = min((int64_t)ctr->n_list, list_cap);
+    const int lane = threadIdx.x & 63;
+    for (int64_t i0 = (int64_t)blockIdx.x * NT; i0 < n; i0 += (int64_t)gridDim.x * NT) {
+        const int64_t i = i0 + threadIdx.x;
+        bool cand = false;
+        int32_t b = -1, u = 0, blo = 0, bhi = 0;
+        if (i < n) {
+            b = cl_b[i];
+            const uint32_t x = bk_c[i];
+            blo = (int32_t)(x & 0xFFFFu);
+            bhi = (int32_t)(x >> 16);
+            cand = bhi <= qi[b].beta;
+            u = cl_u[i];
+        }
+        // the lanes of one query share one atomic, all leaders' in flight at once
+        uint64_t todo = __builtin_amdgcn_ballot_w64(cand);
+        int32_t lead = 0, ahead = 0, count = 0;
+        while (todo) {
+            const int l = __ffsll((unsigned long long)todo) - 1;
+            const int32_t lb = __shfl(b, l, 64);
+            const uint64_t same = __builtin_amdgcn_ballot_w64(cand && b == lb);
+            if (cand && b == lb) {
+                lead = l;
+                ahead = (int32_t)__popcll(same & ((1ull << lane) - 1));
+                count = (int32_t)__popcll(same);
+            }
+            todo &= ~same;
+        }
+        int32_t place = 0;
+        if (cand && lane == lead) place = atomicAdd(&qi[b].fill, count);
+        place = __shfl(place, lead, 64) + ahead;
+        if (!cand) continue;
+        const int64_t slot = qi[b].cand_off + place;
+        const int32_t lbs = blo == S ? (int32_t)n_item : ranks[blo];
+        const int32_t ubs = bhi == 0 ? 0 : ranks[bhi - 1] + 1;
+        int32_t rank = lbs;
+        if (lbs != ubs) {
+            const int32_t r = atomicAdd(refine_total, 1);
+            atomicAdd(&qi[b].n_refine, 1);
+            rank = ~r;
+            refine_user[r] = u;
+            refine_query[r] = b;
+            refine_thr[r] = qip[(int64_t)b * n_user + u];
+            cnt[r] = 0;
+        }
+        cand_user[slot] = u;
+        cand_rank[slot] = rank;
+    }
+}
+
+// gv[u * kGuardRow + f] = gc[f * pitch + u] = T[u][col_f], -inf past the fine
+// columns, rows [u0, u0 + n_rows): by rows for the searches of one user, by
+// columns for the lists, which read one column of many users.
+__global__ void __launch_bounds__(NT) k_gather_guards(const float *__restrict__ T, int64_t S, FineCols fc, int64_t u0,
+                                                      int64_t n_rows, float *__restrict__ gv, float *__restrict__ gc,
+                                                      int64_t pitch) {
+    __shared__ float tile[64][GP];
+    const int64_t r0 = (int64_t)blockIdx.x * 64;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < 64 * GW; i += NT) {
+        const int r = i / GW, f = i % GW;
+        if (r0 + r >= n_rows) break;
+        const int64_t u = u0 + r0 + r;
+        const float v = f < fc.n ? T[u * S + fc.col[f]] : -INFINITY;
+        gv[u * GW + f] = v;
+        tile[r][f] = v;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 64 * GW; i += NT) {
+        const int f = i / 64, r = i % 64;
+        if (r0 + r < n_rows) gc[f * pitch + u0 + r0 + r] = tile[r][f];
+    }
+}
+
+bool fine_ok(const FineCols &fc, int64_t S) {
+    if (fc.n < 1 || fc.n > kMaxFine) return false;
+    for (int f = 0; f < fc.n; ++f)
+        if (fc.col[f] < 0 || fc.col[f] >= S || (f > 0 && fc.col[f] <= fc.col[f - 1])) return false;
+    return true;
+}
+
+}  // namespace
+
+hipError_t launch_gather_guards(hipStream_t s, const float *T, int64_t S, const FineCols &fc, int64_t u0,
+                                int64_t n_rows, float *gv, float *gc, int64_t pitch) {
+    if (n_rows <= 0) return hipSuccess;
+    if ((fc.n > 0 && !fine_ok(fc, S)) || u0 + n_rows > pitch) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_gather_guards, dim3((unsigned)((n_rows + 63) / 64)), dim3(NT), 0, s, T, S, fc, u0, n_rows, gv,
+                       gc, pitch);
+    return hipGetLastError();
+}
+
+#define RKR_KS_SWITCH(kp, CASE)             \
+    switch ((kp) / 32) {                    \
+        CASE(1) CASE(2) CASE(3) CASE(4)     \
+        CASE(5) CASE(6) CASE(7) CASE(8)     \
+        default: return hipErrorInvalidValue; \
+    }
+
+hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L) {
+    if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
+    if (!fine_ok(L.fc, L.S) || !L.gvals || !L.gcols || L.pitch < L.n_user || !L.user_hi || !L.q_hi) return hipErrorInvalidValue;
+    ListScreen P{L.user_hi, L.user_norm, L.gvals, L.gcols, L.pitch, L.q_hi, L.q_cs, L.nq, L.Kp, L.fc.n, L.C, L.floor};
+    const int64_t n_s = (L.n_user + L.stride - 1) / L.stride, n_sb = (n_s + 127) / 128;
+    const unsigned qg = (unsigned)((L.nq + QST - 1) / QST);
+    // two workgroups of the sample fit a CU
+    const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(n_sb, (2 * L.n_cu + qg - 1) / qg));
+#define RKR_SAMPLE_CASE(ks)                                                                                       \
+    case ks:                                                                                                      \
+        hipLaunchKernelGGL(k_sample_screen<ks>, dim3(gx, qg), dim3(NT), 0, s, P, n_s, L.stride, L.hist);           \
+        break;
+    RKR_KS_SWITCH(L.Kp, RKR_SAMPLE_CASE)
+#undef RKR_SAMPLE_CASE
+    hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
+                       L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
+    const int64_t ub = L.Kp <= 160 ? 256 : 128;
+    const int64_t units = (L.n_user + ub - 1) / ub * ((L.nq + kSlice - 1) / kSlice);
+    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(units, (int64_t)L.n_cu * (L.Kp <= 160 ? 3 : 2))));
+#define RKR_LIST_CASE(ks)                                                                                          \
+    case ks:                                                                                                       \
+        hipLaunchKernelGGL((k_list_screen<ks, ks <= 5 ? 4 : 2>), grid, dim3(NT), 0, s, P, L.n_user, L.order, \
+                           L.colg, L.fc, L.S, L.qi, L.ghist, L.ctr, L.cl_u, L.cl_b, L.list_cap);                   \
+        break;
+    RKR_KS_SWITCH(L.Kp, RKR_LIST_CASE)
+#undef RKR_LIST_CASE
+    return hipGetLastError();
+}
+
+hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L) {
+    if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
+    if (!fine_ok(L.fc, L.S) || !L.gvals || !L.gcols || L.pitch < L.n_user) return hipErrorInvalidValue;
+    const int64_t n_s = (L.n_user + L.stride - 1) / L.stride;
+    const unsigned qg = (unsigned)((L.nq + 15) / 16);
+    const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n_s + 63) / 64, (8 * L.n_cu + qg - 1) / qg));
+    hipLaunchKernelGGL(k_sample_scores, dim3(gx, qg), dim3(NT), 0, s, L.qip, L.n_user, L.nq, L.eps, L.gvals, L.fc.n,
+                       n_s, L.stride, L.hist);
+    hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
+                       L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
+    hipLaunchKernelGGL(k_list_scores,
+                       dim3((unsigned)((L.n_user + NT - 1) / NT), (unsigned)((L.nq + kScoreSlice - 1) / kScoreSlice)),
+                       dim3(NT), 0, s, L.qip, L.n_user, L.eps, L.gcols, L.pitch, L.order, L.colg, L.fc, L.S, L.qi,
+                       L.ghist, L.ctr, L.cl_u, L.cl_b, L.list_cap);
+    return hipGetLastError();
+}
+
+hipError_t launch_list_exact(hipStream_t s, const ListLaunch &L, const float *users, const float *queries, int32_t ld,
+                             int32_t dim, const float *table, bool scores, uint32_t *bk_c) {
+    if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
+    const dim3 grid((unsigned)(L.n_cu * 16));  // a multiple of the 8 XCDs (grid-stride over the list)
+    if (scores)
+        hipLaunchKernelGGL(k_list_exact<true>, grid, dim3(NT), 0, s, users, queries, ld, dim, table, L.S, L.eps, L.gvals,
+                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist);
+    else
+        hipLaunchKernelGGL(k_list_exact<false>, grid, dim3(NT), 0, s, users, queries, ld, dim, table, L.S, L.eps, L.gvals,
+                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist);
+    hipLaunchKernelGGL(k_list_kth, dim3((unsigned)L.nq), dim3(NT), 0, s, L.ghist, L.S, L.eps > 0.0f ? 0 : 1, L.fc,
+                       L.list_cap, L.qi, L.ctr);
+    return hipGetLastError();
+}
+
+hipError_t launch_list_final(hipStream_t s, const ListLaunch &L, const uint32_t *bk_c, const int32_t *ranks,
+                             int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_total,
+                             int32_t *refine_user, int32_t *refine_query, float *refine_thr, int32_t *cnt) {
+    if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_list_final, dim3((unsigned)(L.n_cu * 16)), dim3(NT), 0, s, L.cl_u, L.cl_b, bk_c, L.qip, L.ctr,
+                       L.list_cap, L.S, ranks, n_item, L.n_user, L.qi, cand_user, cand_rank, refine_total, refine_user,
+                       refine_query, refine_thr, cnt);
+    return hipGetLastError();
+}
+
+}  // namespace rkr

@@ -290,14 +290,14 @@ __global__ void __launch_bounds__(NT) k_offsets(QueryInfo *__restrict__ qi, int3
 
 // One workgroup per query, users in ascending order: writes the settled users
 // (reference output, at most k, with rank = bound) and the candidates (with
-// their rank when the bounds fix it, else -1 plus a refine row).
+// their rank when the bounds fix it, else a refine row r and ~r in its place).
 __global__ void __launch_bounds__(NT) k_compact(const uint32_t *__restrict__ bk, const float *__restrict__ qip,
                                                 int64_t n_user, int32_t S, const int32_t *__restrict__ ranks,
                                                 int64_t n_item, QueryInfo *__restrict__ qi,
                                                 int32_t *__restrict__ cand_user, int32_t *__restrict__ cand_rank,
-                                                int32_t *__restrict__ refine_total, int32_t *__restrict__ refine_cand,
+                                                int32_t *__restrict__ refine_total,
                                                 int32_t *__restrict__ refine_user, int32_t *__restrict__ refine_query,
-                                                float *__restrict__ refine_thr) {
+                                                float *__restrict__ refine_thr, int32_t *__restrict__ cnt) {
     __shared__ uint32_t red[NW + 1];
     __shared__ int32_t n_refine;
     const int64_t b = blockIdx.x;
@@ -347,11 +347,13 @@ __global__ void __launch_bounds__(NT) k_compact(const uint32_t *__restrict__ bk,
         if (cand) {
             const int64_t slot = can_base + my_can;
             cand_user[slot] = (int32_t)u;
-            cand_rank[slot] = rank;
-            if (rank < 0) {
+            if (rank >= 0) {
+                cand_rank[slot] = rank;
+            } else {
                 ++my_refine;
                 const int32_t r = atomicAdd(refine_total, 1);
-                refine_cand[r] = (int32_t)slot;
+                cand_rank[slot] = ~r;
+                cnt[r] = 0;
                 refine_user[r] = (int32_t)u;
                 refine_query[r] = (int32_t)b;
                 refine_thr[r] = qb[u];
@@ -374,10 +376,9 @@ __global__ void __launch_bounds__(NT) k_compact_chunks(const uint32_t *__restric
                                                        int64_t n_item, int64_t cu, QueryInfo *__restrict__ qi,
                                                        int32_t *__restrict__ cand_user, int32_t *__restrict__ cand_rank,
                                                        int32_t *__restrict__ refine_total,
-                                                       int32_t *__restrict__ refine_cand,
                                                        int32_t *__restrict__ refine_user,
                                                        int32_t *__restrict__ refine_query,
-                                                       float *__restrict__ refine_thr) {
+                                                       float *__restrict__ refine_thr, int32_t *__restrict__ cnt) {
     __shared__ uint32_t red[NW + 1];
     __shared__ int32_t s_can, s_ref;
     const int64_t b = blockIdx.y;
@@ -415,23 +416,18 @@ __global__ void __launch_bounds__(NT) k_compact_chunks(const uint32_t *__restric
         if (cand) {
             const int64_t slot = off + s_can + (e & 0xFFFFu);
             cand_user[slot] = (int32_t)u;
-            cand_rank[slot] = rank;
-            if (refine) {
+            if (!refine) {
+                cand_rank[slot] = rank;
+            } else {
                 const int32_t r = s_ref + (int32_t)(e >> 16);
-                refine_cand[r] = (int32_t)slot;
+                cand_rank[slot] = ~r;
+                cnt[r] = 0;
                 refine_user[r] = (int32_t)u;
                 refine_query[r] = (int32_t)b;
                 refine_thr[r] = qb[u];
             }
         }
     }
-}
-
-__global__ void k_scatter_counts(const int32_t *__restrict__ refine_total, const int32_t *__restrict__ refine_cand,
-                                 const int32_t *__restrict__ cnt, int64_t max_rows, int32_t *__restrict__ cand_rank) {
-    const int64_t n = min((int64_t)*refine_total, max_rows);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        cand_rank[refine_cand[i]] = cnt[i];
 }
 
 // ---- top-k -----------------------------------------------------------------
@@ -452,15 +448,17 @@ __device__ void bitonic_sort_u64(uint64_t *keys, int n_pow2) {
     }
 }
 
-__device__ __forceinline__ uint64_t make_key(int32_t rank, int32_t user) {
-    return ((uint64_t)(uint32_t)rank << 32) | (uint32_t)user;
+// (rank, userID) of a candidate; a negative rank names the refine row that
+// counted it.
+__device__ __forceinline__ uint64_t make_key(int32_t rank, const int32_t *__restrict__ cnt, int32_t user) {
+    return ((uint64_t)(uint32_t)(rank >= 0 ? rank : cnt[~rank]) << 32) | (uint32_t)user;
 }
 
 // One workgroup per query.  Output row: the settled users (reference
 // output) followed by the smallest (rank, userID) candidates.
 __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, const int32_t *__restrict__ cand_user,
-                                             const int32_t *__restrict__ cand_rank, const float *__restrict__ qip,
-                                             int64_t n_user, int32_t max_k, int32_t *__restrict__ out_user,
+                                             const int32_t *__restrict__ cand_rank, const int32_t *__restrict__ cnt,
+                                             const float *__restrict__ qip, int64_t n_user, int32_t max_k, int32_t *__restrict__ out_user,
                                              int32_t *__restrict__ out_rank, float *__restrict__ out_qip) {
     __shared__ uint64_t keys[SORT_CAP];
     __shared__ uint32_t hist[256];
@@ -492,7 +490,7 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
 
     int n_keys;
     if (nc <= SORT_CAP) {
-        for (int64_t i = threadIdx.x; i < nc; i += NT) keys[i] = make_key(cr[i], cu[i]);
+        for (int64_t i = threadIdx.x; i < nc; i += NT) keys[i] = make_key(cr[i], cnt, cu[i]);
         n_keys = (int)nc;
     } else {
         // MSD radix select of the take-th smallest key, 8 bits at a time;
@@ -505,7 +503,7 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
             const uint64_t pre = sel_prefix;
             const uint64_t mask_hi = (shift == 56) ? 0ull : (~0ull << (shift + 8));
             for (int64_t i = threadIdx.x; i < nc; i += NT) {
-                const uint64_t key = make_key(cr[i], cu[i]);
+                const uint64_t key = make_key(cr[i], cnt, cu[i]);
                 if ((key & mask_hi) == pre) atomicAdd(&hist[(key >> shift) & 255u], 1u);
             }
             __syncthreads();
@@ -524,7 +522,7 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
         if (threadIdx.x == 0) n_sel = 0;
         __syncthreads();
         for (int64_t i = threadIdx.x; i < nc; i += NT) {
-            const uint64_t key = make_key(cr[i], cu[i]);
+            const uint64_t key = make_key(cr[i], cnt, cu[i]);
             if (key <= kth) keys[atomicAdd(&n_sel, 1u)] = key;
         }
         __syncthreads();
@@ -575,41 +573,6 @@ __device__ __forceinline__ int64_t xcd_block(int64_t n_live) {
 }
 inline unsigned xcd_grid(int64_t n_max) { return (unsigned)(((n_max + CNT - 1) / CNT + 7) / 8 * 8); }
 
-// The score rule: FP32 products summed in ascending dimension order.
-__device__ __forceinline__ float rule_dot(const float *__restrict__ a, const float *__restrict__ b, int32_t d) {
-    float s = 0.0f;
-    int32_t k = 0;
-    // 32 terms are loaded before they are summed: lanes of a wavefront read
-    // different rows, and taking a whole 128-byte stretch per lane at once
-    // uses each cache line fully before it can be evicted (the sum's order is
-    // unchanged)
-    for (; k + 32 <= d; k += 32) {
-        float4 x[8], y[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            x[t] = *reinterpret_cast<const float4 *>(a + k + 4 * t);
-            y[t] = *reinterpret_cast<const float4 *>(b + k + 4 * t);
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            s = s + x[t].x * y[t].x;
-            s = s + x[t].y * y[t].y;
-            s = s + x[t].z * y[t].z;
-            s = s + x[t].w * y[t].w;
-        }
-    }
-    for (; k + 4 <= d; k += 4) {
-        const float4 x = *reinterpret_cast<const float4 *>(a + k);
-        const float4 y = *reinterpret_cast<const float4 *>(b + k);
-        s = s + x.x * y.x;
-        s = s + x.y * y.y;
-        s = s + x.z * y.z;
-        s = s + x.w * y.w;
-    }
-    for (; k < d; ++k) s = s + a[k] * b[k];
-    return s;
-}
-
 // Nibble counters of 8 bytes' c_lo (low 3 bits) or c_hi (bits 4..6): bin c
 // at bits 4c..4c+3 (at most 8 per nibble).
 template <int SH>
@@ -638,8 +601,7 @@ __device__ __forceinline__ void widen_add(uint32_t e, uint32_t o, uint32_t (&w)[
 }
 
 // grid (chunks, queries): counts of c_lo and c_hi values 0..6 of the chunk's
-// users, part[(b * n_chunk + chunk) * 16 + {0..6 | 8..14}] (b = qmap[y] when
-// given).  16 users per thread and load, four loads in flight (rows of cb
+// users, part[(b * n_chunk + chunk) * 16 + {0..6 | 8..14}].  16 users per thread and load, four loads in flight (rows of cb
 // are ldc bytes, ldc % 16 == 0, chunks start at multiples of 1024).  Each
 // 16-byte load is counted into nibble counters (8 bytes per word, so no
 // nibble passes 8), added into byte counters (at most 16 per load), and those
@@ -647,10 +609,9 @@ __device__ __forceinline__ void widen_add(uint32_t e, uint32_t o, uint32_t (&w)[
 // sums them by wave reductions (cu < 2^18 keeps the sums in 16 bits).  Only
 // a chunk's last load tests its bytes against the chunk's end.
 __global__ void __launch_bounds__(CNT) k_coarse_hist(const uint8_t *__restrict__ cb, int64_t ldc, int64_t n_user,
-                                                     int64_t cu, int32_t n_chunk, const int32_t *__restrict__ qmap,
-                                                     uint32_t *__restrict__ part) {
+                                                     int64_t cu, int32_t n_chunk, uint32_t *__restrict__ part) {
     __shared__ uint32_t red[CNT / 64][8];
-    const int64_t b = qmap ? qmap[blockIdx.y] : blockIdx.y;
+    const int64_t b = blockIdx.y;
     const uint8_t *v = cb + b * ldc;
     const int64_t u0 = (int64_t)blockIdx.x * cu, u1 = min(n_user, u0 + cu);
     uint32_t elo = 0, olo = 0, ehi = 0, ohi = 0;
@@ -714,11 +675,10 @@ __global__ void __launch_bounds__(CNT) k_coarse_hist(const uint8_t *__restrict__
 // #{c_lo <= c} >= k (-1 when there is none: the query takes the full path)
 // and the number of users with c_hi <= beta_c.  cq[b] = {beta_c, count, -, 0}.
 __global__ void __launch_bounds__(CNT) k_coarse_kth(const uint32_t *__restrict__ part, int32_t n_chunk,
-                                                    int32_t n_guard, const int32_t *__restrict__ qmap,
-                                                    const QueryInfo *__restrict__ qi, int32_t *__restrict__ cq,
-                                                    int32_t *__restrict__ hcnt) {
+                                                    int32_t n_guard, const QueryInfo *__restrict__ qi,
+                                                    int32_t *__restrict__ cq, int32_t *__restrict__ hcnt) {
     __shared__ uint32_t sh[CNT];
-    const int64_t b = qmap ? qmap[blockIdx.x] : blockIdx.x;
+    const int64_t b = blockIdx.x;
     uint32_t acc = 0;
     for (int32_t ch = threadIdx.x >> 4; ch < n_chunk; ch += CNT / 16)
         acc += part[((int64_t)b * n_chunk + ch) * 16 + (threadIdx.x & 15)];
@@ -774,7 +734,7 @@ __global__ void __launch_bounds__(NT) k_coarse_chunk_offsets(const uint32_t *__r
 
 // One workgroup: cbase[ch] = exclusive scan of ctot (chunk-major list).
 __global__ void __launch_bounds__(NT) k_coarse_chunk_base(const int32_t *__restrict__ ctot, int32_t n_chunk,
-                                                          int32_t *__restrict__ cbase, int32_t *__restrict__ total) {
+                                                          int32_t *__restrict__ cbase) {
     __shared__ uint32_t red[NW + 1];
     uint32_t base = 0;
     for (int32_t c0 = 0; c0 < n_chunk; c0 += NT) {
@@ -784,21 +744,6 @@ __global__ void __launch_bounds__(NT) k_coarse_chunk_base(const int32_t *__restr
         const uint32_t e = wg_excl_scan(v, red, &tot);
         if (i < n_chunk) cbase[i] = (int32_t)(base + e);
         base += tot;
-    }
-    if (total && threadIdx.x == 0) *total = (int32_t)base;  // the list's length
-}
-
-// One workgroup: a query whose coarse record has no k-th bound, a list over
-// cap, or a list longer than the bound the host put in field 2 (its first
-// pass's length) is sent to the full path (beta = -1, nothing listed).
-__global__ void __launch_bounds__(NT) k_coarse_mark(int32_t *__restrict__ cq, int32_t nq, int64_t cap) {
-    for (int32_t b = threadIdx.x; b < nq; b += NT) {
-        int32_t *e = cq + (int64_t)b * 4;
-        if (e[0] < 0 || e[1] > cap || e[1] > e[2]) {
-            e[0] = -1;
-            e[1] = 0;
-        }
-        e[3] = 0;
     }
 }
 
@@ -862,51 +807,6 @@ __global__ void __launch_bounds__(CNT) k_coarse_compact(const uint8_t *__restric
     }
 }
 
-// One thread per listed (query, user): the score rule's <u,q>, the exact
-// bucket pair against the full table row, and the query's bucket histograms
-// (ghist[b] = [h_lo | h_hi], S + 1 bins each; h_lo only when same != 0).
-__global__ void __launch_bounds__(CNT) k_coarse_exact(const float *__restrict__ users,
-                                                      const float *__restrict__ queries, int32_t ld, int32_t dim,
-                                                      const float *__restrict__ table, int32_t S, float eps, int same,
-                                                      const GuardCols *__restrict__ gsets,
-                                                      const int32_t *__restrict__ gset, const int32_t *__restrict__ cl_u,
-                                                      const int32_t *__restrict__ cl_b, int64_t n,
-                                                      const int32_t *__restrict__ n_dev,
-                                                      uint32_t *__restrict__ bk_c, float *__restrict__ s_c,
-                                                      uint32_t *__restrict__ ghist) {
-    const int64_t n_live = n_dev ? min(n, (int64_t)*n_dev) : n;
-    const int64_t lb = xcd_block(n_live);
-    const int64_t i = lb * CNT + threadIdx.x;
-    if (lb < 0 || i >= n_live) return;
-    const int64_t u = cl_u[i];
-    const uint32_t packed = (uint32_t)cl_b[i];
-    const int64_t b = packed & 0xFFFFu;
-    const int32_t clo = (int32_t)((packed >> 16) & 7u), chi = (int32_t)((packed >> 20) & 7u);
-    const GuardCols gc = gsets[gset[b]];
-    const float sc = rule_dot(users + u * ld, queries + b * ld, dim);
-    // both buckets lie in [j_{c_hi - 1} + 1, j_{c_lo}] (0 / S at the ends),
-    // j the query's guard columns
-    int32_t r0 = 0, r1 = S;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        if (j == chi - 1) r0 = gc.col[j] + 1;
-        if (j == clo && j < gc.n) r1 = gc.col[j];
-    }
-    const float *row = table + u * (int64_t)S;
-    uint32_t lo, hi;
-    if (eps > 0.0f) {
-        lo = (uint32_t)bucket_gt_in(row, r0, r1, __double2float_rd((double)sc - (double)eps));
-        hi = (uint32_t)bucket_gt_in(row, r0, r1, __double2float_ru((double)sc + (double)eps));
-    } else {
-        lo = hi = (uint32_t)bucket_gt_in(row, r0, r1, sc);
-    }
-    bk_c[i] = lo | (hi << 16);
-    s_c[i] = sc;
-    uint32_t *g = ghist + b * 2 * (int64_t)(S + 1);
-    atomicAdd(&g[lo], 1u);
-    if (!same) atomicAdd(&g[S + 1 + hi], 1u);
-}
-
 // Update path, one thread per listed (query, user): the rank bound values of
 // the exact bounds with pending inserts and deletes (base bucket within the
 // guard range, side rows searched at the score rule's <u,q>), as
@@ -914,7 +814,7 @@ __global__ void __launch_bounds__(CNT) k_coarse_exact(const float *__restrict__ 
 __global__ void __launch_bounds__(CNT) k_coarse_exact_upd(
     const float *__restrict__ users, const float *__restrict__ queries, int32_t ld, int32_t dim,
     const float *__restrict__ table, int32_t S, const int32_t *__restrict__ ranks, int64_t n_item_base, float eps,
-    const GuardCols *__restrict__ gsets, const int32_t *__restrict__ gset, const int32_t *__restrict__ cl_u,
+    GuardCols gc, const int32_t *__restrict__ cl_u,
     const int32_t *__restrict__ cl_b, int64_t n, const float *__restrict__ ins, int32_t n_ins, int32_t ld_ins,
     const float *__restrict__ del, int32_t n_del, int32_t ld_del, int64_t n_user, int32_t *__restrict__ lbs,
     int32_t *__restrict__ ubs, float *__restrict__ qip) {
@@ -925,7 +825,6 @@ __global__ void __launch_bounds__(CNT) k_coarse_exact_upd(
     const uint32_t packed = (uint32_t)cl_b[i];
     const int64_t b = packed & 0xFFFFu;
     const int32_t clo = (int32_t)((packed >> 16) & 7u), chi = (int32_t)((packed >> 20) & 7u);
-    const GuardCols gc = gsets[gset[b]];
     const float sc = rule_dot(users + u * ld, queries + b * ld, dim);
     int32_t r0 = 0, r1 = S;
 #pragma unroll
@@ -948,45 +847,6 @@ __global__ void __launch_bounds__(CNT) k_coarse_exact_upd(
     lbs[o] = (blo == S ? (int32_t)n_item_base : ranks[blo]) + off;
     ubs[o] = max((bhi == 0 ? 0 : ranks[bhi - 1] + 1) + off, 0);
     qip[o] = sc;
-}
-
-// One thread per listed (query, user): the candidates (b_hi <= beta) with
-// their rank when the bounds fix it, else -1 and a refine row; <u,q> of each
-// candidate goes to qip for the top-k.
-__global__ void __launch_bounds__(CNT) k_coarse_final(const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
-                                                      const uint32_t *__restrict__ bk_c, const float *__restrict__ s_c,
-                                                      int64_t n, const int32_t *__restrict__ n_dev, int32_t S,
-                                                      const int32_t *__restrict__ ranks,
-                                                      int64_t n_item, int64_t n_user, QueryInfo *__restrict__ qi,
-                                                      int32_t *__restrict__ cand_user, int32_t *__restrict__ cand_rank,
-                                                      int32_t *__restrict__ refine_total,
-                                                      int32_t *__restrict__ refine_cand,
-                                                      int32_t *__restrict__ refine_user,
-                                                      int32_t *__restrict__ refine_query,
-                                                      float *__restrict__ refine_thr, float *__restrict__ qip) {
-    const int64_t i = (int64_t)blockIdx.x * CNT + threadIdx.x;
-    if (i >= (n_dev ? min(n, (int64_t)*n_dev) : n)) return;
-    const int32_t b = cl_b[i] & 0xFFFF;
-    const uint32_t x = bk_c[i];
-    const int32_t blo = (int32_t)(x & 0xFFFFu), bhi = (int32_t)(x >> 16);
-    if (bhi > qi[b].beta) return;
-    const int32_t u = cl_u[i];
-    const int32_t lbs = blo == S ? (int32_t)n_item : ranks[blo];
-    const int32_t ubs = bhi == 0 ? 0 : ranks[bhi - 1] + 1;
-    const int32_t rank = lbs == ubs ? lbs : -1;
-    const int64_t slot = qi[b].cand_off + atomicAdd(&qi[b].fill, 1);
-    const float sc = s_c[i];
-    cand_user[slot] = u;
-    cand_rank[slot] = rank;
-    qip[(int64_t)b * n_user + u] = sc;
-    if (rank < 0) {
-        const int32_t r = atomicAdd(refine_total, 1);
-        atomicAdd(&qi[b].n_refine, 1);
-        refine_cand[r] = (int32_t)slot;
-        refine_user[r] = u;
-        refine_query[r] = b;
-        refine_thr[r] = sc;
-    }
 }
 
 }  // namespace
@@ -1027,113 +887,66 @@ hipError_t launch_offsets(hipStream_t s, QueryInfo *qi, int32_t nq, int32_t *ref
 hipError_t launch_compact(hipStream_t s, const uint32_t *bk, const float *qip, int64_t n_user, int32_t S,
                           const int32_t *ranks, int64_t n_item, int32_t nq, int output_mode, int64_t cu,
                           QueryInfo *qi, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_total,
-                          int32_t *refine_cand, int32_t *refine_user, int32_t *refine_query, float *refine_thr) {
+                          int32_t *refine_user, int32_t *refine_query, float *refine_thr, int32_t *cnt) {
     if (nq <= 0 || n_user <= 0) return hipSuccess;
     if (output_mode == RKR_OUTPUT_EXACT) {
         const unsigned n_chunk = (unsigned)((n_user + cu - 1) / cu);
         hipLaunchKernelGGL(k_compact_chunks, dim3(n_chunk, (unsigned)nq), dim3(NT), 0, s, bk, qip, n_user, S, ranks,
-                           n_item, cu, qi, cand_user, cand_rank, refine_total, refine_cand, refine_user, refine_query,
-                           refine_thr);
+                           n_item, cu, qi, cand_user, cand_rank, refine_total, refine_user, refine_query, refine_thr,
+                           cnt);
     } else {
         // reference output keeps the users in ascending order (settled users
         // are taken by userID, US.hpp:173-186)
         hipLaunchKernelGGL(k_compact, dim3((unsigned)nq), dim3(NT), 0, s, bk, qip, n_user, S, ranks, n_item, qi,
-                           cand_user, cand_rank, refine_total, refine_cand, refine_user, refine_query, refine_thr);
+                           cand_user, cand_rank, refine_total, refine_user, refine_query, refine_thr, cnt);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_scatter_counts(hipStream_t s, const int32_t *refine_total, const int32_t *refine_cand,
-                                 const int32_t *cnt, int64_t max_rows, int32_t *cand_rank) {
-    if (max_rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter_counts, dim3(1024), dim3(256), 0, s, refine_total, refine_cand, cnt, max_rows,
-                       cand_rank);
-    return hipGetLastError();
-}
-
 hipError_t launch_topk(hipStream_t s, const QueryInfo *qi, int32_t nq, const int32_t *cand_user,
-                       const int32_t *cand_rank, const float *qip, int64_t n_user, int32_t max_k, int32_t *out_user,
-                       int32_t *out_rank, float *out_qip, int64_t *scratch_keys) {
-    (void)scratch_keys;
+                       const int32_t *cand_rank, const int32_t *cnt, const float *qip, int64_t n_user, int32_t max_k,
+                       int32_t *out_user, int32_t *out_rank, float *out_qip) {
     if (nq <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_topk, dim3((unsigned)nq), dim3(NT), 0, s, qi, cand_user, cand_rank, qip, n_user, max_k,
+    hipLaunchKernelGGL(k_topk, dim3((unsigned)nq), dim3(NT), 0, s, qi, cand_user, cand_rank, cnt, qip, n_user, max_k,
                        out_user, out_rank, out_qip);
     return hipGetLastError();
 }
 
 hipError_t launch_coarse_kth(hipStream_t s, const uint8_t *cb, int64_t ldc, int64_t n_user, int32_t nq, int64_t cu,
-                             int32_t n_guard, const int32_t *qmap, uint32_t *part, const QueryInfo *qi, int32_t *cq,
-                             int32_t *hcnt) {
+                             int32_t n_guard, uint32_t *part, const QueryInfo *qi, int32_t *cq, int32_t *hcnt) {
     if (nq <= 0 || n_user <= 0) return hipSuccess;
     if (ldc % 16 || cu % 1024 || cu >= (1 << 18)) return hipErrorInvalidValue;
     const int32_t n_chunk = (int32_t)((n_user + cu - 1) / cu);
     hipLaunchKernelGGL(k_coarse_hist, dim3((unsigned)n_chunk, (unsigned)nq), dim3(CNT), 0, s, cb, ldc, n_user, cu,
-                       n_chunk, qmap, part);
-    hipLaunchKernelGGL(k_coarse_kth, dim3((unsigned)nq), dim3(CNT), 0, s, part, n_chunk, n_guard, qmap, qi, cq,
-                       hcnt);
+                       n_chunk, part);
+    hipLaunchKernelGGL(k_coarse_kth, dim3((unsigned)nq), dim3(CNT), 0, s, part, n_chunk, n_guard, qi, cq, hcnt);
     return hipGetLastError();
 }
 
 hipError_t launch_coarse_compact(hipStream_t s, const uint8_t *cb, int64_t ldc, int64_t n_user, int32_t nq,
                                  int64_t cu, const uint32_t *part, const int32_t *cq, int32_t *loc, int32_t *ctot,
-                                 int32_t *cbase, int32_t *cl_u, int32_t *cl_b, int32_t *total) {
+                                 int32_t *cbase, int32_t *cl_u, int32_t *cl_b) {
     if (nq <= 0 || n_user <= 0) return hipSuccess;
     if (ldc % 16 || cu % 1024 || nq > 65535) return hipErrorInvalidValue;
     const int32_t n_chunk = (int32_t)((n_user + cu - 1) / cu);
     hipLaunchKernelGGL(k_coarse_chunk_offsets, dim3((unsigned)n_chunk), dim3(NT), 0, s, part, n_chunk, nq, cq, loc,
                        ctot);
-    hipLaunchKernelGGL(k_coarse_chunk_base, dim3(1), dim3(NT), 0, s, ctot, n_chunk, cbase, total);
+    hipLaunchKernelGGL(k_coarse_chunk_base, dim3(1), dim3(NT), 0, s, ctot, n_chunk, cbase);
     hipLaunchKernelGGL(k_coarse_compact, dim3((unsigned)n_chunk, (unsigned)nq), dim3(CNT), 0, s, cb, ldc, n_user, cu,
                        nq, cq, loc, cbase, cl_u, cl_b);
     return hipGetLastError();
 }
 
-hipError_t launch_coarse_exact(hipStream_t s, const float *users, const float *queries, int32_t ld, int32_t dim,
-                               const float *table, int32_t S, const int32_t *ranks, int64_t n_item, float eps,
-                               const GuardCols *gsets, const int32_t *gset, int32_t nq, const int32_t *cl_u,
-                               const int32_t *cl_b, int64_t n, const int32_t *n_dev, uint32_t *bk_c, float *s_c,
-                               uint32_t *ghist, QueryInfo *qi) {
-    if (nq <= 0) return hipSuccess;
-    const int same = eps == 0.0f ? 1 : 0;
-    hipError_t e = hipMemsetAsync(ghist, 0, sizeof(uint32_t) * 2 * (size_t)(S + 1) * nq, s);
-    if (e != hipSuccess) return e;
-    if (n > 0)
-        hipLaunchKernelGGL(k_coarse_exact, dim3(xcd_grid(n)), dim3(CNT), 0, s, users, queries, ld,
-                           dim, table, S, eps, same, gsets, gset, cl_u, cl_b, n, n_dev, bk_c, s_c, ghist);
-    hipLaunchKernelGGL(k_hist_kth, dim3((unsigned)nq), dim3(NT), 0, s, ghist, S, same, ranks, n_item,
-                       (int)RKR_OUTPUT_EXACT, qi);
-    return hipGetLastError();
-}
-
 hipError_t launch_coarse_exact_upd(hipStream_t s, const float *users, const float *queries, int32_t ld, int32_t dim,
                                    const float *table, int32_t S, const int32_t *ranks, int64_t n_item_base,
-                                   float eps, const GuardCols *gsets, const int32_t *gset, const int32_t *cl_u,
+                                   float eps, const GuardCols &gc, const int32_t *cl_u,
                                    const int32_t *cl_b, int64_t n, const float *ins, int32_t n_ins, int32_t ld_ins,
                                    const float *del, int32_t n_del, int32_t ld_del, int64_t n_user, int32_t *lbs,
                                    int32_t *ubs, float *qip) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_coarse_exact_upd, dim3(xcd_grid(n)), dim3(CNT), 0, s, users, queries, ld,
-                       dim, table, S, ranks, n_item_base, eps, gsets, gset, cl_u, cl_b, n, ins, n_ins, ld_ins, del,
+                       dim, table, S, ranks, n_item_base, eps, gc, cl_u, cl_b, n, ins, n_ins, ld_ins, del,
                        n_del, ld_del, n_user, lbs, ubs, qip);
-    return hipGetLastError();
-}
-
-hipError_t launch_coarse_mark(hipStream_t s, int32_t *cq, int32_t nq, int64_t cap) {
-    if (nq <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_coarse_mark, dim3(1), dim3(NT), 0, s, cq, nq, cap);
-    return hipGetLastError();
-}
-
-hipError_t launch_coarse_final(hipStream_t s, const int32_t *cl_u, const int32_t *cl_b, const uint32_t *bk_c,
-                               const float *s_c, int64_t n, const int32_t *n_dev, int32_t S, const int32_t *ranks,
-                               int64_t n_item,
-                               int64_t n_user, QueryInfo *qi, int32_t *cand_user, int32_t *cand_rank,
-                               int32_t *refine_total, int32_t *refine_cand, int32_t *refine_user,
-                               int32_t *refine_query, float *refine_thr, float *qip) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_coarse_final, dim3((unsigned)((n + CNT - 1) / CNT)), dim3(CNT), 0, s, cl_u, cl_b, bk_c, s_c, n,
-                       n_dev, S, ranks, n_item, n_user, qi, cand_user, cand_rank, refine_total, refine_cand, refine_user,
-                       refine_query, refine_thr, qip);
     return hipGetLastError();
 }
 

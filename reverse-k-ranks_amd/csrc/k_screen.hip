@@ -58,12 +58,16 @@ union Frag {
 // over the users: |u_hi . q_hi (FP32 sums) - s(u, q)| <= ||u|| cs + the
 // denormal floor.  (u_hi . q_r + u_r . q_hi + u_r . q_r by Cauchy-Schwarz with
 // ||u_hi|| <= (1 + rho) ||u||; g1 the FP32 accumulation of the Kp exact
-// products, g_rule the sequential rule's own rounding.)
+// products, g_rule the sequential rule's own rounding.)  With zero64 it also
+// clears the row's 64 words of the batch's sample histogram.
 __global__ void k_prep_items(const float *__restrict__ items, int64_t n_item, int32_t ld, int32_t K, int32_t Kp,
                              uint16_t *__restrict__ hi, uint16_t *__restrict__ lo, float *__restrict__ norm,
-                             float *__restrict__ cs, const float *__restrict__ rho, double g1, double g_rule) {
+                             float *__restrict__ cs, const float *__restrict__ rho, double g1, double g_rule,
+                             uint32_t *__restrict__ zero64) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.y + threadIdx.y;
     if (p >= n_item) return;
+    if (zero64)
+        for (int k = threadIdx.x; k < 64; k += blockDim.x) zero64[p * 64 + k] = 0u;
     const float *x = items + p * ld;
     double ss = 0.0, sh = 0.0, sr = 0.0;
     for (int k = threadIdx.x; k < Kp; k += blockDim.x) {
@@ -453,48 +457,30 @@ __global__ void k_recheck(const float *__restrict__ users, const float *__restri
 }
 
 
-// Coarse buckets of a query batch.  For every (query b, user u) a screened
-// estimate s^ of <u,q_b> with |s^ - s| <= e = C ||u|| ||q|| + abs_floor is
-// compared with G <= 7 guard values of u's table row, T[u][col_0] >=
-// T[u][col_1] >= ... (col ascending):
+// Coarse buckets of a query batch with updates pending.  For every (query b,
+// user u) the estimate s^ = sum_k u_hi q_hi with |s^ - s| <= e = C ||u|| cs(q) +
+// abs_floor (k_prep_items) is compared with G <= 7 guard values of u's table
+// row, T[u][col_0] >= T[u][col_1] >= ... (col ascending):
 //   c_lo = #{g : guard_g > s^ - e},  c_hi = #{g : guard_g > s^ + e}
-// and cb[row(b) * ldc + u] = c_lo | c_hi << 4.  abs_floor also carries the
-// table's own eps.  The first pass (one guard set) takes the single product
-// s^ = sum_k u_hi q_hi, so C there covers the BF16 rounding of both factors
-// (2^-7 + 2^-16 of sum|u_k q_k|): a wider interval only lists a few more
-// users, and the pass does a third of the matrix work.  The second pass
-// (guard sets inside one bin) keeps the three-product form above.  Queries
-// are the A operand (staged through LDS, 64 per stage in the first pass, 32
-// with guard sets), users the B operand held in VGPRs: lane (lr, lq) of a
-// 16x16 tile owns user lr and queries 4 lq .. 4 lq + 3, so its guards stay in
-// registers.  qmap (optional) maps the launch's queries to rows of q_hi /
-// q_lo / q_norm and cb.
+// and cb[b * ldc + u] = c_lo | c_hi << 4.  abs_floor also carries the table's
+// own eps.  Queries are the A operand (staged through LDS, 64 per stage), users
+// the B operand held in VGPRs: lane (lr, lq) of a 16x16 tile owns user lr and
+// queries 4 lq .. 4 lq + 3, so its guards stay in registers.  (Batches without
+// updates need no buckets: k_list.hip lists against one threshold per query.)
 struct IpCoarseParams {
-    const float *users;           // n_user x ld
     const float *user_norm;       // n_user
-    const uint16_t *user_hi, *user_lo;  // n_user x Kp BF16 split
-    const float *table;           // n_user x S
-    const float *gvals;           // n_user x kGuardRow guard values (all sets), or null
+    const uint16_t *user_hi;      // n_user x Kp BF16 hi halves
+    const float *gvals;           // n_user x kGuardRow guard values
     int64_t n_user;
-    int32_t S;
     GuardCols gc;
-    const uint16_t *q_hi, *q_lo;  // rows of Kp
-    const float *q_norm;
-    const int32_t *qmap;          // nq entries, or null
-    int32_t nq;
-    int32_t ld, K, Kp;
+    const uint16_t *q_hi;         // rows of Kp
+    const float *q_cs;
+    int32_t nq, Kp;
     float C, abs_floor;
     uint8_t *cb;                  // rows of ldc bytes (ldc % 128 == 0)
     int64_t ldc;
     int64_t spare_row;            // row written for the stage's padding queries
-    // per-query guard sets (second pass): query qq uses sets[qset[qq]]
-    const GuardCols *sets;
-    const int32_t *qset;
-    int32_t n_sets;
-    int32_t set_id[7];            // guard-row set of each launch set (with gvals)
 };
-
-constexpr int kMaxGuardSets = 7;
 
 // t + t + b for a lane predicate b: one v_addc_co_u32 with b's lane mask as
 // the carry-in (the ballot of a compare is that compare's mask, so no
@@ -548,136 +534,71 @@ __device__ __forceinline__ uint32_t guard_count_last(const float (&g)[8], float 
     return twice_plus(t, b0);
 }
 
-template <int KS, bool SETS>
-__global__ void __launch_bounds__(NT, SETS ? 2 : coarse_first_pass_wgs(KS)) k_ip_coarse(IpCoarseParams P) {
-    // first pass: one product, so only the queries' hi halves are staged and
-    // only the users' hi halves are held (4 workgroups per CU fit)
-    constexpr bool ONE = !SETS;
-    constexpr int NH = ONE ? 1 : 2;
-    // queries per LDS stage: 64 halves the stage barriers and query refills per
-    // user block; the second pass keeps 32 so its guard sets also fit 3
-    // workgroups per CU in LDS
-    constexpr int QST = SETS ? 32 : 64;
+template <int KS>
+__global__ void __launch_bounds__(NT, coarse_first_pass_wgs(KS)) k_ip_coarse(IpCoarseParams P) {
+    constexpr int QST = 64;  // queries per LDS stage
     constexpr int ROWQ = (KS * 32 + KPAD_LDS) / 8;
     constexpr int KQ = KS * 4;
-    __shared__ uint4 sA[NH][QST * ROWQ];
+    __shared__ uint4 sA[QST * ROWQ];
     __shared__ float sQn[QST];
     __shared__ int64_t sQo[QST];  // byte offset of the query's cb row
-    __shared__ int32_t sQs[QST];
-    __shared__ float4 sG[SETS ? kMaxGuardSets * 128 * 2 : 1];      // [set][user][8 guards]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 15, lq = lane >> 4;
     const int64_t n_rb = (P.n_user + 127) / 128;
     for (int64_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x) {
         const int64_t row_base = rb * 128 + wave * 32;
-        Frag uh[2][KS], ul[2][ONE ? 1 : KS];
+        Frag uh[2][KS];
         float gd[2][8], ar[2], hg[2];
-        bool live[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             const int64_t r = row_base + b * 16 + lr;
-            live[b] = r < P.n_user;
+            const bool live = r < P.n_user;
             // rows past n_user load row 0 and are zeroed after the load (a
             // select between a load and a constant can become a load through
             // a selected pointer, flat and from scratch)
-            const int64_t rr = live[b] ? r : 0;
+            const int64_t rr = live ? r : 0;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                const uint4 z = make_uint4(0, 0, 0, 0);
                 const uint4 h = reinterpret_cast<const uint4 *>(P.user_hi + rr * P.Kp)[ks * 4 + lq];
-                uh[b][ks].q = live[b] ? h : z;
-                if (!ONE) {
-                    const uint4 l = reinterpret_cast<const uint4 *>(P.user_lo + rr * P.Kp)[ks * 4 + lq];
-                    ul[b][ONE ? 0 : ks].q = live[b] ? l : z;
-                }
+                uh[b][ks].q = live ? h : make_uint4(0, 0, 0, 0);
             }
-            if (!SETS) {
-                if (P.gvals) {
-                    // the user's guard values, one 32-byte row
-                    const float4 *g4 = reinterpret_cast<const float4 *>(P.gvals + (live[b] ? r : 0) * kGuardRow);
-                    const float4 x0 = g4[0], x1 = g4[1];
-                    const float ninf = -INFINITY;
-                    gd[b][0] = live[b] ? x0.x : ninf; gd[b][1] = live[b] ? x0.y : ninf;
-                    gd[b][2] = live[b] ? x0.z : ninf; gd[b][3] = live[b] ? x0.w : ninf;
-                    gd[b][4] = live[b] ? x1.x : ninf; gd[b][5] = live[b] ? x1.y : ninf;
-                    gd[b][6] = live[b] ? x1.z : ninf; gd[b][7] = ninf;
-                } else {
-                    const float *trow = P.table + (live[b] ? r : 0) * (int64_t)P.S;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) gd[b][j] = (live[b] && j < P.gc.n) ? trow[P.gc.col[j]] : -INFINITY;
-                }
+            for (int j = 0; j < 8; ++j) {
+                const float x = P.gvals[rr * kGuardRow + P.gc.idx[j]];
+                gd[b][j] = live && j < P.gc.n ? x : -INFINITY;
             }
-            ar[b] = live[b] ? P.C * P.user_norm[r] : 0.0f;
-            if (!SETS) {
-                // half the smallest gap between adjacent guards, rounded down
-                // (differences with -inf padding are +inf or NaN, which
-                // fminf passes over)
-                float m = INFINITY;
+            ar[b] = live ? P.C * P.user_norm[r] : 0.0f;
+            // half the smallest gap between adjacent guards, rounded down
+            // (differences with -inf padding are +inf or NaN, which
+            // fminf passes over)
+            float m = INFINITY;
 #pragma unroll
-                for (int j = 0; j < 6; ++j) m = fminf(m, gd[b][j] - gd[b][j + 1]);
-                hg[b] = __double2float_rd(0.5 * (double)m);
-            }
-        }
-        if (SETS) {
-            __syncthreads();  // the previous row block is done with sG
-            float *g = reinterpret_cast<float *>(sG);
-            for (int t = threadIdx.x; t < P.n_sets * 128 * 8; t += NT) {
-                const int set = t / (128 * 8), ul = (t / 8) % 128, j = t % 8;
-                const int64_t r = rb * 128 + ul;
-                float v = -INFINITY;
-                if (r < P.n_user) {
-                    if (P.gvals) {
-                        // 32 contiguous bytes of the user's guard row
-                        v = P.gvals[r * kGuardRow + P.set_id[set] * 8 + j];
-                    } else {
-                        const GuardCols &gc = P.sets[set];
-                        if (j < gc.n) v = P.table[r * P.S + gc.col[j]];
-                    }
-                }
-                g[t] = v;
-            }
+            for (int j = 0; j < 6; ++j) m = fminf(m, gd[b][j] - gd[b][j + 1]);
+            hg[b] = __double2float_rd(0.5 * (double)m);
         }
         for (int32_t q0 = 0; q0 < P.nq; q0 += QST) {
             __syncthreads();  // every wave is done with the previous stage
             {
                 // the stage's query rows: KS 16-byte pieces per thread, all
                 // loads in flight before the first LDS write (rows past nq
-                // load the last query and are zeroed after the load).  The
-                // query map's entries are all read before the first row load,
-                // so the row loads do not wait for one another.
-                static_assert(NH * QST * KQ == KS * NT, "one piece per thread and k-step");
+                // load the last query and are zeroed after the load)
+                static_assert(QST * KQ == KS * NT, "one piece per thread and k-step");
                 uint4 v[KS];
-                int dst[KS], qr[KS];
-                bool ok[KS];
 #pragma unroll
                 for (int k = 0; k < KS; ++k) {
                     const int c = (int)threadIdx.x + k * NT;
-                    const int rem = c % (QST * KQ);
-                    const int qq = q0 + rem / KQ;
-                    ok[k] = qq < P.nq;
-                    qr[k] = min(qq, P.nq - 1);
-                }
-                if (P.qmap) {
-#pragma unroll
-                    for (int k = 0; k < KS; ++k) qr[k] = P.qmap[qr[k]];
+                    v[k] = reinterpret_cast<const uint4 *>(P.q_hi)[(int64_t)min(q0 + c / KQ, P.nq - 1) * KQ + c % KQ];
                 }
 #pragma unroll
                 for (int k = 0; k < KS; ++k) {
                     const int c = (int)threadIdx.x + k * NT;
-                    const int half = c / (QST * KQ);
-                    const int rem = c % (QST * KQ);
-                    v[k] = reinterpret_cast<const uint4 *>(half ? P.q_lo : P.q_hi)[(int64_t)qr[k] * KQ + rem % KQ];
-                    dst[k] = half * (QST * ROWQ) + (rem / KQ) * ROWQ + rem % KQ;
+                    sA[(c / KQ) * ROWQ + c % KQ] = q0 + c / KQ < P.nq ? v[k] : make_uint4(0, 0, 0, 0);
                 }
-#pragma unroll
-                for (int k = 0; k < KS; ++k) (&sA[0][0])[dst[k]] = ok[k] ? v[k] : make_uint4(0, 0, 0, 0);
             }
             if (threadIdx.x < QST) {
                 const int qq = q0 + (int)threadIdx.x;
-                const int32_t qr = qq < P.nq ? (P.qmap ? P.qmap[qq] : qq) : 0;
-                sQo[threadIdx.x] = (qq < P.nq ? (int64_t)qr : P.spare_row) * P.ldc;
-                sQn[threadIdx.x] = qq < P.nq ? P.q_norm[qr] : 0.f;
-                if (SETS) sQs[threadIdx.x] = qq < P.nq ? P.qset[qq] : 0;
+                sQo[threadIdx.x] = (qq < P.nq ? (int64_t)qq : P.spare_row) * P.ldc;
+                sQn[threadIdx.x] = qq < P.nq ? P.q_cs[qq] : 0.f;
             }
             __syncthreads();
 #pragma unroll
@@ -686,123 +607,69 @@ __global__ void __launch_bounds__(NT, SETS ? 2 : coarse_first_pass_wgs(KS)) k_ip
                 f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
-                    Frag qh, ql;
-                    qh.q = sA[0][it * ROWQ + ks * 4 + lq];
-                    if (!ONE) ql.q = sA[NH - 1][it * ROWQ + ks * 4 + lq];
+                    Frag qh;
+                    qh.q = sA[it * ROWQ + ks * 4 + lq];
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                }
+                // D[4 lq + i][lr]: query q0 + g*16 + 4 lq + i, user row_base + b*16 + lr.
+                // c_hi = #{g > xh} <= c_lo.  When at most one guard can lie
+                // in (xl, xh] -- the interval is narrower than half the
+                // smallest gap between adjacent guards -- c_hi is c_lo less
+                // [g[c_lo - 1] <= xh].  Two guards inside would be closer
+                // than xh - xl (< 2 fl(xh - xl) in FP32), so a wavefront
+                // with any pair failing the test counts xh for all its
+                // pairs.
+                uint32_t byte[4][2];
+                bool redo = false;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float qn = sQn[g * 16 + 4 * lq + i];
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
-                        if (!ONE) {
-                            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, ul[b][ONE ? 0 : ks].v, acc[b], 0,
-                                                                              0, 0);
-                            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql.v, uh[b][ks].v, acc[b], 0, 0, 0);
-                        }
+                        const float e = __fmaf_rn(ar[b], qn, P.abs_floor);
+                        const float xl = acc[b][i] - e, xh = acc[b][i] + e;
+                        float last;
+                        const uint32_t c = guard_count_last(gd[b], xl, last);
+                        redo |= !(xh - xl < hg[b]);
+                        byte[i][b] = c | (c - (last <= xh ? 1u : 0u)) << 4;
                     }
                 }
-                // D[4 lq + i][lr]: query q0 + g*16 + 4 lq + i, user row_base + b*16 + lr
-                if (SETS) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        // rows are padded to whole row blocks and padding queries
-                        // write the spare row, so every lane stores
-                        const int ql_ = g * 16 + 4 * lq + i;
-                        const float qn = sQn[ql_];
-                        uint8_t *out = P.cb + sQo[ql_] + row_base + lr;
-#pragma unroll
-                        for (int b = 0; b < 2; ++b) {
-                            const float4 *gp = sG + (sQs[ql_] * 128 + wave * 32 + b * 16 + lr) * 2;
-                            const float4 x0 = gp[0], x1 = gp[1];
-                            gd[b][0] = x0.x; gd[b][1] = x0.y; gd[b][2] = x0.z; gd[b][3] = x0.w;
-                            gd[b][4] = x1.x; gd[b][5] = x1.y; gd[b][6] = x1.z; gd[b][7] = x1.w;
-                            const float e = __fmaf_rn(ar[b], qn, P.abs_floor);
-                            out[b * 16] = (uint8_t)guard_byte(gd[b], acc[b][i] - e, acc[b][i] + e);
-                        }
-                    }
-                } else {
-                    // c_hi = #{g > xh} <= c_lo.  When at most one guard can lie
-                    // in (xl, xh] -- the interval is narrower than half the
-                    // smallest gap between adjacent guards -- c_hi is c_lo less
-                    // [g[c_lo - 1] <= xh].  Two guards inside would be closer
-                    // than xh - xl (< 2 fl(xh - xl) in FP32), so a wavefront
-                    // with any pair failing the test counts xh for all its
-                    // pairs.
-                    uint32_t byte[4][2];
-                    bool redo = false;
+                if (__builtin_amdgcn_ballot_w64(redo) != 0) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float qn = sQn[g * 16 + 4 * lq + i];
 #pragma unroll
                         for (int b = 0; b < 2; ++b) {
                             const float e = __fmaf_rn(ar[b], qn, P.abs_floor);
-                            const float xl = acc[b][i] - e, xh = acc[b][i] + e;
-                            float last;
-                            const uint32_t c = guard_count_last(gd[b], xl, last);
-                            redo |= !(xh - xl < hg[b]);
-                            byte[i][b] = c | (c - (last <= xh ? 1u : 0u)) << 4;
+                            byte[i][b] = guard_byte(gd[b], acc[b][i] - e, acc[b][i] + e);
                         }
                     }
-                    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
+                }
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float qn = sQn[g * 16 + 4 * lq + i];
+                for (int i = 0; i < 4; ++i) {
+                    // rows are padded to whole row blocks and padding
+                    // queries write the spare row, so every lane stores
+                    uint8_t *out = P.cb + sQo[g * 16 + 4 * lq + i] + row_base + lr;
 #pragma unroll
-                            for (int b = 0; b < 2; ++b) {
-                                const float e = __fmaf_rn(ar[b], qn, P.abs_floor);
-                                byte[i][b] = guard_byte(gd[b], acc[b][i] - e, acc[b][i] + e);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        // rows are padded to whole row blocks and padding
-                        // queries write the spare row, so every lane stores
-                        uint8_t *out = P.cb + sQo[g * 16 + 4 * lq + i] + row_base + lr;
-#pragma unroll
-                        for (int b = 0; b < 2; ++b) out[b * 16] = (uint8_t)byte[i][b];
-                    }
+                    for (int b = 0; b < 2; ++b) out[b * 16] = (uint8_t)byte[i][b];
                 }
             }
         }
     }
 }
 
-// gv[u * kGuardRow + 8 s + j] = T[u][set s column j], -inf past the set's n:
-// the coarse passes' guard values of every user in one 256-byte row (the
-// columns sit in different cache lines of a table row), gathered once per
-// table.
-__global__ void __launch_bounds__(256) k_gather_guards(const float *__restrict__ T, int64_t S, GuardSets gs,
-                                                       int64_t u0, int64_t n_rows, float *__restrict__ gv) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n_rows * kGuardRow) return;
-    const int64_t u = u0 + i / kGuardRow;
-    const int sj = (int)(i % kGuardRow), j = sj & 7;
-    const GuardCols &g = gs.set[sj >> 3];
-    gv[u * kGuardRow + sj] = j < g.n ? T[u * S + g.col[j]] : -INFINITY;
-}
-
 }  // namespace
-
-hipError_t launch_gather_guards(hipStream_t s, const float *T, int64_t S, const GuardSets &gs, int64_t u0,
-                                int64_t n_rows, float *gv) {
-    if (n_rows <= 0) return hipSuccess;
-    for (const GuardCols &g : gs.set) {
-        if (g.n < 0 || g.n > 7) return hipErrorInvalidValue;
-        for (int j = 0; j < g.n; ++j)
-            if (g.col[j] < 0 || g.col[j] >= S) return hipErrorInvalidValue;
-    }
-    hipLaunchKernelGGL(k_gather_guards, dim3((unsigned)((n_rows * kGuardRow + 255) / 256)), dim3(256), 0, s, T, S, gs,
-                       u0, n_rows, gv);
-    return hipGetLastError();
-}
 
 hipError_t launch_prep_items(hipStream_t s, const float *items, int64_t n_item, int32_t ld, int32_t K, int32_t Kp,
                              uint16_t *hi, uint16_t *lo, float *norm, float *cs, const float *rho, double g1,
-                             double g_rule) {
+                             double g_rule, uint32_t *zero64) {
     if (n_item <= 0) return hipSuccess;
     if (cs && !rho) return hipErrorInvalidValue;
     dim3 block(32, 8);
     hipLaunchKernelGGL(k_prep_items, dim3((unsigned)((n_item + 7) / 8)), block, 0, s, items, n_item, ld, K, Kp, hi, lo,
-                       norm, cs, rho, g1, g_rule);
+                       norm, cs, rho, g1, g_rule, zero64);
     return hipGetLastError();
 }
 
@@ -883,25 +750,16 @@ hipError_t launch_recheck(hipStream_t s, const float *users, const float *items,
 
 hipError_t launch_ip_coarse(hipStream_t s, const CoarseLaunch &L) {
     if (L.n_user <= 0 || L.nq <= 0) return hipSuccess;
-    const bool sets = L.sets != nullptr;
-    if (sets ? (L.n_sets < 1 || L.n_sets > kMaxGuardSets || !L.qset) : (L.gc.n < 1 || L.gc.n > 7))
-        return hipErrorInvalidValue;
-    if (L.ldc % 128 || L.ldc < L.n_user) return hipErrorInvalidValue;
-    if (!L.user_hi || !L.user_lo) return hipErrorInvalidValue;
-    IpCoarseParams P{L.users, L.user_norm, L.user_hi, L.user_lo, L.table, L.gvals, L.n_user, L.S, L.gc, L.q_hi,
-                     L.q_lo, L.q_norm, L.qmap, L.nq, L.ld, L.K, L.Kp, L.C, L.abs_floor, L.cb, L.ldc, L.spare_row,
-                     L.sets, L.qset, L.n_sets, {}};
-    if (sets && L.gvals)
-        for (int t = 0; t < L.n_sets; ++t) {
-            if (L.set_id[t] < 1 || L.set_id[t] >= kGuardSets) return hipErrorInvalidValue;
-            P.set_id[t] = L.set_id[t];
-        }
+    if (L.gc.n < 1 || L.gc.n > 7 || L.ldc % 128 || L.ldc < L.n_user || !L.user_hi || !L.gvals) return hipErrorInvalidValue;
+    for (int j = 0; j < 8; ++j)
+        if (L.gc.idx[j] < 0 || L.gc.idx[j] >= kGuardRow) return hipErrorInvalidValue;
+    const IpCoarseParams P{L.user_norm, L.user_hi, L.gvals, L.n_user, L.gc, L.q_hi, L.q_cs, L.nq, L.Kp, L.C,
+                           L.abs_floor, L.cb, L.ldc, L.spare_row};
     const int64_t n_rb = (L.n_user + 127) / 128;
     const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(n_rb, L.grid_cap)));
-#define RKR_COARSE_CASE(ks)                                                                                   \
-    case ks:                                                                                                  \
-        if (sets) hipLaunchKernelGGL((k_ip_coarse<ks, true>), grid, dim3(NT), 0, s, P);                      \
-        else hipLaunchKernelGGL((k_ip_coarse<ks, false>), grid, dim3(NT), 0, s, P);                          \
+#define RKR_COARSE_CASE(ks)                                                    \
+    case ks:                                                                   \
+        hipLaunchKernelGGL((k_ip_coarse<ks>), grid, dim3(NT), 0, s, P);        \
         break;
     switch (L.Kp / 32) {
         RKR_COARSE_CASE(1)

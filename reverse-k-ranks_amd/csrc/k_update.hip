@@ -371,8 +371,9 @@ __global__ void __launch_bounds__(NT) k_compact_values(const int32_t *__restrict
                                                        const float *__restrict__ qip, int64_t n_user, int64_t cu,
                                                        QueryInfo *__restrict__ qi, int32_t *__restrict__ cand_user,
                                                        int32_t *__restrict__ cand_rank, int32_t *__restrict__ refine_total,
-                                                       int32_t *__restrict__ refine_cand, int32_t *__restrict__ refine_user,
-                                                       int32_t *__restrict__ refine_query, float *__restrict__ refine_thr) {
+                                                       int32_t *__restrict__ refine_user,
+                                                       int32_t *__restrict__ refine_query, float *__restrict__ refine_thr,
+                                                       int32_t *__restrict__ cnt) {
     __shared__ uint32_t red[NW + 1];
     __shared__ int32_t s_can, s_ref;
     const int64_t b = blockIdx.y;
@@ -406,10 +407,12 @@ __global__ void __launch_bounds__(NT) k_compact_values(const int32_t *__restrict
         if (cand) {
             const int64_t slot = off + s_can + (e & 0xFFFFu);
             cand_user[slot] = (int32_t)u;
-            cand_rank[slot] = rank;
-            if (refine) {
+            if (!refine) {
+                cand_rank[slot] = rank;
+            } else {
                 const int32_t r = s_ref + (int32_t)(e >> 16);
-                refine_cand[r] = (int32_t)slot;
+                cand_rank[slot] = ~r;
+                cnt[r] = 0;
                 refine_user[r] = (int32_t)u;
                 refine_query[r] = (int32_t)b;
                 refine_thr[r] = qb[u];
@@ -517,12 +520,12 @@ hipError_t launch_kth_values(hipStream_t s, const int32_t *lbs, const int32_t *u
 
 hipError_t launch_compact_values(hipStream_t s, const int32_t *lbs, const int32_t *ubs, const float *qip,
                                  int64_t n_user, int32_t nq, int64_t cu, QueryInfo *qi, int32_t *cand_user,
-                                 int32_t *cand_rank, int32_t *refine_total, int32_t *refine_cand,
-                                 int32_t *refine_user, int32_t *refine_query, float *refine_thr) {
+                                 int32_t *cand_rank, int32_t *refine_total, int32_t *refine_user,
+                                 int32_t *refine_query, float *refine_thr, int32_t *cnt) {
     if (nq <= 0 || n_user <= 0) return hipSuccess;
     const dim3 grid((unsigned)((n_user + cu - 1) / cu), (unsigned)nq);
     hipLaunchKernelGGL(k_compact_values, grid, dim3(NT), 0, s, lbs, ubs, qip, n_user, cu, qi, cand_user, cand_rank,
-                       refine_total, refine_cand, refine_user, refine_query, refine_thr);
+                       refine_total, refine_user, refine_query, refine_thr, cnt);
     return hipGetLastError();
 }
 

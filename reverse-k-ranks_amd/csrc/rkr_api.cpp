@@ -108,14 +108,16 @@ DataSnap snap_of(const Ctx *c) {
     d.qtable = c->qtable;
     d.qranks = c->qranks;
     d.n_qs = c->n_qs;
-    guard_columns(c, d.gcol, d.n_guard);
+    d.fine = fine_columns(c);
+    d.guards = guard_columns(c);
     d.gvals = c->gvals;
+    d.gcols = c->gcols;
+    d.gpitch = c->gpitch;
     d.ranks = c->ranks;
     d.n_sample = c->n_sample;
     d.table_eps = c->table_eps;
     d.qcol = c->qcol;
     d.hrk = std::make_shared<const std::vector<int32_t>>(c->qtable ? c->h_qranks : c->h_ranks);
-    if (d.n_guard > 0) d.gsets = guard_sets(c);
     for (int j = 0; j < 8; ++j) d.ins_gmax[j] = c->ins_gmax[j];
     if (c->qsrp_users && c->qsrp_n_user == c->n_user) {
         d.qsrp_users = c->qsrp_users;
@@ -155,11 +157,11 @@ uint64_t row_hash(const void *p, size_t n, uint32_t salt) {
     return x ^ (x >> 32);
 }
 
-// Guard columns of the coarse bounds: the table columns nearest below ranks
-// 4^j - 1 (3, 15, ..., 16383), at most 7, ascending.
-void guard_columns(const Ctx *c, int32_t *col, int32_t &n) {
-    const std::vector<int32_t> &hr = c->qtable ? c->h_qranks : c->h_ranks;
-    n = 0;
+namespace {
+// The table columns nearest below ranks 4^j - 1 (3, 15, ..., 16383), at most
+// 7, ascending.
+int guard_table_columns(const std::vector<int32_t> &hr, int32_t *col) {
+    int n = 0;
     int32_t last = -1;
     for (int64_t target = 3; target <= 16383 && n < 7; target = target * 4 + 3) {
         const auto it = std::upper_bound(hr.begin(), hr.end(), (int32_t)target);
@@ -169,43 +171,75 @@ void guard_columns(const Ctx *c, int32_t *col, int32_t &n) {
             last = j;
         }
     }
+    return n;
+}
+const std::vector<int32_t> &searched_ranks(const Ctx *c) { return c->qtable ? c->h_qranks : c->h_ranks; }
+}  // namespace
+
+// The guard columns and, inside each of their bins and past the last one, up
+// to 7 more spaced geometrically in rank: neighbouring fine columns differ by a
+// factor of about 1.2 in rank (4 between guard columns), which is how much a
+// list is longer than it has to be.
+FineCols fine_columns(const Ctx *c) {
+    FineCols fc{};
+    const std::vector<int32_t> &hr = searched_ranks(c);
+    if (hr.empty()) return fc;
+    int32_t gcol[8];
+    const int ng = guard_table_columns(hr, gcol);
+    int32_t last = -1;
+    auto take = [&](int32_t j, bool coarse) {
+        if (j <= last || fc.n >= kMaxFine) return;
+        if (coarse) fc.coarse |= 1ull << fc.n;
+        fc.col[fc.n++] = j;
+        last = j;
+    };
+    for (int g = 0; g <= ng; ++g) {
+        const int32_t lo = last + 1, hi = g < ng ? gcol[g] : (int32_t)hr.size() - 1;
+        if (lo > hi) continue;
+        const double ra = (double)hr[lo] + 1.0, rb = (double)hr[hi] + 1.0;
+        for (int m = 0; m < 7; ++m) {
+            const auto it = std::upper_bound(hr.begin() + lo, hr.begin() + hi, (int32_t)(ra * std::pow(rb / ra, m / 7.0) - 1.0));
+            const int32_t j = (int32_t)(it - hr.begin()) - 1;
+            if (j >= lo && j < hi) take(j, false);
+        }
+        take(hi, g < ng);
+    }
+    return fc;
 }
 
-// Set 0: the guard columns.  Set 1 + beta: up to 7 columns inside guard bin
-// beta (the columns after guard beta - 1 up to guard beta, the bin's last
-// column included), spaced geometrically in rank, for the second coarse pass
-// of queries whose k-th bound fell in that bin.
-GuardSets guard_sets(const Ctx *c) {
-    GuardSets gs{};
-    GuardCols &gc = gs.set[0];
-    guard_columns(c, gc.col, gc.n);
-    const std::vector<int32_t> &hrk = c->qtable ? c->h_qranks : c->h_ranks;
-    for (int32_t beta = 0; beta < gc.n; ++beta) {
-        GuardCols &g2 = gs.set[1 + beta];
-        const int32_t lo_col = beta == 0 ? 0 : gc.col[beta - 1] + 1, hi_col = gc.col[beta];
-        if (hi_col <= lo_col) continue;
-        const double ra = (double)hrk[lo_col] + 1.0, rb = (double)hrk[hi_col] + 1.0;
-        int32_t last = lo_col - 1;
-        for (int m = 1; m <= 6; ++m) {
-            const double target = ra * std::pow(rb / ra, m / 7.0) - 1.0;
-            int32_t j = last + 1;
-            while (j + 1 < hi_col && (double)hrk[j + 1] <= target) ++j;
-            if (j < hi_col && j > last && (double)hrk[j] <= target) {
-                g2.col[g2.n++] = j;
-                last = j;
-            }
+GuardCols guard_columns(const Ctx *c) {
+    GuardCols gc{};
+    const FineCols fc = fine_columns(c);
+    for (int f = 0; f < fc.n; ++f)
+        if ((fc.coarse >> f) & 1) {
+            gc.col[gc.n] = fc.col[f];
+            gc.idx[gc.n++] = f;
         }
-        g2.col[g2.n++] = hi_col;
-    }
-    return gs;
+    return gc;
 }
 
 int refresh_guard_values(Ctx *c, int64_t u0, int64_t n) {
     if (!c->gvals || n <= 0) return RKR_OK;
-    const GuardSets gs = guard_sets(c);
+    const FineCols fc = fine_columns(c);
     const float *T = c->qtable ? c->qtable : c->table;
     const int64_t S = c->qtable ? c->n_qs : c->n_sample;
-    RKR_HIP(c, launch_gather_guards(c->stream, T, S, gs, u0, n, c->gvals));
+    RKR_HIP(c, launch_gather_guards(c->stream, T, S, fc, u0, n, c->gvals, c->gcols, c->gpitch));
+    return RKR_OK;
+}
+
+int alloc_guards(Ctx *c, int64_t cap) {
+    float *gv = nullptr, *gc = nullptr;
+    int rc = dev_alloc_t(c, &gv, (size_t)cap * kGuardRow, "guard values");
+    if (!rc) rc = dev_alloc_t(c, &gc, (size_t)cap * kGuardRow, "guard columns");
+    if (rc) {
+        dev_free(c, gv, 0);
+        return rc;
+    }
+    dev_free(c, c->gvals, 0);
+    dev_free(c, c->gcols, 0);
+    c->gvals = gv;
+    c->gcols = gc;
+    c->gpitch = cap;
     return RKR_OK;
 }
 
@@ -309,6 +343,9 @@ void free_table(Ctx *c) {
     dev_free(c, c->qcol, 0);
     dev_free(c, c->qtable, 0);
     dev_free(c, c->gvals, 0);
+    dev_free(c, c->gcols, 0);
+    c->gcols = nullptr;
+    c->gpitch = 0;
     c->ranks = c->qranks = c->qcol = nullptr;
     c->table = c->qtable = c->gvals = nullptr;
     c->n_sample = c->n_qs = 0;
@@ -353,8 +390,7 @@ void free_bufs(Ctx *c, std::initializer_list<DeviceBuf *> bufs) {
 
 void free_scratch(Ctx *c) {
     Slot &s = c->main;
-    free_bufs(c, {&s.q_in, &s.qip, &s.bk, &s.qinfo, &s.cand, &s.refine_idx, &s.counts, &s.out, &s.recheck, &s.small,
-                  &c->misc});
+    free_bufs(c, {&s.io, &s.qip, &s.bk, &s.cand, &s.refine_idx, &s.recheck, &c->misc});
 }
 
 }  // namespace
@@ -374,8 +410,8 @@ int slot_init(Ctx *c, Slot &sl, bool own_stream, const std::vector<uint32_t> *cu
 
 void slot_free(Ctx *c, Slot &sl) {
     if (sl.stream) (void)hipStreamSynchronize(sl.stream);
-    free_bufs(c, {&sl.q_in, &sl.qip, &sl.bk, &sl.qinfo, &sl.cand, &sl.refine_idx, &sl.counts, &sl.out, &sl.recheck,
-                  &sl.small, &sl.hist, &sl.q_split, &sl.coarse_info, &sl.coarse_list});
+    free_bufs(c, {&sl.io, &sl.qip, &sl.bk, &sl.cand, &sl.refine_idx, &sl.recheck, &sl.hist, &sl.q_split, &sl.list_info,
+                  &sl.list});
     free_pinned(sl.stage);
     for (auto &e : sl.ev)
         if (e) { (void)hipEventDestroy(e); e = nullptr; }
@@ -690,7 +726,7 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
     int rc = dev_alloc_t(c, &c->ranks, (size_t)S, "ranks");
     if (rc) return rc;
     rc = dev_alloc_t(c, &c->table, (size_t)std::max(c->u_cap, c->n_user) * S, "table");
-    if (!rc) rc = dev_alloc_t(c, &c->gvals, (size_t)std::max(c->u_cap, c->n_user) * kGuardRow, "guard values");
+    if (!rc) rc = alloc_guards(c, std::max(c->u_cap, c->n_user));
     if (rc) { free_table(c); return rc; }
     c->n_sample = S;
     c->h_ranks.assign(ranks, ranks + S);
@@ -774,7 +810,7 @@ int rkr_set_table(rkr_ctx *c, const int32_t *ranks, int32_t S, const float *tabl
     int rc = dev_alloc_t(c, &c->ranks, (size_t)S, "ranks");
     if (rc) return rc;
     rc = dev_alloc_t(c, &c->table, (size_t)std::max(c->u_cap, c->n_user) * S, "table");
-    if (!rc) rc = dev_alloc_t(c, &c->gvals, (size_t)std::max(c->u_cap, c->n_user) * kGuardRow, "guard values");
+    if (!rc) rc = alloc_guards(c, std::max(c->u_cap, c->n_user));
     if (rc) { free_table(c); return rc; }
     c->n_sample = S;
     c->h_ranks.assign(ranks, ranks + S);
@@ -1341,27 +1377,45 @@ int validate_queries(Ctx *c, const DataSnap &d, const float *queries, int32_t n_
 
 namespace {
 
-// a coarse list longer than max(kCoarseRefineMin, U / 64) gets a second pass:
-// the pass costs about a user row per query, an exact-scored entry about a
-// user row per entry, and the pass narrows a list several times over
-constexpr int64_t kCoarseRefineMin = 4096;
 // users per chunk of the coarse histograms and of the list's chunk-major
-// order: at 1M x 50k (1000 queries) 4096, 8192, 16384 and 65536 ran at 258k,
-// 280k, 285k and 279k queries/s (small chunks cost histogram workgroups,
-// large ones the exact pass's reuse of user rows within a chunk)
+// order (batches with updates pending): at 1M x 50k (1000 queries) 4096, 8192,
+// 16384 and 65536 ran at 258k, 280k, 285k and 279k queries/s (small chunks
+// cost histogram workgroups, large ones the exact pass's reuse of user rows
+// within a chunk)
 constexpr int64_t kCoarseChunk = 16384;
 constexpr int32_t kCoarseMinBatch = 8;
 
-// Device batches of query_on_slot.  allow_coarse: screened-form exact batches
-// take the coarse bounds; queries whose coarse list would be empty of a k-th
-// bound or too long are appended to *fallback (indices into queries) with
-// their outputs left unwritten.
+// Every stride-th user is sampled for the list thresholds: all of up to 16,384
+// users (the threshold is then exact), else a sixteenth of them, at least
+// 16,384 and at most 65,536.
+int64_t sample_stride(int64_t U) {
+    const int64_t n = std::min<int64_t>(std::max<int64_t>(U / 16, 16384), 65536);
+    return std::max<int64_t>(1, U / n);
+}
+
+// List entries of a batch of nq queries: a list is a few hundred users at the
+// median and up to a quarter of them for a query that many users rank first
+// (longer ones take the full search, as estimated lists past half the entries
+// do).  A list entry costs kListBytes with the candidate and refine row it may
+// become.
+constexpr int64_t kListBytes = 4 * 9;
+int64_t list_entries(int64_t U, int64_t nq) {
+    const int64_t per = std::min<int64_t>(std::max<int64_t>(U / 64, 4096), 16384);
+    return std::min<int64_t>({std::max<int64_t>(nq * per, 2 * std::max<int64_t>(4096, U / 4)), nq * U, INT32_MAX / 2});
+}
+
+// Device batches of query_on_slot.  allow_list: exact batches take the
+// threshold lists (k_list.hip), or, with updates pending, the coarse bounds;
+// queries those cannot answer (no threshold, a list too long or too short) are
+// appended to *fallback (indices into queries) with their outputs left
+// unwritten.
 int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int32_t n_query, const int32_t *topk,
                 int32_t max_k, int32_t *out_user, int32_t *out_rank, float *out_qip, rkr_query_stats *stats,
-                rkr_batch_timing &tm, bool allow_coarse, std::vector<int32_t> *fallback) {
+                rkr_batch_timing &tm, bool allow_list, std::vector<int32_t> *fallback) {
     const int64_t U = dv.n_user, I = dv.n_item;
     const int32_t ld = c->ld, d = c->dim;
     const int mode = c->output;
+    const bool screened = c->form == RKR_FORM_SCREENED;
     // exact output searches the query table when there is one (exact under
     // the score rule, eps 0); reference output keeps the sampled table
     const bool use_q = mode == RKR_OUTPUT_EXACT && dv.qtable;
@@ -1374,8 +1428,9 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // the QSRP screen (RKR_OPT_QSRP, built by rkr_qsrp_build) replaces the bound
     // stage of exact batches without pending updates
     const bool qsrp = c->qsrp && dv.qsrp_users && mode == RKR_OUTPUT_EXACT && !upd && U > 0;
-    const bool coarse = !qsrp && allow_coarse && c->coarse && c->form == RKR_FORM_SCREENED &&
-                        mode == RKR_OUTPUT_EXACT && c->kp > 0 && dv.user_norm && dv.n_guard > 0 && U > 0;
+    const bool listable = !qsrp && allow_list && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
+                          dv.guards.n > 0 && U > 0;
+    const bool mfma = screened && c->kp > 0 && dv.user_norm;
     const size_t pair_bytes = upd ? 12 : 8;  // <u,q> + buckets, or + two bound values
 
     // queries per device batch
@@ -1387,71 +1442,76 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         nqb = std::min<int64_t>(nqb, n_query);
         nqb = std::min<int64_t>(nqb, 65535);
     }
+    // The lists, for the screened form and for enough pairs that the search
+    // they spare (one user's table row per query, or per batch of 4 and more)
+    // outweighs their three launches of about 5 us: at 64k users one plain
+    // query is even, and batches of 8 at 4k users.
+    const bool list = listable && !upd &&
+                      (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
+    const bool list_mfma = list && mfma;
     int rc;
-    if ((rc = ensure(c, sl.q_in, sizeof(float) * (size_t)nqb * ld, "query vectors"))) return rc;
+    const BatchIo io_max(nqb, ld, max_k);
+    if ((rc = ensure(c, sl.io, io_max.end, "queries and outputs"))) return rc;
     if ((rc = ensure(c, sl.qip, sizeof(float) * (size_t)nqb * U, "query scores"))) return rc;
     // coarse bucket rows: whole row blocks of 128 users, plus a spare row
     const int64_t ldc = (U + 127) / 128 * 128;
-    if ((rc = ensure(c, sl.bk, std::max((pair_bytes - 4) * (size_t)U * nqb, (size_t)ldc * (nqb + 1)),
-                     "bucket pairs")))
+    if (!list && (rc = ensure(c, sl.bk, std::max((pair_bytes - 4) * (size_t)U * nqb, (size_t)ldc * (nqb + 1)),
+                              "bucket pairs")))
         return rc;
-    if ((rc = ensure(c, sl.qinfo, sizeof(QueryInfo) * (size_t)nqb + 64, "query info"))) return rc;
-    if ((rc = ensure(c, sl.out, (sizeof(int32_t) * 2 + sizeof(float)) * (size_t)nqb * max_k, "outputs"))) return rc;
     if ((rc = ensure(c, sl.hist, sizeof(uint32_t) * hist_words((int32_t)nqb, S), "bound histograms"))) return rc;
     if (qsrp && (rc = ensure(c, sl.q_split, sizeof(float) * (size_t)nqb * (dv.qsrp_ldr + 3), "QSRP query rows")))
         return rc;
-    GuardCols gc{};
-    if (coarse) {
-        if ((rc = ensure(c, sl.q_split, (sizeof(uint16_t) * 2 * c->kp + 2 * sizeof(float)) * (size_t)nqb, "query BF16 rows")))
-            return rc;
-        for (int j = 0; j < dv.n_guard; ++j) gc.col[j] = dv.gcol[j];
-        gc.n = dv.n_guard;
-    }
-    // ranks of the searched table's columns (guard placement; the coarse
-    // bounds and the update path run in exact output only, which searches the
-    // query table when there is one)
+    if (listable && mfma &&
+        (rc = ensure(c, sl.q_split, (sizeof(uint16_t) * 2 * c->kp + 2 * sizeof(float)) * (size_t)nqb, "query BF16 rows")))
+        return rc;
+    // ranks of the searched table's columns (guard placement; the lists and
+    // the update path run in exact output only, which searches the query
+    // table when there is one)
     const std::vector<int32_t> &hrk = *dv.hrk;
-    // coarse lists longer than refine_min get a second, finer pass; a list
-    // longer than coarse_cap takes the full path instead
-    const int64_t coarse_cap = std::max<int64_t>(4096, U / 4);
-    const int64_t refine_min = std::max<int64_t>(kCoarseRefineMin, U / 64);
-
-    // pinned staging: queries | query info | outputs (the device layout of
-    // sl.out) | coarse rows, bin counts, guard sets, maps | recheck counts,
-    // scalars; sections 256-byte aligned
-    const size_t out_words = 3 * (size_t)nqb * max_k;
-    size_t sz[10] = {sizeof(float) * (size_t)nqb * ld, sizeof(QueryInfo) * (size_t)nqb, 4 * out_words,
-                     sizeof(int32_t) * 4 * (size_t)nqb, sizeof(int32_t) * 8 * (size_t)nqb, sizeof(GuardCols) * 8,
-                     sizeof(int32_t) * 3 * (size_t)nqb, sizeof(int32_t) * (size_t)nqb, 64, 0};
-    size_t off[10], tot = 0;
-    for (int i = 0; i < 10; ++i) {
-        off[i] = tot;
-        tot += (sz[i] + 255) & ~(size_t)255;
+    const GuardCols &gc = dv.guards;
+    // an (estimated) list longer than list_max takes the full path instead
+    const int64_t list_max = std::max<int64_t>(4096, U / 4);
+    int64_t list_cap = 0;
+    if (list) {
+        // what is held already, or what a quarter of the free budget allows
+        const int64_t avail = (int64_t)((c->budget > c->held ? c->budget - c->held : 0) / 4);
+        const int64_t have = (int64_t)std::min({sl.list.bytes / 12, sl.cand.bytes / 8, sl.refine_idx.bytes / 16});
+        list_cap = std::min<int64_t>(list_entries(U, nqb), std::max<int64_t>({have, avail / kListBytes, 1}));
+        if ((rc = ensure(c, sl.list, 12 * (size_t)list_cap, "listed pairs")) ||
+            (rc = ensure(c, sl.list_info, sizeof(uint32_t) * (66 * (size_t)nqb + 64), "list thresholds")) ||
+            (rc = ensure(c, sl.cand, sizeof(int32_t) * 2 * (size_t)list_cap, "candidates")) ||
+            (rc = ensure(c, sl.refine_idx, sizeof(int32_t) * 4 * (size_t)list_cap, "refine rows")))
+            return rc;
     }
-    if ((rc = ensure_pinned(c, sl.stage, tot))) return rc;
+
+    // pinned staging: the batch's transfer layout | coarse rows and bin counts
+    const size_t stage_io = (io_max.end + 255) & ~(size_t)255;
+    if ((rc = ensure_pinned(c, sl.stage, stage_io + sizeof(int32_t) * 12 * (size_t)nqb))) return rc;
     char *stg = reinterpret_cast<char *>(sl.stage.p);
-    float *hq = reinterpret_cast<float *>(stg + off[0]);
-    QueryInfo *hqi = reinterpret_cast<QueryInfo *>(stg + off[1]);
-    int32_t *ho_user = reinterpret_cast<int32_t *>(stg + off[2]);
-    int32_t *ho_rank = ho_user + (size_t)nqb * max_k;
-    float *ho_qip = reinterpret_cast<float *>(ho_rank + (size_t)nqb * max_k);
-    int32_t *hcq = reinterpret_cast<int32_t *>(stg + off[3]);
-    int32_t *hhc = reinterpret_cast<int32_t *>(stg + off[4]);
-    GuardCols *hsets = reinterpret_cast<GuardCols *>(stg + off[5]);
-    int32_t *hgset = reinterpret_cast<int32_t *>(stg + off[6]);  // then qmap, qset
-    int32_t *h_qrecheck = reinterpret_cast<int32_t *>(stg + off[7]);
-    int32_t *h_scalars = reinterpret_cast<int32_t *>(stg + off[8]);  // refine total, recheck count, error bits
+    int32_t *hcq = reinterpret_cast<int32_t *>(stg + stage_io);
+    int32_t *hhc = hcq + 4 * (size_t)nqb;
 
     for (int64_t q0 = 0; q0 < n_query; q0 += nqb) {
         const int32_t nq = (int32_t)std::min<int64_t>(nqb, n_query - q0);
-        float *q_in = reinterpret_cast<float *>(sl.q_in.p);
+        const BatchIo io(nq, ld, max_k);
+        char *dev = reinterpret_cast<char *>(sl.io.p);
+        float *q_in = reinterpret_cast<float *>(dev);
+        QueryInfo *qi = reinterpret_cast<QueryInfo *>(dev + io.info);
+        int32_t *q_recheck = reinterpret_cast<int32_t *>(dev + io.recheck);
+        ListCounters *ctr = reinterpret_cast<ListCounters *>(dev + io.counters);
+        int32_t *o_user = reinterpret_cast<int32_t *>(dev + io.out);
+        int32_t *o_rank = o_user + (size_t)nq * max_k;
+        float *o_qip = reinterpret_cast<float *>(o_rank + (size_t)nq * max_k);
+        int32_t *refine_total = &ctr->n_refine;
+        float *hq = reinterpret_cast<float *>(stg);
+        QueryInfo *hqi = reinterpret_cast<QueryInfo *>(stg + io.info);
+        const int32_t *h_qrecheck = reinterpret_cast<const int32_t *>(stg + io.recheck);
+        const ListCounters *hctr = reinterpret_cast<const ListCounters *>(stg + io.counters);
+        const int32_t *ho_user = reinterpret_cast<const int32_t *>(stg + io.out);
+        const int32_t *ho_rank = ho_user + (size_t)nq * max_k;
+        const float *ho_qip = reinterpret_cast<const float *>(ho_rank + (size_t)nq * max_k);
         float *qip = reinterpret_cast<float *>(sl.qip.p);
         uint32_t *bk = reinterpret_cast<uint32_t *>(sl.bk.p);
-        QueryInfo *qi = reinterpret_cast<QueryInfo *>(sl.qinfo.p);
-        int32_t *refine_total = reinterpret_cast<int32_t *>(reinterpret_cast<char *>(sl.qinfo.p) + sizeof(QueryInfo) * nqb);
-        int32_t *o_user = reinterpret_cast<int32_t *>(sl.out.p);
-        int32_t *o_rank = o_user + (size_t)nqb * max_k;
-        float *o_qip = reinterpret_cast<float *>(o_rank + (size_t)nqb * max_k);
 
         float q_amax = 0.0f;  // largest |query value| of the batch (validated finite)
         for (int32_t i = 0; i < nq; ++i) {
@@ -1465,46 +1525,59 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             hqi[i] = QueryInfo{};
             hqi[i].topk = topk[q0 + i];
         }
+        std::memset(stg + io.recheck, 0, io.out - io.recheck);
         RKR_HIP(c, hipEventRecord(sl.ev[0], sl.stream));
-        RKR_HIP(c, hipMemcpyAsync(q_in, hq, sizeof(float) * (size_t)nq * ld, hipMemcpyHostToDevice, sl.stream));
-        RKR_HIP(c, hipMemcpyAsync(qi, hqi, sizeof(QueryInfo) * nq, hipMemcpyHostToDevice, sl.stream));
+        RKR_HIP(c, hipMemcpyAsync(dev, stg, io.out, hipMemcpyHostToDevice, sl.stream));
         RKR_HIP(c, hipEventRecord(sl.ev[1], sl.stream));
         int32_t *lbv = reinterpret_cast<int32_t *>(bk);
         int32_t *ubv = lbv + (size_t)nq * U;
         const int64_t cu = chunk_users(U, nq, c->n_cu);
         uint32_t *ghist = reinterpret_cast<uint32_t *>(sl.hist.p);
-        // a few queries are answered faster by the full path: the coarse
-        // kernel converts every user row once per launch
-        const bool coarse_b = coarse && nq >= kCoarseMinBatch;
-        int32_t *cl_u = nullptr, *cl_b = nullptr;
+        // a few queries with updates pending are answered faster by the full
+        // path: the coarse kernel converts every user row once per launch
+        const bool coarse = listable && upd && mfma && nq >= kCoarseMinBatch;
+        uint16_t *q_hi = reinterpret_cast<uint16_t *>(sl.q_split.p);
+        uint16_t *q_lo = q_hi + (size_t)nqb * c->kp;
+        float *qn = reinterpret_cast<float *>(q_lo + (size_t)nqb * c->kp);
+        float *qcs = qn + nqb;  // error scales of the one-product estimate
+        // e = C ||u|| cs + floor, C = 1 + 2^-20 covering the FP32 evaluation of
+        // that product and sum
+        const float est_C = 1.0f + 0x1p-20f;
+        const float est_floor = std::nextafter(
+            (float)(((double)screen_abs_floor(c->kp, dv.max_abs_user, q_amax) + (double)eps) * (1.0 + std::ldexp(1.0, -18))),
+            INFINITY);
+        ListLaunch LL{};
         uint32_t *bk_c = nullptr;
-        float *s_c = nullptr;
-        int64_t n_listed = 0;             // the list length, or a bound on it when dev_lists
-        bool dev_lists = false;           // the lists' true length and fallbacks are on the device
-        int32_t *d_list_n = nullptr;      // the list length (device), when dev_lists
-        int32_t *cq_dev = nullptr;        // the coarse per-query records (device)
         std::vector<int32_t> deep_check;  // update path: queries listed without the deepest bin
-        if (coarse_b) {
+        if (list) {
+            LL.n_user = U; LL.nq = nq; LL.S = S; LL.Kp = c->kp; LL.n_cu = c->n_cu;
+            LL.user_hi = dv.user_hi; LL.user_norm = dv.user_norm; LL.gvals = dv.gvals; LL.gcols = dv.gcols; LL.pitch = dv.gpitch;
+            LL.q_hi = q_hi; LL.q_cs = qcs; LL.fc = dv.fine; LL.C = est_C; LL.floor = est_floor; LL.eps = eps;
+            LL.qip = qip; LL.stride = sample_stride(U); LL.cap = list_max; LL.list_cap = list_cap;
+            LL.hist = reinterpret_cast<uint32_t *>(sl.list_info.p);
+            LL.order = reinterpret_cast<int32_t *>(LL.hist + 64 * (size_t)nq);
+            LL.colg = LL.order + nq;
+            LL.qi = qi; LL.ctr = ctr; LL.ghist = ghist;
+            LL.cl_u = reinterpret_cast<int32_t *>(sl.list.p);
+            LL.cl_b = LL.cl_u + list_cap;
+            bk_c = reinterpret_cast<uint32_t *>(LL.cl_b + list_cap);
+        }
+        if (list_mfma) {
+            RKR_HIP(c, launch_prep_items(sl.stream, q_in, nq, ld, d, c->kp, q_hi, q_lo, qn, qcs, dv.rho, c->coarse_g1,
+                                         c->coarse_grule, LL.hist));
+            RKR_HIP(c, launch_list_screen(sl.stream, LL));
+            RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
+            RKR_HIP(c, launch_list_exact(sl.stream, LL, dv.users, q_in, ld, d, T, false, bk_c));
+            RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+        } else if (coarse) {
             // coarse buckets on the matrix cores, the coarse k-th bound and
-            // list sizes; exact scores and bucket pairs of the listed users
-            uint16_t *q_hi = reinterpret_cast<uint16_t *>(sl.q_split.p);
-            uint16_t *q_lo = q_hi + (size_t)nqb * c->kp;
-            float *qn = reinterpret_cast<float *>(q_lo + (size_t)nqb * c->kp);
-            float *qcs = qn + nqb;  // the first pass's error scales
+            // list sizes; exact scores and bound values of the listed users
             RKR_HIP(c, launch_prep_items(sl.stream, q_in, nq, ld, d, c->kp, q_hi, q_lo, qn, qcs, dv.rho, c->coarse_g1,
                                          c->coarse_grule));
-            const double mq = q_amax;
-            const double absf = ((double)screen_abs_floor(c->kp, dv.max_abs_user, mq) + (double)eps) *
-                                (1.0 + std::ldexp(1.0, -18));
             uint8_t *cb = reinterpret_cast<uint8_t *>(bk);
             CoarseLaunch L{};
-            L.users = dv.users; L.user_norm = dv.user_norm; L.table = T; L.gvals = dv.gvals; L.n_user = U; L.S = S;
-            L.gc = gc;
-            L.user_hi = dv.user_hi; L.user_lo = dv.user_lo;
-            // first pass: e = C ||u|| cs + floor, C = 1 + 2^-20 covering the
-            // FP32 evaluation of that product and sum
-            L.q_hi = q_hi; L.q_lo = q_lo; L.q_norm = qcs; L.qmap = nullptr; L.nq = nq; L.ld = ld; L.K = d;
-            L.Kp = c->kp; L.C = 1.0f + 0x1p-20f; L.abs_floor = std::nextafter((float)absf, INFINITY); L.cb = cb;
+            L.user_norm = dv.user_norm; L.gvals = dv.gvals; L.user_hi = dv.user_hi; L.n_user = U; L.gc = gc;
+            L.q_hi = q_hi; L.q_cs = qcs; L.nq = nq; L.Kp = c->kp; L.C = est_C; L.abs_floor = est_floor; L.cb = cb;
             L.ldc = ldc; L.spare_row = nqb;
             L.grid_cap = (int64_t)c->n_cu * coarse_first_pass_wgs(c->kp / 32);
             RKR_HIP(c, launch_ip_coarse(sl.stream, L));
@@ -1513,36 +1586,30 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // still fill the device and the list stays chunk-major
             const int64_t ccu = kCoarseChunk;
             const int64_t n_chunk = (U + ccu - 1) / ccu;
-            // part | cq | loc | ctot | cbase | guard sets | gset | qmap | qset
-            const size_t w_sets = sizeof(GuardCols) * 8 / 4;
-            if ((rc = ensure(c, sl.coarse_info, sizeof(uint32_t) * (17 * (size_t)nq * n_chunk + 15 * (size_t)nqb +
-                                                                   2 * (size_t)n_chunk + w_sets + 64),
+            // part | cq | loc | ctot | cbase | hcnt
+            if ((rc = ensure(c, sl.list_info, sizeof(uint32_t) * (17 * (size_t)nq * n_chunk + 12 * (size_t)nqb +
+                                                                  2 * (size_t)n_chunk + 64),
                              "coarse counts")))
                 return rc;
-            uint32_t *part = reinterpret_cast<uint32_t *>(sl.coarse_info.p);
+            uint32_t *part = reinterpret_cast<uint32_t *>(sl.list_info.p);
             int32_t *cq = reinterpret_cast<int32_t *>(part + 16 * (size_t)nq * n_chunk);
-            cq_dev = cq;
             int32_t *loc = cq + 4 * (size_t)nqb;
             int32_t *ctot = loc + (size_t)nq * n_chunk;
             int32_t *cbase = ctot + n_chunk;
-            GuardCols *gsets = reinterpret_cast<GuardCols *>(cbase + n_chunk);
-            int32_t *gset = reinterpret_cast<int32_t *>(gsets + 8);
-            int32_t *qmap = gset + nqb;  // then qset (nqb)
-            int32_t *hcnt = qmap + 2 * (size_t)nqb;
-            RKR_HIP(c, launch_coarse_kth(sl.stream, cb, ldc, U, nq, ccu, dv.n_guard, nullptr, part, qi, cq, hcnt));
+            int32_t *hcnt = cbase + n_chunk;
+            RKR_HIP(c, launch_coarse_kth(sl.stream, cb, ldc, U, nq, ccu, gc.n, part, qi, cq, hcnt));
             RKR_HIP(c, hipMemcpyAsync(hcq, cq, sizeof(int32_t) * 4 * nq, hipMemcpyDeviceToHost, sl.stream));
-            if (upd)
-                RKR_HIP(c, hipMemcpyAsync(hhc, hcnt, sizeof(int32_t) * 8 * nq, hipMemcpyDeviceToHost, sl.stream));
+            RKR_HIP(c, hipMemcpyAsync(hhc, hcnt, sizeof(int32_t) * 8 * nq, hipMemcpyDeviceToHost, sl.stream));
             RKR_HIP(c, hipStreamSynchronize(sl.stream));
-            if (upd) {
-                // pending inserts move ranks: a user at or above guard m has
-                // rank <= R[j_m] + ins_gmax[m], so the k-th bound is at most
-                // V = R[j_beta] + ins_gmax[beta]; a user below guard c_hi - 1
-                // has rank >= R[j_{c_hi - 1}] + 1 - n_del, and is listed when
-                // that can be <= V
-                for (int32_t i = 0; i < nq; ++i) {
-                    int32_t *e = &hcq[(size_t)i * 4];
-                    if (e[0] < 0) continue;
+            int64_t n_listed = 0;
+            for (int32_t i = 0; i < nq; ++i) {
+                int32_t *e = &hcq[(size_t)i * 4];
+                if (e[0] >= 0) {
+                    // pending inserts move ranks: a user at or above guard m has
+                    // rank <= R[j_m] + ins_gmax[m], so the k-th bound is at most
+                    // V = R[j_beta] + ins_gmax[beta]; a user below guard c_hi - 1
+                    // has rank >= R[j_{c_hi - 1}] + 1 - n_del, and is listed when
+                    // that can be <= V
                     const int64_t V = (int64_t)hrk[gc.col[e[0]]] + dv.ins_gmax[e[0]];
                     int32_t bl = 0;
                     while (bl < gc.n && (int64_t)hrk[gc.col[bl]] + 1 - dv.n_del <= V) ++bl;
@@ -1558,124 +1625,31 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                     e[0] = bl;
                     e[1] = (int32_t)std::min<int64_t>(n, INT32_MAX);
                 }
+                if (e[0] < 0 || e[1] > list_max) {
+                    if (fallback) fallback->push_back((int32_t)(q0 + i));
+                    tm.n_fallback += 1;
+                    e[0] = -1;
+                    e[1] = 0;
+                }
+                e[2] = (int32_t)n_listed;
+                e[3] = 0;
+                n_listed += e[1];
             }
-            // second pass for long lists: the queries whose k-th bound fell in
-            // guard bin beta are bucketed again against up to 7 columns inside
-            // that bin (the bin's last column included), spaced geometrically
-            // in rank
-            std::vector<GuardCols> sets{gc};
-            std::vector<int32_t> hqmap;
-            for (int32_t i = 0; i < nq; ++i) hgset[i] = 0;
-            std::vector<std::pair<int32_t, int32_t>> groups;  // (set, first index in hqmap)
-            // (not with pending updates: the rank shift bounds are kept for
-            // the first pass's guards only)
-            std::vector<int32_t> set_ids;  // guard-row set of each second-pass set
-            for (int32_t beta = 0; beta < gc.n && !upd; ++beta) {
-                const GuardCols &g2 = dv.gsets.set[1 + beta];
-                if (g2.n == 0) continue;
-                const size_t first = hqmap.size();
-                for (int32_t i = 0; i < nq; ++i)
-                    if (hcq[(size_t)i * 4] == beta && hcq[(size_t)i * 4 + 1] > refine_min) hqmap.push_back(i);
-                if (hqmap.size() == first) continue;
-                for (size_t t = first; t < hqmap.size(); ++t) hgset[hqmap[t]] = (int32_t)sets.size();
-                groups.push_back({(int32_t)sets.size(), (int32_t)first});
-                sets.push_back(g2);
-                set_ids.push_back(1 + beta);
-            }
-            // With a second pass the lists stay on the device: the batch goes
-            // on without reading the new counts.  A second-pass list is a
-            // subset of the query's first-pass list (its guards lie inside the
-            // bin that held the k-th bound), so the first-pass lengths bound
-            // the list; k_coarse_mark sends a query whose list exceeds its
-            // bound or the cap to the full path, and the final counts and
-            // those queries are read with the outputs.
-            dev_lists = !groups.empty();
-            if (dev_lists) {
-                const int32_t nr = (int32_t)hqmap.size();
-                for (int32_t i = 0; i < nq; ++i) {
-                    int32_t *e = &hcq[(size_t)i * 4];
-                    const int32_t b1 = e[0] >= 0 ? (int32_t)std::min<int64_t>(e[1], coarse_cap) : 0;
-                    e[2] = b1;  // field 2 carries the bound to k_coarse_mark
-                    n_listed += b1;
-                }
-                // one launch for every refined query: set of each (local)
-                // query in qset; every set is uploaded once, set 0 (the first
-                // pass's guards) first, and the second pass reads from set 1
-                int32_t *h_map = hgset + nqb, *h_set = h_map + nr;
-                for (int32_t t = 0; t < nr; ++t) {
-                    h_map[t] = hqmap[t];
-                    h_set[t] = hgset[hqmap[t]] - 1;
-                }
-                for (size_t t = 0; t < sets.size(); ++t) hsets[t] = sets[t];
-                int32_t *qset = qmap + nr;
-                RKR_HIP(c, hipMemcpyAsync(cq, hcq, sizeof(int32_t) * 4 * nq, hipMemcpyHostToDevice, sl.stream));
-                RKR_HIP(c, hipMemcpyAsync(qmap, h_map, sizeof(int32_t) * 2 * nr, hipMemcpyHostToDevice, sl.stream));
-                RKR_HIP(c, hipMemcpyAsync(gsets, hsets, sizeof(GuardCols) * sets.size(), hipMemcpyHostToDevice,
-                                          sl.stream));
-                CoarseLaunch L2 = L;
-                L2.C = c->screen_C;  // the second pass's three-product estimate
-                L2.q_norm = qn;
-                L2.grid_cap = (int64_t)c->n_cu * 3;
-                L2.qmap = qmap;
-                L2.nq = nr;
-                L2.sets = gsets + 1;
-                L2.qset = qset;
-                L2.n_sets = (int32_t)sets.size() - 1;
-                for (int32_t t = 0; t < L2.n_sets; ++t) L2.set_id[t] = set_ids[t];
-                RKR_HIP(c, launch_ip_coarse(sl.stream, L2));
-                for (size_t gi = 0; gi < groups.size(); ++gi) {
-                    const int32_t first = groups[gi].second;
-                    const int32_t end = gi + 1 < groups.size() ? groups[gi + 1].second : nr;
-                    RKR_HIP(c, launch_coarse_kth(sl.stream, cb, ldc, U, end - first, ccu, sets[groups[gi].first].n,
-                                                 qmap + first, part, qi, cq, hcnt));
-                }
-                RKR_HIP(c, launch_coarse_mark(sl.stream, cq, nq, coarse_cap));
-                tm.n_coarse_refined += (int64_t)hqmap.size();
-            } else {
-                for (int32_t i = 0; i < nq; ++i) {
-                    int32_t *e = &hcq[(size_t)i * 4];
-                    if (e[0] < 0 || e[1] > coarse_cap) {
-                        if (fallback) fallback->push_back((int32_t)(q0 + i));
-                        tm.n_fallback += 1;
-                        e[0] = -1;
-                        e[1] = 0;
-                    }
-                    e[2] = (int32_t)n_listed;
-                    e[3] = 0;
-                    n_listed += e[1];
-                }
-                tm.n_listed += n_listed;
-            }
+            tm.n_listed += n_listed;
             if (n_listed >= INT32_MAX) return set_err(c, RKR_ERR_NOMEM, "query: coarse list exceeds 2^31; lower the query batch");
-            if ((rc = ensure(c, sl.coarse_list, 16 * (size_t)std::max<int64_t>(n_listed, 1), "coarse list"))) return rc;
-            cl_u = reinterpret_cast<int32_t *>(sl.coarse_list.p);
-            cl_b = cl_u + std::max<int64_t>(n_listed, 1);
-            bk_c = reinterpret_cast<uint32_t *>(cl_b + std::max<int64_t>(n_listed, 1));
-            s_c = reinterpret_cast<float *>(bk_c + std::max<int64_t>(n_listed, 1));
-            if (!dev_lists) {
-                for (size_t t = 0; t < sets.size(); ++t) hsets[t] = sets[t];
-                RKR_HIP(c, hipMemcpyAsync(cq, hcq, sizeof(int32_t) * 4 * nq, hipMemcpyHostToDevice, sl.stream));
-                RKR_HIP(c, hipMemcpyAsync(gsets, hsets, sizeof(GuardCols) * sets.size(), hipMemcpyHostToDevice,
-                                          sl.stream));
-            }
-            RKR_HIP(c, hipMemcpyAsync(gset, hgset, sizeof(int32_t) * nq, hipMemcpyHostToDevice, sl.stream));
-            d_list_n = dev_lists ? hcnt + 8 * (size_t)nqb : nullptr;  // in the spare words of coarse_info
-            RKR_HIP(c, launch_coarse_compact(sl.stream, cb, ldc, U, nq, ccu, part, cq, loc, ctot, cbase, cl_u, cl_b,
-                                             d_list_n));
-            if (upd) {
-                // bound values of the listed pairs only (the rest are ruled
-                // out), then the value selection of the update path; the
-                // bound arrays reuse the coarse rows, read by now
-                RKR_HIP(c, hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(lbv), kNoBound, 2 * (size_t)nq * U,
-                                             sl.stream));
-                RKR_HIP(c, launch_coarse_exact_upd(sl.stream, dv.users, q_in, ld, d, T, S, R, dv.n_item_base, eps, gsets,
-                                                   gset, cl_u, cl_b, n_listed, dv.side_ins, dv.n_ins, dv.ld_ins,
-                                                   dv.side_del, dv.n_del, dv.ld_del, U, lbv, ubv, qip));
-                RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));
-            } else {
-                RKR_HIP(c, launch_coarse_exact(sl.stream, dv.users, q_in, ld, d, T, S, R, I, eps, gsets, gset, nq, cl_u,
-                                               cl_b, n_listed, d_list_n, bk_c, s_c, ghist, qi));
-            }
+            if ((rc = ensure(c, sl.list, 8 * (size_t)std::max<int64_t>(n_listed, 1), "coarse list"))) return rc;
+            int32_t *cl_u = reinterpret_cast<int32_t *>(sl.list.p);
+            int32_t *cl_b = cl_u + std::max<int64_t>(n_listed, 1);
+            RKR_HIP(c, hipMemcpyAsync(cq, hcq, sizeof(int32_t) * 4 * nq, hipMemcpyHostToDevice, sl.stream));
+            RKR_HIP(c, launch_coarse_compact(sl.stream, cb, ldc, U, nq, ccu, part, cq, loc, ctot, cbase, cl_u, cl_b));
+            // bound values of the listed pairs only (the rest are ruled
+            // out), then the value selection of the update path; the
+            // bound arrays reuse the coarse rows, read by now
+            RKR_HIP(c, hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(lbv), kNoBound, 2 * (size_t)nq * U, sl.stream));
+            RKR_HIP(c, launch_coarse_exact_upd(sl.stream, dv.users, q_in, ld, d, T, S, R, dv.n_item_base, eps, gc, cl_u,
+                                               cl_b, n_listed, dv.side_ins, dv.n_ins, dv.ld_ins, dv.side_del, dv.n_del,
+                                               dv.ld_del, U, lbv, ubv, qip));
+            RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));
             RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
         } else if (qsrp) {
             // QSRP screen: rotated queries and their part norms, the left-part
@@ -1684,17 +1658,17 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // over those, then the exact score and table search for the users
             // they keep, and the k-th bound again (the exact path's from here)
             float *qrot = reinterpret_cast<float *>(sl.q_split.p);
-            float *qn = qrot + (size_t)nqb * dv.qsrp_ldr;
+            float *qpn = qrot + (size_t)nqb * dv.qsrp_ldr;
             RKR_HIP(c, launch_scores_store(sl.stream, q_in, nq, ld, dv.qsrp_rot, d, ld, d, qrot,
                                            dv.qsrp_ldr, true));
-            RKR_HIP(c, launch_qsrp_qnorms(sl.stream, qrot, dv.qsrp_ldr, q_in, ld, d, dv.qsrp_cd, nq, qn));
+            RKR_HIP(c, launch_qsrp_qnorms(sl.stream, qrot, dv.qsrp_ldr, q_in, ld, d, dv.qsrp_cd, nq, qpn));
             RKR_HIP(c, launch_scores_store(sl.stream, dv.qsrp_users, U, dv.qsrp_ldr, qrot, nq, dv.qsrp_ldr,
                                            dv.qsrp_cd, qip, U, false));
             RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
             // eps widens the interval as the exact path widens its search; the
             // floor covers gradual underflow in the d products of a score
             const float absf = std::nextafter((float)((double)eps + (double)d * std::ldexp(1.0, -140)), INFINITY);
-            RKR_HIP(c, launch_qsrp_bounds(sl.stream, qip, U, nq, dv.qsrp_par, qn, dv.qsrp_gcd, dv.qsrp_crot, absf,
+            RKR_HIP(c, launch_qsrp_bounds(sl.stream, qip, U, nq, dv.qsrp_par, qpn, dv.qsrp_gcd, dv.qsrp_crot, absf,
                                           dv.n_sample, use_q ? dv.qcol : nullptr, S, bk));
             RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode, 0, cu, ghist, qi));
             RKR_HIP(c, launch_qsrp_exact(sl.stream, dv.users, q_in, ld, d, T, S, eps, U, nq, qi, qip, bk));
@@ -1706,27 +1680,35 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip));
             else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false));
             RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
-            if (upd)
+            if (list) {
+                RKR_HIP(c, hipMemsetAsync(LL.hist, 0, sizeof(uint32_t) * 64 * (size_t)nq, sl.stream));
+                RKR_HIP(c, launch_list_scores(sl.stream, LL));
+                RKR_HIP(c, launch_list_exact(sl.stream, LL, dv.users, q_in, ld, d, T, true, bk_c));
+                RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+            } else if (upd) {
                 RKR_HIP(c, launch_bounds_upd(sl.stream, qip, T, U, S, R, dv.n_item_base, eps, dv.side_ins,
                                              dv.n_ins, dv.ld_ins, dv.side_del, dv.n_del, dv.ld_del, nq, lbv, ubv));
-            else
+                RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+                RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));
+            } else {
                 RKR_HIP(c, launch_bounds(sl.stream, qip, T, U, S, nq, eps, mode == RKR_OUTPUT_REFERENCE ? 1 : 0, bk));
-            RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
-            if (upd) RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));
-            else
+                RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
                 RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode,
                                            (mode == RKR_OUTPUT_EXACT && eps == 0.0f) ? 1 : 0, cu, ghist, qi));
+            }
         }
-        RKR_HIP(c, launch_offsets(sl.stream, qi, nq, refine_total));
-        // Coarse bounds without pending updates: every candidate is a listed
-        // pair, so the list length bounds the candidate and refine arrays and
-        // the batch goes on without waiting for the counts (the refinement and
-        // top-k read them on the device).  Otherwise the counts size them.
-        const bool sized_by_list = coarse_b && !upd;
-        int64_t total = n_listed, total_cand = n_listed;
-        if (!sized_by_list) {
+        // With lists every candidate is a listed pair, so the list's entries
+        // bound the candidate and refine arrays and the batch goes on without
+        // waiting for the counts (the refinement and top-k read them on the
+        // device).  Otherwise the counts size them.
+        int64_t total = list_cap, total_cand = list_cap;
+        if (!list) {
+            RKR_HIP(c, launch_offsets(sl.stream, qi, nq, refine_total));
             RKR_HIP(c, hipMemcpyAsync(hqi, qi, sizeof(QueryInfo) * nq, hipMemcpyDeviceToHost, sl.stream));
             RKR_HIP(c, hipStreamSynchronize(sl.stream));
+            total = hqi[nq - 1].cand_off + hqi[nq - 1].n_settled + hqi[nq - 1].n_cand;
+            total_cand = 0;
+            for (int32_t i = 0; i < nq; ++i) total_cand += hqi[i].n_cand;
         }
         if (!deep_check.empty()) {
             // a user below the deepest guard has rank >= r[j_last] + 1 - n_del:
@@ -1734,50 +1716,32 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // L (QueryInfo.gamma of the value selection) is below that
             const int64_t floor_rank = (int64_t)hrk[gc.col[gc.n - 1]] + 1 - dv.n_del;
             for (int32_t i : deep_check)
-                if ((int64_t)hqi[i].gamma >= floor_rank) {
+                if (hcq[(size_t)i * 4] >= 0 && (int64_t)hqi[i].gamma >= floor_rank) {
                     if (fallback) fallback->push_back((int32_t)(q0 + i));
                     tm.n_fallback += 1;
                 }
-        }
-        if (!sized_by_list) {
-            total = hqi[nq - 1].cand_off + hqi[nq - 1].n_settled + hqi[nq - 1].n_cand;
-            total_cand = 0;
-            for (int32_t i = 0; i < nq; ++i) total_cand += hqi[i].n_cand;
         }
         if (total >= INT32_MAX) return set_err(c, RKR_ERR_NOMEM, "query: candidate count exceeds 2^31; lower the query batch");
         const size_t cap = (size_t)std::max<int64_t>(total, 1);
         const size_t rcap = (size_t)std::max<int64_t>(total_cand, 1);
         if ((rc = ensure(c, sl.cand, sizeof(int32_t) * 2 * cap, "candidates"))) return rc;
-        if ((rc = ensure(c, sl.refine_idx, (sizeof(int32_t) * 3 + sizeof(float)) * rcap, "refine rows"))) return rc;
-        if ((rc = ensure(c, sl.counts, sizeof(int32_t) * rcap, "refine counts"))) return rc;
-        if ((rc = ensure(c, sl.small, sizeof(int32_t) * ((size_t)nqb + 8), "query counters"))) return rc;
+        if ((rc = ensure(c, sl.refine_idx, sizeof(int32_t) * 4 * rcap, "refine rows"))) return rc;
         int32_t *cand_user = reinterpret_cast<int32_t *>(sl.cand.p);
         int32_t *cand_rank = cand_user + cap;
-        int32_t *refine_cand = reinterpret_cast<int32_t *>(sl.refine_idx.p);
-        int32_t *refine_user = refine_cand + rcap;
+        int32_t *refine_user = reinterpret_cast<int32_t *>(sl.refine_idx.p);
         int32_t *refine_query = refine_user + rcap;
         float *refine_thr = reinterpret_cast<float *>(refine_query + rcap);
-        int32_t *cnt = reinterpret_cast<int32_t *>(sl.counts.p);
-        int32_t *q_recheck = reinterpret_cast<int32_t *>(sl.small.p);  // per query
-        int32_t *recheck_n = q_recheck + nqb;
-        uint32_t *max_err_bits = reinterpret_cast<uint32_t *>(recheck_n + 1);
-        const bool screened = c->form == RKR_FORM_SCREENED;
+        int32_t *cnt = reinterpret_cast<int32_t *>(refine_thr + rcap);
 
-        if (coarse_b && !upd)
-            RKR_HIP(c, launch_coarse_final(sl.stream, cl_u, cl_b, bk_c, s_c, n_listed, d_list_n, S, R, I, U, qi, cand_user,
-                                           cand_rank, refine_total, refine_cand, refine_user, refine_query, refine_thr,
-                                           qip));
+        if (list)
+            RKR_HIP(c, launch_list_final(sl.stream, LL, bk_c, R, I, cand_user, cand_rank, refine_total, refine_user,
+                                         refine_query, refine_thr, cnt));
         else if (upd)
             RKR_HIP(c, launch_compact_values(sl.stream, lbv, ubv, qip, U, nq, cu, qi, cand_user, cand_rank,
-                                             refine_total, refine_cand, refine_user, refine_query, refine_thr));
+                                             refine_total, refine_user, refine_query, refine_thr, cnt));
         else
             RKR_HIP(c, launch_compact(sl.stream, bk, qip, U, S, R, I, nq, mode, cu, qi, cand_user, cand_rank,
-                                      refine_total, refine_cand, refine_user, refine_query, refine_thr));
-        int32_t &h_refine_total = h_scalars[0], &h_recheck_n = h_scalars[1];
-        uint32_t &h_err_bits = reinterpret_cast<uint32_t *>(h_scalars)[2];
-        h_refine_total = h_recheck_n = 0;
-        h_err_bits = 0;
-        for (int32_t i = 0; i < nq; ++i) h_qrecheck[i] = 0;
+                                      refine_total, refine_user, refine_query, refine_thr, cnt));
         // refinement + top-k; re-run when the recheck list overflowed
         for (int attempt = 0; attempt < 3; ++attempt) {
             int64_t rec_cap = 0;
@@ -1785,9 +1749,12 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 const int64_t want = std::max<int64_t>(1 << 20, (int64_t)sl.recheck.bytes / 16);
                 if ((rc = ensure(c, sl.recheck, 16 * (size_t)want, "recheck list"))) return rc;
                 rec_cap = (int64_t)(sl.recheck.bytes / 16);
-                RKR_HIP(c, hipMemsetAsync(sl.small.p, 0, sizeof(int32_t) * ((size_t)nqb + 8), sl.stream));
             }
-            RKR_HIP(c, hipMemsetAsync(cnt, 0, sizeof(int32_t) * rcap, sl.stream));
+            if (attempt > 0) {  // the compaction cleared the counts, the upload the recheck counters
+                RKR_HIP(c, hipMemsetAsync(cnt, 0, sizeof(int32_t) * rcap, sl.stream));
+                RKR_HIP(c, hipMemsetAsync(q_recheck, 0, sizeof(int32_t) * (size_t)nq, sl.stream));
+                RKR_HIP(c, hipMemsetAsync(&ctr->n_recheck, 0, sizeof(int32_t) * 2, sl.stream));
+            }
             RKR_HIP(c, hipEventRecord(sl.ev[4], sl.stream));
             // events 4..8 bracket exactly the refinement (or screening) kernel
             if (screened) {
@@ -1798,7 +1765,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 L.n_item = I; L.ld = ld; L.K = d; L.Kp = c->kp;
                 L.rows_user = refine_user; L.rows_thr = refine_thr; L.n_rows_dev = refine_total;
                 L.max_rows = (int64_t)rcap; L.C = c->screen_C; L.abs_floor = dv.screen_abs;
-                L.cnt = cnt; L.recheck_n = recheck_n; L.recheck = sl.recheck.p; L.recheck_cap = rec_cap;
+                L.cnt = cnt; L.recheck_n = &ctr->n_recheck; L.recheck = sl.recheck.p; L.recheck_cap = rec_cap;
                 L.target_units = (int64_t)c->n_cu * 8;
                 L.grid_cap = (int64_t)c->n_cu * 4;
                 L.chunk_items = c->screen_chunk > 0 ? c->screen_chunk : (1 << 30);
@@ -1806,50 +1773,37 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 RKR_HIP(c, launch_refine_screen(sl.stream, L));
                 RKR_HIP(c, hipEventRecord(sl.ev[8], sl.stream));
                 RKR_HIP(c, launch_recheck(sl.stream, dv.users, dv.items, ld, d, refine_user, refine_thr, refine_query,
-                                          recheck_n, sl.recheck.p, rec_cap, cnt, q_recheck, max_err_bits));
+                                          &ctr->n_recheck, sl.recheck.p, rec_cap, cnt, q_recheck, &ctr->max_err_bits));
             } else {
                 RKR_HIP(c, launch_refine_count(sl.stream, dv.users, dv.items, I, ld, d, refine_user, refine_thr,
                                                refine_total, (int64_t)rcap, cnt));
                 RKR_HIP(c, hipEventRecord(sl.ev[8], sl.stream));
             }
             RKR_HIP(c, hipEventRecord(sl.ev[5], sl.stream));
-            RKR_HIP(c, launch_scatter_counts(sl.stream, refine_total, refine_cand, cnt, (int64_t)rcap, cand_rank));
-            RKR_HIP(c, launch_topk(sl.stream, qi, nq, cand_user, cand_rank, qip, U, max_k, o_user, o_rank, o_qip,
-                                   nullptr));
+            RKR_HIP(c, launch_topk(sl.stream, qi, nq, cand_user, cand_rank, cnt, qip, U, max_k, o_user, o_rank, o_qip));
             RKR_HIP(c, hipEventRecord(sl.ev[6], sl.stream));
-            // outputs in one copy (the device layout), then the counters
-            RKR_HIP(c, hipMemcpyAsync(ho_user, o_user, 4 * out_words, hipMemcpyDeviceToHost, sl.stream));
-            RKR_HIP(c, hipMemcpyAsync(hqi, qi, sizeof(QueryInfo) * nq, hipMemcpyDeviceToHost, sl.stream));
-            RKR_HIP(c, hipMemcpyAsync(&h_refine_total, refine_total, sizeof(int32_t), hipMemcpyDeviceToHost, sl.stream));
-            if (dev_lists) {
-                // the lists' length and the queries k_coarse_mark sent to the full path
-                RKR_HIP(c, hipMemcpyAsync(hcq, cq_dev, sizeof(int32_t) * 4 * nq, hipMemcpyDeviceToHost, sl.stream));
-                RKR_HIP(c, hipMemcpyAsync(&h_scalars[3], d_list_n, sizeof(int32_t), hipMemcpyDeviceToHost, sl.stream));
-            }
-            if (screened) {
-                // q_recheck, recheck_n, max_err_bits are adjacent in sl.small
-                RKR_HIP(c, hipMemcpyAsync(h_qrecheck, q_recheck, sizeof(int32_t) * nq, hipMemcpyDeviceToHost, sl.stream));
-                RKR_HIP(c, hipMemcpyAsync(&h_recheck_n, recheck_n, sizeof(int32_t) * 2, hipMemcpyDeviceToHost,
-                                          sl.stream));
-            }
+            // query info, counters and outputs in one copy (the device layout)
+            RKR_HIP(c, hipMemcpyAsync(stg + io.info, dev + io.info, io.end - io.info, hipMemcpyDeviceToHost, sl.stream));
             RKR_HIP(c, hipEventRecord(sl.ev[7], sl.stream));
             RKR_HIP(c, hipStreamSynchronize(sl.stream));
-            if (!screened || (int64_t)h_recheck_n <= rec_cap) break;
+            const int64_t n_recheck = hctr->n_recheck;
+            if (!screened || n_recheck <= rec_cap) break;
             // the list overflowed: grow it and run the refinement again
-            const size_t need = 16 * ((size_t)h_recheck_n + (size_t)h_recheck_n / 4 + 1024);
+            const size_t need = 16 * ((size_t)n_recheck + (size_t)n_recheck / 4 + 1024);
             dev_free(c, sl.recheck.p, sl.recheck.bytes);
             sl.recheck.p = nullptr;
             sl.recheck.bytes = 0;
             if ((rc = ensure(c, sl.recheck, need, "recheck list"))) return rc;
             if (attempt == 2) return set_err(c, RKR_ERR_NOMEM, "query: recheck list kept overflowing");
         }
-        if (dev_lists) {
+        if (list) {
             for (int32_t i = 0; i < nq; ++i)
-                if (hcq[(size_t)i * 4] < 0) {
+                if (hqi[i].thr < 0) {
                     if (fallback) fallback->push_back((int32_t)(q0 + i));
                     tm.n_fallback += 1;
                 }
-            tm.n_listed += h_scalars[3];
+            tm.n_listed += hctr->n_list;
+            tm.n_coarse_refined += hctr->n_finer;
         }
         if (qsrp)
             for (int32_t i = 0; i < nq; ++i) tm.n_listed += hqi[i].n_screen;
@@ -1888,12 +1842,12 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         tm.topk_ms += ev_ms(sl.ev, 5, 6);
         tm.d2h_ms += ev_ms(sl.ev, 6, 7);
         tm.n_batches += 1;
-        tm.n_refined += h_refine_total;
+        tm.n_refined += hctr->n_refine;
         if (screened) {
-            tm.n_rechecked += h_recheck_n;
-            tm.n_screened += (int64_t)h_refine_total * I;
+            tm.n_rechecked += hctr->n_recheck;
+            tm.n_screened += (int64_t)hctr->n_refine * I;
             float e;
-            std::memcpy(&e, &h_err_bits, sizeof(e));
+            std::memcpy(&e, &hctr->max_err_bits, sizeof(e));
             tm.max_screen_err = std::max(tm.max_screen_err, (double)e);
         }
     }

@@ -45,9 +45,10 @@ struct Slot {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     hipEvent_t ev[16] = {};
-    DeviceBuf q_in, qip, bk, qinfo, cand, refine_idx, counts, out, recheck, small, hist;
-    DeviceBuf q_split, coarse_info, coarse_list;  // coarse bounds
-    PinnedBuf stage;                               // host side of the batch copies
+    DeviceBuf io;                // queries | query info, counters | outputs (BatchIo)
+    DeviceBuf qip, bk, cand, refine_idx, recheck, hist;
+    DeviceBuf q_split, list_info, list;  // threshold and coarse lists
+    PinnedBuf stage;                     // host side of the batch copies
 };
 
 struct Ctx {
@@ -121,10 +122,11 @@ struct Ctx {
     int32_t *qcol = nullptr;    // n_sample
     float *qtable = nullptr;    // [u_cap][n_qs]
     std::vector<int32_t> h_qranks;
-    // guard rows of the coarse bounds: [u_cap][kGuardRow], the values of the
-    // searched table at the columns of every guard set, -inf past each set's
-    // length; kept with the table
+    // guard rows: [u_cap][kGuardRow], the values of the searched table at its
+    // fine columns, -inf past them; kept with the table
     float *gvals = nullptr;
+    float *gcols = nullptr;     // the same values by column: [kGuardRow][u_cap at allocation]
+    int64_t gpitch = 0;
     int dense_top = 2;          // query table mode (RKR_OPT_DENSE_TOP)
 
     // screened form: hi/lo BF16 item rows (n_item x kp), norm bounds
@@ -218,24 +220,27 @@ inline float screen_abs_floor(int32_t kp, double max_abs_user, double max_abs_it
     return std::nextafter((float)absf, INFINITY);
 }
 
+// Guard columns of the coarse bounds (updates pending): col[j] the table
+// column, idx[j] its place in the guard row.
 struct GuardCols {
     int32_t col[8];
+    int32_t idx[8];
     int32_t n;
 };
-// Guard sets of the coarse bounds: set 0 holds the first pass's columns, set
-// 1 + beta the second pass's columns inside guard bin beta (empty when the bin
-// has no column of its own).  Each user keeps the values of all of them in one
-// row of kGuardRow floats, set s at floats 8 s .. 8 s + 7 (-inf past its n).
-constexpr int kGuardSets = 8;
-// Workgroups per CU of the coarse first pass (256 threads, users' BF16 hi
+// Fine columns of the searched table, ascending; each user keeps their values
+// in a guard row of kGuardRow floats (-inf past n).  The guard columns are
+// among them (bit f of coarse: column f is one).
+constexpr int kGuardRow = 64;
+constexpr int kMaxFine = 63;
+struct FineCols {
+    int32_t col[kMaxFine];
+    int32_t n;
+    uint64_t coarse;
+};
+// Workgroups per CU of the coarse pass (256 threads, users' BF16 hi
 // halves in VGPRs) for Kp = 32 ks: its launch bound and its persistent grid.
 // (Five fit at ks <= 5 only by spilling the staged query pieces: slower.)
 constexpr int coarse_first_pass_wgs(int ks) { return ks >= 7 ? 3 : 4; }
-constexpr int kGuardRow = 8 * kGuardSets;
-struct GuardSets {
-    GuardCols set[kGuardSets];
-};
-
 
 // Everything a query batch reads from the data and table state, captured
 // when the batch starts.  Outside a snapshot-mode server it is the context's
@@ -255,9 +260,11 @@ struct DataSnap {
     const float *qtable = nullptr;   // query table (exact output), or null
     const int32_t *qranks = nullptr;
     int32_t n_qs = 0;
-    int32_t n_guard = 0;             // guard columns of the coarse bounds
-    int32_t gcol[8] = {};
-    const float *gvals = nullptr;    // guard values per user (kGuardRow floats, all sets), or null
+    GuardCols guards{};              // guard columns of the coarse bounds
+    FineCols fine{};                 // columns of the guard rows
+    const float *gvals = nullptr;    // guard values per user (kGuardRow floats)
+    const float *gcols = nullptr;    // and by column, rows of gpitch users
+    int64_t gpitch = 0;
     // the sampled table's ranks (device), count and eps, the query table's
     // column of each sampled column, and the searched table's ranks on the
     // host (the guard placement): captured with the table, so a batch never
@@ -267,7 +274,6 @@ struct DataSnap {
     float table_eps = 0.0f;
     const int32_t *qcol = nullptr;
     std::shared_ptr<const std::vector<int32_t>> hrk;
-    GuardSets gsets{};               // the coarse guard sets of that table
     // pending inserts: the most inserted items any user has above its value
     // at guard column j (a bound on the rank shift at that guard)
     int32_t ins_gmax[8] = {};
@@ -277,17 +283,19 @@ struct DataSnap {
     float qsrp_gcd = 0.0f, qsrp_crot = 0.0f;
 };
 DataSnap snap_of(const Ctx *c);
-GuardSets guard_sets(const Ctx *c);
-// Guard columns of the coarse bounds for the context's searched table.
-void guard_columns(const Ctx *c, int32_t *col, int32_t &n);
+// Fine columns and guard columns of the context's searched table.
+FineCols fine_columns(const Ctx *c);
+GuardCols guard_columns(const Ctx *c);
 // The table over the current items at sampled ranks S (build_table), and the
 // same at uniform ranks of the current n_sample (rebuild_table): the pending
 // item updates fold into the new table; keep_update_buffers leaves their
 // buffers allocated for the updates that follow.
 int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool keep_update_buffers);
 int rebuild_table(Ctx *c);
-// Fills Ctx::gvals rows [u0, u0 + n) from the searched table.
+// Fills Ctx::gvals and gcols of users [u0, u0 + n) from the searched table.
 int refresh_guard_values(Ctx *c, int64_t u0, int64_t n);
+// New (unfilled) guard arrays for `cap` users; the old ones go through dev_free.
+int alloc_guards(Ctx *c, int64_t cap);
 // Recomputes Ctx::ins_gmax after inserted items or users changed.
 int refresh_ins_guard_max(Ctx *c);
 // Ranks of the query table: the sample ranks and the dense top ranks below
@@ -368,42 +376,32 @@ struct ScreenLaunch {
 // norm upper bounds; used for items, queries and users.  With cs (queries of
 // the coarse first pass): each row's error scale of the one-product
 // estimate, given rho (device) >= ||u - bf16(u)|| / ||u|| over the users and
-// the accumulation and rule rounding factors g1, g_rule.
+// the accumulation and rule rounding factors g1, g_rule.  With zero64, 64 words
+// per row are cleared.
 hipError_t launch_prep_items(hipStream_t s, const float *items, int64_t n_item, int32_t ld, int32_t K, int32_t Kp,
                              uint16_t *hi, uint16_t *lo, float *norm, float *cs = nullptr, const float *rho = nullptr,
-                             double g1 = 0.0, double g_rule = 0.0);
+                             double g1 = 0.0, double g_rule = 0.0, uint32_t *zero64 = nullptr);
 // Users' norm upper bounds; with rho (device), raises *rho to at least every
 // user's ||u - bf16(u)|| / ||u||.
 hipError_t launch_user_norms(hipStream_t s, const float *users, int64_t n_user, int32_t ld, int32_t K, float *norm,
                              float *rho);
 hipError_t launch_refine_screen(hipStream_t s, const ScreenLaunch &L);
-// Guard columns of the coarse bounds: n (1..7) ascending table columns.
-
-// Coarse buckets of a batch (screened <u,q> against the guard columns of
-// every user's table row): cb[row(b) * ldc + u] = c_lo | c_hi << 4, with
-// row(b) = qmap[b] (or b when qmap is null), which also picks the query rows.
+// Coarse buckets of a batch with updates pending (screened <u,q> against the
+// guard columns of every user's table row): cb[b * ldc + u] = c_lo | c_hi << 4.
 struct CoarseLaunch {
-    const float *users, *user_norm, *table;
-    const float *gvals = nullptr;       // n_user x kGuardRow guard values, or null: read the table
-    const uint16_t *user_hi, *user_lo;  // BF16 split of the user rows (n_user x Kp)
+    const float *user_norm;
+    const float *gvals;                 // n_user x kGuardRow guard values
+    const uint16_t *user_hi;            // BF16 hi halves of the user rows (n_user x Kp)
     int64_t n_user;
-    int32_t S;
     GuardCols gc;
-    const uint16_t *q_hi, *q_lo;
-    const float *q_norm;
-    const int32_t *qmap;
-    int32_t nq, ld, K, Kp;
+    const uint16_t *q_hi;
+    const float *q_cs;                  // error scales of the queries
+    int32_t nq, Kp;
     float C, abs_floor;
     uint8_t *cb;            // rows of ldc bytes, ldc % 128 == 0
     int64_t ldc;
     int64_t spare_row;      // a row no query owns (written by padding lanes)
     int64_t grid_cap;
-    // second pass: query b uses sets[qset[b]] (<= 7 sets) instead of gc;
-    // set_id[i] is the guard-row set (1 + beta) of launch set i
-    const GuardCols *sets = nullptr;
-    const int32_t *qset = nullptr;
-    int32_t n_sets = 0;
-    int32_t set_id[7] = {};
 };
 hipError_t launch_ip_coarse(hipStream_t s, const CoarseLaunch &L);
 hipError_t launch_recheck(hipStream_t s, const float *users, const float *items, int32_t ld, int32_t K,
@@ -451,7 +449,76 @@ struct QueryInfo {          // one per query of a device batch
     int32_t fill;           // candidates written so far (chunked compaction)
     int32_t n_screen;       // users a screen kept and scored exactly (QSRP)
     int64_t cand_off;       // offset of this query's candidates
+    int32_t thr;            // fine column of the query's list, -1: the full search answers it
+    int32_t pad2;
 };
+
+// Counters of a device batch, uploaded as zeros with the queries and read back
+// with the outputs.
+struct alignas(64) ListCounters {
+    int32_t n_slots;        // queries with a threshold
+    int32_t n_list;         // listed pairs (past the list's capacity when it overflowed)
+    int32_t n_cand;         // candidates
+    int32_t n_finer;        // queries listed against a column finer than the guard columns
+    int32_t n_refine;       // refine rows
+    int32_t n_recheck;      // screened form: undecided pairs
+    uint32_t max_err_bits;  // screened form: largest screen error seen
+};
+
+// One transfer each way per device batch: the queries, the query info with
+// topk, the recheck counts and counters go up, and the last three come back
+// with the outputs.  Byte offsets for nq queries.
+struct BatchIo {
+    size_t queries = 0, info, recheck, counters, out, end;
+    BatchIo(int64_t nq, int32_t ld, int32_t max_k) {
+        auto up = [](size_t x) { return (x + 63) & ~(size_t)63; };
+        info = up(sizeof(float) * (size_t)nq * ld);
+        recheck = info + up(sizeof(QueryInfo) * (size_t)nq);
+        counters = recheck + up(sizeof(int32_t) * (size_t)nq);
+        out = counters + sizeof(ListCounters);
+        end = out + 3 * sizeof(int32_t) * (size_t)nq * max_k;
+    }
+};
+
+// ---- threshold lists of exact output (k_list.hip) ----------------------------
+struct ListScreen {          // the screened scores of a batch
+    const uint16_t *user_hi; // n_user x Kp BF16 hi halves
+    const float *user_norm, *gvals, *gcols;
+    int64_t pitch;           // of gcols
+    const uint16_t *q_hi;    // nq x Kp
+    const float *q_cs;       // error scales: |s^ - s| <= C ||u|| cs + floor
+    int32_t nq, Kp, n_fine;
+    float C, floor;
+};
+struct ListLaunch {
+    int64_t n_user;
+    int32_t nq, S, Kp, n_cu;
+    const uint16_t *user_hi, *q_hi;
+    const float *user_norm, *gvals, *gcols, *q_cs;
+    int64_t pitch;           // of gcols
+    FineCols fc;
+    float C, floor, eps;
+    float *qip;              // exact scores (read with scores, else written for listed pairs)
+    int64_t stride;          // every stride-th user is sampled
+    int64_t cap;             // a longer estimated list takes the full search
+    int64_t list_cap;        // entries of cl_u, cl_b
+    uint32_t *hist;          // nq x 64, zeroed
+    int32_t *order, *colg;   // nq slots, nq / 4 threshold columns
+    QueryInfo *qi;
+    ListCounters *ctr;
+    uint32_t *ghist;         // nq x 2 (S + 1) bucket histograms
+    int32_t *cl_u, *cl_b;
+};
+// Threshold per query and the listed pairs, from the matrix cores or from qip.
+hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L);
+hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L);
+// Exact scores (read from qip with scores) and buckets of the listed pairs,
+// then the k-th bound and the candidates' place per query.
+hipError_t launch_list_exact(hipStream_t s, const ListLaunch &L, const float *users, const float *queries, int32_t ld,
+                             int32_t dim, const float *table, bool scores, uint32_t *bk_c);
+hipError_t launch_list_final(hipStream_t s, const ListLaunch &L, const uint32_t *bk_c, const int32_t *ranks,
+                             int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_total,
+                             int32_t *refine_user, int32_t *refine_query, float *refine_thr, int32_t *cnt);
 
 // Table rows staged per workgroup by the batched bounds kernels: 16 rows of
 // S + 1 floats (<= 32 KB at S = 511), fewer for long rows; 0 when one row
@@ -479,6 +546,41 @@ __device__ __forceinline__ void stage_rows(float *rows, const float *__restrict_
         for (int64_t i = threadIdx.x; i < nu * S; i += blockDim.x) rows[(i / S) * (S + 1) + i % S] = src[(i / S) * src_ld + i % S];
     }
 }
+
+// The score rule: FP32 products summed in ascending dimension order.
+__device__ __forceinline__ float rule_dot(const float *__restrict__ a, const float *__restrict__ b, int32_t d) {
+    float s = 0.0f;
+    int32_t k = 0;
+    // 32 terms are loaded before they are summed: lanes of a wavefront read
+    // different rows, and taking a whole 128-byte stretch per lane at once
+    // uses each cache line fully before it can be evicted (the sum's order is
+    // unchanged)
+    for (; k + 32 <= d; k += 32) {
+        float4 x[8], y[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            x[t] = *reinterpret_cast<const float4 *>(a + k + 4 * t);
+            y[t] = *reinterpret_cast<const float4 *>(b + k + 4 * t);
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            s = s + x[t].x * y[t].x;
+            s = s + x[t].y * y[t].y;
+            s = s + x[t].z * y[t].z;
+            s = s + x[t].w * y[t].w;
+        }
+    }
+    for (; k + 4 <= d; k += 4) {
+        const float4 x = *reinterpret_cast<const float4 *>(a + k);
+        const float4 y = *reinterpret_cast<const float4 *>(b + k);
+        s = s + x.x * y.x;
+        s = s + x.y * y.y;
+        s = s + x.z * y.z;
+        s = s + x.w * y.w;
+    }
+    for (; k < d; ++k) s = s + a[k] * b[k];
+    return s;
+}
 #endif
 
 // Users per chunk of the chunked prune kernels: enough workgroups per query
@@ -504,56 +606,39 @@ hipError_t launch_bounds(hipStream_t s, const float *qip, const float *table, in
 hipError_t launch_hist_kth(hipStream_t s, const uint32_t *bk, int64_t n_user, int32_t S, const int32_t *ranks,
                            int64_t n_item, int32_t nq, int output_mode, int same, int64_t cu, uint32_t *ghist,
                            QueryInfo *qi);
-// Coarse-bound pipeline of exact output (k_query.hip): guard values per
-// user, the coarse k-th bound and list size per query (cq[b] = {beta_c,
-// count, offset, fill}), the listed users, their exact scores and bucket
-// pairs with the exact k-th bound (into qi), and the final candidates.
-// cb rows are ldc bytes (ldc % 16 == 0, bytes past n_user unread); cu % 1024 == 0
+// Coarse bounds with updates pending (k_query.hip): the coarse k-th bound and
+// list size per query (cq[b] = {beta_c, count, offset, fill}) and the listed
+// users.  cb rows are ldc bytes (ldc % 16 == 0, bytes past n_user unread);
+// cu % 1024 == 0.
 // hcnt[b * 8 + c] = #{users with c_hi == c}, c < 7
 hipError_t launch_coarse_kth(hipStream_t s, const uint8_t *cb, int64_t ldc, int64_t n_user, int32_t nq, int64_t cu,
-                             int32_t n_guard, const int32_t *qmap, uint32_t *part, const QueryInfo *qi, int32_t *cq,
-                             int32_t *hcnt);
-// Update path: exact rank bound values of the listed pairs (lbs / ubs /
-// qip at b * n_user + u; other pairs keep what the caller filled in).
+                             int32_t n_guard, uint32_t *part, const QueryInfo *qi, int32_t *cq, int32_t *hcnt);
+// Exact rank bound values of the listed pairs (lbs / ubs / qip at
+// b * n_user + u; other pairs keep what the caller filled in).
 hipError_t launch_coarse_exact_upd(hipStream_t s, const float *users, const float *queries, int32_t ld, int32_t dim,
                                    const float *table, int32_t S, const int32_t *ranks, int64_t n_item_base,
-                                   float eps, const GuardCols *gsets, const int32_t *gset, const int32_t *cl_u,
+                                   float eps, const GuardCols &gc, const int32_t *cl_u,
                                    const int32_t *cl_b, int64_t n, const float *ins, int32_t n_ins, int32_t ld_ins,
                                    const float *del, int32_t n_del, int32_t ld_del, int64_t n_user, int32_t *lbs,
                                    int32_t *ubs, float *qip);
 // max over users of #{inserted scores > T[u][gc.col[j]]} into out[j] (zeroed here)
 hipError_t launch_ins_guard_max(hipStream_t s, const float *table, int64_t n_user, int32_t S, const GuardCols &gc,
                                 const float *ins, int32_t n_ins, int32_t ld_ins, int32_t *out);
-// chunk-major list: loc (n_chunk x nq), ctot and cbase (n_chunk) are scratch;
-// total (optional) receives the list's length
+// chunk-major list: loc (n_chunk x nq), ctot and cbase (n_chunk) are scratch
 hipError_t launch_coarse_compact(hipStream_t s, const uint8_t *cb, int64_t ldc, int64_t n_user, int32_t nq,
                                  int64_t cu, const uint32_t *part, const int32_t *cq, int32_t *loc, int32_t *ctot,
-                                 int32_t *cbase, int32_t *cl_u, int32_t *cl_b, int32_t *total);
-// cq[b] = {-1, 0, -, 0} for a query with no k-th bound, a count over cap or a
-// count over the bound in field 2 (the full path answers it)
-hipError_t launch_coarse_mark(hipStream_t s, int32_t *cq, int32_t nq, int64_t cap);
-hipError_t launch_coarse_exact(hipStream_t s, const float *users, const float *queries, int32_t ld, int32_t dim,
-                               const float *table, int32_t S, const int32_t *ranks, int64_t n_item, float eps,
-                               const GuardCols *gsets, const int32_t *gset, int32_t nq, const int32_t *cl_u,
-                               const int32_t *cl_b, int64_t n, const int32_t *n_dev, uint32_t *bk_c, float *s_c,
-                               uint32_t *ghist, QueryInfo *qi);
-// n_dev (optional): the list's length on the device (at most n; n sizes the grid)
-hipError_t launch_coarse_final(hipStream_t s, const int32_t *cl_u, const int32_t *cl_b, const uint32_t *bk_c,
-                               const float *s_c, int64_t n, const int32_t *n_dev, int32_t S, const int32_t *ranks,
-                               int64_t n_item,
-                               int64_t n_user, QueryInfo *qi, int32_t *cand_user, int32_t *cand_rank,
-                               int32_t *refine_total, int32_t *refine_cand, int32_t *refine_user,
-                               int32_t *refine_query, float *refine_thr, float *qip);
+                                 int32_t *cbase, int32_t *cl_u, int32_t *cl_b);
+// The compaction kernels give a candidate its rank when the bounds fix it and
+// ~r otherwise, r its refine row, whose count cnt[r] they clear.
 hipError_t launch_offsets(hipStream_t s, QueryInfo *qi, int32_t nq, int32_t *refine_total);
 hipError_t launch_compact(hipStream_t s, const uint32_t *bk, const float *qip, int64_t n_user, int32_t S,
                           const int32_t *ranks, int64_t n_item, int32_t nq, int output_mode, int64_t cu,
                           QueryInfo *qi, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_total,
-                          int32_t *refine_cand, int32_t *refine_user, int32_t *refine_query, float *refine_thr);
-hipError_t launch_scatter_counts(hipStream_t s, const int32_t *refine_total, const int32_t *refine_cand,
-                                 const int32_t *cnt, int64_t max_rows, int32_t *cand_rank);
+                          int32_t *refine_user, int32_t *refine_query, float *refine_thr, int32_t *cnt);
+// cnt: the refine rows' counts
 hipError_t launch_topk(hipStream_t s, const QueryInfo *qi, int32_t nq, const int32_t *cand_user,
-                       const int32_t *cand_rank, const float *qip, int64_t n_user, int32_t max_k,
-                       int32_t *out_user, int32_t *out_rank, float *out_qip, int64_t *scratch_keys);
+                       const int32_t *cand_rank, const int32_t *cnt, const float *qip, int64_t n_user, int32_t max_k,
+                       int32_t *out_user, int32_t *out_rank, float *out_qip);
 
 // ---- update path (k_update.hip) ---------------------------------------------
 // QSRP screen kernels (k_qsrp.hip).  qn holds 3 floats per query: upper bounds
@@ -568,10 +653,10 @@ hipError_t launch_qsrp_exact(hipStream_t s, const float *users, const float *q_i
                              const float *T, int32_t S, float eps, int64_t n_user, int32_t nq, QueryInfo *qi,
                              float *qip, uint32_t *bk);
 
-// gv[u * kGuardRow + 8 s + j] = T[u][gs.set[s].col[j]] (-inf for j >= its n),
-// rows [u0, u0 + n_rows).
-hipError_t launch_gather_guards(hipStream_t s, const float *T, int64_t S, const GuardSets &gs, int64_t u0,
-                                int64_t n_rows, float *gv);
+// gv[u * kGuardRow + f] = gc[f * pitch + u] = T[u][fc.col[f]] (-inf for
+// f >= fc.n), rows [u0, u0 + n_rows).
+hipError_t launch_gather_guards(hipStream_t s, const float *T, int64_t S, const FineCols &fc, int64_t u0,
+                                int64_t n_rows, float *gv, float *gc, int64_t pitch);
 
 // The sort scratch of rkr_sorted_scores_noalloc: looks up its device address
 // on `device` (current) once per device.
@@ -590,8 +675,8 @@ hipError_t launch_kth_values(hipStream_t s, const int32_t *lbs, const int32_t *u
                              int64_t cu, uint32_t *ghist, QueryInfo *qi);
 hipError_t launch_compact_values(hipStream_t s, const int32_t *lbs, const int32_t *ubs, const float *qip,
                                  int64_t n_user, int32_t nq, int64_t cu, QueryInfo *qi, int32_t *cand_user,
-                                 int32_t *cand_rank, int32_t *refine_total, int32_t *refine_cand,
-                                 int32_t *refine_user, int32_t *refine_query, float *refine_thr);
+                                 int32_t *cand_rank, int32_t *refine_total, int32_t *refine_user,
+                                 int32_t *refine_query, float *refine_thr, int32_t *cnt);
 // dst[r][j] = src[r][cols[j]] for r < n_rows, j < n_cols
 hipError_t launch_gather_cols(hipStream_t s, const float *src, int64_t ld_src, const int32_t *cols, int32_t n_cols,
                               int64_t n_rows, float *dst, int64_t ld_dst);

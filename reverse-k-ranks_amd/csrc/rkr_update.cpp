@@ -78,23 +78,22 @@ int reserve_users(Ctx *c, int64_t need) {
     const int32_t ld = c->ld, S = c->n_sample;
     const int32_t QS = c->n_qs;
     float *users = nullptr, *panels = nullptr, *unorm = nullptr, *table = nullptr, *qtable = nullptr, *si = nullptr,
-          *sd = nullptr, *gv = nullptr;
+          *sd = nullptr;
     int rc = RKR_OK;
-    if ((c->gvals && (rc = dev_alloc_t(c, &gv, (size_t)cap * kGuardRow, "guard values"))) ||
-        (rc = dev_alloc_t(c, &users, (size_t)cap * ld, "users")) ||
+    if ((rc = dev_alloc_t(c, &users, (size_t)cap * ld, "users")) ||
         (rc = dev_alloc_t(c, &panels, (size_t)((cap + 63) / 64) * 64 * ld, "user panels")) ||
         (c->kp && (rc = dev_alloc_t(c, &unorm, (size_t)cap, "user norms"))) ||
         (rc = dev_alloc_t(c, &table, (size_t)cap * S, "table")) ||
         (QS && (rc = dev_alloc_t(c, &qtable, (size_t)cap * QS, "query table"))) ||
         (c->ld_ins && (rc = dev_alloc_t(c, &si, (size_t)cap * c->ld_ins, "side array"))) ||
         (c->ld_del && (rc = dev_alloc_t(c, &sd, (size_t)cap * c->ld_del, "side array")))) {
-        for (float *p : {users, panels, unorm, table, qtable, si, sd, gv}) dev_free(c, p, 0);
+        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
         return rc;
     }
     uint16_t *uhi = nullptr, *ulo = nullptr;
     if (c->kp && ((rc = dev_alloc_t(c, &uhi, (size_t)cap * c->kp, "user hi")) ||
                   (rc = dev_alloc_t(c, &ulo, (size_t)cap * c->kp, "user lo")))) {
-        for (float *p : {users, panels, unorm, table, qtable, si, sd, gv}) dev_free(c, p, 0);
+        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
         dev_free(c, uhi, 0);
         dev_free(c, ulo, 0);
         return rc;
@@ -110,15 +109,13 @@ int reserve_users(Ctx *c, int64_t need) {
         (c->kp && (rc = copy_rows(c, unorm, 1, c->user_norm, 1, U, 1))) ||
         (rc = copy_rows(c, table, S, c->table, S, U, S)) ||
         (QS && (rc = copy_rows(c, qtable, QS, c->qtable, QS, U, QS))) ||
-        (gv && (rc = copy_rows(c, gv, kGuardRow, c->gvals, kGuardRow, U, kGuardRow))) ||
         (si && (rc = copy_rows(c, si, c->ld_ins, c->side_ins, c->ld_ins, U, c->n_ins))) ||
         (sd && (rc = copy_rows(c, sd, c->ld_del, c->side_del, c->ld_del, U, c->n_del))))
         return rc;
     RKR_HIP(c, hipStreamSynchronize(c->stream));
     for (float *p : {c->users, c->usersT, c->user_norm, c->table, c->qtable, c->side_ins, c->side_del,
-                     c->side_ins_spare, c->side_del_spare, c->gvals})
+                     c->side_ins_spare, c->side_del_spare})
         dev_free(c, p, 0);
-    c->gvals = gv;
     dev_free(c, c->user_hi, 0);
     dev_free(c, c->user_lo, 0);
     c->user_hi = uhi;
@@ -132,6 +129,8 @@ int reserve_users(Ctx *c, int64_t need) {
     c->side_del = sd;
     c->side_ins_spare = c->side_del_spare = nullptr;
     c->u_cap = cap;
+    if (c->gvals && ((rc = alloc_guards(c, cap)) || (rc = refresh_guard_values(c, 0, U)))) return rc;
+    RKR_HIP(c, hipStreamSynchronize(c->stream));
     return RKR_OK;
 }
 
@@ -337,8 +336,7 @@ int rkr::refresh_ins_guard_max(Ctx *c) {
     const float *T = c->qtable ? c->qtable : c->table;
     const int32_t S = c->qtable ? c->n_qs : c->n_sample;
     if (!c->n_ins || !T || c->n_user <= 0) return RKR_OK;
-    GuardCols gc{};
-    guard_columns(c, gc.col, gc.n);
+    const GuardCols gc = guard_columns(c);
     if (gc.n <= 0) return RKR_OK;
     int rc;
     if ((rc = ensure(c, c->upd_scratch, std::max<size_t>(c->upd_scratch.bytes, 64), "update scratch"))) return rc;
@@ -561,7 +559,7 @@ int rkr_delete_users(rkr_ctx *c, const int64_t *ids, int64_t n) {
     rc = keep_user_rows(c, &c->users, ld, ld, d_keep, nk, "users");
     if (!rc) rc = keep_user_rows(c, &c->table, c->n_sample, c->n_sample, d_keep, nk, "table");
     if (!rc) rc = keep_user_rows(c, &c->qtable, c->n_qs, c->n_qs, d_keep, nk, "query table");
-    if (!rc) rc = keep_user_rows(c, &c->gvals, kGuardRow, kGuardRow, d_keep, nk, "guard values");
+    if (!rc && c->gvals && !(rc = alloc_guards(c, c->u_cap))) rc = refresh_guard_values(c, 0, nk);
     if (!rc) rc = keep_user_rows(c, &c->side_ins, c->n_ins, c->ld_ins, d_keep, nk, "side array");
     if (!rc) rc = keep_user_rows(c, &c->side_del, c->n_del, c->ld_del, d_keep, nk, "side array");
     dev_free(c, d_keep, 0);

@@ -1,5 +1,6 @@
 """GPU tests of kernel edges: tile remainders of the score product, bin
-lengths of the row sort.  Every value is compared bit for bit with the oracle."""
+lengths of the row sort, threshold lists.  Every value is compared bit for bit
+with the oracle or with the search over every user."""
 import numpy as np
 import pytest
 
@@ -42,3 +43,69 @@ def test_row_sort_bin_lengths(orc, copies, odd):
         idx.set_data(users, items)
         got = idx.sorted_scores()
     assert np.array_equal(got, orc.sorted_score_rows(orc.normalize_users(users), items))
+
+
+def _lists_and_search(idx, queries, ks):
+    """The answers with threshold lists and those of the search over every user."""
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    full = idx.query(queries, ks)
+    idx.set_option(9, 1)
+    got = idx.query(queries, ks)
+    for i, k in enumerate(ks):
+        for f in ("users", "ranks", "qips"):
+            assert np.array_equal(getattr(full, f)[i, :k], getattr(got, f)[i, :k]), f"query {i}: {f} differ"
+        for f in ("n_candidate", "n_refine_user", "n_prune_user", "n_result_user"):
+            assert full.stats[i][f] == got.stats[i][f], f"query {i}: {f}"
+    return got
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+@pytest.mark.parametrize("U,nq,d,dense", [(1, 9, 5, 2), (255, 8, 33, 2), (257, 65, 64, 0), (4097, 17, 150, 2),
+                                          (16385, 64, 31, 1), (40003, 5, 161, 2), (70001, 1, 40, 2), (70001, 600, 20, 0)])
+def test_threshold_lists(gpu_index_factory, form, U, nq, d, dense):
+    """Lists against the full search: user counts at the edges of a unit and of
+    the sample, batches of one query to more than a slice, k from 1 to thousands,
+    queries that are items, that nobody and that everybody ranks first."""
+    _case(f"threshold lists {form} U={U} nq={nq} d={d} dense={dense}")
+    rng = np.random.default_rng(U + nq + d)
+    I = 1500
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    users[U // 2] = 0.0
+    items = (rng.standard_normal((I, d), dtype=np.float32) * rng.lognormal(0, 0.5, (I, 1))).astype(np.float32)
+    queries = items[rng.integers(0, I, nq)].copy()
+    if nq > 4:
+        queries[1] = 0.0
+        queries[2] *= 50.0
+        queries[3] = -queries[3]
+        queries[4] *= 1e-3
+    ks = [int(min(U, k)) for k in np.exp(rng.uniform(0, np.log(3000), nq))]
+    idx, _ = gpu_index_factory(users, items, 64, dense_top=dense)
+    idx.set_form(form)
+    res = _lists_and_search(idx, queries, ks)
+    if U >= 70000 or (nq >= 8 and (form == "screened" or U >= 4096)):  # the calls that take lists
+        assert res.timing["n_listed"] > 0 or res.timing["n_fallback"] > 0
+    idx.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+def test_threshold_lists_eps_and_sample(gpu_index_factory, form):
+    """A table with eps > 0, and users ordered so that no sampled one is among a
+    query's best: the threshold is too tight or the list too long, and the query
+    is answered all the same."""
+    _case(f"threshold lists {form}: eps, unrepresentative sample")
+    rng = np.random.default_rng(3)
+    U, I, d = 70001, 800, 16
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    users[::4] = -items[7] + 0.05 * rng.standard_normal((len(users[::4]), d), dtype=np.float32)  # every fourth is sampled
+    users[1:400:4] = items[7] + 0.01 * rng.standard_normal((100, d), dtype=np.float32)
+    queries = np.concatenate([items[:12], -items[:12]])
+    ks = [int(k) for k in rng.integers(1, 300, len(queries))]
+    idx, ranks = gpu_index_factory(users, items, 48)
+    idx.set_form(form)
+    _lists_and_search(idx, queries, ks)
+    T = idx.get_table()
+    idx.set_table(ranks, T + np.float32(5e-5), eps=1e-4)  # off by less than eps
+    res = _lists_and_search(idx, queries, ks)
+    assert res.users.shape == (24, max(ks))
+    idx.close()
