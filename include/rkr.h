@@ -102,7 +102,9 @@ typedef struct rkr_query_stats {
     int64_t n_screened;      /* screened form: (user, item) scores screened     */
 } rkr_query_stats;
 
-/* Batch-level timings (device time from HIP events, milliseconds). */
+/* Batch-level timings (device time, milliseconds: clock readings of the stages'
+ * kernels, HIP events around the copies and in batches with updates pending or
+ * the QSRP screen). */
 typedef struct rkr_batch_timing {
     double total_ms;        /* host wall time of the rkr_query call            */
     double ip_ms;           /* <u,q> GEMV/GEMM                                 */

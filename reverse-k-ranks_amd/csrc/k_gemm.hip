@@ -177,7 +177,8 @@ template <bool ROW_M>
 __global__ void __launch_bounds__(NT, 3) k_scores_store(const float *__restrict__ A, int64_t M, int32_t lda,
                                                      const float *__restrict__ B, int64_t N,
                                                      int32_t ldb, int32_t K, float *__restrict__ C, int64_t ldc,
-                                                     int vec, int64_t n_tiles_m, int64_t n_tiles_n) {
+                                                     int vec, int64_t n_tiles_m, int64_t n_tiles_n, uint64_t *t) {
+    stamp(t);
     __shared__ TileSmem sm;
     int64_t tm, tn;
     if (!tile_of_block(n_tiles_m, n_tiles_n, tm, tn)) return;
@@ -218,7 +219,8 @@ __global__ void __launch_bounds__(NT, 3) k_refine_count(const float *__restrict_
                                                      const int32_t *__restrict__ rows_user,
                                                      const float *__restrict__ rows_thr,
                                                      const int32_t *__restrict__ n_rows_dev, int64_t max_rows,
-                                                     int32_t *__restrict__ cnt) {
+                                                     int32_t *__restrict__ cnt, uint64_t *t) {
+    stamp(t);
     __shared__ TileSmem sm;
     __shared__ int32_t red[BM];
     __shared__ float s_thr[BM];
@@ -274,7 +276,8 @@ __global__ void __launch_bounds__(NT, 3) k_refine_count(const float *__restrict_
 template <int NQ>
 __global__ void __launch_bounds__(NT) k_gemv_panels(const float *__restrict__ usersT, int64_t n_user, int32_t ld,
                                                     int32_t K, const float *__restrict__ q, int32_t nq,
-                                                    float *__restrict__ qip) {
+                                                    float *__restrict__ qip, uint64_t *t) {
+    stamp(t);
     extern __shared__ float qs[];  // nq x K
     for (int i = threadIdx.x; i < nq * K; i += NT) qs[i] = q[(i / K) * (int64_t)ld + (i % K)];
     __syncthreads();
@@ -319,21 +322,21 @@ __global__ void k_make_panels(const float *__restrict__ users, int64_t n_user, i
 
 hipError_t launch_scores_store(hipStream_t s, const float *A, int64_t M, int32_t lda,
                                const float *B, int64_t N, int32_t ldb, int32_t K, float *C, int64_t ldc,
-                               bool c_row_major_m) {
+                               bool c_row_major_m, uint64_t *t) {
     if (M <= 0 || N <= 0) return hipSuccess;
     const int64_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
     const dim3 grid((unsigned)((tm * tn + 7) / 8 * 8));
     const int vec = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0 ? 1 : 0;
     if (c_row_major_m)
-        hipLaunchKernelGGL(k_scores_store<true>, grid, dim3(NT), 0, s, A, M, lda, B, N, ldb, K, C, ldc, vec, tm, tn);
+        hipLaunchKernelGGL(k_scores_store<true>, grid, dim3(NT), 0, s, A, M, lda, B, N, ldb, K, C, ldc, vec, tm, tn, t);
     else
-        hipLaunchKernelGGL(k_scores_store<false>, grid, dim3(NT), 0, s, A, M, lda, B, N, ldb, K, C, ldc, vec, tm, tn);
+        hipLaunchKernelGGL(k_scores_store<false>, grid, dim3(NT), 0, s, A, M, lda, B, N, ldb, K, C, ldc, vec, tm, tn, t);
     return hipGetLastError();
 }
 
 hipError_t launch_refine_count(hipStream_t s, const float *users, const float *items, int64_t n_item, int32_t ld,
                                int32_t K, const int32_t *rows_user, const float *rows_thr, const int32_t *n_rows_dev,
-                               int64_t max_rows, int32_t *cnt) {
+                               int64_t max_rows, int32_t *cnt, uint64_t *t) {
     if (max_rows <= 0 || n_item <= 0) return hipSuccess;
     int dev = 0, n_cu = 256;
     (void)hipGetDevice(&dev);
@@ -342,21 +345,21 @@ hipError_t launch_refine_count(hipStream_t s, const float *users, const float *i
     const int64_t max_units = ((max_rows + BM - 1) / BM) * ((n_it + kGroup - 1) / kGroup);
     const int64_t grid = std::min<int64_t>(max_units, (int64_t)n_cu * 3);  // three workgroups fit a CU
     hipLaunchKernelGGL(k_refine_count, dim3((unsigned)grid), dim3(NT), 0, s, users, items, n_item, ld, K, rows_user,
-                       rows_thr, n_rows_dev, max_rows, cnt);
+                       rows_thr, n_rows_dev, max_rows, cnt, t);
     return hipGetLastError();
 }
 
 hipError_t launch_gemv_panels(hipStream_t s, const float *usersT, int64_t n_user, int32_t ld, int32_t K,
-                              const float *q, int32_t nq, float *qip) {
+                              const float *q, int32_t nq, float *qip, uint64_t *t) {
     if (n_user <= 0 || nq <= 0) return hipSuccess;
     const int64_t n_panel = (n_user + 63) / 64;
     const unsigned grid = (unsigned)((n_panel + 3) / 4);
     const size_t smem = sizeof(float) * (size_t)nq * K;
-    if (nq <= 1) hipLaunchKernelGGL(k_gemv_panels<1>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip);
-    else if (nq <= 2) hipLaunchKernelGGL(k_gemv_panels<2>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip);
-    else if (nq <= 4) hipLaunchKernelGGL(k_gemv_panels<4>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip);
-    else if (nq <= 8) hipLaunchKernelGGL(k_gemv_panels<8>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip);
-    else hipLaunchKernelGGL(k_gemv_panels<16>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip);
+    if (nq <= 1) hipLaunchKernelGGL(k_gemv_panels<1>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
+    else if (nq <= 2) hipLaunchKernelGGL(k_gemv_panels<2>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
+    else if (nq <= 4) hipLaunchKernelGGL(k_gemv_panels<4>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
+    else if (nq <= 8) hipLaunchKernelGGL(k_gemv_panels<8>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
+    else hipLaunchKernelGGL(k_gemv_panels<16>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
     return hipGetLastError();
 }
 

@@ -178,7 +178,8 @@ __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScree
 // The same counts from exact scores qip[b * n_user + u].
 __global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ qip, int64_t n_user, int32_t nq, float eps,
                                                       const float *__restrict__ gvals, int32_t n_fine, int64_t n_s,
-                                                      int64_t stride, uint32_t *__restrict__ hist) {
+                                                      int64_t stride, uint32_t *__restrict__ hist, uint64_t *t) {
+    stamp(t);
     constexpr int UB = 64, QB = 16;
     __shared__ float sG[UB * GP];
     __shared__ uint32_t sH[QB * GW];
@@ -705,7 +706,8 @@ __global__ void __launch_bounds__(NT) k_list_exact(const float *__restrict__ use
                                                    const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
                                                    int64_t n_user, const QueryInfo *__restrict__ qi,
                                                    uint32_t *__restrict__ bk_c, float *__restrict__ qip,
-                                                   uint32_t *__restrict__ ghist) {
+                                                   uint32_t *__restrict__ ghist, uint64_t *t) {
+    stamp(t);
     __shared__ int32_t col[GW];
     __shared__ f32x4 sd[SCORES ? 1 : NT / 64][2][SCORES ? 1 : 64 * DP / 4];
     if (threadIdx.x < GW) col[threadIdx.x] = threadIdx.x < kMaxFine ? fc.col[threadIdx.x] : 0;
@@ -810,7 +812,9 @@ __global__ void __launch_bounds__(NT) k_list_final(const int32_t *__restrict__ c
                                                    QueryInfo *__restrict__ qi, int32_t *__restrict__ cand_user,
                                                    int32_t *__restrict__ cand_rank, int32_t *__restrict__ refine_total,
                                                    int32_t *__restrict__ refine_user, int32_t *__restrict__ refine_query,
-                                                   float *__restrict__ refine_thr, int32_t *__restrict__ cnt) {
+                                                   float *__restrict__ refine_thr, int32_t *__restrict__ cnt,
+                                                   uint64_t *t) {
+    stamp(t);
     const int64_t n = min((int64_t)ctr->n_list, list_cap);
     const int lane = threadIdx.x & 63;
     for (int64_t i0 = (int64_t)blockIdx.x * NT; i0 < n; i0 += (int64_t)gridDim.x * NT) {
@@ -946,7 +950,7 @@ hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L) {
     const unsigned qg = (unsigned)((L.nq + 15) / 16);
     const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n_s + 63) / 64, (8 * L.n_cu + qg - 1) / qg));
     hipLaunchKernelGGL(k_sample_scores, dim3(gx, qg), dim3(NT), 0, s, L.qip, L.n_user, L.nq, L.eps, L.gvals, L.fc.n,
-                       n_s, L.stride, L.hist);
+                       n_s, L.stride, L.hist, L.t_bound);
     hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
                        L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
     hipLaunchKernelGGL(k_list_scores,
@@ -962,10 +966,10 @@ hipError_t launch_list_exact(hipStream_t s, const ListLaunch &L, const float *us
     const dim3 grid((unsigned)(L.n_cu * 16));  // a multiple of the 8 XCDs (grid-stride over the list)
     if (scores)
         hipLaunchKernelGGL(k_list_exact<true>, grid, dim3(NT), 0, s, users, queries, ld, dim, table, L.S, L.eps, L.gvals,
-                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist);
+                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist, nullptr);
     else
         hipLaunchKernelGGL(k_list_exact<false>, grid, dim3(NT), 0, s, users, queries, ld, dim, table, L.S, L.eps, L.gvals,
-                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist);
+                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist, L.t_bound);
     hipLaunchKernelGGL(k_list_kth, dim3((unsigned)L.nq), dim3(NT), 0, s, L.ghist, L.S, L.eps > 0.0f ? 0 : 1, L.fc,
                        L.list_cap, L.qi, L.ctr);
     return hipGetLastError();
@@ -977,7 +981,7 @@ hipError_t launch_list_final(hipStream_t s, const ListLaunch &L, const uint32_t 
     if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_list_final, dim3((unsigned)(L.n_cu * 16)), dim3(NT), 0, s, L.cl_u, L.cl_b, bk_c, L.qip, L.ctr,
                        L.list_cap, L.S, ranks, n_item, L.n_user, L.qi, cand_user, cand_rank, refine_total, refine_user,
-                       refine_query, refine_thr, cnt);
+                       refine_query, refine_thr, cnt, L.t_prune);
     return hipGetLastError();
 }
 

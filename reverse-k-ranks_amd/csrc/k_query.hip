@@ -76,7 +76,8 @@ __device__ __forceinline__ void bucket_pair(const float *row, int32_t S, float q
 // grid: (user blocks, queries).  bk[b * U + u] = b_lo | b_hi << 16.
 __global__ void __launch_bounds__(256) k_bounds(const float *__restrict__ qip, const float *__restrict__ table,
                                                 int64_t n_user, int32_t S, float eps, int ref_mode,
-                                                uint32_t *__restrict__ bk) {
+                                                uint32_t *__restrict__ bk, uint64_t *t) {
+    stamp(t);
     const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t b = blockIdx.y;
     if (u >= n_user) return;
@@ -94,7 +95,8 @@ __global__ void __launch_bounds__(256) k_bounds(const float *__restrict__ qip, c
 // probe the same index of different rows, fall in different LDS banks.
 __global__ void __launch_bounds__(256) k_bounds_lds(const float *__restrict__ qip, const float *__restrict__ table,
                                                     int64_t n_user, int32_t S, int32_t nq, int32_t ut, float eps,
-                                                    int ref_mode, uint32_t *__restrict__ bk) {
+                                                    int ref_mode, uint32_t *__restrict__ bk, uint64_t *t) {
+    stamp(t);
     extern __shared__ float rows[];  // ut x (S + 1)
     const int64_t u0 = (int64_t)blockIdx.x * ut;
     const int64_t nu = min((int64_t)ut, n_user - u0);
@@ -150,7 +152,8 @@ __device__ uint32_t wg_excl_scan(uint32_t v, uint32_t *red, uint32_t *total) {
 // same != 0: b_lo == b_hi for every user (exact output, eps = 0), so only
 // h_lo is built and the selection reads it for both.
 __global__ void __launch_bounds__(NT) k_hist_chunks(const uint32_t *__restrict__ bk, int64_t n_user, int32_t S,
-                                                    int same, int64_t cu, uint32_t *__restrict__ ghist) {
+                                                    int same, int64_t cu, uint32_t *__restrict__ ghist, uint64_t *t) {
+    stamp(t);
     __shared__ uint32_t h_lo[SMAXQ + 1];
     __shared__ uint32_t h_hi[SMAXQ + 1];
     const int64_t b = blockIdx.y;
@@ -271,6 +274,86 @@ __global__ void __launch_bounds__(NT) k_hist_kth(const uint32_t *__restrict__ gh
         q.pad = Lk;
     }
     qi[b] = q;
+}
+
+// Exact output over at most kSmallUsers users, one workgroup per query: the
+// bucket pairs stay in LDS between the search, the histogram, the k-th bound
+// and the candidates.  Through global memory these are five launches of 2 to 5
+// us and a wait for the candidate counts, three quarters of a one-query call
+// over 1000 users.  A query's candidates take their place from one atomic on the
+// batch's counter.
+__global__ void __launch_bounds__(NT) k_small_select(const float *__restrict__ qip, const float *__restrict__ table,
+                                                     int32_t n_user, int32_t S, const int32_t *__restrict__ ranks,
+                                                     int64_t n_item, float eps, QueryInfo *__restrict__ qi,
+                                                     ListCounters *__restrict__ ctr, int32_t *__restrict__ cand_user,
+                                                     int32_t *__restrict__ cand_rank, int32_t *__restrict__ refine_user,
+                                                     int32_t *__restrict__ refine_query, float *__restrict__ refine_thr,
+                                                     int32_t *__restrict__ cnt) {
+    __shared__ uint32_t bk[kSmallUsers], h_lo[SMAXQ + 1], h_hi[SMAXQ + 1], red[NW + 1];
+    __shared__ int32_t s_beta, s_off, s_fill, s_refine;
+    stamp(&ctr->t[kTimeBound]);
+    const int64_t b = blockIdx.x;
+    const float *qb = qip + b * n_user;
+    for (int i = threadIdx.x; i <= S; i += NT) { h_lo[i] = 0; h_hi[i] = 0; }
+    if (threadIdx.x == 0) { s_beta = S; s_fill = 0; s_refine = 0; }
+    __syncthreads();
+    for (int32_t u = threadIdx.x; u < n_user; u += NT) {
+        uint32_t lo, hi;
+        bucket_pair(table + u * (int64_t)S, S, qb[u], eps, 0, lo, hi);
+        bk[u] = lo | (hi << 16);
+        atomicAdd(&h_lo[lo], 1u);
+        atomicAdd(&h_hi[hi], 1u);
+    }
+    __syncthreads();
+    const uint32_t k = (uint32_t)qi[b].topk;
+    const int32_t per = (S + 1 + NT - 1) / NT;
+    const int32_t j0 = threadIdx.x * per, j1 = min(S + 1, j0 + per);
+    uint32_t mine = 0, tot;
+    for (int32_t j = j0; j < j1; ++j) mine += h_lo[j];
+    uint32_t cum = wg_excl_scan(mine, red, &tot);
+    if (cum < k && cum + mine >= k)
+        for (int32_t j = j0; j < j1; ++j) {
+            cum += h_lo[j];
+            if (cum >= k) { s_beta = j; break; }
+        }
+    __syncthreads();
+    const int32_t beta = s_beta;
+    uint32_t nh = 0;
+    for (int32_t j = j0; j < min(j1, beta + 1); ++j) nh += h_hi[j];
+    (void)wg_excl_scan(nh, red, &tot);
+    if (threadIdx.x == 0) s_off = atomicAdd(&ctr->n_cand, (int32_t)tot);
+    __syncthreads();
+    for (int32_t u = threadIdx.x; u < n_user; u += NT) {
+        const int32_t blo = (int32_t)(bk[u] & 0xFFFFu), bhi = (int32_t)(bk[u] >> 16);
+        if (bhi > beta) continue;
+        const int32_t slot = s_off + atomicAdd(&s_fill, 1);
+        const int32_t lbs = blo == S ? (int32_t)n_item : ranks[blo];
+        const int32_t ubs = bhi == 0 ? 0 : ranks[bhi - 1] + 1;
+        int32_t rank = lbs;
+        if (lbs != ubs) {
+            const int32_t r = atomicAdd(&ctr->n_refine, 1);
+            atomicAdd(&s_refine, 1);
+            rank = ~r;
+            refine_user[r] = u;
+            refine_query[r] = (int32_t)b;
+            refine_thr[r] = qb[u];
+            cnt[r] = 0;
+        }
+        cand_user[slot] = u;
+        cand_rank[slot] = rank;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        QueryInfo q = qi[b];
+        q.beta = q.gamma = beta;
+        q.mode = MODE_EXACT;
+        q.n_cand = (int32_t)tot;
+        q.n_settled = 0;
+        q.n_refine = s_refine;
+        q.fill = (int32_t)tot;
+        q.cand_off = s_off;
+        qi[b] = q;
+    }
 }
 
 // Exclusive offsets of each query's [settled | candidates] slice.
@@ -459,7 +542,9 @@ __device__ __forceinline__ uint64_t make_key(int32_t rank, const int32_t *__rest
 __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, const int32_t *__restrict__ cand_user,
                                              const int32_t *__restrict__ cand_rank, const int32_t *__restrict__ cnt,
                                              const float *__restrict__ qip, int64_t n_user, int32_t max_k, int32_t *__restrict__ out_user,
-                                             int32_t *__restrict__ out_rank, float *__restrict__ out_qip) {
+                                             int32_t *__restrict__ out_rank, float *__restrict__ out_qip,
+                                             uint64_t *t_start, uint64_t *t_end) {
+    stamp(t_start);
     __shared__ uint64_t keys[SORT_CAP];
     __shared__ uint32_t hist[256];
     __shared__ uint64_t sel_prefix;
@@ -483,7 +568,10 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
     }
     const int32_t need = k - ns;
     const int64_t nc = q.n_cand;
-    if (need <= 0 || nc <= 0) return;
+    if (need <= 0 || nc <= 0) {
+        if (t_end && threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned long long *>(t_end), wall_clock64());
+        return;
+    }
     const int32_t *cu = cand_user + q.cand_off + q.n_settled;
     const int32_t *cr = cand_rank + q.cand_off + q.n_settled;
     const int32_t take = (int32_t)(nc < need ? nc : need);
@@ -540,6 +628,7 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
         orank[ns + i] = (int32_t)(key >> 32);
         oq[ns + i] = qb[u];
     }
+    if (t_end && threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned long long *>(t_end), wall_clock64());
 }
 
 
@@ -852,30 +941,41 @@ __global__ void __launch_bounds__(CNT) k_coarse_exact_upd(
 }  // namespace
 
 hipError_t launch_bounds(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S, int32_t nq,
-                         float eps, int ref_mode, uint32_t *bk) {
+                         float eps, int ref_mode, uint32_t *bk, uint64_t *t) {
     if (n_user <= 0 || nq <= 0) return hipSuccess;
     const int ut = bounds_rows_per_wg(S);
     if (nq >= 4 && ut > 0) {
         const unsigned grid = (unsigned)((n_user + ut - 1) / ut);
         hipLaunchKernelGGL(k_bounds_lds, dim3(grid), dim3(256), (size_t)ut * (S + 1) * 4, s, qip, table, n_user, S, nq,
-                           ut, eps, ref_mode, bk);
+                           ut, eps, ref_mode, bk, t);
         return hipGetLastError();
     }
     dim3 grid((unsigned)((n_user + 255) / 256), (unsigned)nq);
-    hipLaunchKernelGGL(k_bounds, grid, dim3(256), 0, s, qip, table, n_user, S, eps, ref_mode, bk);
+    hipLaunchKernelGGL(k_bounds, grid, dim3(256), 0, s, qip, table, n_user, S, eps, ref_mode, bk, t);
     return hipGetLastError();
 }
 
 hipError_t launch_hist_kth(hipStream_t s, const uint32_t *bk, int64_t n_user, int32_t S, const int32_t *ranks,
                            int64_t n_item, int32_t nq, int output_mode, int same, int64_t cu, uint32_t *ghist,
-                           QueryInfo *qi) {
+                           QueryInfo *qi, uint64_t *t) {
     if (nq <= 0) return hipSuccess;
     hipError_t e = hipMemsetAsync(ghist, 0, sizeof(uint32_t) * 2 * (size_t)(S + 1) * nq, s);
     if (e != hipSuccess) return e;
     const unsigned n_chunk = (unsigned)((n_user + cu - 1) / cu);
     if (n_user > 0)
-        hipLaunchKernelGGL(k_hist_chunks, dim3(n_chunk, (unsigned)nq), dim3(NT), 0, s, bk, n_user, S, same, cu, ghist);
+        hipLaunchKernelGGL(k_hist_chunks, dim3(n_chunk, (unsigned)nq), dim3(NT), 0, s, bk, n_user, S, same, cu, ghist, t);
     hipLaunchKernelGGL(k_hist_kth, dim3((unsigned)nq), dim3(NT), 0, s, ghist, S, same, ranks, n_item, output_mode, qi);
+    return hipGetLastError();
+}
+
+hipError_t launch_small_select(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
+                               const int32_t *ranks, int64_t n_item, int32_t nq, float eps, QueryInfo *qi,
+                               ListCounters *ctr, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
+                               int32_t *refine_query, float *refine_thr, int32_t *cnt) {
+    if (nq <= 0) return hipSuccess;
+    if (n_user > kSmallUsers || S > kMaxSample) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_small_select, dim3((unsigned)nq), dim3(NT), 0, s, qip, table, (int32_t)n_user, S, ranks, n_item,
+                       eps, qi, ctr, cand_user, cand_rank, refine_user, refine_query, refine_thr, cnt);
     return hipGetLastError();
 }
 
@@ -905,10 +1005,10 @@ hipError_t launch_compact(hipStream_t s, const uint32_t *bk, const float *qip, i
 
 hipError_t launch_topk(hipStream_t s, const QueryInfo *qi, int32_t nq, const int32_t *cand_user,
                        const int32_t *cand_rank, const int32_t *cnt, const float *qip, int64_t n_user, int32_t max_k,
-                       int32_t *out_user, int32_t *out_rank, float *out_qip) {
+                       int32_t *out_user, int32_t *out_rank, float *out_qip, uint64_t *t_start, uint64_t *t_end) {
     if (nq <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_topk, dim3((unsigned)nq), dim3(NT), 0, s, qi, cand_user, cand_rank, cnt, qip, n_user, max_k,
-                       out_user, out_rank, out_qip);
+                       out_user, out_rank, out_qip, t_start, t_end);
     return hipGetLastError();
 }
 

@@ -63,7 +63,8 @@ union Frag {
 __global__ void k_prep_items(const float *__restrict__ items, int64_t n_item, int32_t ld, int32_t K, int32_t Kp,
                              uint16_t *__restrict__ hi, uint16_t *__restrict__ lo, float *__restrict__ norm,
                              float *__restrict__ cs, const float *__restrict__ rho, double g1, double g_rule,
-                             uint32_t *__restrict__ zero64) {
+                             uint32_t *__restrict__ zero64, uint64_t *t) {
+    stamp(t);
     const int64_t p = (int64_t)blockIdx.x * blockDim.y + threadIdx.y;
     if (p >= n_item) return;
     if (zero64)
@@ -135,12 +136,14 @@ struct ScreenParams {
     int32_t *recheck_n;        // appended rechecks (may exceed capacity)
     int4 *recheck;             // (row, item, s^ bits, 0)
     int64_t recheck_cap;
+    uint64_t *t;
 };
 
 // RB row blocks of 16 per wave: 2 (32 rows, two waves per SIMD) or 4 (64
 // rows, one wave per SIMD, half the LDS reads per matrix-core operation).
 template <int KS, int RB>
 __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenParams P) {
+    stamp(P.t);
     constexpr int RW = 4 * 16 * RB;  // rows per workgroup
     // items per LDS stage: 32 keeps the two prefetch register sets at 8 KS
     // VGPRs
@@ -405,7 +408,8 @@ __global__ void k_recheck(const float *__restrict__ users, const float *__restri
                           const int32_t *__restrict__ rows_user, const float *__restrict__ rows_thr,
                           const int32_t *__restrict__ rows_query, const int32_t *__restrict__ recheck_n,
                           const int4 *__restrict__ recheck, int64_t cap, int32_t *__restrict__ cnt,
-                          int32_t *__restrict__ q_recheck, uint32_t *__restrict__ max_err_bits) {
+                          int32_t *__restrict__ q_recheck, uint32_t *__restrict__ max_err_bits, uint64_t *t) {
+    stamp(t);
     const int64_t n = min((int64_t)*recheck_n, cap);
     float worst = 0.0f;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -664,12 +668,12 @@ __global__ void __launch_bounds__(NT, coarse_first_pass_wgs(KS)) k_ip_coarse(IpC
 
 hipError_t launch_prep_items(hipStream_t s, const float *items, int64_t n_item, int32_t ld, int32_t K, int32_t Kp,
                              uint16_t *hi, uint16_t *lo, float *norm, float *cs, const float *rho, double g1,
-                             double g_rule, uint32_t *zero64) {
+                             double g_rule, uint32_t *zero64, uint64_t *t) {
     if (n_item <= 0) return hipSuccess;
     if (cs && !rho) return hipErrorInvalidValue;
     dim3 block(32, 8);
     hipLaunchKernelGGL(k_prep_items, dim3((unsigned)((n_item + 7) / 8)), block, 0, s, items, n_item, ld, K, Kp, hi, lo,
-                       norm, cs, rho, g1, g_rule, zero64);
+                       norm, cs, rho, g1, g_rule, zero64, t);
     return hipGetLastError();
 }
 
@@ -708,6 +712,7 @@ hipError_t launch_refine_screen(hipStream_t s, const ScreenLaunch &L) {
     P.recheck_n = L.recheck_n;
     P.recheck = reinterpret_cast<int4 *>(L.recheck);
     P.recheck_cap = L.recheck_cap;
+    P.t = L.t;
     P.target_units = std::max<int64_t>(1, L.target_units);
     P.chunk_items = std::max(1, L.chunk_items);
     // persistent grid: enough workgroups to fill the device, never more than
@@ -741,10 +746,10 @@ hipError_t launch_refine_screen(hipStream_t s, const ScreenLaunch &L) {
 hipError_t launch_recheck(hipStream_t s, const float *users, const float *items, int32_t ld, int32_t K,
                           const int32_t *rows_user, const float *rows_thr, const int32_t *rows_query,
                           const int32_t *recheck_n, const void *recheck, int64_t cap, int32_t *cnt,
-                          int32_t *q_recheck, uint32_t *max_err_bits) {
+                          int32_t *q_recheck, uint32_t *max_err_bits, uint64_t *t) {
     if (cap <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_recheck, dim3(2048), dim3(256), 0, s, users, items, ld, K, rows_user, rows_thr, rows_query,
-                       recheck_n, reinterpret_cast<const int4 *>(recheck), cap, cnt, q_recheck, max_err_bits);
+                       recheck_n, reinterpret_cast<const int4 *>(recheck), cap, cnt, q_recheck, max_err_bits, t);
     return hipGetLastError();
 }
 

@@ -108,8 +108,8 @@ DataSnap snap_of(const Ctx *c) {
     d.qtable = c->qtable;
     d.qranks = c->qranks;
     d.n_qs = c->n_qs;
-    d.fine = fine_columns(c);
-    d.guards = guard_columns(c);
+    d.fine = c->fine;
+    d.guards = c->guards;
     d.gvals = c->gvals;
     d.gcols = c->gcols;
     d.gpitch = c->gpitch;
@@ -117,7 +117,7 @@ DataSnap snap_of(const Ctx *c) {
     d.n_sample = c->n_sample;
     d.table_eps = c->table_eps;
     d.qcol = c->qcol;
-    d.hrk = std::make_shared<const std::vector<int32_t>>(c->qtable ? c->h_qranks : c->h_ranks);
+    d.hrk = c->hrk;
     for (int j = 0; j < 8; ++j) d.ins_gmax[j] = c->ins_gmax[j];
     if (c->qsrp_users && c->qsrp_n_user == c->n_user) {
         d.qsrp_users = c->qsrp_users;
@@ -173,16 +173,14 @@ int guard_table_columns(const std::vector<int32_t> &hr, int32_t *col) {
     }
     return n;
 }
-const std::vector<int32_t> &searched_ranks(const Ctx *c) { return c->qtable ? c->h_qranks : c->h_ranks; }
 }  // namespace
 
 // The guard columns and, inside each of their bins and past the last one, up
 // to 7 more spaced geometrically in rank: neighbouring fine columns differ by a
 // factor of about 1.2 in rank (4 between guard columns), which is how much a
 // list is longer than it has to be.
-FineCols fine_columns(const Ctx *c) {
+static FineCols fine_columns(const std::vector<int32_t> &hr) {
     FineCols fc{};
-    const std::vector<int32_t> &hr = searched_ranks(c);
     if (hr.empty()) return fc;
     int32_t gcol[8];
     const int ng = guard_table_columns(hr, gcol);
@@ -207,23 +205,22 @@ FineCols fine_columns(const Ctx *c) {
     return fc;
 }
 
-GuardCols guard_columns(const Ctx *c) {
-    GuardCols gc{};
-    const FineCols fc = fine_columns(c);
-    for (int f = 0; f < fc.n; ++f)
-        if ((fc.coarse >> f) & 1) {
-            gc.col[gc.n] = fc.col[f];
-            gc.idx[gc.n++] = f;
+void set_table_columns(Ctx *c) {
+    c->hrk = std::make_shared<const std::vector<int32_t>>(c->qtable ? c->h_qranks : c->h_ranks);
+    c->fine = fine_columns(*c->hrk);
+    c->guards = GuardCols{};
+    for (int f = 0; f < c->fine.n; ++f)
+        if ((c->fine.coarse >> f) & 1) {
+            c->guards.col[c->guards.n] = c->fine.col[f];
+            c->guards.idx[c->guards.n++] = f;
         }
-    return gc;
 }
 
 int refresh_guard_values(Ctx *c, int64_t u0, int64_t n) {
     if (!c->gvals || n <= 0) return RKR_OK;
-    const FineCols fc = fine_columns(c);
     const float *T = c->qtable ? c->qtable : c->table;
     const int64_t S = c->qtable ? c->n_qs : c->n_sample;
-    RKR_HIP(c, launch_gather_guards(c->stream, T, S, fc, u0, n, c->gvals, c->gcols, c->gpitch));
+    RKR_HIP(c, launch_gather_guards(c->stream, T, S, c->fine, u0, n, c->gvals, c->gcols, c->gpitch));
     return RKR_OK;
 }
 
@@ -351,6 +348,7 @@ void free_table(Ctx *c) {
     c->n_sample = c->n_qs = 0;
     c->h_ranks.clear();
     c->h_qranks.clear();
+    set_table_columns(c);
     c->table_eps = 0.0f;
 }
 
@@ -481,6 +479,8 @@ int rkr_create(int device, size_t mem_budget_bytes, rkr_ctx **out) {
     int n_cu = 0;
     if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && n_cu > 0)
         c->n_cu = n_cu;
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0) c->clock_khz = khz;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return RKR_ERR_HIP; }
     for (auto &e : c->ev)
         if (hipEventCreate(&e) != hipSuccess) { rkr_destroy(c); return RKR_ERR_HIP; }
@@ -757,6 +757,8 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
         }
     }
 
+    set_table_columns(c);
+
     // user batch: the score block [nb x n_item] lives in HBM between the
     // GEMM and the selection; size it from the remaining budget (the
     // reference sizes its batch from free memory the same way,
@@ -815,6 +817,7 @@ int rkr_set_table(rkr_ctx *c, const int32_t *ranks, int32_t S, const float *tabl
     c->n_sample = S;
     c->h_ranks.assign(ranks, ranks + S);
     c->table_eps = eps;
+    set_table_columns(c);
     RKR_HIP(c, hipMemcpy(c->ranks, ranks, sizeof(int32_t) * S, hipMemcpyHostToDevice));
     RKR_HIP(c, hipMemcpy(c->table, table, sizeof(float) * (size_t)c->n_user * S, hipMemcpyHostToDevice));
     if ((rc = refresh_guard_values(c, 0, c->n_user))) { free_table(c); return rc; }
@@ -1449,17 +1452,25 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     const bool list = listable && !upd &&
                       (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
     const bool list_mfma = list && mfma;
+    // a few users: bounds to candidates in one kernel, its arrays sized for
+    // every pair (6 MB at most)
+    const bool small = !list && !upd && !qsrp && mode == RKR_OUTPUT_EXACT && U <= kSmallUsers && nqb * U <= (1 << 18);
+    // stages are timed by their kernels, or by events where other kernels open them
+    const bool use_ev = upd || qsrp;
     int rc;
     const BatchIo io_max(nqb, ld, max_k);
     if ((rc = ensure(c, sl.io, io_max.end, "queries and outputs"))) return rc;
     if ((rc = ensure(c, sl.qip, sizeof(float) * (size_t)nqb * U, "query scores"))) return rc;
     // coarse bucket rows: whole row blocks of 128 users, plus a spare row
     const int64_t ldc = (U + 127) / 128 * 128;
-    if (!list && (rc = ensure(c, sl.bk, std::max((pair_bytes - 4) * (size_t)U * nqb, (size_t)ldc * (nqb + 1)),
+    if (!list && !small && (rc = ensure(c, sl.bk, std::max((pair_bytes - 4) * (size_t)U * nqb, (size_t)ldc * (nqb + 1)),
                               "bucket pairs")))
         return rc;
     if ((rc = ensure(c, sl.hist, sizeof(uint32_t) * hist_words((int32_t)nqb, S), "bound histograms"))) return rc;
     if (qsrp && (rc = ensure(c, sl.q_split, sizeof(float) * (size_t)nqb * (dv.qsrp_ldr + 3), "QSRP query rows")))
+        return rc;
+    if (small && ((rc = ensure(c, sl.cand, sizeof(int32_t) * 2 * (size_t)(nqb * U), "candidates")) ||
+                  (rc = ensure(c, sl.refine_idx, sizeof(int32_t) * 4 * (size_t)(nqb * U), "refine rows"))))
         return rc;
     if (listable && mfma &&
         (rc = ensure(c, sl.q_split, (sizeof(uint16_t) * 2 * c->kp + 2 * sizeof(float)) * (size_t)nqb, "query BF16 rows")))
@@ -1503,6 +1514,9 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         int32_t *o_rank = o_user + (size_t)nq * max_k;
         float *o_qip = reinterpret_cast<float *>(o_rank + (size_t)nq * max_k);
         int32_t *refine_total = &ctr->n_refine;
+        uint64_t *const t = use_ev ? nullptr : ctr->t;  // stage stamps
+        auto at = [t](int i) { return t ? t + i : nullptr; };
+        auto event = [&](int i) { return use_ev ? hipEventRecord(sl.ev[i], sl.stream) : hipSuccess; };
         float *hq = reinterpret_cast<float *>(stg);
         QueryInfo *hqi = reinterpret_cast<QueryInfo *>(stg + io.info);
         const int32_t *h_qrecheck = reinterpret_cast<const int32_t *>(stg + io.recheck);
@@ -1513,14 +1527,11 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         float *qip = reinterpret_cast<float *>(sl.qip.p);
         uint32_t *bk = reinterpret_cast<uint32_t *>(sl.bk.p);
 
-        float q_amax = 0.0f;  // largest |query value| of the batch (validated finite)
+        // largest |query value| of the batch (validated finite)
+        const double q_amax = max_abs(queries + (size_t)q0 * d, (size_t)nq * d);
         for (int32_t i = 0; i < nq; ++i) {
-            const float *src = queries + (size_t)(q0 + i) * d;
             float *dst = &hq[(size_t)i * ld];
-            for (int32_t k = 0; k < d; ++k) {
-                dst[k] = src[k];
-                q_amax = std::max(q_amax, std::fabs(src[k]));
-            }
+            std::memcpy(dst, queries + (size_t)(q0 + i) * d, sizeof(float) * d);
             for (int32_t k = d; k < ld; ++k) dst[k] = 0.0f;
             hqi[i] = QueryInfo{};
             hqi[i].topk = topk[q0 + i];
@@ -1557,18 +1568,18 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             LL.hist = reinterpret_cast<uint32_t *>(sl.list_info.p);
             LL.order = reinterpret_cast<int32_t *>(LL.hist + 64 * (size_t)nq);
             LL.colg = LL.order + nq;
-            LL.qi = qi; LL.ctr = ctr; LL.ghist = ghist;
+            LL.qi = qi; LL.ctr = ctr; LL.ghist = ghist; LL.t_bound = at(kTimeBound); LL.t_prune = at(kTimePrune);
             LL.cl_u = reinterpret_cast<int32_t *>(sl.list.p);
             LL.cl_b = LL.cl_u + list_cap;
             bk_c = reinterpret_cast<uint32_t *>(LL.cl_b + list_cap);
         }
         if (list_mfma) {
             RKR_HIP(c, launch_prep_items(sl.stream, q_in, nq, ld, d, c->kp, q_hi, q_lo, qn, qcs, dv.rho, c->coarse_g1,
-                                         c->coarse_grule, LL.hist));
+                                         c->coarse_grule, LL.hist, at(kTimeIp)));
             RKR_HIP(c, launch_list_screen(sl.stream, LL));
-            RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
+            RKR_HIP(c, event(2));
             RKR_HIP(c, launch_list_exact(sl.stream, LL, dv.users, q_in, ld, d, T, false, bk_c));
-            RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+            RKR_HIP(c, event(3));
         } else if (coarse) {
             // coarse buckets on the matrix cores, the coarse k-th bound and
             // list sizes; exact scores and bound values of the listed users
@@ -1581,7 +1592,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             L.ldc = ldc; L.spare_row = nqb;
             L.grid_cap = (int64_t)c->n_cu * coarse_first_pass_wgs(c->kp / 32);
             RKR_HIP(c, launch_ip_coarse(sl.stream, L));
-            RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
+            RKR_HIP(c, event(2));
             // coarse chunks: a fixed user count, so launches over few queries
             // still fill the device and the list stays chunk-major
             const int64_t ccu = kCoarseChunk;
@@ -1650,7 +1661,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                                                cl_b, n_listed, dv.side_ins, dv.n_ins, dv.ld_ins, dv.side_del, dv.n_del,
                                                dv.ld_del, U, lbv, ubv, qip));
             RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));
-            RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+            RKR_HIP(c, event(3));
         } else if (qsrp) {
             // QSRP screen: rotated queries and their part norms, the left-part
             // scores over the first check_dim dimensions, bounds from the
@@ -1664,7 +1675,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             RKR_HIP(c, launch_qsrp_qnorms(sl.stream, qrot, dv.qsrp_ldr, q_in, ld, d, dv.qsrp_cd, nq, qpn));
             RKR_HIP(c, launch_scores_store(sl.stream, dv.qsrp_users, U, dv.qsrp_ldr, qrot, nq, dv.qsrp_ldr,
                                            dv.qsrp_cd, qip, U, false));
-            RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
+            RKR_HIP(c, event(2));
             // eps widens the interval as the exact path widens its search; the
             // floor covers gradual underflow in the d products of a score
             const float absf = std::nextafter((float)((double)eps + (double)d * std::ldexp(1.0, -140)), INFINITY);
@@ -1672,37 +1683,38 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                                           dv.n_sample, use_q ? dv.qcol : nullptr, S, bk));
             RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode, 0, cu, ghist, qi));
             RKR_HIP(c, launch_qsrp_exact(sl.stream, dv.users, q_in, ld, d, T, S, eps, U, nq, qi, qip, bk));
-            RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+            RKR_HIP(c, event(3));
             RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode, 0, cu, ghist, qi));
         } else {
             // <u, q> for every (query, user): qip[b * U + u]
             if (nq <= 16 && (size_t)nq * d * sizeof(float) <= 65536)
-                RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip));
-            else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false));
-            RKR_HIP(c, hipEventRecord(sl.ev[2], sl.stream));
+                RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip, at(kTimeIp)));
+            else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false, at(kTimeIp)));
+            RKR_HIP(c, event(2));
             if (list) {
                 RKR_HIP(c, hipMemsetAsync(LL.hist, 0, sizeof(uint32_t) * 64 * (size_t)nq, sl.stream));
                 RKR_HIP(c, launch_list_scores(sl.stream, LL));
                 RKR_HIP(c, launch_list_exact(sl.stream, LL, dv.users, q_in, ld, d, T, true, bk_c));
-                RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+                RKR_HIP(c, event(3));
             } else if (upd) {
                 RKR_HIP(c, launch_bounds_upd(sl.stream, qip, T, U, S, R, dv.n_item_base, eps, dv.side_ins,
                                              dv.n_ins, dv.ld_ins, dv.side_del, dv.n_del, dv.ld_del, nq, lbv, ubv));
-                RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+                RKR_HIP(c, event(3));
                 RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));
-            } else {
-                RKR_HIP(c, launch_bounds(sl.stream, qip, T, U, S, nq, eps, mode == RKR_OUTPUT_REFERENCE ? 1 : 0, bk));
-                RKR_HIP(c, hipEventRecord(sl.ev[3], sl.stream));
+            } else if (!small) {
+                RKR_HIP(c, launch_bounds(sl.stream, qip, T, U, S, nq, eps, mode == RKR_OUTPUT_REFERENCE ? 1 : 0, bk,
+                                         at(kTimeBound)));
+                RKR_HIP(c, event(3));
                 RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode,
-                                           (mode == RKR_OUTPUT_EXACT && eps == 0.0f) ? 1 : 0, cu, ghist, qi));
+                                           (mode == RKR_OUTPUT_EXACT && eps == 0.0f) ? 1 : 0, cu, ghist, qi, at(kTimePrune)));
             }
         }
         // With lists every candidate is a listed pair, so the list's entries
         // bound the candidate and refine arrays and the batch goes on without
         // waiting for the counts (the refinement and top-k read them on the
         // device).  Otherwise the counts size them.
-        int64_t total = list_cap, total_cand = list_cap;
-        if (!list) {
+        int64_t total = small ? nqb * U : list_cap, total_cand = total;
+        if (!list && !small) {
             RKR_HIP(c, launch_offsets(sl.stream, qi, nq, refine_total));
             RKR_HIP(c, hipMemcpyAsync(hqi, qi, sizeof(QueryInfo) * nq, hipMemcpyDeviceToHost, sl.stream));
             RKR_HIP(c, hipStreamSynchronize(sl.stream));
@@ -1733,7 +1745,10 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         float *refine_thr = reinterpret_cast<float *>(refine_query + rcap);
         int32_t *cnt = reinterpret_cast<int32_t *>(refine_thr + rcap);
 
-        if (list)
+        if (small)
+            RKR_HIP(c, launch_small_select(sl.stream, qip, T, U, S, R, I, nq, eps, qi, ctr, cand_user, cand_rank, refine_user,
+                                           refine_query, refine_thr, cnt));
+        else if (list)
             RKR_HIP(c, launch_list_final(sl.stream, LL, bk_c, R, I, cand_user, cand_rank, refine_total, refine_user,
                                          refine_query, refine_thr, cnt));
         else if (upd)
@@ -1755,8 +1770,8 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 RKR_HIP(c, hipMemsetAsync(q_recheck, 0, sizeof(int32_t) * (size_t)nq, sl.stream));
                 RKR_HIP(c, hipMemsetAsync(&ctr->n_recheck, 0, sizeof(int32_t) * 2, sl.stream));
             }
-            RKR_HIP(c, hipEventRecord(sl.ev[4], sl.stream));
-            // events 4..8 bracket exactly the refinement (or screening) kernel
+            RKR_HIP(c, event(4));
+            // events 4..8, or the stamps, bracket exactly the refinement (or screening) kernel
             if (screened) {
                 ScreenLaunch L{};
                 L.users = dv.users; L.user_norm = dv.user_norm;
@@ -1769,19 +1784,22 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 L.target_units = (int64_t)c->n_cu * 8;
                 L.grid_cap = (int64_t)c->n_cu * 4;
                 L.chunk_items = c->screen_chunk > 0 ? c->screen_chunk : (1 << 30);
+                L.t = at(kTimeRefine);
                 L.rows_per_wave = c->screen_rows > 0 ? c->screen_rows : (c->kp / 32 >= 6 ? 64 : 32);  // d > 160: 32 rows spill
                 RKR_HIP(c, launch_refine_screen(sl.stream, L));
-                RKR_HIP(c, hipEventRecord(sl.ev[8], sl.stream));
+                RKR_HIP(c, event(8));
                 RKR_HIP(c, launch_recheck(sl.stream, dv.users, dv.items, ld, d, refine_user, refine_thr, refine_query,
-                                          &ctr->n_recheck, sl.recheck.p, rec_cap, cnt, q_recheck, &ctr->max_err_bits));
+                                          &ctr->n_recheck, sl.recheck.p, rec_cap, cnt, q_recheck, &ctr->max_err_bits,
+                                          at(kTimeRecheck)));
             } else {
                 RKR_HIP(c, launch_refine_count(sl.stream, dv.users, dv.items, I, ld, d, refine_user, refine_thr,
-                                               refine_total, (int64_t)rcap, cnt));
-                RKR_HIP(c, hipEventRecord(sl.ev[8], sl.stream));
+                                               refine_total, (int64_t)rcap, cnt, at(kTimeRefine)));
+                RKR_HIP(c, event(8));
             }
-            RKR_HIP(c, hipEventRecord(sl.ev[5], sl.stream));
-            RKR_HIP(c, launch_topk(sl.stream, qi, nq, cand_user, cand_rank, cnt, qip, U, max_k, o_user, o_rank, o_qip));
-            RKR_HIP(c, hipEventRecord(sl.ev[6], sl.stream));
+            RKR_HIP(c, event(5));
+            RKR_HIP(c, launch_topk(sl.stream, qi, nq, cand_user, cand_rank, cnt, qip, U, max_k, o_user, o_rank, o_qip, at(kTimeTopk),
+                                   at(kTimeEnd)));
+            RKR_HIP(c, event(6));
             // query info, counters and outputs in one copy (the device layout)
             RKR_HIP(c, hipMemcpyAsync(stg + io.info, dev + io.info, io.end - io.info, hipMemcpyDeviceToHost, sl.stream));
             RKR_HIP(c, hipEventRecord(sl.ev[7], sl.stream));
@@ -1834,13 +1852,31 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             }
         }
         tm.h2d_ms += ev_ms(sl.ev, 0, 1);
-        tm.ip_ms += ev_ms(sl.ev, 1, 2);
-        tm.bound_ms += ev_ms(sl.ev, 2, 3);
-        tm.prune_ms += ev_ms(sl.ev, 3, 4);
-        tm.refine_ms += ev_ms(sl.ev, 4, 8);
-        tm.recheck_ms += ev_ms(sl.ev, 8, 5);
-        tm.topk_ms += ev_ms(sl.ev, 5, 6);
-        tm.d2h_ms += ev_ms(sl.ev, 6, 7);
+        if (use_ev) {
+            tm.ip_ms += ev_ms(sl.ev, 1, 2);
+            tm.bound_ms += ev_ms(sl.ev, 2, 3);
+            tm.prune_ms += ev_ms(sl.ev, 3, 4);
+            tm.refine_ms += ev_ms(sl.ev, 4, 8);
+            tm.recheck_ms += ev_ms(sl.ev, 8, 5);
+            tm.topk_ms += ev_ms(sl.ev, 5, 6);
+            tm.d2h_ms += ev_ms(sl.ev, 6, 7);
+        } else {
+            // a stage without a kernel of its own starts with the next
+            uint64_t ts[kTimeEnd + 1];
+            for (int i = 0; i <= kTimeEnd; ++i) ts[i] = hctr->t[i];
+            for (int i = kTimeEnd - 1; i > 0; --i)
+                if (ts[i] == 0) ts[i] = ts[i + 1];
+            auto ms = [&](int i) { return ts[i + 1] > ts[i] ? (double)(ts[i + 1] - ts[i]) / c->clock_khz : 0.0; };
+            tm.ip_ms += ms(kTimeIp);
+            tm.bound_ms += ms(kTimeBound);
+            tm.prune_ms += ms(kTimePrune);
+            tm.refine_ms += ms(kTimeRefine);
+            tm.recheck_ms += ms(kTimeRecheck);
+            tm.topk_ms += ms(kTimeTopk);
+            // what is left of the time after the upload
+            const double kernels = ts[kTimeEnd] > ts[kTimeIp] ? (double)(ts[kTimeEnd] - ts[kTimeIp]) / c->clock_khz : 0.0;
+            tm.d2h_ms += std::max(0.0, ev_ms(sl.ev, 1, 7) - kernels);
+        }
         tm.n_batches += 1;
         tm.n_refined += hctr->n_refine;
         if (screened) {

@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -49,6 +50,24 @@ struct Slot {
     DeviceBuf qip, bk, cand, refine_idx, recheck, hist;
     DeviceBuf q_split, list_info, list;  // threshold and coarse lists
     PinnedBuf stage;                     // host side of the batch copies
+};
+
+// Guard columns of the coarse bounds (updates pending): col[j] the table
+// column, idx[j] its place in the guard row.
+struct GuardCols {
+    int32_t col[8];
+    int32_t idx[8];
+    int32_t n;
+};
+// Fine columns of the searched table, ascending; each user keeps their values
+// in a guard row of kGuardRow floats (-inf past n).  The guard columns are
+// among them (bit f of coarse: column f is one).
+constexpr int kGuardRow = 64;
+constexpr int kMaxFine = 63;
+struct FineCols {
+    int32_t col[kMaxFine];
+    int32_t n;
+    uint64_t coarse;
 };
 
 struct Ctx {
@@ -127,6 +146,11 @@ struct Ctx {
     float *gvals = nullptr;
     float *gcols = nullptr;     // the same values by column: [kGuardRow][u_cap at allocation]
     int64_t gpitch = 0;
+    // columns of the guard rows, the guard columns among them and the searched
+    // table's ranks, set with the table
+    FineCols fine{};
+    GuardCols guards{};
+    std::shared_ptr<const std::vector<int32_t>> hrk;
     int dense_top = 2;          // query table mode (RKR_OPT_DENSE_TOP)
 
     // screened form: hi/lo BF16 item rows (n_item x kp), norm bounds
@@ -142,6 +166,7 @@ struct Ctx {
     double coarse_g1 = 0.0, coarse_grule = 0.0;
     float *rho = nullptr;
     int n_cu = 256;
+    double clock_khz = 1e5;  // rate of the device clock (stamp())
 
     // QSRP screen (rkr_qsrp_build): users rotated into the SVD basis, the query
     // rotation, and per-user norms and regression parameters (kQsrp* rows of
@@ -192,15 +217,20 @@ void set_defer_frees(bool on);
 void release_retired(Ctx *c);
 
 // Largest |x| over a row-major matrix; -1 when a value is NaN or infinite.
+// Magnitudes order as their bits, so this is an integer maximum the compiler
+// vectorises (a floating maximum with an early exit took 1 ns per value, 150 us
+// of a 1000-query call).
 inline double max_abs(const float *x, size_t n) {
-    double m = 0.0;
+    int32_t m = 0;
     for (size_t i = 0; i < n; ++i) {
-        const float v = x[i];
-        if (!std::isfinite(v)) return -1.0;
-        const double a = std::fabs((double)v);
-        if (a > m) m = a;
+        int32_t b;
+        std::memcpy(&b, x + i, sizeof(b));
+        b &= 0x7FFFFFFF;
+        m = b > m ? b : m;
     }
-    return m;
+    float f;
+    std::memcpy(&f, &m, sizeof(f));
+    return std::isfinite(f) ? (double)f : -1.0;
 }
 
 // Update-path rank bound values stay below kMaxBoundValue (two-level 11-bit
@@ -220,23 +250,6 @@ inline float screen_abs_floor(int32_t kp, double max_abs_user, double max_abs_it
     return std::nextafter((float)absf, INFINITY);
 }
 
-// Guard columns of the coarse bounds (updates pending): col[j] the table
-// column, idx[j] its place in the guard row.
-struct GuardCols {
-    int32_t col[8];
-    int32_t idx[8];
-    int32_t n;
-};
-// Fine columns of the searched table, ascending; each user keeps their values
-// in a guard row of kGuardRow floats (-inf past n).  The guard columns are
-// among them (bit f of coarse: column f is one).
-constexpr int kGuardRow = 64;
-constexpr int kMaxFine = 63;
-struct FineCols {
-    int32_t col[kMaxFine];
-    int32_t n;
-    uint64_t coarse;
-};
 // Workgroups per CU of the coarse pass (256 threads, users' BF16 hi
 // halves in VGPRs) for Kp = 32 ks: its launch bound and its persistent grid.
 // (Five fit at ks <= 5 only by spilling the staged query pieces: slower.)
@@ -283,9 +296,8 @@ struct DataSnap {
     float qsrp_gcd = 0.0f, qsrp_crot = 0.0f;
 };
 DataSnap snap_of(const Ctx *c);
-// Fine columns and guard columns of the context's searched table.
-FineCols fine_columns(const Ctx *c);
-GuardCols guard_columns(const Ctx *c);
+// Sets Ctx::fine, guards and hrk for the searched table's ranks.
+void set_table_columns(Ctx *c);
 // The table over the current items at sampled ranks S (build_table), and the
 // same at uniform ranks of the current n_sample (rebuild_table): the pending
 // item updates fold into the new table; keep_update_buffers leaves their
@@ -337,16 +349,16 @@ int dev_alloc_t(Ctx *c, T **p, size_t n, const char *what) {
 // C[n * ldc + m] (query-major when A = users, B = queries), or C[m * ldc + n].
 hipError_t launch_scores_store(hipStream_t s, const float *A, int64_t M, int32_t lda,
                                const float *B, int64_t N, int32_t ldb, int32_t K, float *C, int64_t ldc,
-                               bool c_row_major_m);
+                               bool c_row_major_m, uint64_t *t = nullptr);
 // Small-batch <u,q>: qip[b * n_user + u] for b < nq (nq <= 16), users in
 // 64-user panels.
 hipError_t launch_gemv_panels(hipStream_t s, const float *usersT, int64_t n_user, int32_t ld, int32_t K,
-                              const float *q, int32_t nq, float *qip);
+                              const float *q, int32_t nq, float *qip, uint64_t *t = nullptr);
 // Refinement count: cnt[r] = #{item p : score(user(r), p) > thr(r)} for every
 // refine row r < *n_rows_dev (device-side count, persistent grid).
 hipError_t launch_refine_count(hipStream_t s, const float *users, const float *items, int64_t n_item,
                                int32_t ld, int32_t K, const int32_t *rows_user, const float *rows_thr,
-                               const int32_t *n_rows_dev, int64_t max_rows, int32_t *cnt);
+                               const int32_t *n_rows_dev, int64_t max_rows, int32_t *cnt, uint64_t *t = nullptr);
 // Transpose users into 64-user panels.
 hipError_t launch_make_panels(hipStream_t s, const float *users, int64_t n_user, int32_t ld, float *usersT);
 
@@ -371,6 +383,7 @@ struct ScreenLaunch {
     int64_t grid_cap;       // workgroups of the persistent grid
     int32_t chunk_items;    // most items per work-unit chunk (L2-resident slice)
     int32_t rows_per_wave;  // 32 or 64 refine rows per wavefront
+    uint64_t *t = nullptr;
 };
 // BF16 hi/lo rows (Kp columns, zero padded) and, when norm is non-null, row
 // norm upper bounds; used for items, queries and users.  With cs (queries of
@@ -380,7 +393,7 @@ struct ScreenLaunch {
 // per row are cleared.
 hipError_t launch_prep_items(hipStream_t s, const float *items, int64_t n_item, int32_t ld, int32_t K, int32_t Kp,
                              uint16_t *hi, uint16_t *lo, float *norm, float *cs = nullptr, const float *rho = nullptr,
-                             double g1 = 0.0, double g_rule = 0.0, uint32_t *zero64 = nullptr);
+                             double g1 = 0.0, double g_rule = 0.0, uint32_t *zero64 = nullptr, uint64_t *t = nullptr);
 // Users' norm upper bounds; with rho (device), raises *rho to at least every
 // user's ||u - bf16(u)|| / ||u||.
 hipError_t launch_user_norms(hipStream_t s, const float *users, int64_t n_user, int32_t ld, int32_t K, float *norm,
@@ -407,7 +420,7 @@ hipError_t launch_ip_coarse(hipStream_t s, const CoarseLaunch &L);
 hipError_t launch_recheck(hipStream_t s, const float *users, const float *items, int32_t ld, int32_t K,
                           const int32_t *rows_user, const float *rows_thr, const int32_t *rows_query,
                           const int32_t *recheck_n, const void *recheck, int64_t cap, int32_t *cnt,
-                          int32_t *q_recheck, uint32_t *max_err_bits);
+                          int32_t *q_recheck, uint32_t *max_err_bits, uint64_t *t = nullptr);
 int screen_max_kp();
 
 // ---- selection (k_select.hip) ---------------------------------------------
@@ -463,7 +476,19 @@ struct alignas(64) ListCounters {
     int32_t n_refine;       // refine rows
     int32_t n_recheck;      // screened form: undecided pairs
     uint32_t max_err_bits;  // screened form: largest screen error seen
+    int32_t pad;
+    uint64_t t[8];          // device clock at the stages' starts (enum below)
 };
+// Stages of a batch timed by its kernels: the first kernel of a stage writes
+// the device clock when it starts, the top-k when its last workgroup ends.  (An
+// event record between two kernels costs about 3 us; six of them were a tenth
+// of a one-query call.)
+enum { kTimeIp = 0, kTimeBound, kTimePrune, kTimeRefine, kTimeRecheck, kTimeTopk, kTimeEnd };
+#ifdef __HIPCC__
+__device__ __forceinline__ void stamp(uint64_t *t) {
+    if (t && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0) *t = wall_clock64();
+}
+#endif
 
 // One transfer each way per device batch: the queries, the query info with
 // topk, the recheck counts and counters go up, and the last three come back
@@ -506,6 +531,7 @@ struct ListLaunch {
     int32_t *order, *colg;   // nq slots, nq / 4 threshold columns
     QueryInfo *qi;
     ListCounters *ctr;
+    uint64_t *t_bound, *t_prune;  // stamps (or null)
     uint32_t *ghist;         // nq x 2 (S + 1) bucket histograms
     int32_t *cl_u, *cl_b;
 };
@@ -602,10 +628,17 @@ inline size_t hist_words(int32_t nq, int32_t S) {
 }
 
 hipError_t launch_bounds(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
-                         int32_t nq, float eps, int ref_mode, uint32_t *bk);
+                         int32_t nq, float eps, int ref_mode, uint32_t *bk, uint64_t *t = nullptr);
 hipError_t launch_hist_kth(hipStream_t s, const uint32_t *bk, int64_t n_user, int32_t S, const int32_t *ranks,
                            int64_t n_item, int32_t nq, int output_mode, int same, int64_t cu, uint32_t *ghist,
-                           QueryInfo *qi);
+                           QueryInfo *qi, uint64_t *t = nullptr);
+// Exact output without updates over at most kSmallUsers users: bounds, the k-th
+// bound and the candidates, one workgroup per query.
+constexpr int64_t kSmallUsers = 4096;
+hipError_t launch_small_select(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
+                               const int32_t *ranks, int64_t n_item, int32_t nq, float eps, QueryInfo *qi,
+                               ListCounters *ctr, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
+                               int32_t *refine_query, float *refine_thr, int32_t *cnt);
 // Coarse bounds with updates pending (k_query.hip): the coarse k-th bound and
 // list size per query (cq[b] = {beta_c, count, offset, fill}) and the listed
 // users.  cb rows are ldc bytes (ldc % 16 == 0, bytes past n_user unread);
@@ -638,7 +671,8 @@ hipError_t launch_compact(hipStream_t s, const uint32_t *bk, const float *qip, i
 // cnt: the refine rows' counts
 hipError_t launch_topk(hipStream_t s, const QueryInfo *qi, int32_t nq, const int32_t *cand_user,
                        const int32_t *cand_rank, const int32_t *cnt, const float *qip, int64_t n_user, int32_t max_k,
-                       int32_t *out_user, int32_t *out_rank, float *out_qip);
+                       int32_t *out_user, int32_t *out_rank, float *out_qip, uint64_t *t_start = nullptr,
+                       uint64_t *t_end = nullptr);
 
 // ---- update path (k_update.hip) ---------------------------------------------
 // QSRP screen kernels (k_qsrp.hip).  qn holds 3 floats per query: upper bounds

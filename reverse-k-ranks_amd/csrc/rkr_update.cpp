@@ -336,7 +336,7 @@ int rkr::refresh_ins_guard_max(Ctx *c) {
     const float *T = c->qtable ? c->qtable : c->table;
     const int32_t S = c->qtable ? c->n_qs : c->n_sample;
     if (!c->n_ins || !T || c->n_user <= 0) return RKR_OK;
-    const GuardCols gc = guard_columns(c);
+    const GuardCols &gc = c->guards;
     if (gc.n <= 0) return RKR_OK;
     int rc;
     if ((rc = ensure(c, c->upd_scratch, std::max<size_t>(c->upd_scratch.bytes, 64), "update scratch"))) return rc;

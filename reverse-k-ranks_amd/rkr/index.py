@@ -29,7 +29,7 @@ def _f32(a):
 
 
 def _ptr(a):
-    return a.ctypes.data_as(C.c_void_p)
+    return a.ctypes.data  # an int: the argument types are c_void_p
 
 
 @dataclass

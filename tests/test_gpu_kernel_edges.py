@@ -109,3 +109,28 @@ def test_threshold_lists_eps_and_sample(gpu_index_factory, form):
     res = _lists_and_search(idx, queries, ks)
     assert res.users.shape == (24, max(ks))
     idx.close()
+
+
+@pytest.mark.parametrize("U,nq,dense", [(1, 1, 2), (63, 5, 0), (1024, 7, 2), (4096, 64, 2), (4096, 65, 0), (4097, 3, 2)])
+def test_few_users(orc, gpu_index_factory, U, nq, dense):
+    """Calls on either side of the one-kernel selection's limits (4096 users,
+    2^18 pairs), with ties, a zero user and k up to every user, against brute force."""
+    _case(f"few users U={U} nq={nq} dense={dense}")
+    rng = np.random.default_rng(U + nq)
+    I, d = 600, 12
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    users[U // 3] = 0.0
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    items[100:140] = items[0]
+    queries = np.concatenate([items[rng.integers(0, 160, (nq + 1) // 2)],
+                              rng.standard_normal((nq // 2, d), dtype=np.float32)])
+    ks = [int(min(U, k)) for k in rng.integers(1, 200, nq)]
+    ks[0] = min(U, 4096)
+    idx, _ = gpu_index_factory(users, items, 40, dense_top=dense)
+    res = idx.query(queries, ks)
+    bu, br, bq = orc.bruteforce(orc.normalize_users(users), items, queries, max(ks))
+    for i, k in enumerate(ks):
+        assert np.array_equal(res.users[i, :k], bu[i, :k]) and np.array_equal(res.ranks[i, :k], br[i, :k])
+        assert np.array_equal(res.qips[i, :k], bq[i, :k])
+        assert np.all(res.users[i, k:] == -1)
+    idx.close()
