@@ -134,3 +134,19 @@ def test_few_users(orc, gpu_index_factory, U, nq, dense):
         assert np.array_equal(res.qips[i, :k], bq[i, :k])
         assert np.all(res.users[i, k:] == -1)
     idx.close()
+
+
+@pytest.mark.parametrize("U,S,nq", [(300, 600, 1), (3000, 40, 2), (12_000, 4, 3)])
+def test_refine_group_sizes(orc, gpu_index_factory, U, S, nq):
+    """Refinement with few rows (a unit is one item tile), some, and more than a full group for every workgroup."""
+    _case(f"refine groups U={U} S={S} nq={nq}")
+    rng = np.random.default_rng(U)
+    users = rng.standard_normal((U, 18), dtype=np.float32)
+    items = rng.standard_normal((5001, 18), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, S)
+    queries = items[rng.choice(5001, nq, replace=False)]
+    res = idx.query(queries, 10)
+    bu, br, _ = orc.bruteforce(orc.normalize_users(users), items, queries, 10)
+    for i in range(nq):
+        print(f"refined {res.stats[i]['n_refine_user']} users", flush=True)
+        assert np.array_equal(res.users[i], bu[i]) and np.array_equal(res.ranks[i], br[i])
