@@ -53,6 +53,7 @@ thread_local bool tl_defer_frees = false;
 }
 
 void set_defer_frees(bool on) { tl_defer_frees = on; }
+bool defer_frees() { return tl_defer_frees; }
 
 // The size recorded at allocation is what returns to the budget; `bytes` is
 // only used for a pointer this context did not allocate.
@@ -375,7 +376,6 @@ void free_data(Ctx *c) {
     c->users = c->usersT = c->items = nullptr;
     c->n_user = c->n_item = 0;
     c->dim = c->ld = 0;
-    c->h_users.clear();
 }
 
 void free_bufs(Ctx *c, std::initializer_list<DeviceBuf *> bufs) {
@@ -422,10 +422,10 @@ namespace {
 // FP32 normalisation exactly as VectorMatrix::vectorNormalize
 // (src/include/struct/VectorMatrix.hpp:51-66).  This file is compiled with
 // -ffp-contract=off, so x*x is rounded before the add.
-void normalize_rows(float *u, int64_t n, int32_t d) {
+void normalize_rows(float *u, int64_t n, int32_t d, int64_t stride) {
 #pragma omp parallel for schedule(static)
     for (int64_t i = 0; i < n; ++i) {
-        float *row = u + i * d;
+        float *row = u + i * stride;
         float l2 = 0.0f;
         for (int32_t j = 0; j < d; ++j) {
             const float sq = row[j] * row[j];
@@ -590,7 +590,7 @@ int rkr_sync(rkr_ctx *c) {
 
 int rkr_normalize_users(float *users, int64_t n_user, int32_t dim) {
     if (!users || n_user < 0 || dim <= 0) return RKR_ERR_INVALID;
-    normalize_rows(users, n_user, dim);
+    normalize_rows(users, n_user, dim, dim);
     return RKR_OK;
 }
 
@@ -632,11 +632,9 @@ int rkr_set_data(rkr_ctx *c, const float *users, int64_t n_user, const float *it
     c->normalize_users = normalize_users != 0;
     c->dim = dim;
     c->ld = ld;
-    // host staging with padding
-    c->h_users.assign(users, users + (size_t)n_user * dim);
-    if (normalize_users) normalize_rows(c->h_users.data(), n_user, dim);
-    // upload row-major with rows padded to ld floats (pad columns zero)
-    auto upload = [&](const float *src, int64_t n, float **dst, const char *what) -> int {
+    // upload row-major with rows padded to ld floats (pad columns zero), users
+    // normalised on the way
+    auto upload = [&](const float *src, int64_t n, float **dst, bool normalize, const char *what) -> int {
         int rc = dev_alloc_t(c, dst, (size_t)n * ld, what);
         if (rc) return rc;
         const int64_t chunk = 65536;
@@ -645,13 +643,14 @@ int rkr_set_data(rkr_ctx *c, const float *users, int64_t n_user, const float *it
             const int64_t nr = std::min<int64_t>(chunk, n - r0);
             for (int64_t r = 0; r < nr; ++r)
                 std::memcpy(&tmp[(size_t)r * ld], src + (size_t)(r0 + r) * dim, sizeof(float) * dim);
+            if (normalize) normalize_rows(tmp.data(), nr, dim, ld);
             RKR_HIP(c, hipMemcpy(*dst + r0 * ld, tmp.data(), sizeof(float) * (size_t)nr * ld, hipMemcpyHostToDevice));
         }
         return RKR_OK;
     };
-    int rc = upload(c->h_users.data(), n_user, &c->users, "users");
+    int rc = upload(users, n_user, &c->users, normalize_users != 0, "users");
     if (rc) { free_data(c); return rc; }
-    rc = upload(items, n_item, &c->items, "items");
+    rc = upload(items, n_item, &c->items, false, "items");
     if (rc) { free_data(c); return rc; }
     rc = dev_alloc_t(c, &c->usersT, (size_t)((n_user + 63) / 64) * 64 * ld, "user panels");
     if (rc) { free_data(c); return rc; }

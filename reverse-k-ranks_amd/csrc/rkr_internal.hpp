@@ -97,7 +97,6 @@ struct Ctx {
     float *users = nullptr;     // n_user x ld, row-major (normalised)
     float *usersT = nullptr;    // panels of 64 users: [panel][ld][64]
     float *items = nullptr;     // n_item x ld, row-major (original order)
-    std::vector<float> h_users; // host copy (normalised)
     double max_abs_user = 1.0;  // bound on |u_i| after normalisation
 
     // update path: the table describes the base item set; inserted items and
@@ -211,8 +210,10 @@ constexpr double kQsrpPhiDevErr = 2e-6;
 // Frees the QSRP screen's buffers (the table or the users changed).
 void free_qsrp(Ctx *c);
 
-// Frees made by this thread go to Ctx::retired instead of hipFree.
+// Frees made by this thread go to Ctx::retired instead of hipFree: batches may be
+// reading what an update of this thread replaces, so nothing is moved in place.
 void set_defer_frees(bool on);
+bool defer_frees();
 // Releases the retired buffers (call only when no batch can still read them).
 void release_retired(Ctx *c);
 
@@ -308,8 +309,9 @@ int rebuild_table(Ctx *c);
 int refresh_guard_values(Ctx *c, int64_t u0, int64_t n);
 // New (unfilled) guard arrays for `cap` users; the old ones go through dev_free.
 int alloc_guards(Ctx *c, int64_t cap);
-// Recomputes Ctx::ins_gmax after inserted items or users changed.
-int refresh_ins_guard_max(Ctx *c);
+// Recomputes Ctx::ins_gmax after inserted items changed (u0 = 0), or raises it
+// for the new users u0 and up.
+int refresh_ins_guard_max(Ctx *c, int64_t u0);
 // Ranks of the query table: the sample ranks and the dense top ranks below
 // n_item, ascending; empty when they would exceed kMaxSample.
 // mode 1: all of 0..255, every 8th to 1023, every 32nd to 4095; mode 2: every

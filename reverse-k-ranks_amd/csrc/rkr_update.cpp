@@ -194,6 +194,10 @@ int reserve_list(Ctx *c, float **arr, int64_t *cap, int64_t n, int64_t need, con
 // into one side array of every user.  The result is written to the spare (or
 // a fresh buffer when the rows must grow), never to the rows batches read.
 int update_side(Ctx *c, bool ins_side, const float *X, int64_t n, int sign) {
+    if (sign < 0 && n == (ins_side ? c->n_ins : c->n_del)) {  // every score leaves
+        (ins_side ? c->n_ins : c->n_del) = 0;
+        return RKR_OK;
+    }
     float **side = ins_side ? &c->side_ins : &c->side_del;
     float **spare = ins_side ? &c->side_ins_spare : &c->side_del_spare;
     int32_t *ld = ins_side ? &c->ld_ins : &c->ld_del;
@@ -314,6 +318,28 @@ void init_item_map(Ctx *c) {
     c->base_deleted.assign((size_t)c->n_item_base, 0);
 }
 
+// Moves the kept rows idx[0..n) (device, ascending, idx[j] > first + j) of an
+// array to rows first, first + 1, ... of the same array, through a scratch
+// block: a block's rows are all read before it is written, and its places lie
+// before every row still to be read.
+constexpr size_t kMoveBytes = (size_t)64 << 20;
+int64_t move_block(int64_t n, int64_t ld) {
+    return std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)(kMoveBytes / sizeof(float)) / ld));
+}
+// upd_scratch holds move_block(n, ld) rows.
+int move_rows_down(Ctx *c, float *arr, int64_t ld, int64_t first, const int64_t *idx, int64_t n) {
+    if (!arr || n <= 0) return RKR_OK;
+    const int64_t blk = move_block(n, ld);
+    float *tmp = reinterpret_cast<float *>(c->upd_scratch.p);
+    for (int64_t j = 0; j < n; j += blk) {
+        const int64_t m = std::min(blk, n - j);
+        RKR_HIP(c, launch_gather_rows(c->stream, arr, ld, idx + j, m, ld, tmp, ld));
+        RKR_HIP(c, hipMemcpyAsync(arr + (first + j) * ld, tmp, sizeof(float) * (size_t)(m * ld), hipMemcpyDeviceToDevice,
+                                  c->stream));
+    }
+    return RKR_OK;
+}
+
 // Row compaction of a per-user array ([u_cap][ld], w floats used per row)
 // into a new buffer of the same shape.
 int keep_user_rows(Ctx *c, float **arr, int64_t w, int64_t ld, const int64_t *d_keep, int64_t n_keep,
@@ -331,19 +357,23 @@ int keep_user_rows(Ctx *c, float **arr, int64_t w, int64_t ld, const int64_t *d_
 
 }  // namespace
 
-int rkr::refresh_ins_guard_max(Ctx *c) {
-    for (int j = 0; j < 8; ++j) c->ins_gmax[j] = 0;
+int rkr::refresh_ins_guard_max(Ctx *c, int64_t u0) {
+    if (u0 == 0)
+        for (int j = 0; j < 8; ++j) c->ins_gmax[j] = 0;
     const float *T = c->qtable ? c->qtable : c->table;
     const int32_t S = c->qtable ? c->n_qs : c->n_sample;
-    if (!c->n_ins || !T || c->n_user <= 0) return RKR_OK;
+    if (!c->n_ins || !T || c->n_user <= u0) return RKR_OK;
     const GuardCols &gc = c->guards;
     if (gc.n <= 0) return RKR_OK;
     int rc;
     if ((rc = ensure(c, c->upd_scratch, std::max<size_t>(c->upd_scratch.bytes, 64), "update scratch"))) return rc;
     int32_t *d = reinterpret_cast<int32_t *>(c->upd_scratch.p);
-    RKR_HIP(c, launch_ins_guard_max(c->stream, T, c->n_user, S, gc, c->side_ins, c->n_ins, c->ld_ins, d));
-    RKR_HIP(c, hipMemcpyAsync(c->ins_gmax, d, sizeof(int32_t) * 8, hipMemcpyDeviceToHost, c->stream));
+    int32_t h[8];
+    RKR_HIP(c, launch_ins_guard_max(c->stream, T + u0 * S, c->n_user - u0, S, gc, c->side_ins + u0 * c->ld_ins, c->n_ins,
+                                    c->ld_ins, d));
+    RKR_HIP(c, hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     RKR_HIP(c, hipStreamSynchronize(c->stream));
+    for (int j = 0; j < 8; ++j) c->ins_gmax[j] = std::max(c->ins_gmax[j], h[j]);
     return RKR_OK;
 }
 
@@ -385,7 +415,7 @@ int rkr_insert_items(rkr_ctx *c, const float *items, int64_t n) {
     if (c->kp) c->screen_abs = screen_abs_floor(c->kp, c->max_abs_user, c->max_abs_item);
     for (int64_t j = 0; j < n; ++j) c->cur_src.push_back(-(1 + (int64_t)ins0 + j));
     c->n_item = I0 + n;
-    return rkr::refresh_ins_guard_max(c);
+    return rkr::refresh_ins_guard_max(c, 0);
 }
 
 int rkr_delete_items(rkr_ctx *c, const int64_t *ids, int64_t n) {
@@ -438,6 +468,29 @@ int rkr_delete_items(rkr_ctx *c, const int64_t *ids, int64_t n) {
         std::vector<int64_t> keep;
         for (int64_t j = 0; j < n_ins_old; ++j)
             if (!gone[j]) keep.push_back(j);
+        if (del_base.empty() && c->n_del == 0 && !defer_frees()) {
+            // the current items are the base and then the inserted items, and
+            // no batch is running: only the inserted rows move
+            const int64_t I0 = c->n_item_base, nk = (int64_t)keep.size();
+            if (nk > 0) {
+                float *kept = nullptr;
+                if ((rc = gather_items(c, c->items_ins, keep, &kept))) return rc;
+                if (!(rc = copy_rows(c, c->items_ins, ld, kept, ld, nk, ld))) rc = copy_rows(c, c->items + I0 * ld, ld, kept, ld, nk, ld);
+                if (!rc && c->kp) {
+                    const hipError_t e = launch_prep_items(c->stream, c->items + I0 * ld, nk, ld, c->dim, c->kp,
+                                                           c->item_hi + I0 * c->kp, c->item_lo + I0 * c->kp, c->item_norm + I0);
+                    if (e != hipSuccess) rc = set_err(c, RKR_ERR_HIP, hipGetErrorString(e));
+                }
+                const hipError_t e = hipStreamSynchronize(c->stream);
+                dev_free(c, kept, 0);
+                if (rc) return rc;
+                RKR_HIP(c, e);
+            }
+            c->n_item = I0 + nk;
+            c->cur_src.resize((size_t)I0);
+            for (int64_t j = 0; j < nk; ++j) c->cur_src.push_back(-(1 + j));
+            return RKR_OK;
+        }
         // the kept rows go to a new list: the old one may still be read
         float *next = nullptr;
         if ((rc = dev_alloc_t(c, &next, (size_t)std::max<int64_t>(c->ins_cap, 1) * ld, "inserted items"))) return rc;
@@ -524,12 +577,11 @@ int rkr_insert_users(rkr_ctx *c, const float *users, int64_t n) {
         RKR_HIP(c, launch_sort_rows_desc(c->stream, rows, n, ns, lds));
     }
     RKR_HIP(c, hipStreamSynchronize(c->stream));
-    c->h_users.insert(c->h_users.end(), h.begin(), h.end());
     c->max_abs_user_raw = mu_raw;
     c->max_abs_user = mu_new;
     if (c->kp) c->screen_abs = screen_abs_floor(c->kp, c->max_abs_user, c->max_abs_item);
     c->n_user = U1;
-    return rkr::refresh_ins_guard_max(c);
+    return rkr::refresh_ins_guard_max(c, U0);  // the other users' counts stand
 }
 
 int rkr_delete_users(rkr_ctx *c, const int64_t *ids, int64_t n) {
@@ -552,7 +604,38 @@ int rkr_delete_users(rkr_ctx *c, const int64_t *ids, int64_t n) {
     for (int64_t u = 0; u < U0; ++u)
         if (!gone[u]) keep.push_back(u);
     const int64_t nk = (int64_t)keep.size();
+    int64_t first = 0;  // users before it keep their rows
+    while (first < nk && keep[first] == first) ++first;
     int64_t *d_keep = nullptr;
+    if (!defer_frees()) {
+        // no batch is running: later users shift down inside the arrays.
+        // (Copies of every array, 1.6 GB of query table at 100k users, and
+        // their allocation took 19 ms whatever was deleted.)
+        const int64_t n_mv = nk - first;
+        const struct { float *p; int64_t ld; } arr[] = {
+            {c->users, ld}, {c->table, c->n_sample}, {c->qtable, c->n_qs}, {c->n_ins ? c->side_ins : nullptr, c->ld_ins},
+            {c->n_del ? c->side_del : nullptr, c->ld_del}, {c->user_norm, 1},
+            {reinterpret_cast<float *>(c->user_hi), c->kp / 2}, {reinterpret_cast<float *>(c->user_lo), c->kp / 2}};
+        if (n_mv > 0) {
+            // everything that can be refused for memory comes before the first move
+            size_t need = 0;
+            for (const auto &x : arr)
+                if (x.p) need = std::max(need, sizeof(float) * (size_t)(move_block(n_mv, x.ld) * x.ld));
+            if ((rc = ensure(c, c->upd_scratch, need, "update scratch")) ||
+                (rc = dev_alloc_t(c, &d_keep, (size_t)n_mv, "gather index")))
+                return rc;
+            RKR_HIP(c, hipMemcpyAsync(d_keep, keep.data() + first, sizeof(int64_t) * n_mv, hipMemcpyHostToDevice, c->stream));
+            for (const auto &x : arr)
+                if (!rc) rc = move_rows_down(c, x.p, x.ld, first, d_keep, n_mv);
+        }
+        c->n_user = nk;
+        if (!rc && c->gvals) rc = refresh_guard_values(c, first, n_mv);
+        const int64_t p0 = first / 64;  // first panel that changes
+        if (!rc) RKR_HIP(c, launch_make_panels(c->stream, c->users + p0 * 64 * ld, nk - p0 * 64, ld, c->usersT + p0 * 64 * ld));
+        RKR_HIP(c, hipStreamSynchronize(c->stream));
+        dev_free(c, d_keep, 0);
+        return rc;
+    }
     if ((rc = dev_alloc_t(c, &d_keep, (size_t)nk, "gather index"))) return rc;
     RKR_HIP(c, hipMemcpyAsync(d_keep, keep.data(), sizeof(int64_t) * nk, hipMemcpyHostToDevice, c->stream));
     // SampleSearchUpdate::DeleteUser (SampleSearchUpdate.hpp:89-109): later users shift down
@@ -564,10 +647,6 @@ int rkr_delete_users(rkr_ctx *c, const int64_t *ids, int64_t n) {
     if (!rc) rc = keep_user_rows(c, &c->side_del, c->n_del, c->ld_del, d_keep, nk, "side array");
     dev_free(c, d_keep, 0);
     if (rc) return rc;
-    std::vector<float> hu((size_t)nk * c->dim);
-    for (int64_t i = 0; i < nk; ++i)
-        std::memcpy(&hu[(size_t)i * c->dim], &c->h_users[(size_t)keep[i] * c->dim], sizeof(float) * c->dim);
-    c->h_users.swap(hu);
     c->n_user = nk;
     float *panels = nullptr, *unorm = nullptr;
     uint16_t *uhi = nullptr, *ulo = nullptr;

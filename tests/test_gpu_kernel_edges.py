@@ -150,3 +150,70 @@ def test_refine_group_sizes(orc, gpu_index_factory, U, S, nq):
     for i in range(nq):
         print(f"refined {res.stats[i]['n_refine_user']} users", flush=True)
         assert np.array_equal(res.users[i], bu[i]) and np.array_equal(res.ranks[i], br[i])
+
+
+@pytest.mark.parametrize("U,which", [(500, "first"), (500, "middle"), (500, "last"), (500, "all_but_one"),
+                                     (70_000, "first_and_last")])
+def test_delete_users_in_place(orc, gpu_index_factory, U, which):
+    """Users leave from every place (also more rows than one move block holds,
+    and a tail that is not touched), with inserted and deleted items pending."""
+    _case(f"delete users U={U} {which}")
+    from test_gpu_update import Mirror
+    rng = np.random.default_rng(U)
+    d, I = 20, 600
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 300)
+    m = Mirror(orc, users, items)
+    new = rng.standard_normal((40, d), dtype=np.float32)
+    idx.insert_items(new)
+    m.insert_items(new)
+    idx.delete_items(np.array([3, 50], np.int64))
+    m.delete_items([3, 50])
+    queries = items[rng.choice(I, 5, replace=False)]
+    gone = {"first": np.arange(0, 70), "middle": np.array([130, 131, 200]), "last": np.arange(440, 500),
+            "all_but_one": np.arange(1, 500), "first_and_last": np.array([0, 33_000, U - 1])}[which].astype(np.int64)
+    for form in ("plain", "screened"):
+        m.check(idx, queries, min(10, len(m.users)), form)
+    idx.delete_users(gone)
+    m.delete_users(gone)
+    for form in ("plain", "screened"):
+        m.check(idx, queries, min(10, len(m.users)), form)
+    more = rng.standard_normal((90, d), dtype=np.float32)
+    idx.insert_users(more)
+    m.insert_users(more)
+    m.check(idx, queries, 12, "screened")
+
+
+@pytest.mark.parametrize("gone", ["first", "some", "all"])
+@pytest.mark.parametrize("reserved", [False, True])
+def test_delete_inserted_items(orc, gpu_index_factory, gone, reserved):
+    """Inserted items leave again while no base item has, then others come and
+    a base item goes too."""
+    _case(f"delete inserted items: {gone}, reserved={reserved}")
+    from test_gpu_update import Mirror
+    rng = np.random.default_rng(7)
+    d, U, I = 24, 3000, 700
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 40)
+    m = Mirror(orc, users, items)
+    if reserved:
+        idx.reserve(4000, 300)
+    queries = items[rng.choice(I, 9, replace=False)]
+    for n in (60, 130):
+        new = rng.standard_normal((n, d), dtype=np.float32) * np.float32(1.3)
+        idx.insert_items(new)
+        m.insert_items(new)
+        n_ins = len(m.ins)
+        ids = I + {"first": np.arange(1), "some": np.arange(1, n_ins, 3), "all": np.arange(n_ins)}[gone].astype(np.int64)
+        idx.delete_items(ids)
+        m.delete_items(ids)
+        for form in ("plain", "screened"):
+            m.check(idx, queries, 20, form)
+    new = rng.standard_normal((20, d), dtype=np.float32)
+    idx.insert_items(new)
+    m.insert_items(new)
+    idx.delete_items(np.array([0, 5, I + 2], np.int64))
+    m.delete_items([0, 5, I + 2])
+    m.check(idx, queries, 20, "screened")
