@@ -289,16 +289,10 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
 }
 
 // ---- list ------------------------------------------------------------------
-// Zeroes the bucket histogram bins of the queries in slots blockIdx.x, +
-// gridDim.x, ... that the exact stage fills: buckets up to the threshold.
-__device__ __forceinline__ void zero_hist(const int32_t *__restrict__ order, int32_t n_slots, const QueryInfo *__restrict__ qi,
-                                          const FineCols &fc, int32_t S, uint32_t *__restrict__ ghist) {
-    for (int32_t s = blockIdx.x; s < n_slots; s += gridDim.x) {
-        const int32_t b = order[s];
-        uint32_t *g = ghist + (int64_t)b * 2 * (S + 1);
-        const int32_t n = fc.col[qi[b].thr] + 1;
-        for (int i = threadIdx.x; i < n; i += NT) { g[i] = 0u; g[S + 1 + i] = 0u; }
-    }
+// Zeroes the list's counts per query and the scatter's cursors behind them.
+__device__ __forceinline__ void zero_counts(int32_t nq, uint32_t *__restrict__ g_cnt) {
+    if (g_cnt && blockIdx.y == 0)
+        for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < 2 * (int64_t)nq; i += (int64_t)gridDim.x * NT) g_cnt[i] = 0u;
 }
 
 constexpr int QCAP = 512;    // listed pairs of a unit queued in LDS
@@ -408,9 +402,8 @@ __device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int32_t bas
 template <int KS, int NB>
 __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen P, int64_t n_user,
                                                                      const int32_t *__restrict__ order,
-                                                                     const int32_t *__restrict__ colg, FineCols fc,
-                                                                     int32_t S, const QueryInfo *__restrict__ qi,
-                                                                     uint32_t *__restrict__ ghist,
+                                                                     const int32_t *__restrict__ colg,
+                                                                     uint32_t *__restrict__ g_cnt,
                                                                      ListCounters *__restrict__ ctr,
                                                                      int32_t *__restrict__ cl_u,
                                                                      int32_t *__restrict__ cl_b, int64_t list_cap) {
@@ -426,7 +419,7 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
     __shared__ int32_t sN[NT / 64], sBase;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
     const int32_t n_slots = ctr->n_slots;
-    zero_hist(order, n_slots, qi, fc, S, ghist);
+    zero_counts(P.nq, g_cnt);
     const int64_t n_rb = (n_user + UB - 1) / UB;
     const int64_t n_sl = (n_slots + kSlice - 1) / kSlice, n_units = n_rb * n_sl;
     for (int64_t unit = blockIdx.x; unit < n_units; unit += gridDim.x) {
@@ -569,14 +562,13 @@ constexpr int kScoreSlice = 64;
 __global__ void __launch_bounds__(NT) k_list_scores(const float *__restrict__ qip, int64_t n_user, float eps,
                                                     const float *__restrict__ gcols, int64_t pitch,
                                                     const int32_t *__restrict__ order, const int32_t *__restrict__ colg,
-                                                    FineCols fc, int32_t S, const QueryInfo *__restrict__ qi,
-                                                    uint32_t *__restrict__ ghist, ListCounters *__restrict__ ctr,
-                                                    int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b,
-                                                    int64_t list_cap) {
+                                                    int32_t nq, uint32_t *__restrict__ g_cnt,
+                                                    ListCounters *__restrict__ ctr, int32_t *__restrict__ cl_u,
+                                                    int32_t *__restrict__ cl_b, int64_t list_cap) {
     __shared__ ListQueue sq;
     __shared__ int32_t sB[kScoreSlice], sCol[kScoreSlice / 4];
     const int32_t n_slots = ctr->n_slots;
-    if (blockIdx.y == 0) zero_hist(order, n_slots, qi, fc, S, ghist);
+    zero_counts(nq, g_cnt);
     const int32_t s0 = (int32_t)blockIdx.y * kScoreSlice, ns = min(n_slots - s0, kScoreSlice);
     if (ns <= 0) return;
     if (threadIdx.x == 0) sq.n = 0;
@@ -604,6 +596,113 @@ __global__ void __launch_bounds__(NT) k_list_scores(const float *__restrict__ qi
     }
     __syncthreads();
     list_flush(sq, cl_u, cl_b, list_cap, &ctr->n_list);
+}
+
+// ---- the listed pairs by query ------------------------------------------------
+// Batches of more than kFilterQueries queries have their list ordered by query:
+// pairs per query, their places, and the pairs moved there.  The k-th bound and
+// the candidates then are one workgroup's work per query, in LDS.  (With counts
+// and places by global atomics per pair, the adds to one query's counter follow
+// one another: with queries that 100k users rank first, 3.8M pairs of 1024 queries,
+// the exact stage took 2.2 ms and the candidates' 0.9; now 0.54 and 0.30, and
+// 0.18 for the order.)
+// One contiguous chunk of the list per workgroup, counted in LDS, so a query
+// takes one global add per chunk.
+constexpr int CT = 1024;
+constexpr int kGroupQ = 4096;       // queries counted in LDS at a time
+constexpr int64_t kChunk = 1024;    // pairs of a workgroup, at least
+
+__device__ __forceinline__ bool list_chunk(const ListCounters *ctr, int64_t cap, int64_t &first, int64_t &last) {
+    const int64_t n = ctr->n_list <= cap ? ctr->n_list : 0;  // an overflowed list is not used
+    const int64_t per = max(kChunk, (n + gridDim.x - 1) / gridDim.x);
+    first = min(n, (int64_t)blockIdx.x * per);
+    last = min(n, first + per);
+    return first < last;
+}
+
+__device__ __forceinline__ void count_queries(uint32_t *h, const int32_t *__restrict__ raw_b, int64_t first,
+                                              int64_t last, int32_t q0) {
+    for (int j = threadIdx.x; j < kGroupQ; j += CT) h[j] = 0u;
+    __syncthreads();
+    for (int64_t i = first + threadIdx.x; i < last; i += CT) {
+        const uint32_t j = (uint32_t)(raw_b[i] - q0);
+        if (j < (uint32_t)kGroupQ) atomicAdd(&h[j], 1u);
+    }
+    __syncthreads();
+}
+
+// Pairs per query.
+__global__ void __launch_bounds__(CT) k_list_count(const int32_t *__restrict__ raw_b, int64_t cap, int32_t nq,
+                                                   uint32_t *__restrict__ g_cnt, const ListCounters *__restrict__ ctr,
+                                                   uint64_t *t) {
+    stamp(t);
+    __shared__ uint32_t h[kGroupQ];
+    int64_t first, last;
+    if (!list_chunk(ctr, cap, first, last)) return;
+    for (int32_t q0 = 0; q0 < nq; q0 += kGroupQ) {
+        count_queries(h, raw_b, first, last, q0);
+        for (int j = threadIdx.x; j < kGroupQ; j += CT)
+            if (h[j]) atomicAdd(&g_cnt[q0 + j], h[j]);
+        __syncthreads();
+    }
+}
+
+// Every workgroup sums the counts to places itself (a last workgroup that does
+// it for all needs a device-wide fence per workgroup: 36 us for 64 queries,
+// where the count takes 5), the first one writes them for the candidates.
+__global__ void __launch_bounds__(CT) k_list_scatter(const int32_t *__restrict__ raw_u, const int32_t *__restrict__ raw_b,
+                                                     int64_t cap, int32_t nq, const uint32_t *__restrict__ g_cnt,
+                                                     uint32_t *__restrict__ g_off, uint32_t *__restrict__ g_cur,
+                                                     const ListCounters *__restrict__ ctr, int32_t *__restrict__ cl_u,
+                                                     int32_t *__restrict__ cl_b) {
+    constexpr int PER = kGroupQ / CT;
+    __shared__ uint32_t h[kGroupQ], red[CT / 64];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    int64_t first, last;
+    const bool work = list_chunk(ctr, cap, first, last);
+    if (!work && blockIdx.x != 0) return;
+    uint32_t before = 0;
+    for (int32_t q0 = 0; q0 < nq; q0 += kGroupQ) {
+        count_queries(h, raw_b, first, last, q0);
+        // the thread's PER queries: places of the query and, in it, of the chunk
+        const int32_t j0 = (int32_t)threadIdx.x * PER;
+        uint32_t v[PER], own = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            v[i] = q0 + j0 + i < nq ? g_cnt[q0 + j0 + i] : 0u;
+            own += v[i];
+        }
+        uint32_t x = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) red[w] = x;
+        __syncthreads();
+        uint32_t base = before + x - own;
+        for (int i = 0; i < CT / 64; ++i) {
+            base += i < w ? red[i] : 0u;
+            before += red[i];
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int32_t j = j0 + i;
+            if (blockIdx.x == 0 && q0 + j < nq) g_off[q0 + j] = base;
+            if (h[j]) h[j] = base + atomicAdd(&g_cur[q0 + j], h[j]);
+            base += v[i];
+        }
+        __syncthreads();
+        for (int64_t i = first + threadIdx.x; i < last; i += CT) {
+            const int32_t b = raw_b[i];
+            const uint32_t j = (uint32_t)(b - q0);
+            if (j >= (uint32_t)kGroupQ) continue;
+            const uint32_t at = atomicAdd(&h[j], 1u);
+            cl_u[at] = raw_u[i];
+            cl_b[at] = b;
+        }
+        __syncthreads();
+    }
 }
 
 // ---- exact scores, buckets and the k-th bound of the listed pairs -----------
@@ -704,9 +803,8 @@ __global__ void __launch_bounds__(NT) k_list_exact(const float *__restrict__ use
                                                    float eps, const float *__restrict__ gvals, FineCols fc,
                                                    const ListCounters *__restrict__ ctr, int64_t list_cap,
                                                    const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
-                                                   int64_t n_user, const QueryInfo *__restrict__ qi,
-                                                   uint32_t *__restrict__ bk_c, float *__restrict__ qip,
-                                                   uint32_t *__restrict__ ghist, uint64_t *t) {
+                                                   int64_t n_user, uint32_t *__restrict__ bk_c,
+                                                   float *__restrict__ qip, uint64_t *t) {
     stamp(t);
     __shared__ int32_t col[GW];
     __shared__ f32x4 sd[SCORES ? 1 : NT / 64][2][SCORES ? 1 : 64 * DP / 4];
@@ -734,134 +832,261 @@ __global__ void __launch_bounds__(NT) k_list_exact(const float *__restrict__ use
             lo = hi = bucket_of(grow, row, col, fc.n, S, s);
         }
         bk_c[i] = (uint32_t)lo | ((uint32_t)hi << 16);
-        // only buckets up to the threshold can hold the k-th bound or a candidate
-        const int32_t last = col[qi[b].thr];
-        uint32_t *g = ghist + b * 2 * (int64_t)(S + 1);
-        if (lo <= last) atomicAdd(&g[lo], 1u);
-        if (eps > 0.0f && hi <= last) atomicAdd(&g[S + 1 + hi], 1u);
     }
 }
 
-// One workgroup per query: beta, the bucket of the k-th smallest b_lo, and the
-// candidates' count, from the histogram bins up to the threshold.  A query
-// with fewer than k buckets there (or a list that overflowed) gets thr = -1
-// and no candidates: the full search answers it.
-__global__ void __launch_bounds__(NT) k_list_kth(const uint32_t *__restrict__ ghist, int32_t S, int same, FineCols fc,
-                                                 int64_t list_cap, QueryInfo *__restrict__ qi,
-                                                 ListCounters *__restrict__ ctr) {
-    constexpr int NW = NT / 64;
-    __shared__ uint32_t red[NW];
-    __shared__ int32_t s_beta;
-    const int64_t b = blockIdx.x;
-    const QueryInfo q = qi[b];
-    const uint32_t *lo = ghist + b * 2 * (int64_t)(S + 1), *hi = same ? lo : lo + S + 1;
-    const int32_t n = q.thr >= 0 && (int64_t)ctr->n_list <= list_cap ? fc.col[q.thr] + 1 : 0;
-    const uint32_t k = (uint32_t)q.topk;
+// Adds each lane's one (of the lanes that `on` says) to LDS bin j; lanes of the
+// first two distinct bins add together, since many users of a popular query
+// share a bucket.
+__device__ __forceinline__ void add_bins(uint32_t *h, bool on, int32_t j) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const uint64_t todo = __builtin_amdgcn_ballot_w64(on);
+        if (todo == 0) return;  // uniform
+        const int l = __ffsll((unsigned long long)todo) - 1;
+        const bool mine = on && j == __builtin_amdgcn_readlane(j, l);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+        if (lane == l) atomicAdd(&h[j], (uint32_t)__popcll(m));
+        on = on && !mine;
+    }
+    if (on) atomicAdd(&h[j], 1u);
+}
+
+// Smallest bin j of h[0 .. FB) where `before` plus the counts up to j reach k:
+// res = {j or -1, the sum up to j, the sum before j}; with j = -1 the sum is of
+// all bins.  All threads call it.
+constexpr int FB = 2048;
+struct BinScan {
+    int32_t bin;
+    uint32_t upto, under;
+};
+template <int FT>
+__device__ __forceinline__ void find_bin(const uint32_t *h, uint32_t before, uint32_t k, uint32_t *red, BinScan *res) {
+    constexpr int PER = FB / FT;
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (threadIdx.x == 0) s_beta = -1;
-    uint32_t before = 0, below = 0;  // totals of the bins already scanned
-    for (int32_t j0 = 0; j0 < n; j0 += NT) {
-        const int32_t j = j0 + (int)threadIdx.x;
-        const uint32_t v = j < n ? lo[j] : 0u, h = j < n ? hi[j] : 0u;
-        uint32_t x = v;
+    uint32_t v[PER], own = 0;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (lane == 63) red[w] = x;
-        __syncthreads();
-        uint32_t base = before, tot = 0;
-        for (int i = 0; i < NW; ++i) {
-            base += i < w ? red[i] : 0u;
-            tot += red[i];
-        }
-        if (base + x >= k && base + x - v < k) s_beta = j;
-        __syncthreads();
-        const int32_t beta = s_beta;
-        // candidates: buckets b_hi <= beta
-        uint32_t c = j < n && (beta < 0 || j <= beta) ? h : 0u;
+    for (int i = 0; i < PER; ++i) {
+        v[i] = h[threadIdx.x * PER + i];
+        own += v[i];
+    }
+    uint32_t x = own;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-        if (lane == 0) red[w] = c;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) red[w] = x;
+    __syncthreads();
+    uint32_t sum = before, tot = before;
+    for (int i = 0; i < FT / 64; ++i) {
+        sum += i < w ? red[i] : 0u;
+        tot += red[i];
+    }
+    sum += x - own;
+    if (threadIdx.x == 0 && tot < k) *res = {-1, tot, tot};
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (sum < k && sum + v[i] >= k) *res = {(int32_t)threadIdx.x * PER + i, sum + v[i], sum};
+        sum += v[i];
+    }
+    __syncthreads();
+}
+
+// One workgroup per query, over its pairs of the grouped list (FILTER: over the
+// whole list of a few queries, skipping other queries' pairs): beta, the bucket
+// of the k-th smallest b_lo, then the candidates (b_hi <= beta) with their rank
+// when the bounds fix it, else ~(refine row).  A query with fewer than k buckets
+// up to its threshold, or a list that overflowed, gets thr = -1 and no
+// candidates: the full search answers it.
+//
+// Many candidates are users of bucket beta itself (an item that most of 100k
+// users rank first).  When that bucket fixes the rank, the answer takes the
+// smallest userIDs of it, as many as the buckets below leave: a histogram of
+// their userIDs gives a bound, and the users past it are counted but not
+// written, so the top-k sorts a few hundred keys and not 188k.
+//
+// Bound: latency of a few passes over some hundred pairs; a list of 250k pairs
+// is read three times by one workgroup, 4096 pairs at a time.
+template <bool FILTER, int FT>
+__global__ void __launch_bounds__(FT) k_list_final(const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
+                                                   const uint32_t *__restrict__ bk_c, const uint32_t *__restrict__ g_off,
+                                                   const uint32_t *__restrict__ g_cnt, const float *__restrict__ qip,
+                                                   ListCounters *__restrict__ ctr, int64_t list_cap, FineCols fc, int32_t S,
+                                                   int same, const int32_t *__restrict__ ranks, int64_t n_item,
+                                                   int64_t n_user, QueryInfo *__restrict__ qi,
+                                                   int32_t *__restrict__ cand_user, int32_t *__restrict__ cand_rank,
+                                                   int32_t *__restrict__ refine_user, int32_t *__restrict__ refine_query,
+                                                   float *__restrict__ refine_thr, int32_t *__restrict__ cnt, uint64_t *t) {
+    stamp(t);
+    constexpr int UNR = 4096 / FT;
+    __shared__ alignas(8) uint32_t h[FB];
+    __shared__ uint32_t red[FT / 64];
+    __shared__ BinScan s_beta, s_user;
+    __shared__ int32_t s_cand, s_fill, s_refine;
+    __shared__ int64_t s_off;
+    const int32_t b = (int32_t)blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    const QueryInfo q = qi[b];
+    const bool listed = q.thr >= 0 && (int64_t)ctr->n_list <= list_cap;
+    const int64_t first = !listed || FILTER ? 0 : g_off[b];
+    const int64_t end = !listed ? 0 : FILTER ? (int64_t)ctr->n_list : first + g_cnt[b];
+    const uint32_t k = (uint32_t)q.topk;
+    if (threadIdx.x == 0) { s_beta = {-1, 0u, 0u}; s_cand = s_fill = s_refine = 0; }
+    // buckets of UNR pairs per thread, loads in flight together; bit 31 of none: not a pair of b
+    constexpr uint32_t none = 0xFFFFFFFFu;
+    auto load = [&](int64_t i0, uint32_t (&x)[UNR]) {
+        int32_t y[UNR];
+#pragma unroll
+        for (int j = 0; j < UNR; ++j) {  // the last pair again past the end: no branch between the loads
+            const int64_t i = min(i0 + j * FT + threadIdx.x, end - 1);
+            x[j] = bk_c[i];
+            y[j] = FILTER ? cl_b[i] : b;
+        }
+#pragma unroll
+        for (int j = 0; j < UNR; ++j)
+            if (i0 + j * FT + threadIdx.x >= end || y[j] != b) x[j] = none;
+    };
+    // beta: only buckets up to the threshold can hold it
+    const int32_t last = listed ? fc.col[q.thr] : -1;
+    uint32_t before = 0;
+    int32_t beta = -1;
+    __syncthreads();
+    for (int32_t w0 = 0; w0 <= last && beta < 0; w0 += FB) {
+        for (int j = threadIdx.x; j < FB; j += FT) h[j] = 0u;
         __syncthreads();
-        for (int i = 0; i < NW; ++i) below += red[i];
+        for (int64_t i0 = first; i0 < end; i0 += FT * UNR) {
+            uint32_t x[UNR];
+            load(i0, x);
+#pragma unroll
+            for (int j = 0; j < UNR; ++j) {
+                const int32_t lo = (int32_t)(x[j] & 0xFFFFu);
+                add_bins(h, x[j] != none && lo >= w0 && lo <= min(last, w0 + FB - 1), lo - w0);
+            }
+        }
         __syncthreads();
-        if (beta >= 0) break;  // uniform
-        before += tot;
+        find_bin<FT>(h, before, k, red, &s_beta);
+        before = s_beta.upto;
+        if (s_beta.bin >= 0) beta = w0 + s_beta.bin;
+        __syncthreads();  // s_beta is read before the next window's
+    }
+    if (beta < 0) {  // uniform
+        if (threadIdx.x == 0) {
+            qi[b].beta = qi[b].gamma = qi[b].thr = -1;
+            qi[b].n_cand = qi[b].n_dropped = qi[b].n_refine = qi[b].fill = qi[b].n_settled = 0;
+            qi[b].cand_off = 0;
+        }
+        return;
+    }
+    const uint32_t under = s_beta.under;  // pairs with b_lo < beta
+    uint32_t n_cand = s_beta.upto;
+    if (!same) {
+        int32_t c = 0;
+        for (int64_t i0 = first; i0 < end; i0 += FT * UNR) {
+            uint32_t x[UNR];
+            load(i0, x);
+#pragma unroll
+            for (int j = 0; j < UNR; ++j) c += x[j] != none && (int32_t)(x[j] >> 16) <= beta;
+        }
+        if (c) atomicAdd(&s_cand, c);
+        __syncthreads();
+        n_cand = (uint32_t)s_cand;
+    }
+    auto rank_lb = [&](int32_t j) { return j == S ? (int32_t)n_item : ranks[j]; };
+    auto rank_ub = [&](int32_t j) { return j == 0 ? 0 : ranks[j - 1] + 1; };
+    // the users of bucket beta that the answer can hold
+    int32_t u_max = INT32_MAX;
+    uint32_t n_keep = n_cand;
+    if (same && n_cand > 1024u && rank_lb(beta) == rank_ub(beta)) {  // uniform
+        int sh = 0;
+        while (((n_user - 1) >> sh) >= FB) ++sh;
+        for (int j = threadIdx.x; j < FB; j += FT) h[j] = 0u;
+        __syncthreads();
+        for (int64_t i0 = first; i0 < end; i0 += FT * UNR) {
+            uint32_t x[UNR];
+            load(i0, x);
+            int32_t u[UNR];
+#pragma unroll
+            for (int j = 0; j < UNR; ++j) u[j] = cl_u[min(i0 + j * FT + threadIdx.x, end - 1)];
+#pragma unroll
+            for (int j = 0; j < UNR; ++j)
+                if (x[j] != none && (int32_t)(x[j] >> 16) == beta) atomicAdd(&h[u[j] >> sh], 1u);
+        }
+        __syncthreads();
+        find_bin<FT>(h, under, k, red, &s_user);  // found: bucket beta reaches k
+        u_max = (int32_t)(((int64_t)s_user.bin + 1) << sh) - 1;
+        n_keep = s_user.upto;
+    }
+    if (threadIdx.x == 0) s_off = atomicAdd(&ctr->n_cand, (int32_t)n_keep);
+    __syncthreads();
+    const int64_t off = s_off;
+    // refine rows (user, candidate slot) until their number is known, in the histogram's place
+    constexpr int ROWS = FB / 2;
+    uint2 *rows = reinterpret_cast<uint2 *>(h);
+    auto refine_row = [&](int32_t r, int32_t u) {
+        refine_user[r] = u;
+        refine_query[r] = b;
+        refine_thr[r] = qip[(int64_t)b * n_user + u];
+        cnt[r] = 0;
+    };
+    for (int64_t i0 = first; i0 < end; i0 += FT * UNR) {
+        uint32_t x[UNR];
+        int32_t us[UNR];
+        load(i0, x);
+#pragma unroll
+        for (int j = 0; j < UNR; ++j) us[j] = cl_u[min(i0 + j * FT + threadIdx.x, end - 1)];
+#pragma unroll
+        for (int j = 0; j < UNR; ++j) {
+            const int32_t u = us[j];
+            const int32_t blo = (int32_t)(x[j] & 0xFFFFu), bhi = (int32_t)(x[j] >> 16);
+            const bool cand = x[j] != none && (bhi < beta || (bhi == beta && u <= u_max));
+            const uint64_t m = __builtin_amdgcn_ballot_w64(cand);
+            if (m == 0) continue;  // uniform in the wavefront
+            int32_t rank = 0;
+            bool open = false;
+            if (cand) {
+                rank = rank_lb(blo);
+                open = rank != rank_ub(bhi);
+            }
+            int32_t place = 0;
+            if (lane == 0) place = atomicAdd(&s_fill, (int32_t)__popcll(m));
+            place = __shfl(place, 0, 64) + (int32_t)__popcll(m & ((1ull << lane) - 1));
+            if (open) {
+                const int32_t r = atomicAdd(&s_refine, 1);
+                if (r < ROWS) {
+                    rows[r] = make_uint2((uint32_t)u, (uint32_t)place);
+                } else {
+                    const int32_t g = atomicAdd(&ctr->n_refine, 1);
+                    refine_row(g, u);
+                    rank = ~g;
+                }
+            }
+            if (cand) {
+                cand_user[off + place] = u;
+                cand_rank[off + place] = rank;
+            }
+        }
+    }
+    __syncthreads();
+    const int32_t n_rows = min(s_refine, ROWS);
+    if (threadIdx.x == 0 && n_rows > 0) s_cand = atomicAdd(&ctr->n_refine, n_rows);
+    __syncthreads();
+    for (int32_t i = threadIdx.x; i < n_rows; i += FT) {
+        const int32_t r = s_cand + i;
+        refine_row(r, (int32_t)rows[i].x);
+        cand_rank[off + rows[i].y] = ~r;
     }
     if (threadIdx.x == 0) {
-        const bool ok = s_beta >= 0;
         QueryInfo r = q;
-        r.beta = s_beta;
-        r.gamma = s_beta;
-        r.thr = ok ? q.thr : -1;
-        r.n_cand = ok ? (int32_t)below : 0;
-        r.n_refine = r.fill = r.n_settled = 0;
-        r.cand_off = atomicAdd(&ctr->n_cand, r.n_cand);
+        r.beta = r.gamma = beta;
+        r.n_cand = (int32_t)n_cand;
+        r.n_dropped = (int32_t)(n_cand - n_keep);
+        r.n_refine = s_refine;
+        r.fill = (int32_t)n_keep;
+        r.n_settled = 0;
+        r.cand_off = off;
         qi[b] = r;
-    }
-}
-
-// One thread per listed pair: the candidates (b_hi <= beta) with their rank when
-// the bounds fix it, else ~(refine row).
-__global__ void __launch_bounds__(NT) k_list_final(const int32_t *__restrict__ cl_u, const int32_t *__restrict__ cl_b,
-                                                   const uint32_t *__restrict__ bk_c, const float *__restrict__ qip,
-                                                   const ListCounters *__restrict__ ctr, int64_t list_cap, int32_t S,
-                                                   const int32_t *__restrict__ ranks, int64_t n_item, int64_t n_user,
-                                                   QueryInfo *__restrict__ qi, int32_t *__restrict__ cand_user,
-                                                   int32_t *__restrict__ cand_rank, int32_t *__restrict__ refine_total,
-                                                   int32_t *__restrict__ refine_user, int32_t *__restrict__ refine_query,
-                                                   float *__restrict__ refine_thr, int32_t *__restrict__ cnt,
-                                                   uint64_t *t) {
-    stamp(t);
-    const int64_t n = min((int64_t)ctr->n_list, list_cap);
-    const int lane = threadIdx.x & 63;
-    for (int64_t i0 = (int64_t)blockIdx.x * NT; i0 < n; i0 += (int64_t)gridDim.x * NT) {
-        const int64_t i = i0 + threadIdx.x;
-        bool cand = false;
-        int32_t b = -1, u = 0, blo = 0, bhi = 0;
-        if (i < n) {
-            b = cl_b[i];
-            const uint32_t x = bk_c[i];
-            blo = (int32_t)(x & 0xFFFFu);
-            bhi = (int32_t)(x >> 16);
-            cand = bhi <= qi[b].beta;
-            u = cl_u[i];
-        }
-        // the lanes of one query share one atomic, all leaders' in flight at once
-        uint64_t todo = __builtin_amdgcn_ballot_w64(cand);
-        int32_t lead = 0, ahead = 0, count = 0;
-        while (todo) {
-            const int l = __ffsll((unsigned long long)todo) - 1;
-            const int32_t lb = __shfl(b, l, 64);
-            const uint64_t same = __builtin_amdgcn_ballot_w64(cand && b == lb);
-            if (cand && b == lb) {
-                lead = l;
-                ahead = (int32_t)__popcll(same & ((1ull << lane) - 1));
-                count = (int32_t)__popcll(same);
-            }
-            todo &= ~same;
-        }
-        int32_t place = 0;
-        if (cand && lane == lead) place = atomicAdd(&qi[b].fill, count);
-        place = __shfl(place, lead, 64) + ahead;
-        if (!cand) continue;
-        const int64_t slot = qi[b].cand_off + place;
-        const int32_t lbs = blo == S ? (int32_t)n_item : ranks[blo];
-        const int32_t ubs = bhi == 0 ? 0 : ranks[bhi - 1] + 1;
-        int32_t rank = lbs;
-        if (lbs != ubs) {
-            const int32_t r = atomicAdd(refine_total, 1);
-            atomicAdd(&qi[b].n_refine, 1);
-            rank = ~r;
-            refine_user[r] = u;
-            refine_query[r] = b;
-            refine_thr[r] = qip[(int64_t)b * n_user + u];
-            cnt[r] = 0;
-        }
-        cand_user[slot] = u;
-        cand_rank[slot] = rank;
     }
 }
 
@@ -936,7 +1161,7 @@ hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L) {
 #define RKR_LIST_CASE(ks)                                                                                          \
     case ks:                                                                                                       \
         hipLaunchKernelGGL((k_list_screen<ks, ks <= 5 ? 4 : 2>), grid, dim3(NT), 0, s, P, L.n_user, L.order, \
-                           L.colg, L.fc, L.S, L.qi, L.ghist, L.ctr, L.cl_u, L.cl_b, L.list_cap);                   \
+                           L.colg, L.g_cnt, L.ctr, L.raw_u, L.raw_b, L.list_cap);                                  \
         break;
     RKR_KS_SWITCH(L.Kp, RKR_LIST_CASE)
 #undef RKR_LIST_CASE
@@ -955,33 +1180,46 @@ hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L) {
                        L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
     hipLaunchKernelGGL(k_list_scores,
                        dim3((unsigned)((L.n_user + NT - 1) / NT), (unsigned)((L.nq + kScoreSlice - 1) / kScoreSlice)),
-                       dim3(NT), 0, s, L.qip, L.n_user, L.eps, L.gcols, L.pitch, L.order, L.colg, L.fc, L.S, L.qi,
-                       L.ghist, L.ctr, L.cl_u, L.cl_b, L.list_cap);
+                       dim3(NT), 0, s, L.qip, L.n_user, L.eps, L.gcols, L.pitch, L.order, L.colg, L.nq, L.g_cnt, L.ctr,
+                       L.raw_u, L.raw_b, L.list_cap);
     return hipGetLastError();
 }
 
 hipError_t launch_list_exact(hipStream_t s, const ListLaunch &L, const float *users, const float *queries, int32_t ld,
                              int32_t dim, const float *table, bool scores, uint32_t *bk_c) {
     if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
+    uint64_t *t = scores ? nullptr : L.t_bound;
+    if (L.g_cnt) {
+        const dim3 cg((unsigned)std::max(1, L.n_cu / 2));
+        hipLaunchKernelGGL(k_list_count, cg, dim3(CT), 0, s, L.raw_b, L.list_cap, L.nq, L.g_cnt, L.ctr, t);
+        hipLaunchKernelGGL(k_list_scatter, cg, dim3(CT), 0, s, L.raw_u, L.raw_b, L.list_cap, L.nq, L.g_cnt, L.g_off,
+                           L.g_cur, L.ctr, L.cl_u, L.cl_b);
+        t = nullptr;
+    }
     const dim3 grid((unsigned)(L.n_cu * 16));  // a multiple of the 8 XCDs (grid-stride over the list)
     if (scores)
         hipLaunchKernelGGL(k_list_exact<true>, grid, dim3(NT), 0, s, users, queries, ld, dim, table, L.S, L.eps, L.gvals,
-                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist, nullptr);
+                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, bk_c, L.qip, t);
     else
         hipLaunchKernelGGL(k_list_exact<false>, grid, dim3(NT), 0, s, users, queries, ld, dim, table, L.S, L.eps, L.gvals,
-                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, L.qi, bk_c, L.qip, L.ghist, L.t_bound);
-    hipLaunchKernelGGL(k_list_kth, dim3((unsigned)L.nq), dim3(NT), 0, s, L.ghist, L.S, L.eps > 0.0f ? 0 : 1, L.fc,
-                       L.list_cap, L.qi, L.ctr);
+                           L.fc, L.ctr, L.list_cap, L.cl_u, L.cl_b, L.n_user, bk_c, L.qip, t);
     return hipGetLastError();
 }
 
 hipError_t launch_list_final(hipStream_t s, const ListLaunch &L, const uint32_t *bk_c, const int32_t *ranks,
-                             int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_total,
-                             int32_t *refine_user, int32_t *refine_query, float *refine_thr, int32_t *cnt) {
+                             int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
+                             int32_t *refine_query, float *refine_thr, int32_t *cnt) {
     if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_list_final, dim3((unsigned)(L.n_cu * 16)), dim3(NT), 0, s, L.cl_u, L.cl_b, bk_c, L.qip, L.ctr,
-                       L.list_cap, L.S, ranks, n_item, L.n_user, L.qi, cand_user, cand_rank, refine_total, refine_user,
-                       refine_query, refine_thr, cnt, L.t_prune);
+    const dim3 grid((unsigned)L.nq);
+    const int same = L.eps > 0.0f ? 0 : 1;
+    if (L.g_cnt)
+        hipLaunchKernelGGL((k_list_final<false, 512>), grid, dim3(512), 0, s, L.cl_u, L.cl_b, bk_c, L.g_off, L.g_cnt, L.qip, L.ctr,
+                           L.list_cap, L.fc, L.S, same, ranks, n_item, L.n_user, L.qi, cand_user, cand_rank, refine_user,
+                           refine_query, refine_thr, cnt, L.t_prune);
+    else
+        hipLaunchKernelGGL((k_list_final<true, 1024>), grid, dim3(1024), 0, s, L.cl_u, L.cl_b, bk_c, nullptr, nullptr, L.qip, L.ctr,
+                           L.list_cap, L.fc, L.S, same, ranks, n_item, L.n_user, L.qi, cand_user, cand_rank, refine_user,
+                           refine_query, refine_thr, cnt, L.t_prune);
     return hipGetLastError();
 }
 

@@ -567,7 +567,7 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
         oq[i] = qb[u];
     }
     const int32_t need = k - ns;
-    const int64_t nc = q.n_cand;
+    const int64_t nc = q.n_cand - q.n_dropped;
     if (need <= 0 || nc <= 0) {
         if (t_end && threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned long long *>(t_end), wall_clock64());
         return;

@@ -1567,9 +1567,18 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             LL.hist = reinterpret_cast<uint32_t *>(sl.list_info.p);
             LL.order = reinterpret_cast<int32_t *>(LL.hist + 64 * (size_t)nq);
             LL.colg = LL.order + nq;
-            LL.qi = qi; LL.ctr = ctr; LL.ghist = ghist; LL.t_bound = at(kTimeBound); LL.t_prune = at(kTimePrune);
+            LL.qi = qi; LL.ctr = ctr; LL.t_bound = at(kTimeBound); LL.t_prune = at(kTimePrune);
             LL.cl_u = reinterpret_cast<int32_t *>(sl.list.p);
             LL.cl_b = LL.cl_u + list_cap;
+            LL.raw_u = LL.cl_u;
+            LL.raw_b = LL.cl_b;
+            if (nq > kFilterQueries) {  // as listed: where the candidates go later
+                LL.raw_u = reinterpret_cast<int32_t *>(sl.cand.p);
+                LL.raw_b = LL.raw_u + list_cap;
+                LL.g_cnt = ghist;
+                LL.g_cur = LL.g_cnt + nq;
+                LL.g_off = LL.g_cur + nq;
+            }
             bk_c = reinterpret_cast<uint32_t *>(LL.cl_b + list_cap);
         }
         if (list_mfma) {
@@ -1748,8 +1757,8 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             RKR_HIP(c, launch_small_select(sl.stream, qip, T, U, S, R, I, nq, eps, qi, ctr, cand_user, cand_rank, refine_user,
                                            refine_query, refine_thr, cnt));
         else if (list)
-            RKR_HIP(c, launch_list_final(sl.stream, LL, bk_c, R, I, cand_user, cand_rank, refine_total, refine_user,
-                                         refine_query, refine_thr, cnt));
+            RKR_HIP(c, launch_list_final(sl.stream, LL, bk_c, R, I, cand_user, cand_rank, refine_user, refine_query,
+                                         refine_thr, cnt));
         else if (upd)
             RKR_HIP(c, launch_compact_values(sl.stream, lbv, ubv, qip, U, nq, cu, qi, cand_user, cand_rank,
                                              refine_total, refine_user, refine_query, refine_thr, cnt));

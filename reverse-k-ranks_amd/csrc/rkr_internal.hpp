@@ -465,7 +465,7 @@ struct QueryInfo {          // one per query of a device batch
     int32_t n_screen;       // users a screen kept and scored exactly (QSRP)
     int64_t cand_off;       // offset of this query's candidates
     int32_t thr;            // fine column of the query's list, -1: the full search answers it
-    int32_t pad2;
+    int32_t n_dropped;      // candidates counted but not written: the answer cannot hold them
 };
 
 // Counters of a device batch, uploaded as zeros with the queries and read back
@@ -528,25 +528,29 @@ struct ListLaunch {
     float *qip;              // exact scores (read with scores, else written for listed pairs)
     int64_t stride;          // every stride-th user is sampled
     int64_t cap;             // a longer estimated list takes the full search
-    int64_t list_cap;        // entries of cl_u, cl_b
+    int64_t list_cap;        // entries of the lists
     uint32_t *hist;          // nq x 64, zeroed
     int32_t *order, *colg;   // nq slots, nq / 4 threshold columns
     QueryInfo *qi;
     ListCounters *ctr;
     uint64_t *t_bound, *t_prune;  // stamps (or null)
-    uint32_t *ghist;         // nq x 2 (S + 1) bucket histograms
-    int32_t *cl_u, *cl_b;
+    // the pairs as listed, and by query (the same arrays without g_cnt)
+    int32_t *raw_u, *raw_b, *cl_u, *cl_b;
+    uint32_t *g_cnt, *g_off, *g_cur;  // pairs per query and their places (null: kFilterQueries or fewer)
 };
+// Up to this many queries the candidates are looked for in the whole list,
+// which spares the two launches that order it (about 5 us each).
+constexpr int kFilterQueries = 16;
 // Threshold per query and the listed pairs, from the matrix cores or from qip.
 hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L);
 hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L);
 // Exact scores (read from qip with scores) and buckets of the listed pairs,
-// then the k-th bound and the candidates' place per query.
+// ordered by query first with g_cnt; then the k-th bound and the candidates.
 hipError_t launch_list_exact(hipStream_t s, const ListLaunch &L, const float *users, const float *queries, int32_t ld,
                              int32_t dim, const float *table, bool scores, uint32_t *bk_c);
 hipError_t launch_list_final(hipStream_t s, const ListLaunch &L, const uint32_t *bk_c, const int32_t *ranks,
-                             int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_total,
-                             int32_t *refine_user, int32_t *refine_query, float *refine_thr, int32_t *cnt);
+                             int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
+                             int32_t *refine_query, float *refine_thr, int32_t *cnt);
 
 // Table rows staged per workgroup by the batched bounds kernels: 16 rows of
 // S + 1 floats (<= 32 KB at S = 511), fewer for long rows; 0 when one row

@@ -217,3 +217,41 @@ def test_delete_inserted_items(orc, gpu_index_factory, gone, reserved):
     idx.delete_items(np.array([0, 5, I + 2], np.int64))
     m.delete_items([0, 5, I + 2])
     m.check(idx, queries, 20, "screened")
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+@pytest.mark.parametrize("nq,dense", [(16, 2), (17, 2), (200, 0)])
+def test_popular_queries(orc, gpu_index_factory, form, nq, dense):
+    """Queries that thousands of users rank first (more candidates of one rank
+    than k), a list searched whole (16 queries) and one ordered by query."""
+    _case(f"popular queries {form} nq={nq} dense={dense}")
+    rng = np.random.default_rng(5)
+    U, I, d = 30_000, 2000, 16
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    queries = items[rng.choice(I, nq, replace=False)]
+    queries[::2] *= np.float32(2.6)
+    ks = [int(k) for k in np.exp(rng.uniform(0, np.log(400), nq))]
+    idx, _ = gpu_index_factory(users, items, 64, dense_top=dense)
+    idx.set_form(form)
+    res = _lists_and_search(idx, queries, ks)
+    assert res.timing["n_listed"] > 0 and max(s["n_candidate"] for s in res.stats) > 1024
+    bu, br, _ = orc.bruteforce(orc.normalize_users(users), items, queries[:8], max(ks[:8]))
+    for i in range(8):
+        assert np.array_equal(res.users[i, :ks[i]], bu[i, :ks[i]]) and np.array_equal(res.ranks[i, :ks[i]], br[i, :ks[i]])
+    idx.close()
+
+
+def test_list_of_a_large_batch(gpu_index_factory):
+    """More queries in one device batch than the list's order counts at a time."""
+    _case("list of 4500 queries")
+    rng = np.random.default_rng(9)
+    users = rng.standard_normal((900, 12), dtype=np.float32)
+    items = rng.standard_normal((700, 12), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 32)
+    idx.set_option(3, 8192)  # RKR_OPT_QUERY_BATCH
+    idx.set_form("screened")
+    queries = rng.standard_normal((4500, 12), dtype=np.float32)
+    res = _lists_and_search(idx, queries, [int(k) for k in rng.integers(1, 60, 4500)])
+    assert res.timing["n_batches"] == 1 and res.timing["n_listed"] > 0
+    idx.close()
