@@ -29,10 +29,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-// native vectors, not HIP's uint4 struct: a struct copy is a memcpy that keeps
-// staged values in scratch memory
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int NT = 256;
 constexpr int QST = 64;       // queries per LDS stage
 constexpr int KPAD_LDS = 8;   // bf16 pad per LDS row
@@ -359,22 +355,6 @@ __device__ __forceinline__ void list_flush(ListQueue &sq, int32_t *__restrict__ 
         __syncthreads();
         if (threadIdx.x == 0) sq.n = 0;
     }
-}
-
-// Place of 16-byte piece j of staged query row r: rows are not padded (they
-// arrive by direct loads, 16 bytes per lane in lane order), so the pieces of a
-// row are permuted such that the 16 lanes that read piece j of 16 rows together
-// find them in different banks.
-template <int KS>
-__device__ __forceinline__ int swizzled(int r, int j) {
-    return KS % 4 == 0 ? j ^ (r & 15) : KS % 2 == 0 ? j ^ ((r >> 1) & 7) : j ^ ((r >> 2) & 3);
-}
-
-// 16 bytes per lane from global memory straight to LDS, lane l of the wavefront
-// to dst + 16 l (dst the same in every lane).
-__device__ __forceinline__ void load_to_lds(const void *src, void *dst) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                     (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
 }
 
 // A wavefront's listed pairs, user in the unit | slot in the slice << 8, and

@@ -20,10 +20,11 @@
 // sequential FP32 score (k_recheck), so every rank stays bit-exact.
 //
 // Work unit = 128 refine rows (4 waves x 2 blocks of 16 rows; A fragments
-// held in VGPRs) x a chunk of items streamed through LDS 64 items at a time.
-// Units are ordered chunk-major, so the workgroups resident at one time all
-// stream the same item chunk, which stays in each XCD's L2.  The next stage
-// is loaded into registers while the current one is computed from LDS.
+// held in VGPRs) x a chunk of items streamed through LDS 32 items at a time.
+// Units are ordered chunk-major and each XCD takes a contiguous eighth of
+// them, so a chunk's items are read by one XCD (by two at an eighth's ends) and
+// stay in its L2.  The next stage's rows go straight to LDS while the current
+// one is computed.
 #include "rkr_internal.hpp"
 
 namespace rkr {
@@ -33,7 +34,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NT = 256;
-constexpr int ITEMS_STAGE = 64;
 constexpr int KPAD_LDS = 8;  // bf16 pad per LDS row
 
 // Round-to-nearest-even FP32 -> BF16 (finite inputs).
@@ -47,6 +47,7 @@ union Frag {
     bf16x8 v;
     uint16_t h[8];
     uint4 q;
+    u32x4 n;
 };
 
 // Splits every item row into hi/lo BF16 rows (Kp columns, zero padded) and
@@ -139,87 +140,97 @@ struct ScreenParams {
     uint64_t *t;
 };
 
-// RB row blocks of 16 per wave: 2 (32 rows, two waves per SIMD) or 4 (64
-// rows, one wave per SIMD, half the LDS reads per matrix-core operation).
+// Workgroups of the screen that fit a CU by their VGPRs (RB row blocks of 16
+// per wave: 2, or 4, half the LDS reads per matrix-core operation).
+constexpr int screen_wgs(int KS, int RB) { return RB == 4 ? 1 : KS <= 3 ? 3 : 2; }
+
+// Items stream through two LDS buffers, the next stage's rows by direct loads
+// (no registers, and the loads of a stage stay in flight for the whole previous
+// one) while one is computed; one barrier per stage.  The items' rows (32 MB of
+// a 50k x 150 catalogue) come from the memory side, so units that share a chunk
+// of items are given to one XCD, whose L2 then serves all but the first.
+// Bound: the matrix cores with few rows, the L2 with many (a stage's 20 KB per
+// 128 rows).  Measured at 2374 rows x 50k items x 150 dims 194 -> 154 us (760
+// TFLOP/s of products), 650 rows x 50k x 128 94 -> 51 us, 2.5M rows x 30k x 256
+// 155 -> 106 ms; before, stages passed through registers and every XCD read
+// every chunk.  32 rows a wave beat 64 at every width from 30 to 256 dims.
 template <int KS, int RB>
-__global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenParams P) {
+__global__ void __launch_bounds__(NT, screen_wgs(KS, RB)) k_refine_screen(ScreenParams P) {
     stamp(P.t);
     constexpr int RW = 4 * 16 * RB;  // rows per workgroup
-    // items per LDS stage: 32 keeps the two prefetch register sets at 8 KS
-    // VGPRs
-    constexpr int IST = 32;
-    // two stage buffers: stage m of a unit is computed from buffer m & 1
-    // while stage m + 1 is written to the other and stage m + 3 is loaded
-    // into registers, with one barrier per stage
-    __shared__ uint4 sB[2][2][IST * (KS * 32 + KPAD_LDS) / 8];  // [buf][hi|lo][item][k] as 16-byte chunks
-    __shared__ float sN[2][IST];                                // item norm bounds of the stage
+    constexpr int IST = 32;          // items per LDS stage
+    constexpr int KQ = KS * 4;       // 16-byte pieces per item row (Kp = 32 KS)
+    static_assert(2 * IST * KQ == KS * NT, "KS 16-byte pieces per thread and stage");
+    // [hi|lo][item][piece, permuted]; two variables, not one array: a read of
+    // one then does not wait for the loads into the other
+    __shared__ u32x4 sB0[2 * IST * KQ], sB1[2 * IST * KQ];
     // undecided (row, item) pairs of the unit, appended with LDS atomics and
     // flushed to the recheck list when the unit ends (a global atomic that
     // returns a slot would make the stage loop wait for its prefetch loads)
     constexpr int QCAP = 256;
     __shared__ int4 sQ[QCAP];
     __shared__ int32_t sQn, sQbase;
-    constexpr int ROWQ = (KS * 32 + KPAD_LDS) / 8;                   // uint4 per LDS item row
-    constexpr int KQ = KS * 4;                                       // uint4 per global item row (Kp = 32 KS)
-    constexpr int PER_T = 2 * IST * KQ / NT;                 // uint4 each thread stages per stage
-    static_assert(2 * IST * KQ % NT == 0, "stage must split evenly over the workgroup");
     // Persistent grid: the work split is sized here from the refine count the
-    // compaction produced, so the host launches without reading it back.
+    // compaction produced, so the host launches without reading it back.  A
+    // unit starts with a gather of its rows (about three stages' time), so
+    // there is one unit per resident workgroup while the row blocks are few,
+    // and four where they would leave the last round uneven.
     const int64_t n_rows = min((int64_t)*P.n_rows_dev, P.max_rows);
     const int64_t n_rb = (n_rows + RW - 1) / RW;
     const int64_t n_stage_total = (P.n_item + IST - 1) / IST;
-    const int64_t fill_chunks = n_rb > 0 ? (P.target_units + n_rb - 1) / n_rb : 1;
-    const int64_t st_per_chunk =
-        max((int64_t)1, min((int64_t)max(1, P.chunk_items / IST), (n_stage_total + fill_chunks - 1) / fill_chunks));
+    const int64_t fill_chunks =
+        n_rb <= 0 ? 1 : 4 * n_rb <= P.target_units ? P.target_units / n_rb : (4 * P.target_units + n_rb - 1) / n_rb;
+    // a chunk is at most 2 MB of items, half an XCD's L2
+    constexpr int64_t L2_ST = (2 << 20) / (2 * IST * KQ * 16);
+    const int64_t st_per_chunk = max((int64_t)1, min(min((int64_t)max(1, P.chunk_items / IST), L2_ST),
+                                                     (n_stage_total + fill_chunks - 1) / fill_chunks));
     const int64_t n_chunks = (n_stage_total + st_per_chunk - 1) / st_per_chunk;
     const int64_t n_units = n_rb * n_chunks;
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 15, lq = lane >> 4;
-    // Register sets for the stages loaded ahead: with two (where the A
-    // fragments leave room), stage m of a unit lives in set A (m even) or B
-    // (m odd) from its load, three stages ahead, until it is written to LDS;
-    // with one, two stages ahead.  Every lane issues the same
-    // loads in every call, with no branch around them and no use of their
-    // values until the set is written to LDS, so the memory counter then
-    // waits for exactly the older set, never for the loads just issued.  Rows
-    // past n_item load the last item; compute() gives them a norm bound of
-    // -inf, so they never count.
-    constexpr int NSET = (KS <= 4 || (RB == 4 && KS <= 5)) ? 2 : 1;
-    // native vectors, not HIP's uint4 struct: a struct copy is a memcpy that
-    // keeps the sets in scratch memory
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 preA[PER_T], preB[NSET == 2 ? PER_T : 1];
-    float preA_n = -INFINITY, preB_n = -INFINITY;
-#define RKR_LOAD_STAGE(st, dst, dst_n)                                                                        \
-    do {                                                                                                    \
-        const int64_t p0_ = (st) * IST;                                                                     \
-        _Pragma("unroll") for (int j = 0; j < PER_T; ++j) {                                                 \
-            const int c = threadIdx.x + j * NT;                                                             \
-            const int half = c / (IST * KQ);                                                                \
-            const int rem = c % (IST * KQ);                                                                 \
-            const int64_t p = min(p0_ + rem / KQ, P.n_item - 1);                                            \
-            dst[j] = reinterpret_cast<const u32x4 *>(half ? P.item_lo : P.item_hi)[p * KQ + rem % KQ];     \
-        }                                                                                                   \
-        dst_n = P.item_norm[min(p0_ + (int64_t)(threadIdx.x % IST), P.n_item - 1)];                         \
-    } while (0)
-#define RKR_STORE_STAGE(src, src_n, buf)                                                                      \
-    do {                                                                                                    \
-        _Pragma("unroll") for (int j = 0; j < PER_T; ++j) {                                                 \
-            const int c = threadIdx.x + j * NT;                                                             \
-            const int half = c / (IST * KQ);                                                                \
-            const int rem = c % (IST * KQ);                                                                 \
-            *reinterpret_cast<u32x4 *>(&sB[buf][half][(rem / KQ) * ROWQ + rem % KQ]) = src[j];              \
-        }                                                                                                   \
-        if (threadIdx.x < IST) sN[buf][threadIdx.x] = src_n;                                                \
-    } while (0)
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    // workgroup i runs on XCD i % 8, which takes a contiguous eighth of the units
+    const bool by_xcd = gridDim.x % 8 == 0;
+    const int64_t per_xcd = (n_units + 7) / 8;
+    const int64_t u_first = by_xcd ? (blockIdx.x % 8) * per_xcd + blockIdx.x / 8 : blockIdx.x;
+    const int64_t u_end = by_xcd ? min(n_units, (int64_t)(blockIdx.x % 8 + 1) * per_xcd) : n_units;
+    const int64_t u_step = by_xcd ? gridDim.x / 8 : gridDim.x;
 
     if (threadIdx.x == 0) sQn = 0;
     __syncthreads();
-    for (int64_t unit = blockIdx.x; unit < n_units; unit += gridDim.x) {
+    for (int64_t unit = u_first; unit < u_end; unit += u_step) {
         const int64_t chunk = unit / n_rb;
         const int64_t rb = unit % n_rb;
         const int64_t row_base = rb * RW + wave * 16 * RB;
+        const int64_t st0 = chunk * st_per_chunk;
+        const int64_t n_st = max((int64_t)0, min(n_stage_total, st0 + st_per_chunk) - st0);
+        // stage st's rows to dst (waves 0 and 1 the hi halves, 2 and 3 the lo):
+        // lane order in LDS, the pieces of a row permuted; the last item again
+        // past the last
+        auto load_stage = [&](u32x4 *dst, int64_t st) __attribute__((always_inline)) {
+            const u32x4 *base = reinterpret_cast<const u32x4 *>(wave_u >= 2 ? P.item_lo : P.item_hi) + st * (IST * KQ);
+            const uint32_t last = (uint32_t)min((int64_t)(IST - 1), P.n_item - 1 - st * IST);
+#pragma unroll
+            for (int j = 0; j < KS; ++j) {
+                const uint32_t c = (threadIdx.x & 127) + j * 128, r = c / KQ;
+                load_to_lds(base + (min(r, last) * KQ + swizzled<KS>((int)r, (int)(c % KQ))),
+                            dst + (wave_u >> 1) * (IST * KQ) + (wave_u & 1) * 64 + j * 128);
+            }
+        };
+        // norm bounds of the lane's items of a stage; rows past n_item never count
+        static_assert(IST == 32, "two groups of 16 items a stage");
+        float ahead0 = 0.0f, ahead1 = 0.0f;
+        auto load_norms = [&](int64_t st) __attribute__((always_inline)) {
+            const float *base = P.item_norm + st * IST;
+            const uint32_t last = (uint32_t)min((int64_t)(IST - 1), P.n_item - 1 - st * IST);
+            ahead0 = base[min((uint32_t)lr, last)];
+            ahead1 = base[min((uint32_t)lr + 16u, last)];
+        };
+        if (n_st > 0) {
+            load_stage(sB0, st0);
+            load_norms(st0);
+        }
 
         // A fragments: row (row_base + b*16 + lr), k = ks*32 + 8*lq + i
         Frag ah[RB][KS], al[RB][KS];
@@ -260,24 +271,16 @@ __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenPar
 #pragma unroll
             for (int i = 0; i < 4; ++i) cnt[b][i] = 0;
 
-        // Wait here for the unit's A fragments and epilogue constants: the
-        // stage loop's prefetch loads are issued after them, and a use of an
-        // older load inside the loop would otherwise wait for every load in
-        // flight (the memory counter is in order), the prefetch included.
-        __builtin_amdgcn_s_waitcnt(0);
-        const int64_t st0 = chunk * st_per_chunk;
-        const int64_t n_st = max((int64_t)0, min(n_stage_total, st0 + st_per_chunk) - st0);
-        // Stage m (of this unit) is computed from LDS buffer m & 1.  Before it,
-        // stage m + 1 goes from register set (m + 1) & 1 to the other buffer
-        // (its last readers, stage m - 1, passed the barrier that ended it) and
-        // stage m + 3 starts loading into that register set; one barrier per
-        // stage then orders the buffers.
-        auto compute = [&](int buf, int64_t st) {
-            const int64_t p0 = st * IST;
+        auto stage = [&](const u32x4 *rows, u32x4 *other, int64_t m) __attribute__((always_inline)) {
+            const int64_t st = st0 + m, p0 = st * IST;
+            const float n0 = p0 + lr < P.n_item ? ahead0 : -INFINITY, n1 = p0 + lr + 16 < P.n_item ? ahead1 : -INFINITY;
+            if (m + 1 < n_st) {
+                load_stage(other, st + 1);
+                load_norms(st + 1);
+            }
 #pragma unroll 1
             for (int g = 0; g < IST / 16; ++g) {
                 const int it = g * 16 + lr;
-                const int64_t p = p0 + it;
                 // all 3*Kp products of a 16x16 block into one FP32 accumulator
                 // (the bound holds for any order of the additions); B
                 // fragments are read from LDS one k-step at a time
@@ -287,8 +290,8 @@ __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenPar
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
                     Frag bh, bl;
-                    bh.q = sB[buf][0][it * ROWQ + ks * 4 + lq];
-                    bl.q = sB[buf][1][it * ROWQ + ks * 4 + lq];
+                    bh.n = rows[it * KQ + swizzled<KS>(it, ks * 4 + lq)];
+                    bl.n = rows[IST * KQ + it * KQ + swizzled<KS>(it, ks * 4 + lq)];
 #pragma unroll
                     for (int b = 0; b < RB; ++b) {
                         accs[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[b][ks].v, bh.v, accs[b], 0, 0, 0);
@@ -296,9 +299,9 @@ __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenPar
                         accs[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[b][ks].v, bh.v, accs[b], 0, 0, 0);
                     }
                 }
-                // decide the 8 outputs without branches; only undecided ones
+                // decide the outputs without branches; only undecided ones
                 // (rare) take the recheck path
-                const float np = p < P.n_item ? sN[buf][it] : -INFINITY;
+                const float np = g ? n1 : n0;
                 uint32_t undecided = 0;
 #pragma unroll
                 for (int b = 0; b < RB; ++b)
@@ -317,7 +320,7 @@ __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenPar
                         for (int i = 0; i < 4; ++i)
                             if (undecided & (1u << (b * 4 + i))) {
                                 const int64_t r = row_base + b * 16 + 4 * lq + i;
-                                const int4 e = make_int4((int32_t)r, (int32_t)p, __float_as_int(accs[b][i]), 0);
+                                const int4 e = make_int4((int32_t)r, (int32_t)(p0 + it), __float_as_int(accs[b][i]), 0);
                                 const int32_t q = atomicAdd(&sQn, 1);
                                 if (q < QCAP) {
                                     sQ[q] = e;
@@ -329,46 +332,14 @@ __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenPar
                             }
                 }
             }
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's rows of the next stage are in LDS
+            __syncthreads();
         };
-        // stages past the unit's last load its last again (never computed),
-        // so the loads stay unconditional
-        const int64_t st_last = st0 + n_st - 1;
-        auto ahead = [&](int64_t m) { return min(st0 + m, st_last); };
-        if constexpr (NSET == 2) {
-            if (n_st > 0) {
-                RKR_LOAD_STAGE(ahead(0), preA, preA_n);
-                RKR_LOAD_STAGE(ahead(1), preB, preB_n);
-                RKR_STORE_STAGE(preA, preA_n, 0);  // the previous unit ended with a barrier
-                RKR_LOAD_STAGE(ahead(2), preA, preA_n);
-                __syncthreads();
-            }
-            for (int64_t m = 0; m < n_st; m += 2) {
-                // even stage: buffer 0; stage m + 1 is in set B
-                RKR_STORE_STAGE(preB, preB_n, 1);
-                RKR_LOAD_STAGE(ahead(m + 3), preB, preB_n);
-                compute(0, st0 + m);
-                __syncthreads();
-                if (m + 1 >= n_st) break;
-                // odd stage: buffer 1; stage m + 2 is in set A
-                RKR_STORE_STAGE(preA, preA_n, 0);
-                RKR_LOAD_STAGE(ahead(m + 4), preA, preA_n);
-                compute(1, st0 + m + 1);
-                __syncthreads();
-            }
-        } else {
-            if (n_st > 0) {
-                RKR_LOAD_STAGE(ahead(0), preA, preA_n);
-                RKR_STORE_STAGE(preA, preA_n, 0);  // the previous unit ended with a barrier
-                RKR_LOAD_STAGE(ahead(1), preA, preA_n);
-                __syncthreads();
-            }
-            for (int64_t m = 0; m < n_st; ++m) {
-                const int buf = (int)(m & 1);
-                RKR_STORE_STAGE(preA, preA_n, buf ^ 1);
-                RKR_LOAD_STAGE(ahead(m + 2), preA, preA_n);
-                compute(buf, st0 + m);
-                __syncthreads();
-            }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // the first stage's rows, the A fragments and the constants
+        __syncthreads();
+        for (int64_t m = 0; m < n_st; m += 2) {
+            stage(sB0, sB1, m);
+            if (m + 1 < n_st) stage(sB1, sB0, m + 1);
         }
         // the unit's queued rechecks go to the list (the stage loop ended
         // with a barrier, so the queue is complete)
@@ -398,9 +369,6 @@ __global__ void __launch_bounds__(NT, RB == 2 ? 2 : 1) k_refine_screen(ScreenPar
             }
     }
 }
-
-#undef RKR_LOAD_STAGE
-#undef RKR_STORE_STAGE
 
 // Exact decision of the rechecked (row, item) pairs with the sequential FP32
 // rule; also records the largest |s^ - s_fp64| seen (as float bits).
@@ -730,16 +698,13 @@ hipError_t launch_refine_screen(hipStream_t s, const ScreenLaunch &L) {
     P.recheck = reinterpret_cast<int4 *>(L.recheck);
     P.recheck_cap = L.recheck_cap;
     P.t = L.t;
-    P.target_units = std::max<int64_t>(1, L.target_units);
     P.chunk_items = std::max(1, L.chunk_items);
-    // persistent grid: enough workgroups to fill the device, never more than
-    // the largest possible number of units
+    // persistent grid: the workgroups that fit the device, never more than the
+    // largest possible number of units
     const int rb = L.rows_per_wave == 64 ? 4 : 2;
+    P.target_units = std::max<int64_t>(8, (int64_t)L.n_cu * screen_wgs(L.Kp / 32, rb));
     const int64_t n_rb_max = (L.max_rows + 64 * rb - 1) / (64 * rb);
-    const int64_t n_stage = (L.n_item + ITEMS_STAGE - 1) / ITEMS_STAGE;
-    const int64_t max_units = std::max<int64_t>(n_rb_max, std::min<int64_t>(P.target_units, n_rb_max * n_stage));
-    const int64_t cap = rb == 4 ? L.grid_cap / 2 : L.grid_cap;  // one workgroup per CU at 64 rows per wave
-    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(max_units, cap)));
+    const dim3 grid((unsigned)std::min<int64_t>(n_rb_max * ((L.n_item + 31) / 32), P.target_units));
 #define RKR_SCREEN_CASE(ks)                                                                              \
     case ks:                                                                                           \
         if (rb == 4) hipLaunchKernelGGL((k_refine_screen<ks, 4>), grid, dim3(NT), 0, s, P);             \

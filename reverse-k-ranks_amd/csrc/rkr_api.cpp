@@ -1789,11 +1789,10 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 L.rows_user = refine_user; L.rows_thr = refine_thr; L.n_rows_dev = refine_total;
                 L.max_rows = (int64_t)rcap; L.C = c->screen_C; L.abs_floor = dv.screen_abs;
                 L.cnt = cnt; L.recheck_n = &ctr->n_recheck; L.recheck = sl.recheck.p; L.recheck_cap = rec_cap;
-                L.target_units = (int64_t)c->n_cu * 8;
-                L.grid_cap = (int64_t)c->n_cu * 4;
+                L.n_cu = c->n_cu;
                 L.chunk_items = c->screen_chunk > 0 ? c->screen_chunk : (1 << 30);
                 L.t = at(kTimeRefine);
-                L.rows_per_wave = c->screen_rows > 0 ? c->screen_rows : (c->kp / 32 >= 6 ? 64 : 32);  // d > 160: 32 rows spill
+                L.rows_per_wave = c->screen_rows > 0 ? c->screen_rows : 32;
                 RKR_HIP(c, launch_refine_screen(sl.stream, L));
                 RKR_HIP(c, event(8));
                 RKR_HIP(c, launch_recheck(sl.stream, dv.users, dv.items, ld, d, refine_user, refine_thr, refine_query,

@@ -381,8 +381,7 @@ struct ScreenLaunch {
     int32_t *recheck_n;
     void *recheck;          // int4 records (row, item, screened score bits, 0)
     int64_t recheck_cap;
-    int64_t target_units;   // work units wanted to fill the device
-    int64_t grid_cap;       // workgroups of the persistent grid
+    int32_t n_cu;
     int32_t chunk_items;    // most items per work-unit chunk (L2-resident slice)
     int32_t rows_per_wave;  // 32 or 64 refine rows per wavefront
     uint64_t *t = nullptr;
@@ -562,6 +561,26 @@ inline int bounds_rows_per_wg(int32_t S) {
 }
 
 #ifdef __HIPCC__
+// native vectors, not HIP's uint4 struct: a struct copy is a memcpy that keeps
+// staged values in scratch memory
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// Place of 16-byte piece j of staged BF16 row r (Kp = 32 KS): rows are not padded (they
+// arrive by direct loads, 16 bytes per lane in lane order), so the pieces of a
+// row are permuted such that the 16 lanes that read piece j of 16 rows together
+// find them in different banks.
+template <int KS>
+__device__ __forceinline__ int swizzled(int r, int j) {
+    return KS % 4 == 0 ? j ^ (r & 15) : KS % 2 == 0 ? j ^ ((r >> 1) & 7) : j ^ ((r >> 2) & 3);
+}
+
+// 16 bytes per lane from global memory straight to LDS, lane l of the wavefront
+// to dst + 16 l (dst the same in every lane).
+__device__ __forceinline__ void load_to_lds(const void *src, void *dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                     (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+}
+
 // Copies nu rows of S floats (source row stride src_ld) to LDS rows of
 // stride S + 1, 16-byte loads where the rows allow.
 __device__ __forceinline__ void stage_rows(float *rows, const float *__restrict__ src, int64_t nu, int32_t S,

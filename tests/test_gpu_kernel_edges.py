@@ -255,3 +255,25 @@ def test_list_of_a_large_batch(gpu_index_factory):
     res = _lists_and_search(idx, queries, [int(k) for k in rng.integers(1, 60, 4500)])
     assert res.timing["n_batches"] == 1 and res.timing["n_listed"] > 0
     idx.close()
+
+
+@pytest.mark.parametrize("d", [5, 33, 70, 100, 130, 161, 200, 256])
+@pytest.mark.parametrize("U,I", [(40, 31), (3000, 1031), (700, 20_001)])
+def test_screened_refinement(orc, gpu_index_factory, d, U, I):
+    """The screen at every row width, with a last stage of one item, fewer and
+    more row blocks than workgroups, both row counts per wavefront."""
+    _case(f"screened refinement d={d} U={U} I={I}")
+    rng = np.random.default_rng(d + U)
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    queries = np.concatenate([items[:6], rng.standard_normal((6, d), dtype=np.float32)])
+    idx, _ = gpu_index_factory(users, items, 6, dense_top=0)
+    idx.set_form("screened")
+    k = min(U, 30)
+    bu, br, _ = orc.bruteforce(orc.normalize_users(users), items, queries, k)
+    for rows in (32, 64):
+        idx.set_option(7, rows)  # RKR_OPT_SCREEN_ROWS
+        res = idx.query(queries, k)
+        assert res.timing["n_refined"] > 0
+        assert np.array_equal(res.users[:, :k], bu) and np.array_equal(res.ranks[:, :k], br)
+    idx.close()
