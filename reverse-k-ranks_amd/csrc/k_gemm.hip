@@ -277,15 +277,19 @@ __global__ void __launch_bounds__(NT, 3) k_refine_count(const float *__restrict_
 
 // Small-batch <u, q>: one wave per 64-user panel, lane = user.  Users are
 // stored as panels [p][k][lane] so every k step is one coalesced 256-byte
-// load; queries sit in LDS and are read as broadcasts.
+// load, 16 of them in flight ahead of the sums; query values are uniform and
+// come through the scalar cache.  With bk also #{T > score} of every pair, the
+// NQ searches of a user side by side so their loads overlap.
+// Bound: the panels' bytes (7 queries x 250k users x 128 dims, 128 MB: 74 us
+// with one load in flight and the queries in LDS, now 33; 16 x 100k x 150, 60 MB: 133 us, now 44).
+constexpr int GC = 16;
+
 template <int NQ>
 __global__ void __launch_bounds__(NT) k_gemv_panels(const float *__restrict__ usersT, int64_t n_user, int32_t ld,
                                                     int32_t K, const float *__restrict__ q, int32_t nq,
-                                                    float *__restrict__ qip, uint64_t *t) {
+                                                    float *__restrict__ qip, const float *__restrict__ table, int32_t S,
+                                                    uint32_t *__restrict__ bk, uint64_t *t) {
     stamp(t);
-    extern __shared__ float qs[];  // nq x K
-    for (int i = threadIdx.x; i < nq * K; i += NT) qs[i] = q[(i / K) * (int64_t)ld + (i % K)];
-    __syncthreads();
     const int lane = threadIdx.x & 63;
     const int64_t panel = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
     const int64_t u = panel * 64 + lane;
@@ -294,21 +298,54 @@ __global__ void __launch_bounds__(NT) k_gemv_panels(const float *__restrict__ us
     float acc[NQ];
 #pragma unroll
     for (int b = 0; b < NQ; ++b) acc[b] = 0.0f;
-    for (int k = 0; k < K; ++k) {
-        const float x = src[(int64_t)k * 64];
+    float x[GC], y[GC];
+    auto load = [&](int32_t k0, float (&v)[GC]) {
+#pragma unroll
+        for (int j = 0; j < GC; ++j) v[j] = src[(int64_t)min(k0 + j, K - 1) * 64];
+    };
+    load(0, x);
+    int32_t k0 = 0;
+    for (; k0 + GC <= K; k0 += GC) {
+        load(k0 + GC, y);  // past the last term: its value again, unused
 #pragma unroll
         for (int b = 0; b < NQ; ++b) {
-            if (b < nq) {
-                const float p = x * qs[b * K + k];
+            const float *qb = q + min(b, nq - 1) * (int64_t)ld + k0;
+#pragma unroll
+            for (int j = 0; j < GC; ++j) {
+                const float p = x[j] * qb[j];
                 acc[b] = acc[b] + p;
             }
         }
-    }
-    if (u < n_user) {
 #pragma unroll
-        for (int b = 0; b < NQ; ++b)
-            if (b < nq) qip[(int64_t)b * n_user + u] = acc[b];
+        for (int j = 0; j < GC; ++j) x[j] = y[j];
     }
+#pragma unroll
+    for (int j = 0; j < GC; ++j)
+        if (k0 + j < K)
+#pragma unroll
+            for (int b = 0; b < NQ; ++b) {
+                const float p = x[j] * q[min(b, nq - 1) * (int64_t)ld + k0 + j];
+                acc[b] = acc[b] + p;
+            }
+    if (u >= n_user) return;
+#pragma unroll
+    for (int b = 0; b < NQ; ++b)
+        if (b < nq) qip[(int64_t)b * n_user + u] = acc[b];
+    if (!bk) return;
+    const float *row = table + u * (int64_t)S;
+    int32_t pos[NQ];
+#pragma unroll
+    for (int b = 0; b < NQ; ++b) pos[b] = 0;
+    for (int32_t step = 1 << (31 - __clz(S)); step > 0; step >>= 1)
+#pragma unroll
+        for (int b = 0; b < NQ; ++b) {
+            const int32_t at = pos[b] + step;
+            const float v = row[min(at, S) - 1];
+            pos[b] = at <= S && v > acc[b] ? at : pos[b];
+        }
+#pragma unroll
+    for (int b = 0; b < NQ; ++b)
+        if (b < nq) bk[(int64_t)b * n_user + u] = (uint32_t)pos[b] | (uint32_t)pos[b] << 16;
 }
 
 __global__ void k_make_panels(const float *__restrict__ users, int64_t n_user, int32_t ld, float *__restrict__ usersT) {
@@ -355,16 +392,19 @@ hipError_t launch_refine_count(hipStream_t s, const float *users, const float *i
 }
 
 hipError_t launch_gemv_panels(hipStream_t s, const float *usersT, int64_t n_user, int32_t ld, int32_t K,
-                              const float *q, int32_t nq, float *qip, uint64_t *t) {
+                              const float *q, int32_t nq, float *qip, const float *table, int32_t S, uint32_t *bk,
+                              uint64_t *t) {
     if (n_user <= 0 || nq <= 0) return hipSuccess;
+    if (nq > 16 || (bk && (!table || S <= 0))) return hipErrorInvalidValue;
     const int64_t n_panel = (n_user + 63) / 64;
-    const unsigned grid = (unsigned)((n_panel + 3) / 4);
-    const size_t smem = sizeof(float) * (size_t)nq * K;
-    if (nq <= 1) hipLaunchKernelGGL(k_gemv_panels<1>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
-    else if (nq <= 2) hipLaunchKernelGGL(k_gemv_panels<2>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
-    else if (nq <= 4) hipLaunchKernelGGL(k_gemv_panels<4>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
-    else if (nq <= 8) hipLaunchKernelGGL(k_gemv_panels<8>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
-    else hipLaunchKernelGGL(k_gemv_panels<16>, dim3(grid), dim3(NT), smem, s, usersT, n_user, ld, K, q, nq, qip, t);
+    const dim3 grid((unsigned)((n_panel + 3) / 4)), block(NT);
+#define RKR_GEMV(n) hipLaunchKernelGGL(k_gemv_panels<n>, grid, block, 0, s, usersT, n_user, ld, K, q, nq, qip, table, S, bk, t)
+    if (nq <= 1) RKR_GEMV(1);
+    else if (nq <= 2) RKR_GEMV(2);
+    else if (nq <= 4) RKR_GEMV(4);
+    else if (nq <= 8) RKR_GEMV(8);
+    else RKR_GEMV(16);
+#undef RKR_GEMV
     return hipGetLastError();
 }
 

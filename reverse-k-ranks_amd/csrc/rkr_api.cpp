@@ -1697,8 +1697,8 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode, 0, cu, ghist, qi));
         } else {
             // <u, q> for every (query, user): qip[b * U + u]
-            if (nq <= 16 && (size_t)nq * d * sizeof(float) <= 65536)
-                RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip, at(kTimeIp)));
+            if (nq <= 16)
+                RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip, nullptr, 0, nullptr, at(kTimeIp)));
             else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false, at(kTimeIp)));
             RKR_HIP(c, event(2));
             if (list) {

@@ -355,7 +355,8 @@ hipError_t launch_scores_store(hipStream_t s, const float *A, int64_t M, int32_t
 // Small-batch <u,q>: qip[b * n_user + u] for b < nq (nq <= 16), users in
 // 64-user panels.
 hipError_t launch_gemv_panels(hipStream_t s, const float *usersT, int64_t n_user, int32_t ld, int32_t K,
-                              const float *q, int32_t nq, float *qip, uint64_t *t = nullptr);
+                              const float *q, int32_t nq, float *qip, const float *table, int32_t S, uint32_t *bk,
+                              uint64_t *t = nullptr);
 // Refinement count: cnt[r] = #{item p : score(user(r), p) > thr(r)} for every
 // refine row r < *n_rows_dev (device-side count, persistent grid).
 hipError_t launch_refine_count(hipStream_t s, const float *users, const float *items, int64_t n_item,
