@@ -113,7 +113,8 @@ typedef struct rkr_batch_timing {
     double refine_ms;       /* exact-rank refinement (screening kernel when screened) */
     double recheck_ms;      /* screened form: exact recheck of undecided items */
     double topk_ms;         /* top-k selection                                 */
-    double h2d_ms, d2h_ms;  /* copies of queries and results                   */
+    double h2d_ms, d2h_ms;  /* copies of queries and results (d2h 0 where the
+                               top-k writes them to the host: up to 8 MB)      */
     int64_t n_batches;
     int64_t n_refined;      /* (query, user) pairs counted                     */
     int64_t n_rechecked;

@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(NT) k_hist_kth(const uint32_t *__restrict__ gh
 // over 1000 users.  A query's candidates take their place from one atomic on the
 // batch's counter.
 __global__ void __launch_bounds__(NT) k_small_select(const float *__restrict__ qip, const float *__restrict__ table,
-                                                     int32_t n_user, int32_t S, const int32_t *__restrict__ ranks,
+                                                     const uint32_t *__restrict__ bk_in, int32_t n_user, int32_t S, const int32_t *__restrict__ ranks,
                                                      int64_t n_item, float eps, QueryInfo *__restrict__ qi,
                                                      ListCounters *__restrict__ ctr, int32_t *__restrict__ cand_user,
                                                      int32_t *__restrict__ cand_rank, int32_t *__restrict__ refine_user,
@@ -299,7 +299,13 @@ __global__ void __launch_bounds__(NT) k_small_select(const float *__restrict__ q
     __syncthreads();
     for (int32_t u = threadIdx.x; u < n_user; u += NT) {
         uint32_t lo, hi;
-        bucket_pair(table + u * (int64_t)S, S, qb[u], eps, 0, lo, hi);
+        if (bk_in) {
+            const uint32_t x = bk_in[b * n_user + u];
+            lo = x & 0xFFFFu;
+            hi = x >> 16;
+        } else {
+            bucket_pair(table + u * (int64_t)S, S, qb[u], eps, 0, lo, hi);
+        }
         bk[u] = lo | (hi << 16);
         atomicAdd(&h_lo[lo], 1u);
         atomicAdd(&h_hi[hi], 1u);
@@ -543,7 +549,7 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
                                              const int32_t *__restrict__ cand_rank, const int32_t *__restrict__ cnt,
                                              const float *__restrict__ qip, int64_t n_user, int32_t max_k, int32_t *__restrict__ out_user,
                                              int32_t *__restrict__ out_rank, float *__restrict__ out_qip,
-                                             uint64_t *t_start, uint64_t *t_end) {
+                                             uint64_t *t_start, uint64_t *t_end, HostResult hr) {
     stamp(t_start);
     __shared__ uint64_t keys[SORT_CAP];
     __shared__ uint32_t hist[256];
@@ -557,8 +563,6 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
     float *oq = out_qip + b * (int64_t)max_k;
     const float *qb = qip + b * n_user;
 
-    for (int i = threadIdx.x; i < max_k; i += NT) { ou[i] = -1; orank[i] = -1; oq[i] = -1.0f; }
-    __syncthreads();
     const int32_t ns = q.n_settled < k ? q.n_settled : k;
     for (int i = threadIdx.x; i < ns; i += NT) {
         const int32_t u = cand_user[q.cand_off + i];
@@ -568,13 +572,29 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
     }
     const int32_t need = k - ns;
     const int64_t nc = q.n_cand - q.n_dropped;
-    if (need <= 0 || nc <= 0) {
-        if (t_end && threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned long long *>(t_end), wall_clock64());
+    const int32_t take = need <= 0 || nc <= 0 ? 0 : (int32_t)(nc < need ? nc : need);
+    for (int i = ns + take + threadIdx.x; i < max_k; i += NT) { ou[i] = -1; orank[i] = -1; oq[i] = -1.0f; }
+    auto finish = [&] {
+        if (hr.qi) {  // the query's info and the batch's counters leave with the outputs
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                QueryInfo r = q;
+                r.pad = (int32_t)(uint32_t)wall_clock64();
+                hr.qi[b] = r;
+                hr.recheck_out[b] = hr.recheck[b];
+            }
+            if (b == 0 && threadIdx.x < sizeof(ListCounters) / 4)
+                reinterpret_cast<uint32_t *>(hr.ctr_out)[threadIdx.x] = reinterpret_cast<const uint32_t *>(hr.ctr)[threadIdx.x];
+        } else if (t_end && threadIdx.x == 0) {
+            atomicMax(reinterpret_cast<unsigned long long *>(t_end), wall_clock64());
+        }
+    };
+    if (take == 0) {  // uniform
+        finish();
         return;
     }
     const int32_t *cu = cand_user + q.cand_off + q.n_settled;
     const int32_t *cr = cand_rank + q.cand_off + q.n_settled;
-    const int32_t take = (int32_t)(nc < need ? nc : need);
 
     int n_keys;
     if (nc <= SORT_CAP) {
@@ -628,7 +648,17 @@ __global__ void __launch_bounds__(NT) k_topk(const QueryInfo *__restrict__ qi, c
         orank[ns + i] = (int32_t)(key >> 32);
         oq[ns + i] = qb[u];
     }
-    if (t_end && threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned long long *>(t_end), wall_clock64());
+    finish();
+}
+
+// A batch's upload, read from pinned host memory.  Also clears n_zero 16-byte
+// words at zero.
+__global__ void __launch_bounds__(256) k_upload(const uint4 *__restrict__ src, uint4 *__restrict__ dst, int64_t n,
+                                                uint4 *__restrict__ zero, int64_t n_zero, uint64_t *t) {
+    stamp(t);
+    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    for (int64_t i = i0; i < n; i += step) dst[i] = src[i];
+    for (int64_t i = i0; i < n_zero; i += step) zero[i] = make_uint4(0, 0, 0, 0);
 }
 
 
@@ -968,14 +998,15 @@ hipError_t launch_hist_kth(hipStream_t s, const uint32_t *bk, int64_t n_user, in
     return hipGetLastError();
 }
 
-hipError_t launch_small_select(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
+hipError_t launch_small_select(hipStream_t s, const float *qip, const float *table, const uint32_t *bk_in,
+                               int64_t n_user, int32_t S,
                                const int32_t *ranks, int64_t n_item, int32_t nq, float eps, QueryInfo *qi,
                                ListCounters *ctr, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
                                int32_t *refine_query, float *refine_thr, int32_t *cnt) {
     if (nq <= 0) return hipSuccess;
     if (n_user > kSmallUsers || S > kMaxSample) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_small_select, dim3((unsigned)nq), dim3(NT), 0, s, qip, table, (int32_t)n_user, S, ranks, n_item,
-                       eps, qi, ctr, cand_user, cand_rank, refine_user, refine_query, refine_thr, cnt);
+    hipLaunchKernelGGL(k_small_select, dim3((unsigned)nq), dim3(NT), 0, s, qip, table, bk_in, (int32_t)n_user,
+                       S, ranks, n_item, eps, qi, ctr, cand_user, cand_rank, refine_user, refine_query, refine_thr, cnt);
     return hipGetLastError();
 }
 
@@ -1005,10 +1036,20 @@ hipError_t launch_compact(hipStream_t s, const uint32_t *bk, const float *qip, i
 
 hipError_t launch_topk(hipStream_t s, const QueryInfo *qi, int32_t nq, const int32_t *cand_user,
                        const int32_t *cand_rank, const int32_t *cnt, const float *qip, int64_t n_user, int32_t max_k,
-                       int32_t *out_user, int32_t *out_rank, float *out_qip, uint64_t *t_start, uint64_t *t_end) {
+                       int32_t *out_user, int32_t *out_rank, float *out_qip, uint64_t *t_start, uint64_t *t_end,
+                       const HostResult &hr) {
     if (nq <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_topk, dim3((unsigned)nq), dim3(NT), 0, s, qi, cand_user, cand_rank, cnt, qip, n_user, max_k,
-                       out_user, out_rank, out_qip, t_start, t_end);
+                       out_user, out_rank, out_qip, t_start, t_end, hr);
+    return hipGetLastError();
+}
+
+hipError_t launch_upload(hipStream_t s, const void *src, void *dst, size_t bytes, void *zero, size_t zero_bytes, uint64_t *t) {
+    if (bytes % 16 || zero_bytes % 16) return hipErrorInvalidValue;
+    const int64_t n = (int64_t)(bytes / 16), n_zero = (int64_t)(zero_bytes / 16);
+    const int64_t blocks = std::min<int64_t>(256, std::max<int64_t>(1, (std::max(n, n_zero) + 255) / 256));
+    hipLaunchKernelGGL(k_upload, dim3((unsigned)blocks), dim3(256), 0, s, reinterpret_cast<const uint4 *>(src),
+                       reinterpret_cast<uint4 *>(dst), n, reinterpret_cast<uint4 *>(zero), n_zero, t);
     return hipGetLastError();
 }
 

@@ -1458,12 +1458,15 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     const bool small = !list && !upd && !qsrp && mode == RKR_OUTPUT_EXACT && U <= kSmallUsers && nqb * U <= (1 << 18);
     // stages are timed by their kernels, or by events where other kernels open them
     const bool use_ev = upd || qsrp;
+    // transfers without copy commands
+    auto direct_of = [&](const BatchIo &io) { return !use_ev && io.end <= kDirectBytes; };
     int rc;
     const BatchIo io_max(nqb, ld, max_k);
     if ((rc = ensure(c, sl.io, io_max.end, "queries and outputs"))) return rc;
     if ((rc = ensure(c, sl.qip, sizeof(float) * (size_t)nqb * U, "query scores"))) return rc;
     // coarse bucket rows: whole row blocks of 128 users, plus a spare row
     const int64_t ldc = (U + 127) / 128 * 128;
+    if (small && (rc = ensure(c, sl.bk, sizeof(uint32_t) * (size_t)(nqb * U), "bucket pairs"))) return rc;
     if (!list && !small && (rc = ensure(c, sl.bk, std::max((pair_bytes - 4) * (size_t)U * nqb, (size_t)ldc * (nqb + 1)),
                               "bucket pairs")))
         return rc;
@@ -1498,7 +1501,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
 
     // pinned staging: the batch's transfer layout | coarse rows and bin counts
     const size_t stage_io = (io_max.end + 255) & ~(size_t)255;
-    if ((rc = ensure_pinned(c, sl.stage, stage_io + sizeof(int32_t) * 12 * (size_t)nqb))) return rc;
+    if ((rc = ensure_pinned(c, sl.stage, stage_io + std::max<size_t>(sizeof(int32_t) * 12 * (size_t)nqb, 64)))) return rc;
     char *stg = reinterpret_cast<char *>(sl.stage.p);
     int32_t *hcq = reinterpret_cast<int32_t *>(stg + stage_io);
     int32_t *hhc = hcq + 4 * (size_t)nqb;
@@ -1506,16 +1509,20 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     for (int64_t q0 = 0; q0 < n_query; q0 += nqb) {
         const int32_t nq = (int32_t)std::min<int64_t>(nqb, n_query - q0);
         const BatchIo io(nq, ld, max_k);
+        const bool direct = direct_of(io);
         char *dev = reinterpret_cast<char *>(sl.io.p);
         float *q_in = reinterpret_cast<float *>(dev);
         QueryInfo *qi = reinterpret_cast<QueryInfo *>(dev + io.info);
         int32_t *q_recheck = reinterpret_cast<int32_t *>(dev + io.recheck);
         ListCounters *ctr = reinterpret_cast<ListCounters *>(dev + io.counters);
-        int32_t *o_user = reinterpret_cast<int32_t *>(dev + io.out);
+        int32_t *o_user = reinterpret_cast<int32_t *>((direct ? stg : dev) + io.out);
         int32_t *o_rank = o_user + (size_t)nq * max_k;
         float *o_qip = reinterpret_cast<float *>(o_rank + (size_t)nq * max_k);
         int32_t *refine_total = &ctr->n_refine;
         uint64_t *const t = use_ev ? nullptr : ctr->t;  // stage stamps
+        // few users and queries: the scores' kernel also searches the table
+        uint32_t *const small_bk = small && nq <= 16 && eps == 0.0f ? reinterpret_cast<uint32_t *>(sl.bk.p) : nullptr;
+        uint64_t *t_up = reinterpret_cast<uint64_t *>(hcq);  // when the direct upload began
         auto at = [t](int i) { return t ? t + i : nullptr; };
         auto event = [&](int i) { return use_ev ? hipEventRecord(sl.ev[i], sl.stream) : hipSuccess; };
         float *hq = reinterpret_cast<float *>(stg);
@@ -1538,9 +1545,15 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             hqi[i].topk = topk[q0 + i];
         }
         std::memset(stg + io.recheck, 0, io.out - io.recheck);
-        RKR_HIP(c, hipEventRecord(sl.ev[0], sl.stream));
-        RKR_HIP(c, hipMemcpyAsync(dev, stg, io.out, hipMemcpyHostToDevice, sl.stream));
-        RKR_HIP(c, hipEventRecord(sl.ev[1], sl.stream));
+        const bool plain_list = list && !list_mfma;  // its sample histogram is cleared here
+        if (direct) {
+            RKR_HIP(c, launch_upload(sl.stream, stg, dev, io.out, plain_list ? sl.list_info.p : nullptr,
+                                     plain_list ? sizeof(uint32_t) * 64 * (size_t)nq : 0, t_up));
+        } else {
+            RKR_HIP(c, hipEventRecord(sl.ev[0], sl.stream));
+            RKR_HIP(c, hipMemcpyAsync(dev, stg, io.out, hipMemcpyHostToDevice, sl.stream));
+            RKR_HIP(c, hipEventRecord(sl.ev[1], sl.stream));
+        }
         int32_t *lbv = reinterpret_cast<int32_t *>(bk);
         int32_t *ubv = lbv + (size_t)nq * U;
         const int64_t cu = chunk_users(U, nq, c->n_cu);
@@ -1698,11 +1711,11 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         } else {
             // <u, q> for every (query, user): qip[b * U + u]
             if (nq <= 16)
-                RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip, nullptr, 0, nullptr, at(kTimeIp)));
+                RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip, T, S, small_bk, at(kTimeIp)));
             else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false, at(kTimeIp)));
             RKR_HIP(c, event(2));
             if (list) {
-                RKR_HIP(c, hipMemsetAsync(LL.hist, 0, sizeof(uint32_t) * 64 * (size_t)nq, sl.stream));
+                if (!direct) RKR_HIP(c, hipMemsetAsync(LL.hist, 0, sizeof(uint32_t) * 64 * (size_t)nq, sl.stream));
                 RKR_HIP(c, launch_list_scores(sl.stream, LL));
                 RKR_HIP(c, launch_list_exact(sl.stream, LL, dv.users, q_in, ld, d, T, true, bk_c));
                 RKR_HIP(c, event(3));
@@ -1756,8 +1769,8 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         int32_t *cnt = reinterpret_cast<int32_t *>(refine_thr + rcap);
 
         if (small)
-            RKR_HIP(c, launch_small_select(sl.stream, qip, T, U, S, R, I, nq, eps, qi, ctr, cand_user, cand_rank, refine_user,
-                                           refine_query, refine_thr, cnt));
+            RKR_HIP(c, launch_small_select(sl.stream, qip, T, small_bk, U, S, R, I, nq, eps, qi, ctr, cand_user, cand_rank,
+                                           refine_user, refine_query, refine_thr, cnt));
         else if (list)
             RKR_HIP(c, launch_list_final(sl.stream, LL, bk_c, R, I, cand_user, cand_rank, refine_user, refine_query,
                                          refine_thr, cnt));
@@ -1807,11 +1820,16 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             }
             RKR_HIP(c, event(5));
             RKR_HIP(c, launch_topk(sl.stream, qi, nq, cand_user, cand_rank, cnt, qip, U, max_k, o_user, o_rank, o_qip, at(kTimeTopk),
-                                   at(kTimeEnd)));
+                                   at(kTimeEnd),
+                                   direct ? HostResult{hqi, reinterpret_cast<int32_t *>(stg + io.recheck),
+                                                       reinterpret_cast<ListCounters *>(stg + io.counters), q_recheck, ctr}
+                                          : HostResult{}));
             RKR_HIP(c, event(6));
-            // query info, counters and outputs in one copy (the device layout)
-            RKR_HIP(c, hipMemcpyAsync(stg + io.info, dev + io.info, io.end - io.info, hipMemcpyDeviceToHost, sl.stream));
-            RKR_HIP(c, hipEventRecord(sl.ev[7], sl.stream));
+            if (!direct) {
+                // query info, counters and outputs in one copy (the device layout)
+                RKR_HIP(c, hipMemcpyAsync(stg + io.info, dev + io.info, io.end - io.info, hipMemcpyDeviceToHost, sl.stream));
+                RKR_HIP(c, hipEventRecord(sl.ev[7], sl.stream));
+            }
             RKR_HIP(c, hipStreamSynchronize(sl.stream));
             const int64_t n_recheck = hctr->n_recheck;
             if (!screened || n_recheck <= rec_cap) break;
@@ -1860,7 +1878,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 }
             }
         }
-        tm.h2d_ms += ev_ms(sl.ev, 0, 1);
+        if (!direct) tm.h2d_ms += ev_ms(sl.ev, 0, 1);
         if (use_ev) {
             tm.ip_ms += ev_ms(sl.ev, 1, 2);
             tm.bound_ms += ev_ms(sl.ev, 2, 3);
@@ -1873,6 +1891,11 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // a stage without a kernel of its own starts with the next
             uint64_t ts[kTimeEnd + 1];
             for (int i = 0; i <= kTimeEnd; ++i) ts[i] = hctr->t[i];
+            if (direct) {  // the last workgroup's end, from the low words
+                uint32_t end = 0;
+                for (int32_t i = 0; i < nq; ++i) end = std::max(end, (uint32_t)hqi[i].pad - (uint32_t)ts[kTimeTopk]);
+                ts[kTimeEnd] = ts[kTimeTopk] + end;
+            }
             for (int i = kTimeEnd - 1; i > 0; --i)
                 if (ts[i] == 0) ts[i] = ts[i + 1];
             auto ms = [&](int i) { return ts[i + 1] > ts[i] ? (double)(ts[i + 1] - ts[i]) / c->clock_khz : 0.0; };
@@ -1882,9 +1905,12 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             tm.refine_ms += ms(kTimeRefine);
             tm.recheck_ms += ms(kTimeRecheck);
             tm.topk_ms += ms(kTimeTopk);
-            // what is left of the time after the upload
-            const double kernels = ts[kTimeEnd] > ts[kTimeIp] ? (double)(ts[kTimeEnd] - ts[kTimeIp]) / c->clock_khz : 0.0;
-            tm.d2h_ms += std::max(0.0, ev_ms(sl.ev, 1, 7) - kernels);
+            if (direct) {  // the outputs leave within the top-k
+                tm.h2d_ms += ts[kTimeIp] > *t_up ? (double)(ts[kTimeIp] - *t_up) / c->clock_khz : 0.0;
+            } else {  // what is left of the time after the upload
+                const double kernels = ts[kTimeEnd] > ts[kTimeIp] ? (double)(ts[kTimeEnd] - ts[kTimeIp]) / c->clock_khz : 0.0;
+                tm.d2h_ms += std::max(0.0, ev_ms(sl.ev, 1, 7) - kernels);
+            }
         }
         tm.n_batches += 1;
         tm.n_refined += hctr->n_refine;

@@ -460,7 +460,7 @@ struct QueryInfo {          // one per query of a device batch
     int32_t n_settled;      // reference output: users settled by the bounds
     int32_t n_refine;       // candidates whose rank is counted
     int32_t mode;           // classification case (reference output)
-    int32_t pad;
+    int32_t pad;            // scratch of a stage
     int32_t fill;           // candidates written so far (chunked compaction)
     int32_t n_screen;       // users a screen kept and scored exactly (QSRP)
     int64_t cand_off;       // offset of this query's candidates
@@ -505,6 +505,21 @@ struct BatchIo {
         out = counters + sizeof(ListCounters);
         end = out + 3 * sizeof(int32_t) * (size_t)nq * max_k;
     }
+};
+
+// A batch whose transfers take at most kDirectBytes goes without copy commands:
+// a kernel reads the upload from the pinned staging buffer, and the top-k writes
+// outputs, query info and counters to it.  Two copies and the three events that
+// timed them took 25 us of any call (one query over 1000 users 54 -> 30 us in
+// the library, 64 over 500k 279 -> 250, 1000 over 1M with 1.3 MB 1337 -> 1300);
+// past 8 MB, more than any measured, the copy engine is left the work.
+constexpr size_t kDirectBytes = (size_t)8 << 20;
+struct HostResult {         // where the top-k puts what the host reads (qi null: a copy follows)
+    QueryInfo *qi;          // pad: low word of the device clock when the query's workgroup ended
+    int32_t *recheck_out;
+    ListCounters *ctr_out;
+    const int32_t *recheck;
+    const ListCounters *ctr;
 };
 
 // ---- threshold lists of exact output (k_list.hip) ----------------------------
@@ -661,7 +676,8 @@ hipError_t launch_hist_kth(hipStream_t s, const uint32_t *bk, int64_t n_user, in
 // Exact output without updates over at most kSmallUsers users: bounds, the k-th
 // bound and the candidates, one workgroup per query.
 constexpr int64_t kSmallUsers = 4096;
-hipError_t launch_small_select(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
+hipError_t launch_small_select(hipStream_t s, const float *qip, const float *table, const uint32_t *bk_in,
+                               int64_t n_user, int32_t S,
                                const int32_t *ranks, int64_t n_item, int32_t nq, float eps, QueryInfo *qi,
                                ListCounters *ctr, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
                                int32_t *refine_query, float *refine_thr, int32_t *cnt);
@@ -697,8 +713,9 @@ hipError_t launch_compact(hipStream_t s, const uint32_t *bk, const float *qip, i
 // cnt: the refine rows' counts
 hipError_t launch_topk(hipStream_t s, const QueryInfo *qi, int32_t nq, const int32_t *cand_user,
                        const int32_t *cand_rank, const int32_t *cnt, const float *qip, int64_t n_user, int32_t max_k,
-                       int32_t *out_user, int32_t *out_rank, float *out_qip, uint64_t *t_start = nullptr,
-                       uint64_t *t_end = nullptr);
+                       int32_t *out_user, int32_t *out_rank, float *out_qip, uint64_t *t_start, uint64_t *t_end,
+                       const HostResult &hr);
+hipError_t launch_upload(hipStream_t s, const void *src, void *dst, size_t bytes, void *zero, size_t zero_bytes, uint64_t *t);
 
 // ---- update path (k_update.hip) ---------------------------------------------
 // QSRP screen kernels (k_qsrp.hip).  qn holds 3 floats per query: upper bounds

@@ -277,3 +277,28 @@ def test_screened_refinement(orc, gpu_index_factory, d, U, I):
         assert res.timing["n_refined"] > 0
         assert np.array_equal(res.users[:, :k], bu) and np.array_equal(res.ranks[:, :k], br)
     idx.close()
+
+
+@pytest.mark.parametrize("U,nq,k,max_k", [(1, 1, 1, 1), (65, 16, 20, 33), (3000, 17, 5, 300), (9000, 600, 40, 1500)])
+def test_results_written_to_the_host(orc, gpu_index_factory, U, nq, k, max_k):
+    """Outputs written by the top-k itself (up to 8 MB, the last one is past it):
+    padding past k, stats and counters, twice in a row."""
+    _case(f"host results U={U} nq={nq} k={k} max_k={max_k}")
+    rng = np.random.default_rng(U)
+    users = rng.standard_normal((U, 10), dtype=np.float32)
+    items = rng.standard_normal((500, 10), dtype=np.float32)
+    queries = rng.standard_normal((nq, 10), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 20)
+    n = min(8, nq)
+    bu, br, bq = orc.bruteforce(orc.normalize_users(users), items, queries[:n], min(k, U))
+    for form in ("plain", "screened"):
+        idx.set_form(form)
+        for _ in range(2):
+            res = idx.query(queries, min(k, U), max_k=max_k)
+            m = min(k, U)
+            assert np.array_equal(res.users[:n, :m], bu) and np.array_equal(res.ranks[:n, :m], br)
+            assert np.array_equal(res.qips[:n, :m], bq)
+            assert np.all(res.users[:, m:] == -1) and np.all(res.ranks[:, m:] == -1) and np.all(res.qips[:, m:] == -1)
+            assert all(s["n_candidate"] >= m and s["n_prune_user"] == U - s["n_candidate"] for s in res.stats)
+            assert res.timing["total_ms"] > 0 and res.timing["topk_ms"] > 0
+    idx.close()
