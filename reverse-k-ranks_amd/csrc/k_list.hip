@@ -221,19 +221,20 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
     if (threadIdx.x == 0) n_finer = 0;
     __syncthreads();
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
-        const uint4 *h4 = reinterpret_cast<const uint4 *>(hist + (int64_t)b * GW);
+        // the row's 64 counts in flight together (read one after the other, the
+        // early end of the search costs more than it saves)
+        u32x4 v[GW / 4];
+#pragma unroll
+        for (int j = 0; j < GW / 4; ++j) v[j] = reinterpret_cast<const u32x4 *>(hist + (int64_t)b * GW)[j];
         const int64_t k = qi[b].topk;
         const double mean = (double)k / (double)stride;
         const int64_t want = stride == 1 ? k : (int64_t)(mean + 3.0 * sqrt(mean) + 4.0) + 1;
         int32_t t = -1;
         int64_t cum = 0, n = 0;
-        for (int j = 0; j < GW / 4 && t < 0; ++j) {
-            const uint4 v = h4[j];
-            const uint32_t x[4] = {v.x, v.y, v.z, v.w};
-            for (int c = 0; c < 4; ++c) {
-                cum += x[c];
-                if (t < 0 && 4 * j + c < n_fine && cum >= want) { t = 4 * j + c; n = cum; }
-            }
+#pragma unroll
+        for (int f = 0; f < GW; ++f) {
+            cum += v[f / 4][f % 4];
+            if (t < 0 && f < n_fine && cum >= want) { t = f; n = cum; }
         }
         n = min(n * stride, n_user);
         if (n > cap) t = -1;
@@ -244,17 +245,23 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
         }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        // columns in order while their estimated lists fit
-        int32_t s = 0;
-        int64_t sum = 0;
-        for (int t = 0; t < GW; ++t) {
-            sum += load[t];
-            const bool fits = 2 * sum <= list_cap;
-            at[t] = fits ? s : -1;
-            if (fits) s += bin[t];
+    if (threadIdx.x < 64) {
+        // columns in order while their estimated lists fit: a column per lane
+        static_assert(GW == 64, "one wavefront");
+        const int t = threadIdx.x;
+        int64_t sum = load[t];
+        int32_t s = bin[t];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int64_t y = __shfl_up(sum, o, 64);
+            const int32_t z = __shfl_up(s, o, 64);
+            if (t >= o) { sum += y; s += z; }
         }
-        n_slots = s;
+        const bool fits = 2 * sum <= list_cap;  // loads are not negative: true up to some column
+        at[t] = fits ? s - bin[t] : -1;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(fits);
+        if (t == 0 && m == 0) n_slots = 0;
+        if (m != 0 && t == 63 - __clzll((long long)m)) n_slots = s;
     }
     __syncthreads();
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
