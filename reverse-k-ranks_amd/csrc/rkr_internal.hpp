@@ -448,6 +448,13 @@ hipError_t launch_rank_hist(hipStream_t s, const float *sorted, int64_t ld, int6
 hipError_t launch_transit(hipStream_t s, const int64_t *C, int32_t Q, const int32_t *pos, const int32_t *col,
                           const int64_t *end_cost, int32_t R, int64_t *T);
 // One DP layer: dp_cur[r] = min(dp_prev[r], min_{p<r} dp_prev[p] + T[r][p]).
+// All n_layer rows of the DP (dp, path: n_layer x R; row 0 given, the others of
+// dp set to kDpUnset) for ranks that dp_in_one_launch; *err is set where a value
+// was waited for spin_max times.
+constexpr int64_t kDpUnset = (int64_t)0x8080808080808080ull;  // no sum of costs
+bool dp_in_one_launch(int64_t R);
+hipError_t launch_dp_layers(hipStream_t s, const int64_t *T, int32_t R, int32_t n_layer, int64_t *dp, int32_t *path,
+                            int32_t spin_max, int32_t *err);
 hipError_t launch_dp_layer(hipStream_t s, const int64_t *T, const int64_t *dp_prev, const int32_t *pos_prev, int32_t R,
                            int64_t *dp_cur, int32_t *pos_cur);
 

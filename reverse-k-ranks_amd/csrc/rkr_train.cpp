@@ -204,10 +204,15 @@ int rkr_find_optimal_sample(rkr_ctx *c, int64_t n_user, int64_t n_item, int32_t 
     RKR_HIP(c, hipSetDevice(c->device));
     RKR_HIP(c, hipStreamSynchronize(c->stream));
     DevArr<int64_t> dC{c}, dEnd{c}, dT{c}, dDp{c};
-    DevArr<int32_t> dPos{c}, dPath{c};
+    DevArr<int32_t> dPos{c}, dPath{c}, dErr{c};
+    // one launch keeps every layer's row, if the budget has room beside the rest
+    const size_t dp_need = sizeof(int64_t) * (C.size() + (size_t)R + (size_t)(R * (R - 1) / 2) + (size_t)n_sample * R) +
+                           sizeof(int32_t) * ((size_t)(2 * R) + (size_t)n_sample * R + 64);
+    const bool one = dp_in_one_launch(R) && c->held + dp_need <= c->budget;
+    const int64_t dp_rows = one ? n_sample : 2;
     int rc;
     if ((rc = dC.alloc(C.size(), "training prefix sums")) || (rc = dEnd.alloc((size_t)R, "training costs")) ||
-        (rc = dT.alloc((size_t)(R * (R - 1) / 2), "transit costs")) || (rc = dDp.alloc((size_t)(2 * R), "DP row")) ||
+        (rc = dT.alloc((size_t)(R * (R - 1) / 2), "transit costs")) || (rc = dDp.alloc((size_t)(dp_rows * R), "DP rows")) || (rc = dErr.alloc(1, "DP state")) ||
         (rc = dPos.alloc((size_t)(2 * R), "query positions")) ||
         (rc = dPath.alloc((size_t)n_sample * R, "DP positions")))
         return rc;
@@ -219,15 +224,23 @@ int rkr_find_optimal_sample(rkr_ctx *c, int64_t n_user, int64_t n_item, int32_t 
     RKR_HIP(c, hipMemcpyAsync(dDp.p, dp0.data(), sizeof(int64_t) * R, hipMemcpyHostToDevice, s));
     RKR_HIP(c, hipMemcpyAsync(dPath.p, pos0.data(), sizeof(int32_t) * R, hipMemcpyHostToDevice, s));
     RKR_HIP(c, launch_transit(s, dC.p, (int32_t)Q, dPos.p, dPos.p + R, dEnd.p, (int32_t)R, dT.p));
-    for (int32_t l = 1; l < n_sample; ++l)
+    if (one) {
+        RKR_HIP(c, hipMemsetAsync(dErr.p, 0, sizeof(int32_t), s));
+        if (n_sample > 1) RKR_HIP(c, hipMemsetAsync(dDp.p + R, 0x80, sizeof(int64_t) * (size_t)((n_sample - 1) * R), s));
+        RKR_HIP(c, launch_dp_layers(s, dT.p, (int32_t)R, n_sample, dDp.p, dPath.p, 1 << 20, dErr.p));
+    }
+    for (int32_t l = 1; !one && l < n_sample; ++l)
         RKR_HIP(c, launch_dp_layer(s, dT.p, dDp.p + ((l - 1) & 1) * R, dPath.p + (int64_t)(l - 1) * R, (int32_t)R,
                                    dDp.p + (l & 1) * R, dPath.p + (int64_t)l * R));
     std::vector<int64_t> last((size_t)R);
     std::vector<int32_t> path((size_t)n_sample * R);
-    RKR_HIP(c, hipMemcpyAsync(last.data(), dDp.p + ((n_sample - 1) & 1) * R, sizeof(int64_t) * R,
+    int32_t err = 0;
+    if (one) RKR_HIP(c, hipMemcpyAsync(&err, dErr.p, sizeof(err), hipMemcpyDeviceToHost, s));
+    RKR_HIP(c, hipMemcpyAsync(last.data(), dDp.p + (one ? n_sample - 1 : (n_sample - 1) & 1) * R, sizeof(int64_t) * R,
                               hipMemcpyDeviceToHost, s));
     RKR_HIP(c, hipMemcpyAsync(path.data(), dPath.p, sizeof(int32_t) * path.size(), hipMemcpyDeviceToHost, s));
     RKR_HIP(c, hipStreamSynchronize(s));
+    if (err) return set_err(c, RKR_ERR_HIP, "find_optimal_sample: the DP's workgroups waited too long for each other");
 
     // smallest final cost, first index on ties (unsigned compare as the reference's)
     uint64_t min_cost = UINT64_MAX;

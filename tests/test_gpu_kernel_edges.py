@@ -302,3 +302,57 @@ def test_results_written_to_the_host(orc, gpu_index_factory, U, nq, k, max_k):
             assert all(s["n_candidate"] >= m and s["n_prune_user"] == U - s["n_candidate"] for s in res.stats)
             assert res.timing["total_ms"] > 0 and res.timing["topk_ms"] > 0
     idx.close()
+
+
+def _sample_rank_dp(n_user, kth, accu, n_sample):
+    """Cost and path of the sample-rank DP over prefix sums, 64-bit whole numbers."""
+    Q = len(kth)
+    rank = np.array(sorted({int(k) for k in kth} | {int(k) - 1 for k in kth if k > 0}))
+    pos = np.searchsorted(kth, rank, side="right")
+    S = np.zeros((Q + 1, len(rank)), np.int64)  # S[x, j] = sum of accu[q][rank_j] over q < x
+    S[1:] = np.cumsum(accu[:, rank].astype(np.int64), axis=0)
+    j = np.arange(len(rank))
+    end = (Q - pos) * n_user - (S[Q] - S[pos, j])
+    between = (S[pos, j][:, None] - S[pos][:, j].T) - (S[pos][:, j] - S[pos, j][None, :])
+    between[(pos[None, :] >= pos[:, None]) | (pos[None, :] >= Q)] = 0
+    T = -end[None, :] + between + end[:, None]
+    T[j[None, :] >= j[:, None]] = 1 << 60
+    dp, path = S[pos, j] + end, [j.copy()]
+    for _ in range(1, n_sample):
+        c = dp[None, :] + T
+        p = c.argmin(axis=1)
+        better = c[j, p] < dp
+        path.append(np.where(better, p, path[-1]))
+        dp = np.where(better, c[j, p], dp)
+    i = int(dp.argmin())
+    cost, out = int(dp[i]), []
+    for p in reversed(path):
+        out.append(int(rank[i]))
+        i = int(p[i])
+    return out[::-1], cost
+
+
+@pytest.mark.parametrize("I,Q,n_sample", [(60, 3, 2), (400, 33, 20), (3000, 120, 12), (6000, 530, 40), (9000, 1015, 25),
+                                          (14_000, 2100, 9), (30_000, 2300, 6)])
+def test_sample_rank_dp_sizes(orc, I, Q, n_sample):
+    """The DP of sample-rank training at every number of ranks it holds in
+    registers (up to 512, 1024, 2048) and past it."""
+    from rkr import train
+    from test_gpu_train import _synthetic_distribution
+    import rkr
+    rng = np.random.default_rng(Q)
+    accu = _synthetic_distribution(rng, 40, I, Q, I // 2)
+    kth, order = train.sort_kth_rank(accu, 5)
+    acc_s = accu[order]
+    want, cost = _sample_rank_dp(40, kth, acc_s, n_sample)
+    n_rank = len(set(kth.tolist()) | {int(k) - 1 for k in kth if k > 0})
+    _case(f"sample-rank DP Q={Q}: {n_rank} ranks, {n_sample} layers")
+    if n_rank < 200:  # the oracle's own DP is cubic
+        oranks, ocost = orc.find_optimal_sample_fast(40, I, kth, acc_s, 0, n_sample)
+        assert ocost == cost and (len(set(want)) < n_sample or list(oranks) == want)
+    with rkr.Index(0) as idx:
+        for _ in range(2):
+            ranks, got = train.find_optimal_sample(idx, 40, I, kth, acc_s, n_sample, "OptimalPart")
+            assert got == cost
+            if len(set(want)) == n_sample:  # a rank kept for several samples is filled up from others
+                assert ranks.tolist() == want
