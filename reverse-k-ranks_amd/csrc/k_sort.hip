@@ -5,8 +5,8 @@
 // (src/include/score_computation/ComputeScoreTableBatch.hpp:83-89).  Only the values are kept, so the
 // order of equal values is irrelevant and the sort need not be stable.
 //
-// One 1024-thread workgroup per CU, taking rows in turn.  Rows of up to NMAX values are sorted in LDS
-// (bucket path):
+// Persistent workgroups of 256, 512 or 1024 threads by the rows' length, taking rows in turn.  Rows of up
+// to 28 values per thread are sorted in LDS (bucket path):
 //   1. the row is in registers (coalesced loads, issued while the workgroup's previous row was
 //      sorted), and each wavefront's min and max of it were taken before that row's last barrier;
 //   2. a histogram over NBK value bins, descending, and its exclusive scan.  The bins are
@@ -22,6 +22,9 @@
 // LDS operations and barriers set the pace.  Ranking each value by counting over its bin read about
 // 14 LDS words per value, the bins' networks 3.3 and as many writes: 10,007 rows of 20,000 took 1263 us
 // (in 24 launches) and take 814 us, 1.97 TB/s of the 4.7 a large copy reaches.
+// With 1024 threads for every length the shorter rows left most of a CU waiting at barriers: 50,000 rows
+// of 10,000 take 2.3 ms with 512 threads a row, two rows on a CU (3.6 with 1024), and 8,398 rows of 1,617
+// 0.2 with 256, four on a CU (0.5).
 // A row longer than NMAX, or one with a bin over BIN_MAX values (heavy ties, extreme skew), takes
 // the merge path instead:
 //   1. tiles of TILE values are sorted in LDS by a bitonic network (a partial last tile is padded with
@@ -37,43 +40,9 @@
 namespace rkr {
 namespace {
 
-constexpr int NT = 1024;                 // threads per row
-constexpr int NW = NT / 64;              // wavefronts per row
 constexpr int TILE = 8192;               // values sorted in LDS at a time (32 KB)
-constexpr int PER = TILE / 2 / NT;       // compare-exchange pairs per thread and stage
-constexpr int NBK = 8192;                // value bins of the bucket path
-constexpr int NMAX = 28672;              // longest row of the bucket path (112 KB of LDS)
-constexpr int EPT = NMAX / NT;           // values per thread
 constexpr uint32_t BIN_MAX = 192;        // largest bin the bucket path ranks by counting
-constexpr int NB1 = 1024;                // linear coarse bins that apportion the NBK bins
 constexpr int KPAD = 16;                 // zero keys past the row's end, read by the bins' sort windows
-
-struct alignas(16) SortSmem {
-    union {
-        float tile[TILE];                // merge path
-        struct {
-            uint32_t key[NMAX + KPAD];   // the row's keys, bin by bin, then KPAD zero keys
-            uint32_t cnt[NBK];           // bin counts, then scatter cursors, then the long bins' list
-            uint32_t fseg[NB1];          // bins of coarse bin c: s0 | s1 << 16, bins s0 .. s1 - 1
-            uint32_t coarse[NB1];        // coarse counts (zero between rows)
-            float red_f[2 * NW];         // the row's min and max per wavefront, then the largest bin
-            uint32_t red_u[NW + 1];      // wavefront sums of the scans; [NW]: bins ranked by wavefronts
-        } b;
-    } u;
-};
-
-// Bin of x, descending: its coarse bin c (NB1 linear bins from hi down)
-// owns bins s0 .. s1 - 1 (fseg[c] = s0 | s1 << 16: one LDS read), and x takes the one its place
-// inside c falls in.  t is clamped to [0, NB1] (NaN from 0 * inf at x == hi
-// to 0), so c = NB1 - 1 with frac 1 at and past the range's end.
-__device__ __forceinline__ int sort_bin(const uint32_t *fseg, float x, float hi, float scale1) {
-    const float t = fminf(fmaxf((hi - x) * scale1, 0.0f), (float)NB1);
-    const int c = min((int)t, NB1 - 1);
-    const float frac = t - (float)c;
-    const uint32_t g = fseg[c];
-    const int s0 = (int)(g & 0xFFFFu), nc = (int)(g >> 16) - s0;  // nc >= 1
-    return s0 + min(nc - 1, (int)(frac * (float)nc));
-}
 
 // Order-preserving key of a float: key(a) < key(b) whenever a < b.  Every NaN
 // maps to the largest key (the bins put NaN first); -0 keys just below +0.
@@ -107,10 +76,62 @@ __device__ __forceinline__ void sort_desc(uint32_t (&z)[N]) {
                     }
 }
 
+// Number of elements of A among the first d outputs of the descending merge of
+// A[0..na) and B[0..nb), where A goes first on ties.
+__device__ inline int merge_split(const float *A, int na, const float *B, int nb, int d) {
+    int lo = max(0, d - nb), hi = min(d, na);
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (A[mid] >= B[d - 1 - mid]) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// The sort of a row by NT threads.  All sizes go with NT, so a row of a quarter
+// of the longest takes a quarter of a CU's threads, registers and LDS, and the
+// barriers of one row pass while others on the CU work: a CU holds 1024 / NT
+// workgroups.
+template <int NT>
+struct RowSort {
+static constexpr int NW = NT / 64;              // wavefronts per row
+static constexpr int PER = TILE / 2 / NT;       // compare-exchange pairs per thread and stage
+static constexpr int NBK = 8 * NT;              // value bins of the bucket path
+static constexpr int NMAX = 28 * NT;            // longest row of the bucket path (112 KB of LDS at NT = 1024)
+static constexpr int EPT = NMAX / NT;           // values per thread
+static constexpr int NB1 = NT;                  // linear coarse bins that apportion the NBK bins
+
+struct alignas(16) SortSmem {
+    union {
+        float tile[TILE];                // merge path
+        struct {
+            uint32_t key[NMAX + KPAD];   // the row's keys, bin by bin, then KPAD zero keys
+            uint32_t cnt[NBK];           // bin counts, then scatter cursors, then the long bins' list
+            uint32_t fseg[NB1];          // bins of coarse bin c: s0 | s1 << 16, bins s0 .. s1 - 1
+            uint32_t coarse[NB1];        // coarse counts (zero between rows)
+            float red_f[2 * NW];         // the row's min and max per wavefront, then the largest bin
+            uint32_t red_u[NW + 1];      // wavefront sums of the scans; [NW]: bins ranked by wavefronts
+        } b;
+    } u;
+};
+
+// Bin of x, descending: its coarse bin c (NB1 linear bins from hi down)
+// owns bins s0 .. s1 - 1 (fseg[c] = s0 | s1 << 16: one LDS read), and x takes the one its place
+// inside c falls in.  t is clamped to [0, NB1] (NaN from 0 * inf at x == hi
+// to 0), so c = NB1 - 1 with frac 1 at and past the range's end.
+static __device__ __forceinline__ int sort_bin(const uint32_t *fseg, float x, float hi, float scale1) {
+    const float t = fminf(fmaxf((hi - x) * scale1, 0.0f), (float)NB1);
+    const int c = min((int)t, NB1 - 1);
+    const float frac = t - (float)c;
+    const uint32_t g = fseg[c];
+    const int s0 = (int)(g & 0xFFFFu), nc = (int)(g >> 16) - s0;  // nc >= 1
+    return s0 + min(nc - 1, (int)(frac * (float)nc));
+}
+
 // Sorts s[0..TILE) in descending order.  Stage (k, j) compares i with i + j for
 // the i whose bit j is clear; blocks of k elements alternate direction so that
 // each merge step sees bitonic sequences, and the final k = TILE is descending.
-__device__ inline void bitonic_desc(float *s) {
+static __device__ inline void bitonic_desc(float *s) {
     for (int k = 2; k <= TILE; k <<= 1) {
         for (int j = k >> 1; j > 0; j >>= 1) {
 #pragma unroll
@@ -129,18 +150,6 @@ __device__ inline void bitonic_desc(float *s) {
     }
 }
 
-// Number of elements of A among the first d outputs of the descending merge of
-// A[0..na) and B[0..nb), where A goes first on ties.
-__device__ inline int merge_split(const float *A, int na, const float *B, int nb, int d) {
-    int lo = max(0, d - nb), hi = min(d, na);
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (A[mid] >= B[d - 1 - mid]) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // A row of n <= NMAX values in registers, EPT slots per thread.  Rows of a
 // multiple of 4 values whose rows start 16-byte aligned (vec) take 16 bytes
 // per slot group (slot 4k + c holds value 4 (t + k NT) + c), others 4 bytes
@@ -148,19 +157,19 @@ __device__ inline int merge_split(const float *A, int na, const float *B, int nb
 // test is uniform, so the slots past a short row are skipped, not run with no
 // lanes active); in_row says whether this thread's slot e holds one.
 template <bool vec>
-__device__ __forceinline__ int row_slots(int n) {
+static __device__ __forceinline__ int row_slots(int n) {
     return vec ? 4 * ((n / 4 + NT - 1) / NT) : (n + NT - 1) / NT;
 }
 
 template <bool vec>
-__device__ __forceinline__ bool in_row(int t, int e, int n) {
+static __device__ __forceinline__ bool in_row(int t, int e, int n) {
     return vec ? t + (e >> 2) * NT < (n >> 2) : t + e * NT < n;
 }
 
 // Issues every load of the thread's slots before any is used, from clamped
 // addresses; the caller's first use of v waits for them.
 template <bool vec>
-__device__ __forceinline__ void load_row(int t, float (&v)[EPT], const float *x, int n) {
+static __device__ __forceinline__ void load_row(int t, float (&v)[EPT], const float *x, int n) {
     if constexpr (vec) {
         const float4 *x4 = reinterpret_cast<const float4 *>(x);
         const int n4 = n / 4;
@@ -177,7 +186,7 @@ __device__ __forceinline__ void load_row(int t, float (&v)[EPT], const float *x,
 
 // The inverse of load_row: each slot's value back to its place in y.
 template <bool vec>
-__device__ __forceinline__ void store_row(int t, const float (&v)[EPT], float *y, int n) {
+static __device__ __forceinline__ void store_row(int t, const float (&v)[EPT], float *y, int n) {
     if constexpr (vec) {
         float4 *y4 = reinterpret_cast<float4 *>(y);
 #pragma unroll
@@ -197,7 +206,7 @@ __device__ __forceinline__ void store_row(int t, const float (&v)[EPT], float *y
 // Each wavefront's min and max of the row held in v, into red_f (read by the
 // row's bucket path after the next barrier).
 template <bool vec>
-__device__ __forceinline__ void row_partials(SortSmem &sm, const float (&v)[EPT], int32_t n, int t) {
+static __device__ __forceinline__ void row_partials(SortSmem &sm, const float (&v)[EPT], int32_t n, int t) {
     const int lane = t & 63, w = t >> 6;
     float mn = INFINITY, mx = -INFINITY;
 #pragma unroll
@@ -225,7 +234,7 @@ __device__ __forceinline__ void row_partials(SortSmem &sm, const float (&v)[EPT]
 // min/max partials in red_f.  On entry red_f holds this row's partials and
 // coarse is zero.  y may be the row v came from.
 template <bool vec>
-__device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], int32_t n, float *y, bool out_vec,
+static __device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], int32_t n, float *y, bool out_vec,
                                                 const float *xn, int t) {
     const int lane = t & 63, w = t >> 6;
     const int ne = row_slots<vec>(n);
@@ -421,7 +430,7 @@ __device__ __forceinline__ bool bucket_sort_row(SortSmem &sm, float (&v)[EPT], i
 
 // Merge path for one row; x and y may be the same row: every value of x is
 // read before y is written where it lies.
-__device__ void merge_sort_row(float *s, const float *x, int32_t n, float *out_row, float *tmp_row) {
+static __device__ void merge_sort_row(float *s, const float *x, int32_t n, float *out_row, float *tmp_row) {
     int passes = 0;
     for (int64_t w = TILE; w < n; w <<= 1) ++passes;
     float *a = (passes & 1) ? tmp_row : out_row;  // sorted tiles
@@ -465,30 +474,32 @@ __device__ void merge_sort_row(float *s, const float *x, int32_t n, float *out_r
         b = t;
     }
 }
+};
 
 // Workgroup p sorts rows p, p + G, p + 2G, ... (G = gridDim.x); its merge
 // passes use scratch row p.  vec (every row starts 16-byte aligned and n is a
 // multiple of 4): on the bucket path the next row's loads are in flight while
 // the current row is sorted.
-template <bool vec>
-__global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_src, int64_t n_rows, int32_t n,
+template <bool vec, int NT>
+__global__ void __launch_bounds__(NT, 4) k_sort_rows(const float *src, int64_t ld_src, int64_t n_rows, int32_t n,
                                                   float *out, float *tmp, int64_t ld, int out_vec) {
-    __shared__ SortSmem sm;
+    using RS = RowSort<NT>;
+    __shared__ typename RS::SortSmem sm;
     int64_t row = blockIdx.x;
     float *tmp_row = tmp + (int64_t)blockIdx.x * ld;
-    if (n > NMAX) {
+    if (n > RS::NMAX) {
         for (; row < n_rows; row += gridDim.x) {
-            merge_sort_row(sm.u.tile, src + row * ld_src, n, out + row * ld, tmp_row);
+            RS::merge_sort_row(sm.u.tile, src + row * ld_src, n, out + row * ld, tmp_row);
             __syncthreads();  // the tiles are free before the next row's first tile
         }
         return;
     }
-    float v[EPT];
+    float v[RS::EPT];
     if (row >= n_rows) return;
-    for (int i = threadIdx.x; i < NB1; i += NT) sm.u.b.coarse[i] = 0u;
+    for (int i = threadIdx.x; i < RS::NB1; i += NT) sm.u.b.coarse[i] = 0u;
     if constexpr (vec) {
-        load_row<vec>(threadIdx.x, v, src + row * ld_src, n);
-        row_partials<vec>(sm, v, n, threadIdx.x);
+        RS::template load_row<vec>(threadIdx.x, v, src + row * ld_src, n);
+        RS::template row_partials<vec>(sm, v, n, threadIdx.x);
         __syncthreads();
     }
     for (; row < n_rows; row += gridDim.x) {
@@ -501,8 +512,8 @@ __global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_s
         asm volatile("" : "+s"(nn), "+v"(t));
         const float *x = src + row * ld_src;
         if constexpr (!vec) {
-            load_row<vec>(t, v, x, nn);
-            row_partials<vec>(sm, v, nn, t);
+            RS::template load_row<vec>(t, v, x, nn);
+            RS::template row_partials<vec>(sm, v, nn, t);
             __syncthreads();
         }
         // the next row's loads are issued unconditionally (so v is dead across
@@ -510,12 +521,12 @@ __global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_s
         // it has just read, and the values are not used
         const int64_t next = row + gridDim.x;
         const float *xn = src + (next < n_rows ? next : row) * ld_src;
-        if (!bucket_sort_row<vec>(sm, v, nn, out + row * ld, out_vec != 0, xn, t)) {
+        if (!RS::template bucket_sort_row<vec>(sm, v, nn, out + row * ld, out_vec != 0, xn, t)) {
             __syncthreads();  // the bucket path's LDS is done with before the tiles reuse it
-            merge_sort_row(sm.u.tile, x, n, out + row * ld, tmp_row);
+            RS::merge_sort_row(sm.u.tile, x, n, out + row * ld, tmp_row);
             if constexpr (vec) {
-                load_row<vec>(t, v, xn, nn);
-                row_partials<vec>(sm, v, nn, t);
+                RS::template load_row<vec>(t, v, xn, nn);
+                RS::template row_partials<vec>(sm, v, nn, t);
             }
         }
         __syncthreads();  // this row's LDS is done with, the next row's partials are visible
@@ -524,6 +535,13 @@ __global__ void __launch_bounds__(NT) k_sort_rows(const float *src, int64_t ld_s
 
 }  // namespace
 
+// Threads per row: the fewest that hold it in the bucket path.
+static int sort_threads(int64_t n_item) {
+    return n_item <= RowSort<256>::NMAX ? 256 : n_item <= RowSort<512>::NMAX ? 512 : 1024;
+}
+
+int64_t sort_rows_in_flight(int64_t n_item, int n_cu) { return (int64_t)n_cu * (1024 / sort_threads(n_item)); }
+
 hipError_t launch_sort_rows(hipStream_t s, const float *src, int64_t ld_src, int64_t nb, int64_t n_item, float *out,
                             float *tmp, int64_t tmp_rows, int64_t ld, int n_cu) {
     if (nb <= 0 || n_item <= 0) return hipSuccess;
@@ -531,12 +549,22 @@ hipError_t launch_sort_rows(hipStream_t s, const float *src, int64_t ld_src, int
         return hipErrorInvalidValue;
     const bool vec = (n_item & 3) == 0 && (ld_src & 3) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
     const int out_vec = (n_item & 3) == 0 && (ld & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 ? 1 : 0;
-    // one workgroup fits a CU, and each needs a scratch row of its own
-    const dim3 grid((unsigned)std::min<int64_t>({nb, (int64_t)n_cu, tmp_rows}));
-    if (vec)
-        hipLaunchKernelGGL(k_sort_rows<true>, grid, dim3(NT), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, ld, out_vec);
-    else
-        hipLaunchKernelGGL(k_sort_rows<false>, grid, dim3(NT), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, ld, out_vec);
+    const int nt = sort_threads(n_item);
+    // each workgroup needs a scratch row of its own
+    const dim3 grid((unsigned)std::min<int64_t>({nb, sort_rows_in_flight(n_item, n_cu), tmp_rows}));
+#define RKR_SORT(v, threads)                                                                                      \
+    hipLaunchKernelGGL((k_sort_rows<v, threads>), grid, dim3(threads), 0, s, src, ld_src, nb, (int32_t)n_item, out, tmp, \
+                       ld, out_vec)
+    if (vec) {
+        if (nt == 256) RKR_SORT(true, 256);
+        else if (nt == 512) RKR_SORT(true, 512);
+        else RKR_SORT(true, 1024);
+    } else {
+        if (nt == 256) RKR_SORT(false, 256);
+        else if (nt == 512) RKR_SORT(false, 512);
+        else RKR_SORT(false, 1024);
+    }
+#undef RKR_SORT
     return hipGetLastError();
 }
 

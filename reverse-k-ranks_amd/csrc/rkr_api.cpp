@@ -958,7 +958,7 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
     if (nb <= 0) return set_err(c, RKR_ERR_NOMEM, std::string(what) + ": no memory for a score block");
     // the build scratch, kept between calls (allocating and freeing the block
     // took 1 ms of a call over 13k users)
-    const int64_t tmp_rows = std::min<int64_t>(nb, c->n_cu);  // one per workgroup of the row sort
+    const int64_t tmp_rows = std::min<int64_t>(nb, sort_rows_in_flight(I, c->n_cu));
     const size_t blk_bytes = ((size_t)nb * row_bytes + 255) & ~(size_t)255;
     const size_t tmp_bytes = ((size_t)tmp_rows * row_bytes + 255) & ~(size_t)255;
     int rc = ensure(c, c->misc, blk_bytes + tmp_bytes + sizeof(float) * (size_t)(nb * extra), "score block");

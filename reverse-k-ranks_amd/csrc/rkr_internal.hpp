@@ -432,8 +432,9 @@ hipError_t launch_select_rows(hipStream_t s, const float *scores, int64_t nb, in
 
 // ---- full sorted rows (k_sort.hip) ------------------------------------------
 // out[b * ld + i] = i-th largest of src[b * ld_src + 0..n_item), b < nb; tmp is
-// scratch of tmp_rows rows of stride ld.  out may be src (ld == ld_src).  One
-// workgroup fits a CU; at most min(n_cu, tmp_rows) run, taking rows in turn.
+// scratch of tmp_rows rows of stride ld.  out may be src (ld == ld_src).  A
+// CU holds sort_rows_in_flight / n_cu workgroups; at most tmp_rows run, taking rows in turn.
+int64_t sort_rows_in_flight(int64_t n_item, int n_cu);  // scratch rows that keep every workgroup busy
 hipError_t launch_sort_rows(hipStream_t s, const float *src, int64_t ld_src, int64_t nb, int64_t n_item, float *out,
                             float *tmp, int64_t tmp_rows, int64_t ld, int n_cu);
 

@@ -356,3 +356,18 @@ def test_sample_rank_dp_sizes(orc, I, Q, n_sample):
             assert got == cost
             if len(set(want)) == n_sample:  # a rank kept for several samples is filled up from others
                 assert ranks.tolist() == want
+
+
+@pytest.mark.parametrize("I", [2, 255, 1617, 7168, 7169, 7172, 14_336, 14_340, 28_672, 28_676])
+def test_row_sort_thread_counts(orc, I):
+    """Rows on either side of the lengths that take 256, 512 and 1024 threads, some with equal values only."""
+    _case(f"row sort I={I}")
+    import rkr
+    rng = np.random.default_rng(I)
+    users = rng.standard_normal((70, 5), dtype=np.float32)
+    users[3] = 0.0
+    items = rng.standard_normal((I, 5), dtype=np.float32)
+    with rkr.Index(0) as idx:
+        idx.set_data(users, items)
+        got = idx.sorted_scores()
+    assert np.array_equal(got, orc.sorted_score_rows(orc.normalize_users(users), items))
