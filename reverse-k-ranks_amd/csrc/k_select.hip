@@ -18,14 +18,20 @@
 //      fl(x - lo) and fl(t * scale) are monotone in x, so the bin is too); a
 //      reverse prefix sum tells, for every r_j, its bin and the elements
 //      above that bin;
-//   3. one more pass over the row gathers the elements of the bins holding
-//      targets into LDS (the histogram's storage), with a bitmap of target
-//      bins deciding membership -- several passes only when they exceed it;
+//   3. one more pass over the row (its bins kept in registers, two to a word)
+//      gathers the elements of the bins holding targets into LDS (the
+//      histogram's storage).  A table of half that storage says which target
+//      bin a bin is, or a bitmap and its prefix where more than half is
+//      gathered -- in several passes only when all of it is exceeded;
 //   4. bins of up to 64 elements are ranked element-parallel (each element
 //      counts the elements of its bin that order before it), larger ones by
 //      one wavefront (register bitonic sort up to 256, counting above) or
 //      the whole workgroup (wg_select, which narrows the bin by repeated
 //      histograms -- this also makes ties and skewed rows exact).
+// Bound: LDS operations and the barriers between phases; a row's load is a
+// fifth of its time.  150k rows of 50,000 values, 4096 ranks: 29.4 ms with the
+// bins computed again and two LDS reads per value in the gather, now 26.2 (its
+// 30 GB take 6.4 at copy rate).
 #include "rkr_internal.hpp"
 
 namespace rkr {
@@ -75,7 +81,7 @@ struct SelSmem {
     uint16_t srk[SMAX];           // the target ranks, when n_item <= 65536
     float red_f[2 * NW];
     uint32_t red_u[NW + 1];
-    int32_t nfb, ngrp, ncoop, nmid, sel_b;
+    int32_t nfb, ngrp, ncoop, nmid, sel_b, few;
 };
 
 // Monotone in x for x >= lo with FP32 arithmetic (every rounding step is
@@ -129,7 +135,8 @@ __device__ __forceinline__ void fine_bins(const uint32_t *fseg, const float (&v)
 template <int C4>
 struct RowRegs {
     float4 r[C4];
-    int nv;  // float4s this thread owns
+    uint32_t bins[2 * C4];  // level-0 bins of the values, two to a word
+    int nv;                 // float4s this thread owns
     __device__ __forceinline__ void load(const float *__restrict__ x, int64_t n) {
         const float4 *x4 = reinterpret_cast<const float4 *>(x);
         const int n4 = (int)(n >> 2), t = threadIdx.x;
@@ -140,7 +147,8 @@ struct RowRegs {
 #pragma unroll
         for (int k = 0; k < C4; ++k) r[k] = x4[min(t + k * NT, max(n4 - 1, 0))];
     }
-    // f(const float (&v)[4]) for every float4 the thread owns
+    // f(const float (&v)[4]) for every float4 the thread owns, or f(v, b) with
+    // the values' bins, which `bin` (v, b) finds and for_each_bin keeps
     template <class F>
     __device__ __forceinline__ void for_each(F &&f) const {
 #pragma unroll
@@ -148,6 +156,30 @@ struct RowRegs {
             if (k < nv) {
                 const float v[4] = {r[k].x, r[k].y, r[k].z, r[k].w};
                 f(v);
+            }
+    }
+    template <class B, class F>
+    __device__ __forceinline__ void for_each_bin(B &&bin, F &&f) {
+#pragma unroll
+        for (int k = 0; k < C4; ++k)
+            if (k < nv) {
+                const float v[4] = {r[k].x, r[k].y, r[k].z, r[k].w};
+                int b[4];
+                bin(v, b);
+                bins[2 * k] = (uint32_t)b[0] | (uint32_t)b[1] << 16;
+                bins[2 * k + 1] = (uint32_t)b[2] | (uint32_t)b[3] << 16;
+                f(v, b);
+            }
+    }
+    template <class F>
+    __device__ __forceinline__ void for_each_kept(F &&f) const {
+#pragma unroll
+        for (int k = 0; k < C4; ++k)
+            if (k < nv) {
+                const float v[4] = {r[k].x, r[k].y, r[k].z, r[k].w};
+                const int b[4] = {(int)(bins[2 * k] & 0xFFFFu), (int)(bins[2 * k] >> 16),
+                                  (int)(bins[2 * k + 1] & 0xFFFFu), (int)(bins[2 * k + 1] >> 16)};
+                f(v, b);
             }
     }
 };
@@ -298,38 +330,28 @@ __device__ __forceinline__ void wg_reverse_incl(SelSmem &sm, uint32_t *h) {
     const int base = threadIdx.x * per;
     if constexpr (per == 16) {
         const int rot = (threadIdx.x >> 1) & 3;
-        u32x4 q[4], nat[4];
+        u32x4 q[4];  // step i: granule (i + rot) mod 4
+        uint32_t sum[4], s = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) q[i] = *reinterpret_cast<const u32x4 *>(&h[base + 4 * ((i + rot) & 3)]);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {  // granule g was read in step (g - rot) mod 4
-            const int i = (g - rot) & 3;
-            u32x4 v = q[0];
-#pragma unroll
-            for (int k = 1; k < 4; ++k) v = __builtin_unpredictable(i == k) ? q[k] : v;
-            nat[g] = v;
+        for (int i = 0; i < 4; ++i) {
+            sum[i] = q[i].x + q[i].y + q[i].z + q[i].w;
+            s += sum[i];
         }
-        uint32_t s = 0;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) s += nat[g].x + nat[g].y + nat[g].z + nat[g].w;
         uint32_t total;
-        uint32_t e = wg_excl_scan(sm, s, &total);
+        const uint32_t below = wg_excl_scan(sm, s, &total), e0 = total - below;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
+        for (int i = 0; i < 4; ++i) {
+            uint32_t left = e0;  // elements of this granule's bins and all above
+#pragma unroll
+            for (int j = 0; j < 4; ++j) left -= ((j + rot) & 3) < ((i + rot) & 3) ? sum[j] : 0u;
             u32x4 o;
-            o.x = total - e; e += nat[g].x;
-            o.y = total - e; e += nat[g].y;
-            o.z = total - e; e += nat[g].z;
-            o.w = total - e; e += nat[g].w;
-            nat[g] = o;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {  // step i writes granule (i + rot) mod 4
-            const int g = (i + rot) & 3;
-            u32x4 v = nat[0];
-#pragma unroll
-            for (int k = 1; k < 4; ++k) v = __builtin_unpredictable(g == k) ? nat[k] : v;
-            *reinterpret_cast<u32x4 *>(&h[base + 4 * g]) = v;
+            o.x = left; left -= q[i].x;
+            o.y = left; left -= q[i].y;
+            o.z = left; left -= q[i].z;
+            o.w = left;
+            *reinterpret_cast<u32x4 *>(&h[base + 4 * ((i + rot) & 3)]) = o;
         }
     } else {
         uint32_t loc[per];
@@ -390,11 +412,12 @@ __device__ float wg_select(SelSmem &sm, const float *src, int64_t n, float lo, f
 }
 
 // One group of target bins of the row (a pass of the gather over the row, or
-// one bin larger than LDS narrowed on its own): `each` visits the row's values.
+// one bin larger than LDS narrowed on its own): `each` visits the row's values
+// and bins.
 template <class Each>
 __device__ __forceinline__ void select_group(SelSmem &sm, int g, int ngrp, int nfb, const float *__restrict__ x,
                                              int64_t n_item, const Ranks &ranks, int32_t S, float *T,
-                                             float lo0, float scale1, Each &&each) {
+                                             bool few, Each &&each) {
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     const bool deep = (sm.grp[g] & DEEP) != 0;
     const int f0 = sm.grp[g] & ~DEEP;
@@ -405,10 +428,8 @@ __device__ __forceinline__ void select_group(SelSmem &sm, int g, int ngrp, int n
         const int j1 = (f0 + 1 < nfb) ? sm.fb[f0 + 1] : S;
         const int b = sm.tb[j0];
         float bmn = INFINITY, bmx = -INFINITY;
-        each([&](const auto &v) {
+        each([&](const auto &v, const auto &bv) {
             constexpr int N = sizeof(v) / sizeof(float);
-            int bv[N];
-            fine_bins<N>(sm.fseg, v, lo0, scale1, bv);
 #pragma unroll
             for (int q = 0; q < N; ++q)
                 if (bv[q] == b) { bmn = fminf(bmn, v[q]); bmx = fmaxf(bmx, v[q]); }
@@ -421,52 +442,76 @@ __device__ __forceinline__ void select_group(SelSmem &sm, int g, int ngrp, int n
         }
         return;
     }
-    // member bins: bitmap bits, then segment starts (bins descending in f)
-    for (int f = f0 + tid; f < f1; f += NT) {
-        const int b = sm.tb[sm.fb[f]];
-        atomicOr(&sm.tbits[b >> 5], 1u << (b & 31));
-    }
-    if (ngrp > 1) {
-        // several passes: offsets restart at each group's first bin
-        __syncthreads();
-        const uint32_t base = sm.fcur[f0];
-        __syncthreads();
-        for (int f = f0 + tid; f < f1; f += NT) sm.fcur[f] -= base;
-    }
     for (int i = tid; i < GCAP / 32; i += NT) sm.sbits[i] = 0;
     if (tid == 0) { sm.ncoop = 0; sm.nmid = 0; }
-    __syncthreads();
-    {
-        // member bins below each bitmap word (ascending bins)
-        const uint32_t cnt = tid < NB / 32 ? (uint32_t)__popc(sm.tbits[tid]) : 0u;
-        uint32_t tot;
-        const uint32_t pre = wg_excl_scan(sm, cnt, &tot);
-        if (tid < NB / 32) sm.tpre[tid] = (uint16_t)pre;
-    }
-    __syncthreads();
-    // gather: the member bin of rank m in ascending bin order is f1 - 1 - m
-    // A batch's bins, bitmap words and prefixes are read together, and its
-    // members' slots are all claimed before the first is written.
-    each([&](const auto &v) {
-        constexpr int N = sizeof(v) / sizeof(float);
-        int b[N];
-        fine_bins<N>(sm.fseg, v, lo0, scale1, b);
-        uint32_t word[N], pre[N];
+    if (few) {
+        // one pass of at most half the gather buffer: the other half says, per
+        // bin, which distinct bin it is (0: none), one LDS read per value
+        uint16_t *of = reinterpret_cast<uint16_t *>(sm.u.gbuf + GCAP / 2);
+        static_assert(NB * sizeof(uint16_t) == GCAP / 2 * sizeof(float), "half of the buffer");
+        for (int i = tid; i < NB / 8; i += NT) reinterpret_cast<u32x4 *>(of)[i] = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads();
+        for (int f = f0 + tid; f < f1; f += NT) of[sm.tb[sm.fb[f]]] = (uint16_t)(f + 1);
+        __syncthreads();
+        each([&](const auto &v, const auto &b) {
+            constexpr int N = sizeof(v) / sizeof(float);
+            int f[N];
+            uint32_t slot[N];
 #pragma unroll
-        for (int q = 0; q < N; ++q) { word[q] = sm.tbits[b[q] >> 5]; pre[q] = sm.tpre[b[q] >> 5]; }
-        uint32_t slot[N];
-        bool mem[N];
+            for (int q = 0; q < N; ++q) f[q] = of[b[q]];
 #pragma unroll
-        for (int q = 0; q < N; ++q) {
-            const uint32_t bit = 1u << (b[q] & 31);
-            mem[q] = (word[q] & bit) != 0;
-            slot[q] = 0;
-            if (mem[q]) slot[q] = atomicAdd(&sm.fcur[f1 - 1 - ((int)pre[q] + __popc(word[q] & (bit - 1u)))], 1u);
+            for (int q = 0; q < N; ++q) {
+                slot[q] = 0;
+                if (f[q]) slot[q] = atomicAdd(&sm.fcur[f[q] - 1], 1u);
+            }
+#pragma unroll
+            for (int q = 0; q < N; ++q)
+                if (f[q]) sm.u.gbuf[slot[q]] = v[q];
+        });
+    } else {
+        // member bins: bitmap bits, then segment starts (bins descending in f)
+        for (int f = f0 + tid; f < f1; f += NT) {
+            const int b = sm.tb[sm.fb[f]];
+            atomicOr(&sm.tbits[b >> 5], 1u << (b & 31));
         }
+        if (ngrp > 1) {
+            // several passes: offsets restart at each group's first bin
+            __syncthreads();
+            const uint32_t base = sm.fcur[f0];
+            __syncthreads();
+            for (int f = f0 + tid; f < f1; f += NT) sm.fcur[f] -= base;
+        }
+        __syncthreads();
+        {
+            // member bins below each bitmap word (ascending bins)
+            const uint32_t cnt = tid < NB / 32 ? (uint32_t)__popc(sm.tbits[tid]) : 0u;
+            uint32_t tot;
+            const uint32_t pre = wg_excl_scan(sm, cnt, &tot);
+            if (tid < NB / 32) sm.tpre[tid] = (uint16_t)pre;
+        }
+        __syncthreads();
+        // gather: the member bin of rank m in ascending bin order is f1 - 1 - m
+        // A batch's bitmap words and prefixes are read together, and its
+        // members' slots are all claimed before the first is written.
+        each([&](const auto &v, const auto &b) {
+            constexpr int N = sizeof(v) / sizeof(float);
+            uint32_t word[N], pre[N];
 #pragma unroll
-        for (int q = 0; q < N; ++q)
-            if (mem[q]) sm.u.gbuf[slot[q]] = v[q];
-    });
+            for (int q = 0; q < N; ++q) { word[q] = sm.tbits[b[q] >> 5]; pre[q] = sm.tpre[b[q] >> 5]; }
+            uint32_t slot[N];
+            bool mem[N];
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const uint32_t bit = 1u << (b[q] & 31);
+                mem[q] = (word[q] & bit) != 0;
+                slot[q] = 0;
+                if (mem[q]) slot[q] = atomicAdd(&sm.fcur[f1 - 1 - ((int)pre[q] + __popc(word[q] & (bit - 1u)))], 1u);
+            }
+#pragma unroll
+            for (int q = 0; q < N; ++q)
+                if (mem[q]) sm.u.gbuf[slot[q]] = v[q];
+        });
+    }
     __syncthreads();
     // Bins of up to EMAX elements are ranked element-parallel: each gathered
     // element finds its bin from the segment starts (a bitmap over the gather
@@ -561,7 +606,7 @@ __device__ __forceinline__ void select_group(SelSmem &sm, int g, int ngrp, int n
         }
     }
     // release the member bins
-    for (int f = f0 + tid; f < f1; f += NT) {
+    for (int f = f0 + tid; !few && f < f1; f += NT) {
         const int b = sm.tb[sm.fb[f]];
         sm.tbits[b >> 5] = 0;
     }
@@ -639,13 +684,21 @@ __global__ void __launch_bounds__(NT) k_select_rows(const float *__restrict__ sc
     for (int i = tid; i < NB; i += NT) sm.u.incl[i] = 0;
     for (int i = tid; i < NB / 32; i += NT) sm.tbits[i] = 0;
     __syncthreads();
-    each([&](const auto &v) {
-        constexpr int N = sizeof(v) / sizeof(float);
-        int b[N];
-        fine_bins<N>(sm.fseg, v, lo0, scale1, b);
+    auto bin = [&](const auto &v, auto &b) { fine_bins<sizeof(v) / sizeof(float)>(sm.fseg, v, lo0, scale1, b); };
+    auto count = [&](const auto &v, const auto &b) {
 #pragma unroll
-        for (int q = 0; q < N; ++q) atomicAdd(&sm.u.incl[b[q]], 1u);
-    });
+        for (int q = 0; q < (int)(sizeof(v) / sizeof(float)); ++q) atomicAdd(&sm.u.incl[b[q]], 1u);
+    };
+    // the row from memory, values and bins
+    auto from_memory = [&](auto &&f) {
+        row_for_each(x, n_item, [&](const auto &v) {
+            int b[sizeof(v) / sizeof(float)];
+            bin(v, b);
+            f(v, b);
+        });
+    };
+    if constexpr (C4 > 0) rr.for_each_bin(bin, count);
+    else from_memory(count);
     __syncthreads();
     wg_reverse_incl<NB>(sm, sm.u.incl);
 
@@ -725,6 +778,7 @@ __global__ void __launch_bounds__(NT) k_select_rows(const float *__restrict__ sc
                 sm.grp[0] = 0;
                 sm.grp[1] = (uint16_t)nfb;
                 sm.ngrp = 1;
+                sm.few = total <= GCAP / 2;
             } else {
                 int ngrp = 0;
                 uint32_t fill = GCAP;
@@ -740,6 +794,7 @@ __global__ void __launch_bounds__(NT) k_select_rows(const float *__restrict__ sc
                 }
                 sm.grp[ngrp] = (uint16_t)nfb;
                 sm.ngrp = ngrp;
+                sm.few = 0;
             }
         }
     }
@@ -749,10 +804,13 @@ __global__ void __launch_bounds__(NT) k_select_rows(const float *__restrict__ sc
     // the first group reads the row from wherever the kernel holds it; any
     // later one (rows whose target bins exceed LDS) reads it from memory, so
     // the registers of a register-held row are free after the first gather
-    if (ngrp > 0) select_group(sm, 0, ngrp, nfb, x, n_item, ranks, S, T, lo0, scale1, each);
-    for (int g = 1; g < ngrp; ++g)
-        select_group(sm, g, ngrp, nfb, x, n_item, ranks, S, T, lo0, scale1,
-                     [&](auto &&f) { row_for_each(x, n_item, f); });
+    const bool few = sm.few != 0;
+    auto each_bin = [&](auto &&f) {
+        if constexpr (C4 > 0) rr.for_each_kept(f);
+        else from_memory(f);
+    };
+    if (ngrp > 0) select_group(sm, 0, ngrp, nfb, x, n_item, ranks, S, T, few, each_bin);
+    for (int g = 1; g < ngrp; ++g) select_group(sm, g, ngrp, nfb, x, n_item, ranks, S, T, false, from_memory);
 }
 
 }  // namespace

@@ -371,3 +371,26 @@ def test_row_sort_thread_counts(orc, I):
         idx.set_data(users, items)
         got = idx.sorted_scores()
     assert np.array_equal(got, orc.sorted_score_rows(orc.normalize_users(users), items))
+
+
+@pytest.mark.parametrize("I,S", [(4000, 100), (9000, 4096), (20_000, 4096), (20_001, 700), (52_000, 4096)])
+@pytest.mark.parametrize("ties", [0, 1])
+def test_select_gather_sizes(orc, I, S, ties):
+    """Target bins that fill less and more than half of the gather buffer, rows
+    in registers and not, rows whose values crowd into few bins."""
+    _case(f"select I={I} S={S} ties={ties}")
+    import rkr
+    rng = np.random.default_rng(I + S)
+    users = rng.standard_normal((9, 7), dtype=np.float32)
+    items = rng.standard_normal((I, 7), dtype=np.float32)
+    if ties:
+        items[I // 3:] = items[rng.integers(0, I // 3, I - I // 3)]
+        items[:50] *= 1e4
+    with rkr.Index(0) as idx:
+        idx.set_option(8, 0)  # RKR_OPT_DENSE_TOP: the sampled table alone
+        idx.set_data(users, items)
+        ranks = np.unique(np.concatenate([np.arange(S // 2), rng.choice(I, S, replace=False)]))[:S].astype(np.int32)
+        idx.build_table(ranks)
+        got = idx.get_table()
+    want = orc.sorted_score_rows(orc.normalize_users(users), items)[:, ranks]
+    assert np.array_equal(got, want)
