@@ -1097,12 +1097,13 @@ int rkr_query_rank_distribution(rkr_ctx *c, const int32_t *item_ids, int32_t n_s
         RKR_HIP(c, hipEventRecord(c->ev[3], c->stream));
         RKR_HIP(c, launch_scores_store(c->stream, c->users + u * c->ld, m, c->ld, smat.as<float>(), ns, c->ld,
                                        c->dim, qbuf, ns, true));
-        RKR_HIP(c, launch_rank_hist(c->stream, rows, I, m, I, qbuf, ns, (int32_t)ns, h));
+        RKR_HIP(c, launch_rank_hist(c->stream, rows, I, m, I, qbuf, ns, (int32_t)ns, h,
+                                    reinterpret_cast<uint16_t *>(qbuf + m * ns + (m * ns & 1))));
         RKR_HIP(c, hipEventRecord(c->ev[4], c->stream));
         RKR_HIP(c, hipEventSynchronize(c->ev[4]));
         ms += ev_ms(c->ev, 0, 2) + ev_ms(c->ev, 3, 4);
         return (int)RKR_OK;
-    }, nullptr, nullptr, ns);
+    }, nullptr, nullptr, ns + rank_row(ns) / 2 + 1);  // a batch's scores (rounded to 8 bytes) and 16-bit ranks
     if (rc) return rc;
     // The counts leave through the pinned staging buffers in chunks of whole
     // rows; host threads turn each chunk's counts per rank into users with

@@ -441,8 +441,9 @@ hipError_t launch_sort_rows(hipStream_t s, const float *src, int64_t ld_src, int
 // ---- QS sample-rank training (k_train.hip) ----------------------------------
 // hist[s * (n_item + 1) + #{i : sorted[u * ld + i] > q[u * ldq + s]}] += 1 for
 // u < nb, s < ns (sorted rows descending).
+inline int64_t rank_row(int64_t ns) { return (ns + 3) / 4 * 4; }
 hipError_t launch_rank_hist(hipStream_t s, const float *sorted, int64_t ld, int64_t nb, int64_t n_item, const float *q,
-                            int64_t ldq, int32_t ns, int32_t *hist);
+                            int64_t ldq, int32_t ns, int32_t *hist, uint16_t *ranks);
 // Transit-cost triangle T[lb * (lb - 1) / 2 + ub], 0 <= ub < lb < R, from the
 // query positions pos[j], End(j) and the prefix sums kept at the breakpoints:
 // C[col[j'] * R + j] = sum over queries q < pos[j'] of accu[q][rank_j].
