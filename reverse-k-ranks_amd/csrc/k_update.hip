@@ -155,7 +155,8 @@ __global__ void __launch_bounds__(256) k_subtract_rows(const float *__restrict__
 
 // Bounds with side-array offsets (exact output).  lbs/ubs as values:
 //   off = #{ins > q} - #{del > q};  lbs' = lbs + off;  ubs' = ubs + off.
-__device__ __forceinline__ void bounds_values(const float *row, int32_t S, float q, float eps,
+template <class Bucket>  // bucket(x) = #{row > x}
+__device__ __forceinline__ void bounds_values(Bucket &&bucket, int32_t S, float q, float eps,
                                               const int32_t *__restrict__ ranks, int64_t n_item_base,
                                               const float *ins_row, int32_t n_ins, const float *del_row,
                                               int32_t n_del, int32_t &lb, int32_t &ub) {
@@ -164,7 +165,7 @@ __device__ __forceinline__ void bounds_values(const float *row, int32_t S, float
         qlo = __double2float_rd((double)q - (double)eps);
         qhi = __double2float_ru((double)q + (double)eps);
     }
-    const int32_t blo = count_gt(row, S, qlo), bhi = eps > 0.0f ? count_gt(row, S, qhi) : blo;
+    const int32_t blo = bucket(qlo), bhi = eps > 0.0f ? bucket(qhi) : blo;
     int32_t off = 0;
     if (n_ins) off += count_gt(ins_row, n_ins, q);
     if (n_del) off -= count_gt(del_row, n_del, q);
@@ -199,10 +200,53 @@ __global__ void __launch_bounds__(256) k_bounds_upd(const float *__restrict__ qi
     const int64_t b = blockIdx.y;
     if (u >= n_user) return;
     int32_t lb, ub;
-    bounds_values(table + u * (int64_t)S, S, qip[b * n_user + u], eps, ranks, n_item_base, ins + u * (int64_t)ld_ins,
+    const float *row = table + u * (int64_t)S;
+    bounds_values([&](float x) { return count_gt(row, S, x); }, S, qip[b * n_user + u], eps, ranks, n_item_base, ins + u * (int64_t)ld_ins,
                   n_ins, del + u * (int64_t)ld_del, n_del, lb, ub);
     lbs[b * n_user + u] = lb;
     ubs[b * n_user + u] = ub;
+}
+
+// A few queries: 64 users per workgroup, their guard rows in LDS, a query per
+// wavefront at a time.  The guard row leaves the columns between two fine ones,
+// a line or two of the table row, where staging the row reads all of its 16 KB
+// (4096 columns) and leaves two users to a workgroup.  16 queries x 102k users,
+// 500 items pending: 590 us, now 205.
+__global__ void __launch_bounds__(256) k_bounds_upd_guards(const float *__restrict__ qip, const float *__restrict__ table,
+                                                           const float *__restrict__ gvals, FineCols fc, int64_t n_user,
+                                                           int32_t S, int32_t nq, const int32_t *__restrict__ ranks,
+                                                           int64_t n_item_base, float eps, const float *__restrict__ ins,
+                                                           int32_t n_ins, int32_t ld_ins, const float *__restrict__ del,
+                                                           int32_t n_del, int32_t ld_del, int32_t *__restrict__ lbs,
+                                                           int32_t *__restrict__ ubs) {
+    constexpr int GP = kGuardRow + 1;  // an odd stride: the lanes' searches fall in different banks
+    __shared__ float g[64 * GP];
+    __shared__ int32_t col[kGuardRow];
+    const int64_t u0 = (int64_t)blockIdx.x * 64;
+    for (int i = threadIdx.x; i < 64 * kGuardRow; i += 256) {
+        const int64_t u = min(u0 + i / kGuardRow, n_user - 1);
+        g[(i / kGuardRow) * GP + i % kGuardRow] = gvals[u * kGuardRow + i % kGuardRow];
+    }
+    if (threadIdx.x < kGuardRow) col[threadIdx.x] = threadIdx.x < kMaxFine ? fc.col[threadIdx.x] : 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int64_t u = u0 + lane;
+    if (u >= n_user) return;
+    const float *grow = g + lane * GP, *row = table + u * (int64_t)S;
+    auto bucket = [&](float x) {
+        int f = 0;  // -inf past the fine columns
+#pragma unroll
+        for (int st = kGuardRow / 2; st > 0; st >>= 1) f += grow[f + st - 1] > x ? st : 0;
+        const int32_t lo = f > 0 ? col[f - 1] + 1 : 0, hi = f < fc.n ? col[f] : S;
+        return lo + count_gt(row + lo, hi - lo, x);
+    };
+    for (int32_t b = threadIdx.x >> 6; b < nq; b += 4) {
+        int32_t lb, ub;
+        bounds_values(bucket, S, qip[(int64_t)b * n_user + u], eps, ranks, n_item_base, ins + u * (int64_t)ld_ins, n_ins,
+                      del + u * (int64_t)ld_del, n_del, lb, ub);
+        lbs[(int64_t)b * n_user + u] = lb;
+        ubs[(int64_t)b * n_user + u] = ub;
+    }
 }
 
 // Batched form: ut table rows staged in LDS serve all nq queries of those
@@ -237,7 +281,7 @@ __global__ void __launch_bounds__(256) k_bounds_upd_lds(const float *__restrict_
     const float *del_row = stage_side ? rows_del + (int64_t)ul * (n_del + 1) : del + u * (int64_t)ld_del;
     for (int32_t b = threadIdx.x / ut; b < nq; b += lanes_q) {
         int32_t lb, ub;
-        bounds_values(row, S, qip[(int64_t)b * n_user + u], eps, ranks, n_item_base, ins_row, n_ins, del_row, n_del,
+        bounds_values([&](float x) { return count_gt(row, S, x); }, S, qip[(int64_t)b * n_user + u], eps, ranks, n_item_base, ins_row, n_ins, del_row, n_del,
                       lb, ub);
         lbs[(int64_t)b * n_user + u] = lb;
         ubs[(int64_t)b * n_user + u] = ub;
@@ -494,11 +538,23 @@ hipError_t launch_subtract_rows(hipStream_t s, const float *a, int64_t lda, int3
     return hipGetLastError();
 }
 
-hipError_t launch_bounds_upd(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
+// Queries up to which the guard rows' path is taken.  100k users, 20k items, 500
+// pending: 16 queries 0.33 ms against 0.65 with rows staged, 32 0.63 against
+// 0.55; 60k users, 8k items, 40 pending: 32 0.18 against 0.32, 64 0.35 against
+// 0.34 (the staged rows serve any number of queries).
+constexpr int kGuardBounds = 24;
+
+hipError_t launch_bounds_upd(hipStream_t s, const float *qip, const float *table, const float *gvals,
+                             const FineCols &fc, int64_t n_user, int32_t S,
                              const int32_t *ranks, int64_t n_item_base, float eps, const float *ins, int32_t n_ins,
                              int32_t ld_ins, const float *del, int32_t n_del, int32_t ld_del, int32_t nq,
                              int32_t *lbs, int32_t *ubs) {
     if (n_user <= 0 || nq <= 0) return hipSuccess;
+    if (gvals && fc.n > 0 && nq <= kGuardBounds) {
+        hipLaunchKernelGGL(k_bounds_upd_guards, dim3((unsigned)((n_user + 63) / 64)), dim3(256), 0, s, qip, table, gvals, fc,
+                           n_user, S, nq, ranks, n_item_base, eps, ins, n_ins, ld_ins, del, n_del, ld_del, lbs, ubs);
+        return hipGetLastError();
+    }
     if (nq >= 4) {
         // users per workgroup: with their side rows when they fit 40 KB
         const int64_t per_user = (int64_t)(S + 1) + (n_ins ? n_ins + 1 : 0) + (n_del ? n_del + 1 : 0);

@@ -1721,7 +1721,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 RKR_HIP(c, launch_list_exact(sl.stream, LL, dv.users, q_in, ld, d, T, true, bk_c));
                 RKR_HIP(c, event(3));
             } else if (upd) {
-                RKR_HIP(c, launch_bounds_upd(sl.stream, qip, T, U, S, R, dv.n_item_base, eps, dv.side_ins,
+                RKR_HIP(c, launch_bounds_upd(sl.stream, qip, T, dv.gvals, dv.fine, U, S, R, dv.n_item_base, eps, dv.side_ins,
                                              dv.n_ins, dv.ld_ins, dv.side_del, dv.n_del, dv.ld_del, nq, lbv, ubv));
                 RKR_HIP(c, event(3));
                 RKR_HIP(c, launch_kth_values(sl.stream, lbv, ubv, U, nq, cu, ghist, qi));

@@ -753,7 +753,8 @@ hipError_t launch_merge_rows(hipStream_t s, const float *a, int64_t lda, int32_t
                              int32_t nb, float *out, int64_t ldo, int64_t n_rows);
 hipError_t launch_subtract_rows(hipStream_t s, const float *a, int64_t lda, int32_t na, const float *b, int64_t ldb,
                                 int32_t nb, float *out, int64_t ldo, int64_t n_rows);
-hipError_t launch_bounds_upd(hipStream_t s, const float *qip, const float *table, int64_t n_user, int32_t S,
+hipError_t launch_bounds_upd(hipStream_t s, const float *qip, const float *table, const float *gvals,
+                             const FineCols &fc, int64_t n_user, int32_t S,
                              const int32_t *ranks, int64_t n_item_base, float eps, const float *ins, int32_t n_ins,
                              int32_t ld_ins, const float *del, int32_t n_del, int32_t ld_del, int32_t nq,
                              int32_t *lbs, int32_t *ubs);

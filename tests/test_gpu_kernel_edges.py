@@ -394,3 +394,26 @@ def test_select_gather_sizes(orc, I, S, ties):
         got = idx.get_table()
     want = orc.sorted_score_rows(orc.normalize_users(users), items)[:, ranks]
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("U,nq,dense", [(65, 3, 2), (4100, 24, 2), (4100, 25, 0), (1, 1, 0)])
+def test_update_bounds_by_guards(orc, gpu_index_factory, U, nq, dense):
+    """Bounds with updates pending on either side of the guard rows' limit of
+    24 queries, with inserts and deletes, users at the edge of a block of 64."""
+    _case(f"update bounds U={U} nq={nq} dense={dense}")
+    from test_gpu_update import Mirror
+    rng = np.random.default_rng(U + nq)
+    d, I = 14, 900
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 200, dense_top=dense)
+    m = Mirror(orc, users, items)
+    new = rng.standard_normal((30, d), dtype=np.float32) * np.float32(1.2)
+    idx.insert_items(new)
+    m.insert_items(new)
+    idx.delete_items(np.array([0, 7, 9, I + 2], np.int64))
+    m.delete_items([0, 7, 9, I + 2])
+    queries = np.concatenate([items[:nq // 2], rng.standard_normal((nq - nq // 2, d), dtype=np.float32)])
+    for form in ("plain", "screened"):
+        m.check(idx, queries, min(U, 12), form)
+    idx.close()
