@@ -748,7 +748,7 @@ hipError_t launch_gather_guards(hipStream_t s, const float *T, int64_t S, const 
 // on `device` (current) once per device.
 hipError_t noalloc_init(int device);
 
-hipError_t launch_sort_rows_desc(hipStream_t s, float *x, int64_t n_rows, int32_t n, int64_t ld);
+hipError_t launch_sort_rows_desc(hipStream_t s, float *x, int64_t n_rows, int32_t n, int64_t ld, float *out, int64_t ldo);
 hipError_t launch_merge_rows(hipStream_t s, const float *a, int64_t lda, int32_t na, const float *b, int64_t ldb,
                              int32_t nb, float *out, int64_t ldo, int64_t n_rows);
 hipError_t launch_subtract_rows(hipStream_t s, const float *a, int64_t lda, int32_t na, const float *b, int64_t ldb,

@@ -227,10 +227,12 @@ int update_side(Ctx *c, bool ins_side, const float *X, int64_t n, int sign) {
         float *block = reinterpret_cast<float *>(c->upd_scratch.p);
         RKR_HIP(c, launch_scores_store(c->stream, c->users, U, c->ld, X + x0 * c->ld, m, c->ld, c->dim, block,
                                        m, true));
-        RKR_HIP(c, launch_sort_rows_desc(c->stream, block, U, (int32_t)m, m));
-        if (sign > 0)
+        // the first scores are sorted to their place, later ones merged in
+        const bool place = sign > 0 && *ns == 0 && m <= 1024;
+        RKR_HIP(c, launch_sort_rows_desc(c->stream, block, U, (int32_t)m, m, place ? target : block, place ? ld_t : m));
+        if (!place && sign > 0)
             RKR_HIP(c, launch_merge_rows(c->stream, *side, *ld, *ns, block, m, (int32_t)m, target, ld_t, U));
-        else
+        else if (sign < 0)
             RKR_HIP(c, launch_subtract_rows(c->stream, *side, *ld, *ns, block, m, (int32_t)m, target, ld_t, U));
         RKR_HIP(c, hipStreamSynchronize(c->stream));
         if (*side != published) dev_free(c, *side, 0);  // an intermediate of this call
@@ -574,7 +576,7 @@ int rkr_insert_users(rkr_ctx *c, const float *users, int64_t n) {
         if (!ns) continue;
         float *rows = arr + U0 * lds;
         RKR_HIP(c, launch_scores_store(c->stream, c->users + U0 * ld, n, ld, X, ns, ld, c->dim, rows, lds, true));
-        RKR_HIP(c, launch_sort_rows_desc(c->stream, rows, n, ns, lds));
+        RKR_HIP(c, launch_sort_rows_desc(c->stream, rows, n, ns, lds, rows, lds));
     }
     RKR_HIP(c, hipStreamSynchronize(c->stream));
     c->max_abs_user_raw = mu_raw;

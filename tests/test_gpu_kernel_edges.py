@@ -417,3 +417,34 @@ def test_update_bounds_by_guards(orc, gpu_index_factory, U, nq, dense):
     for form in ("plain", "screened"):
         m.check(idx, queries, min(U, 12), form)
     idx.close()
+
+
+@pytest.mark.parametrize("n_new", [1, 2, 63, 64, 65, 128, 129, 256, 257, 511, 512, 513, 1000, 1024, 1025])
+def test_inserted_score_rows(orc, gpu_index_factory, n_new):
+    """Inserted items' scores sorted in one wavefront at every length, placed,
+    merged with those there, and taken out again."""
+    _case(f"insert {n_new} items")
+    from test_gpu_update import Mirror
+    rng = np.random.default_rng(n_new)
+    d = 9
+    users = rng.standard_normal((300, d), dtype=np.float32)
+    users[5] = 0.0
+    items = rng.standard_normal((400, d), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 30)
+    m = Mirror(orc, users, items)
+    queries = items[:9]
+    for n in (n_new, 77):
+        new = rng.standard_normal((n, d), dtype=np.float32)
+        new[n // 2:] = new[: n - n // 2]  # equal scores
+        idx.insert_items(new)
+        m.insert_items(new)
+        for form in ("plain", "screened"):
+            m.check(idx, queries, 40, form)
+    gone = (400 + np.arange(0, n_new, 2)).astype(np.int64)
+    idx.delete_items(gone)
+    m.delete_items(gone)
+    more = rng.standard_normal((3, d), dtype=np.float32)
+    idx.insert_users(more)
+    m.insert_users(more)
+    m.check(idx, queries, 40)
+    idx.close()
