@@ -216,9 +216,15 @@ __global__ void __launch_bounds__(NT, 3) k_scores_store(const float *__restrict_
 // a unit: with table columns at every top rank there are often fewer than 128
 // rows in all, and groups of 8 tiles then used 98 of 256 CUs (92 rows against
 // 100k items, 150 dims: 300 us; one tile a unit: 94 us).
+//
+// OCC workgroups per CU: 3 hide the start of a unit, its gather of rows, when
+// units are single tiles (300 rows x 100k items x 128 dims: 0.18 ms, with 2
+// 0.245); over many rows 2 are faster, the three run in step and the card
+// clocks lower (125k rows x 21k items x 157 dims: 13.2 ms, with 3 15.7).
 constexpr int kGroup = 8;  // a thread counts at most 8 per tile and row: 8 * kGroup < 256
 
-__global__ void __launch_bounds__(NT, 3) k_refine_count(const float *__restrict__ users, const float *__restrict__ items,
+template <int OCC>
+__global__ void __launch_bounds__(NT, OCC) k_refine_count(const float *__restrict__ users, const float *__restrict__ items,
                                                      int64_t n_item, int32_t ld, int32_t K,
                                                      const int32_t *__restrict__ rows_user,
                                                      const float *__restrict__ rows_thr,
@@ -378,16 +384,21 @@ hipError_t launch_scores_store(hipStream_t s, const float *A, int64_t M, int32_t
 
 hipError_t launch_refine_count(hipStream_t s, const float *users, const float *items, int64_t n_item, int32_t ld,
                                int32_t K, const int32_t *rows_user, const float *rows_thr, const int32_t *n_rows_dev,
-                               int64_t max_rows, int32_t *cnt, uint64_t *t) {
+                               int64_t max_rows, int32_t *cnt, bool many, uint64_t *t) {
     if (max_rows <= 0 || n_item <= 0) return hipSuccess;
     int dev = 0, n_cu = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
     const int64_t n_it = (n_item + BN - 1) / BN;
     const int64_t max_units = ((max_rows + BM - 1) / BM) * n_it;
-    const int64_t grid = std::min<int64_t>(max_units, (int64_t)n_cu * 3);  // three workgroups fit a CU
-    hipLaunchKernelGGL(k_refine_count, dim3((unsigned)grid), dim3(NT), 0, s, users, items, n_item, ld, K, rows_user,
-                       rows_thr, n_rows_dev, max_rows, cnt, t);
+    many = many && max_units >= (int64_t)kGroup * n_cu * 2;
+    const dim3 grid((unsigned)std::min<int64_t>(max_units, (int64_t)n_cu * (many ? 2 : 3)));
+    if (many)
+        hipLaunchKernelGGL(k_refine_count<2>, grid, dim3(NT), 0, s, users, items, n_item, ld, K, rows_user, rows_thr,
+                           n_rows_dev, max_rows, cnt, t);
+    else
+        hipLaunchKernelGGL(k_refine_count<3>, grid, dim3(NT), 0, s, users, items, n_item, ld, K, rows_user, rows_thr,
+                           n_rows_dev, max_rows, cnt, t);
     return hipGetLastError();
 }
 

@@ -1781,6 +1781,9 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         else
             RKR_HIP(c, launch_compact(sl.stream, bk, qip, U, S, R, I, nq, mode, cu, qi, cand_user, cand_rank,
                                       refine_total, refine_user, refine_query, refine_thr, cnt));
+        // without a list the rows' bound is the candidates' count; a list over a
+        // table with every top rank leaves few rows, whatever its capacity
+        const bool many = !list || !use_q;
         // refinement + top-k; re-run when the recheck list overflowed
         for (int attempt = 0; attempt < 3; ++attempt) {
             int64_t rec_cap = 0;
@@ -1816,7 +1819,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                                           at(kTimeRecheck)));
             } else {
                 RKR_HIP(c, launch_refine_count(sl.stream, dv.users, dv.items, I, ld, d, refine_user, refine_thr,
-                                               refine_total, (int64_t)rcap, cnt, at(kTimeRefine)));
+                                               refine_total, (int64_t)rcap, cnt, many, at(kTimeRefine)));
                 RKR_HIP(c, event(8));
             }
             RKR_HIP(c, event(5));

@@ -359,9 +359,10 @@ hipError_t launch_gemv_panels(hipStream_t s, const float *usersT, int64_t n_user
                               uint64_t *t = nullptr);
 // Refinement count: cnt[r] = #{item p : score(user(r), p) > thr(r)} for every
 // refine row r < *n_rows_dev (device-side count, persistent grid).
+// many: max_rows is near the number of rows, or that is unknown and not small
 hipError_t launch_refine_count(hipStream_t s, const float *users, const float *items, int64_t n_item,
                                int32_t ld, int32_t K, const int32_t *rows_user, const float *rows_thr,
-                               const int32_t *n_rows_dev, int64_t max_rows, int32_t *cnt, uint64_t *t = nullptr);
+                               const int32_t *n_rows_dev, int64_t max_rows, int32_t *cnt, bool many, uint64_t *t = nullptr);
 // Transpose users into 64-user panels.
 hipError_t launch_make_panels(hipStream_t s, const float *users, int64_t n_user, int32_t ld, float *usersT);
 
