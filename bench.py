@@ -9,8 +9,8 @@ the device, 1,000 queries drawn from the items, k=50, exact ranks.  One step
 HBM (only the query vectors and the answers cross PCIe).
 
 Prints one JSON line: queries/s (value), single-query p50/p99 latency, table
-build time, the roofline of the dominant kernel (HIP-event time of that
-kernel inside the timed region), the same queries through the other forms
+build time, the roofline of the dominant kernel (device time of its
+stage inside the timed region), the same queries through the other forms
 (sampled table only, plain FP32) so every ratio is like for like, and the
 CPU baseline (the oracle's restatement of the reference's OpenMP US query
 path on every core of this process's CPU share, timed on a bounded sample of
@@ -83,7 +83,7 @@ def parse():
     ap.add_argument("--no-dedup", action="store_true", help="compute byte-equal queries of a call separately")
     ap.add_argument("--dense-top", type=int, default=2, choices=[0, 1, 2],
                     help="query table: 0 none (sampled table only), 1 dense top ranks, 2 every rank to the cap")
-    ap.add_argument("--coarse", type=int, default=1, choices=[0, 1], help="0: no coarse bounds (full bound search)")
+    ap.add_argument("--coarse", type=int, default=1, choices=[0, 1], help="0: no threshold lists (full bound search)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="run a plain 1 GiB device copy (for scaling rocprofv3 byte counters) and exit")
     ap.add_argument("--update-mode", default="snapshot", choices=["snapshot", "barrier"],
@@ -488,10 +488,8 @@ def cpu_baseline(wl, table, ranks, users_norm, gpu_users, k, n_max, seconds):
 # plain 1 GiB device copy gives, bench.py --copy-calibration).  Keyed by
 # (workload, form); other configurations report null.
 PROFILED_TRAFFIC = {
-    ("plain_gpu", "screened"): {"kernel": "k_ip_coarse", "bytes": 1.486e8, "fetch_kib": 23608.4,
-                                "write_kib": 97847.8, "profile": "profiles/k_ip_coarse_100k_x_20k_d150_k50.md"},
-    ("precision", "screened"): {"kernel": "k_ip_coarse", "bytes": 1.484e9, "fetch_kib": 235798.1,
-                                "write_kib": 977734.2, "profile": "profiles/k_ip_coarse_1M_x_50k_d150_k50.md"},
+    ("precision", "screened"): {"kernel": "k_list_screen", "bytes": 1.042e9, "fetch_kib": 484924.0,
+                                "write_kib": 48115.0, "profile": "profiles/query_batch_1M_x_50k_d150_k50.md"},
 }
 
 
@@ -593,7 +591,7 @@ def main():
         lat.append((time.perf_counter() - s) * 1e3)
     lat = np.array(lat)
 
-    # stage times (device, HIP events on the library's stream)
+    # stage times (device clock, or HIP events with updates pending)
     tot = {key: sum(t[key] for t in timings) for key in timings[0]}
     launches = max(1, int(tot["n_batches"]))
     stages = {"ip": tot["ip_ms"], "bound": tot["bound_ms"], "prune": tot["prune_ms"],
@@ -606,20 +604,21 @@ def main():
     coarse_used = tot.get("n_listed", 0) > 0 or tot.get("n_fallback", 0) > 0
     n_distinct = int(len(np.unique(wl.queries, axis=0))) if not args.no_dedup else nq
     if dom != "refine" and coarse_used:
-        # the coarse-bound kernel (first pass) is the largest single kernel of
-        # the ip + bound stages: 2*d flops per (query, user) pair, executed
-        # as one BF16 product over d padded to 32 on the matrix cores
+        # the ip stage is the list pass: thresholds from a sample of the users,
+        # then one estimate per (query, user) pair on the matrix cores
+        # (k_list_screen, nearly four fifths of the stage), 2*d flops executed
+        # as one BF16 product over d padded to 32
         kp = (d + 31) // 32 * 32
         flops = 2.0 * U * d * n_distinct * args.steps
         ach = flops / (tot["ip_ms"] * 1e-3) / 1e12
         executed = ach * kp / d
-        roof = {"kernel": "k_ip_coarse", "bound": "mfma", "achieved": round(ach, 3), "peak": PEAK_BF16_TFLOPS,
+        roof = {"kernel": "k_list_screen", "bound": "mfma", "achieved": round(ach, 3), "peak": PEAK_BF16_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(ach / PEAK_BF16_TFLOPS, 4), "traffic": None,
                 "executed_mfma_tflops": round(executed, 2), "executed_frac": round(executed / PEAK_BF16_TFLOPS, 4),
                 "avg_launch_ms": round(tot["ip_ms"] / launches, 4),
                 "work_per_launch": f"2*U*d algorithmic flops x {n_distinct * args.steps / launches:.0f} distinct queries "
-                                   f"(executed: 2*U*{kp}, one BF16 product); first pass only, the second pass is in "
-                                   "the bound stage"}
+                                   f"(executed: 2*U*{kp}, one BF16 product); the time is the stage's, with the queries' "
+                                   "conversion and the threshold sample before it"}
     elif dom == "refine":
         flops = 2.0 * I * d * tot["n_refined"]
         ach = flops / (tot["refine_ms"] * 1e-3) / 1e12
@@ -720,10 +719,10 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "bf16" if args.form == "screened" else "f32",
-        "dtype_note": ("coarse bounds on BF16 matrix cores (one product per term in the first pass, the "
-                       "3-product hi/lo split in the second), refinement screen with the 3-product split, FP32 "
-                       "accumulation throughout; undecided items rechecked with the exact FP32 rule; answers "
-                       "identical to the f32 form"
+        "dtype_note": ("threshold lists from one BF16 product per term with its error bound, listed users scored with "
+                       "the exact FP32 rule; refinement screen with the 3-product hi/lo split, FP32 accumulation "
+                       "throughout, undecided items rechecked with the exact FP32 rule; answers identical to the "
+                       "f32 form"
                        if args.form == "screened" else "exact sequential FP32 score rule"),
         "data": "synthetic (seeded), inputs resident in HBM",
         "config": {"workload": label, "form": args.form, "queries_per_step": nq,
@@ -734,7 +733,7 @@ def main():
         "distinct_queries_per_s": round(qps * n_distinct / nq, 2),
         "p50_ms": round(float(np.percentile(lat, 50)), 3),
         "p99_ms": round(float(np.percentile(lat, 99)), 3),
-        "latency_note": "single-query calls (batch of 1), host wall time incl. PCIe copies",
+        "latency_note": "single-query calls (batch of 1), host wall time incl. PCIe transfers",
         "table_build_ms": round(build_ms, 2),
         "table_build_wall_s": round(build_wall, 3),
         "stage_ms_per_step": {k_: round(v / args.steps, 3) for k_, v in stages.items()},
@@ -746,7 +745,7 @@ def main():
                       if args.form == "screened" else None),
         "coarse_bounds": ({"listed_per_query": round(tot["n_listed"] / max(1, args.steps) / nq, 1),
                            "fallback_queries_per_step": round(tot["n_fallback"] / max(1, args.steps), 2),
-                           "second_pass_queries_per_step": round(tot["n_coarse_refined"] / max(1, args.steps), 2)}
+                           "fine_column_queries_per_step": round(tot["n_coarse_refined"] / max(1, args.steps), 2)}
                           if tot.get("n_listed", 0) or tot.get("n_fallback", 0) else None),
         "roofline": roof,
         "same_queries_other_forms": compare,
