@@ -143,7 +143,7 @@ struct Ctx {
     // guard rows: [u_cap][kGuardRow], the values of the searched table at its
     // fine columns, -inf past them; kept with the table
     float *gvals = nullptr;
-    float *gcols = nullptr;     // the same values by column: [kGuardRow][u_cap at allocation]
+    float *gcols = nullptr;     // the same values by column behind them: [kGuardRow][u_cap at allocation]
     int64_t gpitch = 0;
     // columns of the guard rows, the guard columns among them and the searched
     // table's ranks, set with the table

@@ -448,3 +448,36 @@ def test_inserted_score_rows(orc, gpu_index_factory, n_new):
     m.insert_users(more)
     m.check(idx, queries, 40)
     idx.close()
+
+
+def test_rebuild_reuses_buffers(orc):
+    """Tables built one after the other on the same data: equal sizes, other
+    sizes, without and with a query table, after users came."""
+    _case("rebuild with equal and other sizes")
+    import rkr
+    rng = np.random.default_rng(4)
+    users = rng.standard_normal((500, 11), dtype=np.float32)
+    items = rng.standard_normal((900, 11), dtype=np.float32)
+    queries = items[:12]
+    nu = orc.normalize_users(users)
+    with rkr.Index(0) as idx:
+        idx.set_data(users, items)
+        for S, dense in ((40, 2), (40, 2), (41, 2), (41, 0), (41, 0), (40, 1), (40, 2)):
+            idx.set_option(8, dense)  # RKR_OPT_DENSE_TOP
+            ranks = np.sort(rng.choice(900, S, replace=False)).astype(np.int32)
+            idx.build_table(ranks)
+            assert np.array_equal(idx.get_table(), orc.sorted_score_rows(nu, items)[:, ranks])
+            for form in ("plain", "screened"):
+                idx.set_form(form)
+                res = idx.query(queries, 15)
+                bu, br, _ = orc.bruteforce(nu, items, queries, 15)
+                assert np.array_equal(res.users, bu) and np.array_equal(res.ranks, br)
+        more = rng.standard_normal((30, 11), dtype=np.float32)
+        idx.insert_users(more)
+        nu = np.concatenate([nu, orc.normalize_users(more)])
+        for _ in range(2):
+            idx.build_table(ranks)
+            assert np.array_equal(idx.get_table(), orc.sorted_score_rows(nu, items)[:, ranks])
+        bu, br, _ = orc.bruteforce(nu, items, queries, 15)
+        res = idx.query(queries, 15)
+        assert np.array_equal(res.users, bu) and np.array_equal(res.ranks, br)
