@@ -300,7 +300,8 @@ int ensure_pinned(Ctx *c, PinnedBuf &b, size_t bytes) {
     if (b.bytes >= bytes) return RKR_OK;
     free_pinned(b);
     const size_t want = std::max(bytes, b.bytes + b.bytes / 2);
-    if (hipHostMalloc(&b.p, want, hipHostMallocDefault) != hipSuccess) {
+    // coherent: kernels read and write it beside the host
+    if (hipHostMalloc(&b.p, want, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         b.p = nullptr;
         return set_err(c, RKR_ERR_NOMEM, "pinned host staging (" + std::to_string(want) + " bytes)");
     }
