@@ -481,3 +481,22 @@ def test_rebuild_reuses_buffers(orc):
         bu, br, _ = orc.bruteforce(nu, items, queries, 15)
         res = idx.query(queries, 15)
         assert np.array_equal(res.users, bu) and np.array_equal(res.ranks, br)
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 192, 193, 250])
+def test_narrow_column_tiles(orc, gpu_index_factory, n):
+    """A last column block on either side of 64 columns: items of sorted rows, queries of a plain batch."""
+    _case(f"narrow tiles n={n}")
+    import rkr
+    rng = np.random.default_rng(n)
+    users = rng.standard_normal((4300, 21), dtype=np.float32)
+    items = rng.standard_normal((n, 21), dtype=np.float32)
+    with rkr.Index(0) as idx:
+        idx.set_data(users[:200], items)
+        assert np.array_equal(idx.sorted_scores(), orc.sorted_score_rows(orc.normalize_users(users[:200]), items))
+    catalogue = rng.standard_normal((400, 21), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, catalogue, 30)
+    res = idx.query(items, 9)
+    bu, br, bq = orc.bruteforce(orc.normalize_users(users), catalogue, items, 9)
+    assert np.array_equal(res.users, bu) and np.array_equal(res.ranks, br) and np.array_equal(res.qips, bq)
+    idx.close()
