@@ -564,7 +564,10 @@ struct ListLaunch {
     uint32_t *g_cnt, *g_off, *g_cur;  // pairs per query and their places (null: kFilterQueries or fewer)
 };
 // Up to this many queries the candidates are looked for in the whole list,
-// which spares the two launches that order it (about 5 us each).
+// which spares the two launches that order it.  Without the order and with it,
+// ms: 16 queries over 1M users 0.31 and 0.35, 6 over 30k 0.13 and 0.14.  Each
+// query reads all of the list, so popular queries pay for it: 16 of them over
+// 1M users 0.59 and 0.42, 8 over 250k 0.22 and 0.19.
 constexpr int kFilterQueries = 16;
 // Threshold per query and the listed pairs, from the matrix cores or from qip.
 hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L);
