@@ -292,6 +292,14 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
 }
 
 // ---- list ------------------------------------------------------------------
+// The list's length as every later stage reads it: none of a list that outgrew
+// its arrays.  Its pairs are not all there, and in a batch that orders them by
+// query the ordered arrays are never written, so no stage may walk them.
+__device__ __forceinline__ int64_t list_len(const ListCounters *ctr, int64_t cap) {
+    const int64_t n = ctr->n_list;
+    return n <= cap ? n : 0;
+}
+
 // Zeroes the list's counts per query and the scatter's cursors behind them.
 __device__ __forceinline__ void zero_counts(int32_t nq, uint32_t *__restrict__ g_cnt) {
     if (g_cnt && blockIdx.y == 0)
@@ -600,7 +608,7 @@ constexpr int kGroupQ = 4096;       // queries counted in LDS at a time
 constexpr int64_t kChunk = 1024;    // pairs of a workgroup, at least
 
 __device__ __forceinline__ bool list_chunk(const ListCounters *ctr, int64_t cap, int64_t &first, int64_t &last) {
-    const int64_t n = ctr->n_list <= cap ? ctr->n_list : 0;  // an overflowed list is not used
+    const int64_t n = list_len(ctr, cap);
     const int64_t per = max(kChunk, (n + gridDim.x - 1) / gridDim.x);
     first = min(n, (int64_t)blockIdx.x * per);
     last = min(n, first + per);
@@ -797,7 +805,7 @@ __global__ void __launch_bounds__(NT) k_list_exact(const float *__restrict__ use
     __shared__ f32x4 sd[SCORES ? 1 : NT / 64][2][SCORES ? 1 : 64 * DP / 4];
     if (threadIdx.x < GW) col[threadIdx.x] = threadIdx.x < kMaxFine ? fc.col[threadIdx.x] : 0;
     __syncthreads();
-    const int64_t n = min((int64_t)ctr->n_list, list_cap);
+    const int64_t n = list_len(ctr, list_cap);
     const int64_t per_round = (int64_t)gridDim.x * NT;
     for (int64_t r0 = 0; r0 < n; r0 += per_round) {
         const int64_t lb = xcd_block(min(n - r0, per_round));
