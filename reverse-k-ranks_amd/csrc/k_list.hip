@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
 // its arrays.  Its pairs are not all there, and in a batch that orders them by
 // query the ordered arrays are never written, so no stage may walk them.
 __device__ __forceinline__ int64_t list_len(const ListCounters *ctr, int64_t cap) {
-    const int64_t n = ctr->n_list;
+    const int64_t n = (int64_t)ctr->n_list;
     return n <= cap ? n : 0;
 }
 
@@ -313,7 +313,8 @@ constexpr int kSlice = 512;
 
 struct ListQueue {
     uint2 e[QCAP];
-    int32_t n, base;
+    int32_t n;
+    int64_t base;  // places are counted in 64 bits, also past the list's capacity
 };
 
 // Appends each lane's pairs (bit 4 b + i of m: user u0 + 16 b, query slot_b[i])
@@ -321,7 +322,7 @@ struct ListQueue {
 // wavefront.  Called by whole wavefronts.
 __device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, const int32_t *slot_b,
                                          int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b, int64_t cap,
-                                         int32_t *__restrict__ list_n) {
+                                         unsigned long long *__restrict__ list_n) {
     const int lane = threadIdx.x & 63;
     const int32_t c = __popc(m);
     int32_t x = c;
@@ -336,10 +337,10 @@ __device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, 
     base = __shfl(base, 0, 64);
     int32_t p = base + x - c;
     // places at and past QCAP: the wavefront's share of the list
-    int32_t over = 0;
+    long long over = 0;
     if (base + tot > QCAP) {
         const int32_t first = max(base, QCAP);
-        if (lane == 0) over = atomicAdd(list_n, base + tot - first);
+        if (lane == 0) over = (long long)atomicAdd(list_n, (unsigned long long)(base + tot - first));
         over = __shfl(over, 0, 64) - first;
     }
     while (m) {
@@ -348,7 +349,7 @@ __device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, 
         const int32_t u = u0 + (t >> 2) * 16, b = slot_b[t & 3];
         if (p < QCAP) {
             sq.e[p] = make_uint2((uint32_t)u, (uint32_t)b);
-        } else if ((int64_t)over + p < cap) {
+        } else if (over + p < cap) {
             cl_u[over + p] = u;
             cl_b[over + p] = b;
         }
@@ -359,10 +360,10 @@ __device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, 
 // The unit's queued pairs go to the list; every wave has passed a barrier
 // since the last push, and passes one before the next.
 __device__ __forceinline__ void list_flush(ListQueue &sq, int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b,
-                                           int64_t cap, int32_t *__restrict__ list_n) {
+                                           int64_t cap, unsigned long long *__restrict__ list_n) {
     const int32_t n = min(sq.n, QCAP);
     if (n > 0) {  // uniform
-        if (threadIdx.x == 0) sq.base = atomicAdd(list_n, n);
+        if (threadIdx.x == 0) sq.base = (int64_t)atomicAdd(list_n, (unsigned long long)n);
         __syncthreads();
         const int64_t base = sq.base;
         for (int i = threadIdx.x; i < n; i += NT)
@@ -376,10 +377,10 @@ __device__ __forceinline__ void list_flush(ListQueue &sq, int32_t *__restrict__ 
 // their number in a register of every lane.
 constexpr int WQ = 256;
 
-__device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int32_t base, int32_t u0, const int32_t *ord,
+__device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int64_t base, int32_t u0, const int32_t *ord,
                                            int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b, int64_t cap) {
     for (int i = threadIdx.x & 63; i < n; i += 64)
-        if ((int64_t)base + i < cap) {
+        if (base + i < cap) {
             cl_u[base + i] = u0 + (int32_t)(q[i] & 0xFFu);
             cl_b[base + i] = ord[q[i] >> 8];
         }
@@ -411,7 +412,8 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
     __shared__ f32x4 sCs[kSlice / 4];
     __shared__ int32_t sCol[kSlice / 4 + QST / 4], sOrd[kSlice];
     __shared__ uint32_t sQ[NT / 64][WQ];
-    __shared__ int32_t sN[NT / 64], sBase;
+    __shared__ int32_t sN[NT / 64];
+    __shared__ int64_t sBase;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
     const int32_t n_slots = ctr->n_slots;
     zero_counts(P.nq, g_cnt);
@@ -510,8 +512,8 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
                             const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
                             if (m != 0) {
                                 if (n_q + 64 > WQ) {  // uniform: make room
-                                    int32_t base = 0;
-                                    if (lane == 0) base = atomicAdd(&ctr->n_list, n_q);
+                                    long long base = 0;
+                                    if (lane == 0) base = (long long)atomicAdd(&ctr->n_list, (unsigned long long)n_q);
                                     wave_flush(sQ[wave], n_q, __shfl(base, 0, 64), (int32_t)(rb * UB), sOrd, cl_u, cl_b,
                                                list_cap);
                                     n_q = 0;
@@ -541,7 +543,7 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
             tot += sN[w];
         }
         if (tot > 0) {  // uniform
-            if (threadIdx.x == 0) sBase = atomicAdd(&ctr->n_list, tot);
+            if (threadIdx.x == 0) sBase = (int64_t)atomicAdd(&ctr->n_list, (unsigned long long)tot);
             __syncthreads();
             wave_flush(sQ[wave], n_q, sBase + before, (int32_t)(rb * UB), sOrd, cl_u, cl_b, list_cap);
         }
@@ -924,7 +926,7 @@ __global__ void __launch_bounds__(FT) k_list_final(const int32_t *__restrict__ c
     const int32_t b = (int32_t)blockIdx.x;
     const int lane = threadIdx.x & 63;
     const QueryInfo q = qi[b];
-    const bool listed = q.thr >= 0 && (int64_t)ctr->n_list <= list_cap;
+    const bool listed = q.thr >= 0 && (int64_t)ctr->n_list <= list_cap;  // list_len, and thr = -1 past it
     const int64_t first = !listed || FILTER ? 0 : g_off[b];
     const int64_t end = !listed ? 0 : FILTER ? (int64_t)ctr->n_list : first + g_cnt[b];
     const uint32_t k = (uint32_t)q.topk;

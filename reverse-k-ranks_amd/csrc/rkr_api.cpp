@@ -1876,7 +1876,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                     if (fallback) fallback->push_back((int32_t)(q0 + i));
                     tm.n_fallback += 1;
                 }
-            if (hctr->n_list <= list_cap) tm.n_listed += hctr->n_list;  // else no stage read the list
+            if ((int64_t)hctr->n_list <= list_cap) tm.n_listed += (int64_t)hctr->n_list;  // else no stage read the list
             tm.n_coarse_refined += hctr->n_finer;
         }
         if (qsrp)

@@ -482,13 +482,14 @@ struct QueryInfo {          // one per query of a device batch
 // with the outputs.
 struct alignas(64) ListCounters {
     int32_t n_slots;        // queries with a threshold
-    int32_t n_list;         // listed pairs (past the list's capacity when it overflowed)
     int32_t n_cand;         // candidates
     int32_t n_finer;        // queries listed against a column finer than the guard columns
     int32_t n_refine;       // refine rows
     int32_t n_recheck;      // screened form: undecided pairs
     uint32_t max_err_bits;  // screened form: largest screen error seen
-    int32_t pad;
+    int32_t pad[2];
+    unsigned long long n_list;  // listed pairs, past the list's capacity when it overflowed: up to
+                                // every pair of the batch, which nothing keeps below 2^32
     uint64_t t[8];          // device clock at the stages' starts (enum below)
 };
 // Stages of a batch timed by its kernels: the first kernel of a stage writes

@@ -46,3 +46,28 @@ def test_list_overflow(gpu_index_factory, form, nq):
     idx.set_option(9, 0)  # RKR_OPT_COARSE
     _same_answers(got, idx.query(queries, ks), ks)
     idx.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+def test_more_listed_pairs_than_31_bits_count(gpu_index_factory, form):
+    """1024 queries whose lists hold 2.2 million users each, 2.29e9 pairs in all,
+    where the sample shows a dozen users a query."""
+    _case(f"2.3e9 listed pairs, {form}")
+    rng = np.random.default_rng(1)
+    U, I, d, nq = 2_300_000, 300, 8, 1024
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    pool = rng.standard_normal((40_000, d), dtype=np.float32)
+    rank = (pool @ items.T > (pool @ items[7])[:, None]).sum(axis=1)
+    users = pool[rng.choice(np.flatnonzero(rank < 100), U)]
+    at = _sampled(U)
+    users[at] = pool[rng.choice(np.flatnonzero(rank >= 280), len(at))]
+    users[at[100:112]] = pool[np.flatnonzero((rank >= 100) & (rank < 110))[:12]]
+    queries = items[7] + np.float32(1e-4) * rng.standard_normal((nq, d), dtype=np.float32)
+    idx, _ = gpu_index_factory(users, items, 64, dense_top=0)
+    idx.set_form(form)
+    ks = [10] * nq
+    got = idx.query(queries, ks)
+    assert got.timing["n_batches"] == 2 and got.timing["n_fallback"] == nq and got.timing["n_listed"] == 0
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    _same_answers(got, idx.query(queries, ks), ks)
+    idx.close()
