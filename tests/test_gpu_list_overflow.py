@@ -56,6 +56,7 @@ def test_more_listed_pairs_than_31_bits_count(gpu_index_factory, form):
     rng = np.random.default_rng(1)
     U, I, d, nq = 2_300_000, 300, 8, 1024
     items = rng.standard_normal((I, d), dtype=np.float32)
+    items /= np.linalg.norm(items, axis=1, keepdims=True)
     pool = rng.standard_normal((40_000, d), dtype=np.float32)
     rank = (pool @ items.T > (pool @ items[7])[:, None]).sum(axis=1)
     users = pool[rng.choice(np.flatnonzero(rank < 100), U)]
