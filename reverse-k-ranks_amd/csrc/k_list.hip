@@ -13,7 +13,7 @@
 // those of a search over every user.  A query for which that fails is answered
 // by the full search instead, so t only decides how long the list is.
 //
-// t comes from a sample of the users, every stride-th (all of them for few
+// t comes from a sample of the users, one of every stride (all of them for few
 // users, where the k-th bound is then exact): the smallest column that as many
 // sampled users reach for certain (s - e) as k users would need, plus a margin
 // of three standard deviations, since a threshold that is too tight costs a
@@ -49,19 +49,30 @@ __device__ __forceinline__ int guard_pos(const float *row, float x) {
     return p;
 }
 
-// Guard rows of NU sampled users (users (r0 + i) * stride, i < NU, clamped to
-// the last) to LDS rows of stride GW + 1: an odd stride, so the lanes' searches
+// Sampled user r: one of the users r * stride .. r * stride + stride - 1, at a
+// place that a hash of r gives.  A fixed place would fall into step with users
+// stored in a periodic order (users of 16 clusters in turn, a stride of 15 or
+// 16): 1000 queries over 1M such users overflowed their lists, 33 ms a call
+// where this sample takes 1.25.  (r * stride < n_user < 2^31.)
+__device__ __forceinline__ int64_t sample_user(int64_t r, int64_t stride, int64_t n_user) {
+    uint32_t h = (uint32_t)r * 0x9E3779B1u;
+    h = (h ^ (h >> 15)) * 0x85EBCA6Bu;
+    return min((uint32_t)r * (uint32_t)stride + __umulhi(h, (uint32_t)stride), (uint32_t)n_user - 1u);
+}
+
+// Guard rows of NU sampled users (r0 + i, i < NU, clamped to the last) to LDS rows of stride GW + 1: an odd stride, so the lanes' searches
 // fall in different banks.  Every load is in flight before the first write.
 constexpr int GP = GW + 1;
 template <int NU>
 __device__ __forceinline__ void stage_guards(float *dst, const float *__restrict__ gvals, int64_t r0, int64_t n_s,
-                                             int64_t stride) {
+                                             int64_t stride, int64_t n_user) {
     constexpr int N = NU * GW / 4 / NT;
     f32x4 v[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) {
         const int c = (int)threadIdx.x + k * NT;
-        v[k] = reinterpret_cast<const f32x4 *>(gvals)[min(r0 + c / (GW / 4), n_s - 1) * stride * (GW / 4) + c % (GW / 4)];
+        v[k] = reinterpret_cast<const f32x4 *>(gvals)[
+            sample_user(min(r0 + c / (GW / 4), n_s - 1), stride, n_user) * (GW / 4) + c % (GW / 4)];
     }
 #pragma unroll
     for (int k = 0; k < N; ++k) {
@@ -100,7 +111,7 @@ __device__ __forceinline__ int guard_pos_reg(const float (&hd)[7], const float *
 // block owns user lr and queries 4 lq .. 4 lq + 3.
 template <int KS>
 __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScreen P, int64_t n_s, int64_t stride,
-                                                         uint32_t *__restrict__ hist) {
+                                                         int64_t n_user, uint32_t *__restrict__ hist) {
     constexpr int ROWQ = (KS * 32 + KPAD_LDS) / 8, KQ = KS * 4;
     __shared__ u32x4 sA[QST * ROWQ];
     __shared__ float sCs[QST];
@@ -124,7 +135,7 @@ __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScree
     const int64_t n_rb = (n_s + 127) / 128;
     for (int64_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x) {
         __syncthreads();  // the previous block is done with sG
-        stage_guards<128>(sG, P.gvals, rb * 128, n_s, stride);
+        stage_guards<128>(sG, P.gvals, rb * 128, n_s, stride, n_user);
         Frag uh[2][KS];
         float ar[2];
         bool live[2];
@@ -132,7 +143,7 @@ __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScree
         for (int b = 0; b < 2; ++b) {
             const int64_t r = rb * 128 + wave * 32 + b * 16 + lr;
             live[b] = r < n_s;
-            const int64_t u = min(r, n_s - 1) * stride;
+            const int64_t u = sample_user(min(r, n_s - 1), stride, n_user);
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) uh[b][ks].q = reinterpret_cast<const u32x4 *>(P.user_hi + u * P.Kp)[ks * 4 + lq];
             ar[b] = P.C * P.user_norm[u];
@@ -184,13 +195,14 @@ __global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ 
     const int64_t n_ub = (n_s + UB - 1) / UB;
     for (int64_t ub = blockIdx.x; ub < n_ub; ub += gridDim.x) {
         __syncthreads();
-        stage_guards<UB>(sG, gvals, ub * UB, n_s, stride);
+        stage_guards<UB>(sG, gvals, ub * UB, n_s, stride, n_user);
         __syncthreads();
         const int ul = threadIdx.x & 63;
         const int64_t r = ub * UB + ul;
+        const int64_t u = sample_user(min(r, n_s - 1), stride, n_user);
         if (r < n_s)
             for (int ql = threadIdx.x >> 6; ql < QB && q0 + ql < nq; ql += NT / 64) {
-                const float s = qip[(int64_t)(q0 + ql) * n_user + r * stride];
+                const float s = qip[(int64_t)(q0 + ql) * n_user + u];
                 const int p = guard_pos(&sG[ul * GP], eps > 0.0f ? __double2float_rd((double)s - (double)eps) : s);
                 if (p < n_fine) atomicAdd(&sH[ql * GW + p], 1u);
             }
@@ -1146,7 +1158,7 @@ hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L) {
     const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(n_sb, (2 * L.n_cu + qg - 1) / qg));
 #define RKR_SAMPLE_CASE(ks)                                                                                       \
     case ks:                                                                                                      \
-        hipLaunchKernelGGL(k_sample_screen<ks>, dim3(gx, qg), dim3(NT), 0, s, P, n_s, L.stride, L.hist);           \
+        hipLaunchKernelGGL(k_sample_screen<ks>, dim3(gx, qg), dim3(NT), 0, s, P, n_s, L.stride, L.n_user, L.hist);           \
         break;
     RKR_KS_SWITCH(L.Kp, RKR_SAMPLE_CASE)
 #undef RKR_SAMPLE_CASE

@@ -1415,7 +1415,7 @@ namespace {
 constexpr int64_t kCoarseChunk = 16384;
 constexpr int32_t kCoarseMinBatch = 8;
 
-// Every stride-th user is sampled for the list thresholds: all of up to 16,384
+// One user of every stride is sampled for the list thresholds: all of up to 16,384
 // users (the threshold is then exact), else a sixteenth of them, at least
 // 16,384 and at most 65,536.
 int64_t sample_stride(int64_t U) {

@@ -552,7 +552,7 @@ struct ListLaunch {
     FineCols fc;
     float C, floor, eps;
     float *qip;              // exact scores (read with scores, else written for listed pairs)
-    int64_t stride;          // every stride-th user is sampled
+    int64_t stride;          // one user of every stride is sampled
     int64_t cap;             // a longer estimated list takes the full search
     int64_t list_cap;        // entries of the lists
     uint32_t *hist;          // nq x 64, zeroed

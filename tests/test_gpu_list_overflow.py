@@ -11,9 +11,12 @@ def _case(msg):
 
 
 def _sampled(U):
-    """The users that the list thresholds are taken from."""
-    n = min(max(U // 16, 16384), 65536)
-    return np.arange(0, U, max(1, U // n))
+    """The users that the list thresholds are taken from: one of every stride, at a hashed place."""
+    stride = max(1, U // min(max(U // 16, 16384), 65536))
+    r = np.arange((U + stride - 1) // stride, dtype=np.uint64)
+    h = r * np.uint64(0x9E3779B1) & np.uint64(0xFFFFFFFF)
+    h = (h ^ (h >> np.uint64(15))) * np.uint64(0x85EBCA6B) & np.uint64(0xFFFFFFFF)
+    return np.minimum(r * np.uint64(stride) + (h * np.uint64(stride) >> np.uint64(32)), U - 1).astype(np.int64)
 
 
 def _same_answers(got, want, ks):
@@ -69,6 +72,30 @@ def test_more_listed_pairs_than_31_bits_count(gpu_index_factory, form):
     ks = [10] * nq
     got = idx.query(queries, ks)
     assert got.timing["n_batches"] == 2 and got.timing["n_fallback"] == nq and got.timing["n_listed"] == 0
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    _same_answers(got, idx.query(queries, ks), ks)
+    idx.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+@pytest.mark.parametrize("U", [66_000, 300_000])
+def test_users_in_a_periodic_order(gpu_index_factory, form, U):
+    """Users of as many clusters as the sample's stride, in turn, and queries near
+    all clusters but the first: every list fits, as the sample says."""
+    _case(f"periodic user order {form} U={U}")
+    rng = np.random.default_rng(U)
+    I, d, nq = 700, 24, 64
+    stride = U // max(U // 16, 16384)
+    centre = rng.standard_normal((stride, d), dtype=np.float32)
+    users = np.float32(0.7) * centre[np.arange(U) % stride] + rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    near = centre[rng.integers(1, stride, nq // 2)] + np.float32(0.5) * rng.standard_normal((nq // 2, d), dtype=np.float32)
+    queries = np.concatenate([items[:nq // 2], near]) * np.float32(0.9)
+    ks = [int(k) for k in rng.integers(1, 50, nq)]
+    idx, _ = gpu_index_factory(users, items, 64)
+    idx.set_form(form)
+    got = idx.query(queries, ks)
+    assert got.timing["n_listed"] > 0 and got.timing["n_fallback"] == 0
     idx.set_option(9, 0)  # RKR_OPT_COARSE
     _same_answers(got, idx.query(queries, ks), ks)
     idx.close()
