@@ -214,11 +214,15 @@ __global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ 
 
 // ---- plan ------------------------------------------------------------------
 // One workgroup.  Each query's threshold column, the queries ordered by it
-// (slot -> query), and for every four neighbouring slots the largest of their
-// columns, which all four take (a larger column lists more users, never
-// fewer).  A query with no such column, with an estimated list over cap, or
-// past the point where the estimates fill half the list gets thr = -1 (the
-// full search answers it) and no slot.
+// (slot -> query), and for every four neighbouring slots the column they share,
+// the largest of theirs (a larger column lists more users, never fewer).  A
+// query with no such column, with an estimated list over cap, or past the point
+// where the estimates fill half the list gets thr = -1 (the full search answers
+// it) and no slot.  Four slots of different columns are estimated again at the
+// shared one: a query that few users rank high can make three others list most
+// users.  Where such a list is over cap, or what all of them add does not fit
+// and the four take more than an equal share of the room, they keep a smaller one
+// of their columns and the deeper queries get thr = -1.
 constexpr int PT = 1024;
 
 __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ hist, int32_t nq, int32_t n_fine,
@@ -226,11 +230,14 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
                                                   uint64_t coarse_mask, QueryInfo *__restrict__ qi,
                                                   int32_t *__restrict__ order, int32_t *__restrict__ colg,
                                                   ListCounters *__restrict__ ctr) {
-    __shared__ int32_t bin[GW], at[GW];
+    __shared__ int32_t bin[GW], at[GW], mix[GW];
     __shared__ int64_t load[GW];
-    __shared__ int32_t n_finer, n_slots;
+    __shared__ int64_t left, added;  // room beside the lists at their own columns, and what sharing adds
+    __shared__ int32_t n_finer, n_slots, n_mix;
+    auto estimate = [&](int64_t sampled) { return min(sampled * stride, n_user); };
+    const int64_t room = list_cap / 2;
     for (int i = threadIdx.x; i < GW; i += PT) { bin[i] = 0; load[i] = 0; }
-    if (threadIdx.x == 0) n_finer = 0;
+    if (threadIdx.x == 0) n_finer = n_slots = n_mix = 0, left = added = 0;
     __syncthreads();
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
         // the row's 64 counts in flight together (read one after the other, the
@@ -248,9 +255,10 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
             cum += v[f / 4][f % 4];
             if (t < 0 && f < n_fine && cum >= want) { t = f; n = cum; }
         }
-        n = min(n * stride, n_user);
+        n = estimate(n);
         if (n > cap) t = -1;
         qi[b].thr = t;
+        qi[b].n_cand = (int32_t)n;  // until the candidates are counted
         if (t >= 0) {
             atomicAdd(&bin[t], 1);
             atomicAdd(reinterpret_cast<unsigned long long *>(&load[t]), (unsigned long long)n);
@@ -269,11 +277,22 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
             const int32_t z = __shfl_up(s, o, 64);
             if (t >= o) { sum += y; s += z; }
         }
-        const bool fits = 2 * sum <= list_cap;  // loads are not negative: true up to some column
-        at[t] = fits ? s - bin[t] : -1;
-        const uint64_t m = __builtin_amdgcn_ballot_w64(fits);
-        if (t == 0 && m == 0) n_slots = 0;
-        if (m != 0 && t == 63 - __clzll((long long)m)) n_slots = s;
+        const bool ok = sum <= room;  // loads are not negative: true up to some column
+        const int32_t first = s - bin[t];
+        at[t] = ok ? first : -1;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(ok);
+        // the groups of four that hold more than one column, at the first of
+        // the columns that start inside them
+        const uint64_t in = __builtin_amdgcn_ballot_w64(ok && bin[t] > 0 && first % 4 != 0);
+        const uint64_t before = in & ((1ull << t) - 1);
+        const int32_t prev = __shfl(first, before ? 63 - __clzll((long long)before) : 0, 64);
+        mix[t] = ((in >> t) & 1) && (!before || prev / 4 != first / 4) ? first / 4 : -1;
+        const int groups = (int)__popcll(__builtin_amdgcn_ballot_w64(mix[t] >= 0));
+        if (m != 0 && t == 63 - __clzll((long long)m)) {
+            n_slots = s;
+            n_mix = groups;
+            left = room - sum;
+        }
     }
     __syncthreads();
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
@@ -292,10 +311,57 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
     __threadfence_block();
     __syncthreads();
     for (int32_t g = threadIdx.x; g < (n_slots + 3) / 4; g += PT) {
-        int32_t c = 0;
-        for (int j = 0; j < 4 && 4 * g + j < n_slots; ++j) c = max(c, qi[order[4 * g + j]].thr);
-        colg[g] = c;
-        for (int j = 0; j < 4 && 4 * g + j < n_slots; ++j) qi[order[4 * g + j]].thr = c;
+        const int32_t c = qi[order[4 * g]].thr;
+        if (qi[order[min(4 * g + 3, n_slots - 1)]].thr == c) colg[g] = c;
+    }
+    // a thread per member of the mixed groups
+    const int32_t g = threadIdx.x < 4 * GW ? mix[threadIdx.x >> 2] : -1;
+    const int32_t slot = 4 * g + (int32_t)(threadIdx.x & 3);
+    const bool member = g >= 0 && slot < n_slots;
+    const int32_t b = member ? order[slot] : 0;
+    const int32_t own = member ? qi[b].thr : -1;
+    // the group's columns: the largest, the next one below it, the smallest
+    auto quad_max = [](int32_t x) {
+        x = max(x, __shfl_xor(x, 1, 64));
+        return max(x, __shfl_xor(x, 2, 64));
+    };
+    const int32_t c0 = quad_max(own), c1 = quad_max(own < c0 ? own : -1);
+    const int32_t least = __shfl(own, (int)(threadIdx.x & 63 & ~3), 64);
+    int64_t more[2] = {0, 0};
+    bool over[2] = {false, false};
+    if (member && own < c0) {
+        const u32x4 *row = reinterpret_cast<const u32x4 *>(hist + (int64_t)b * GW);
+        int64_t cum[2] = {0, 0};
+#pragma unroll
+        for (int j = 0; j < GW / 4; ++j) {
+            const u32x4 v = row[j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                cum[0] += 4 * j + i <= c0 ? v[i] : 0u;
+                cum[1] += 4 * j + i <= c1 ? v[i] : 0u;
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int64_t n = estimate(cum[h]);
+            more[h] = n - qi[b].n_cand;
+            over[h] = n > cap;
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        more[h] += __shfl_xor(more[h], 1, 64);
+        more[h] += __shfl_xor(more[h], 2, 64);
+        over[h] = (__builtin_amdgcn_ballot_w64(over[h]) >> (threadIdx.x & 63 & ~3) & 0xF) != 0;
+    }
+    if (g >= 0 && (threadIdx.x & 3) == 0)
+        atomicAdd(reinterpret_cast<unsigned long long *>(&added), (unsigned long long)more[0]);
+    __syncthreads();
+    if (member) {
+        auto good = [&](int h) { return !over[h] && more[h] <= left / n_mix; };
+        const int32_t c = !over[0] && added <= left ? c0 : good(0) ? c0 : good(1) ? c1 : least;
+        qi[b].thr = own <= c ? c : -1;
+        if ((threadIdx.x & 3) == 0) colg[g] = c;
     }
     if (threadIdx.x == 0) {
         ctr->n_slots = n_slots;

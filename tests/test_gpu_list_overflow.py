@@ -99,3 +99,26 @@ def test_users_in_a_periodic_order(gpu_index_factory, form, U):
     idx.set_option(9, 0)  # RKR_OPT_COARSE
     _same_answers(got, idx.query(queries, ks), ks)
     idx.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+@pytest.mark.parametrize("scale", [0.01, 0.1, 0.3])
+def test_one_deep_query_among_ordinary_ones(gpu_index_factory, form, scale):
+    """A short query that no user ranks high beside 19 ordinary ones: four
+    neighbours in the order of thresholds share one, and the ordinary ones'
+    lists would hold most users at the short one's."""
+    _case(f"one query scaled by {scale}, {form}")
+    rng = np.random.default_rng(11)
+    U, I, d, nq = 100_000, 800, 16, 20
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    queries = items[:nq].copy()
+    queries[3] *= np.float32(scale)
+    idx, _ = gpu_index_factory(users, items, 48)
+    idx.set_form(form)
+    ks = [20] * nq
+    got = idx.query(queries, ks)
+    assert got.timing["n_listed"] > 0 and got.timing["n_fallback"] <= 1
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    _same_answers(got, idx.query(queries, ks), ks)
+    idx.close()
