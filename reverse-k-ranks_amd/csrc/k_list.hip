@@ -216,29 +216,68 @@ __global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ 
 // One workgroup.  Each query's threshold column, the queries ordered by it
 // (slot -> query), and for every four neighbouring slots the column they share,
 // the largest of theirs (a larger column lists more users, never fewer).  A
-// query with no such column, with an estimated list over cap, or past the point
-// where the estimates fill half the list gets thr = -1 (the full search answers
-// it) and no slot.  Four slots of different columns are estimated again at the
-// shared one: a query that few users rank high can make three others list most
-// users.  Where such a list is over cap, or what all of them add does not fit
-// and the four take more than an equal share of the room, they keep a smaller one
-// of their columns and the deeper queries get thr = -1.
+// query with no such column or with an estimated list over cap gets thr = -1 (a
+// search over every user answers it) and no slot.  Lists are taken in order of
+// their length, up to `room` pairs; the longer ones get thr = kNoRoom and
+// ctr->n_need says how many pairs they hold.  (Taken in order of their column,
+// popular queries came first and one of them kept every other out.)
+// Four slots of different columns are estimated again at the shared one: a query
+// that few users rank high can make three others list most users.  Where such a
+// list is over cap, or what all of them add does not fit and the four take more
+// than an equal share of the room, they keep a smaller one of their columns and
+// the deeper queries get thr = kNoRoom.
 constexpr int PT = 1024;
 
 __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ hist, int32_t nq, int32_t n_fine,
-                                                  int64_t stride, int64_t n_user, int64_t cap, int64_t list_cap,
+                                                  int64_t stride, int64_t n_user, int64_t cap, int64_t room,
                                                   uint64_t coarse_mask, QueryInfo *__restrict__ qi,
                                                   int32_t *__restrict__ order, int32_t *__restrict__ colg,
                                                   ListCounters *__restrict__ ctr) {
     __shared__ int32_t bin[GW], at[GW], mix[GW];
-    __shared__ int64_t load[GW];
+    __shared__ int64_t load[GW];  // pairs of the lists of each length class
     __shared__ int64_t left, added;  // room beside the lists at their own columns, and what sharing adds
-    __shared__ int32_t n_finer, n_slots, n_mix;
+    __shared__ int32_t n_finer, n_slots, n_mix, longest;
     auto estimate = [&](int64_t sampled) { return min(sampled * stride, n_user); };
-    const int64_t room = list_cap / 2;
+    // two length classes an octave
+    auto length_class = [](int32_t n) {
+        const int top = 31 - __clz(max(n, 1));
+        return 2 * top + (top > 0 ? n >> (top - 1) & 1 : 0);
+    };
+    // the columns' first slots: a column per lane of one wavefront
+    auto first_slots = [&] {
+        const int t = threadIdx.x;
+        const int32_t own = bin[t];
+        int32_t s = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t z = __shfl_up(s, o, 64);
+            if (t >= o) s += z;
+        }
+        const int32_t first = s - own;
+        at[t] = first;
+        bin[t] = 0;
+        // the groups of four that hold more than one column, at the first of
+        // the columns that start inside them
+        const uint64_t in = __builtin_amdgcn_ballot_w64(own > 0 && first % 4 != 0);
+        const uint64_t before = in & ((1ull << t) - 1);
+        const int32_t prev = __shfl(first, before ? 63 - __clzll((long long)before) : 0, 64);
+        mix[t] = ((in >> t) & 1) && (!before || prev / 4 != first / 4) ? first / 4 : -1;
+        const int groups = (int)__popcll(__builtin_amdgcn_ballot_w64(mix[t] >= 0));
+        if (t == 63) {
+            n_slots = s;
+            n_mix = groups;
+        }
+    };
+    auto column_of = [&](int32_t slot) {  // the last column that starts at or before it
+        int t = 0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) t += at[t + o] <= slot ? o : 0;
+        return t;
+    };
     for (int i = threadIdx.x; i < GW; i += PT) { bin[i] = 0; load[i] = 0; }
-    if (threadIdx.x == 0) n_finer = n_slots = n_mix = 0, left = added = 0;
+    if (threadIdx.x == 0) n_finer = n_slots = n_mix = longest = 0, left = added = 0;
     __syncthreads();
+    int32_t own_thr = -1;  // of the thread's first query, which then needs no reading back
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
         // the row's 64 counts in flight together (read one after the other, the
         // early end of the search costs more than it saves)
@@ -257,53 +296,53 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
         }
         n = estimate(n);
         if (n > cap) t = -1;
+        if (b < PT) own_thr = t;
         qi[b].thr = t;
         qi[b].n_cand = (int32_t)n;  // until the candidates are counted
         if (t >= 0) {
             atomicAdd(&bin[t], 1);
-            atomicAdd(reinterpret_cast<unsigned long long *>(&load[t]), (unsigned long long)n);
+            atomicAdd(reinterpret_cast<unsigned long long *>(&load[length_class((int32_t)n)]), (unsigned long long)n);
         }
     }
     __syncthreads();
+    static_assert(GW == 64, "one wavefront");
     if (threadIdx.x < 64) {
-        // columns in order while their estimated lists fit: a column per lane
-        static_assert(GW == 64, "one wavefront");
         const int t = threadIdx.x;
         int64_t sum = load[t];
-        int32_t s = bin[t];
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const int64_t y = __shfl_up(sum, o, 64);
-            const int32_t z = __shfl_up(s, o, 64);
-            if (t >= o) { sum += y; s += z; }
+            if (t >= o) sum += y;
         }
-        const bool ok = sum <= room;  // loads are not negative: true up to some column
-        const int32_t first = s - bin[t];
-        at[t] = ok ? first : -1;
-        const uint64_t m = __builtin_amdgcn_ballot_w64(ok);
-        // the groups of four that hold more than one column, at the first of
-        // the columns that start inside them
-        const uint64_t in = __builtin_amdgcn_ballot_w64(ok && bin[t] > 0 && first % 4 != 0);
-        const uint64_t before = in & ((1ull << t) - 1);
-        const int32_t prev = __shfl(first, before ? 63 - __clzll((long long)before) : 0, 64);
-        mix[t] = ((in >> t) & 1) && (!before || prev / 4 != first / 4) ? first / 4 : -1;
-        const int groups = (int)__popcll(__builtin_amdgcn_ballot_w64(mix[t] >= 0));
-        if (m != 0 && t == 63 - __clzll((long long)m)) {
-            n_slots = s;
-            n_mix = groups;
-            left = room - sum;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(sum <= room);  // loads are not negative: true up to some class
+        const int last = m ? 63 - __clzll((long long)m) : -1;
+        const int64_t all = __shfl(sum, 63, 64), in = last >= 0 ? __shfl(sum, max(last, 0), 64) : 0;
+        if (t == 0) {
+            longest = last;
+            left = room - in;
+            ctr->n_need = (unsigned long long)(all - in);
         }
+        if (last == 63) first_slots();
+        else bin[t] = 0;
     }
     __syncthreads();
-    for (int32_t b = threadIdx.x; b < nq; b += PT) {
-        const int32_t t = qi[b].thr;
-        if (t < 0) continue;
-        if (at[t] < 0) { qi[b].thr = -1; continue; }
-        bin[t] = 0;
+    if (longest < 63) {  // uniform: some lists find no room
+        for (int32_t b = threadIdx.x; b < nq; b += PT) {
+            const int32_t t = qi[b].thr;
+            if (t < 0) continue;
+            if (length_class(qi[b].n_cand) <= longest) {
+                atomicAdd(&bin[t], 1);
+            } else {
+                qi[b].thr = kNoRoom;
+                if (b < PT) own_thr = kNoRoom;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < 64) first_slots();
+        __syncthreads();
     }
-    __syncthreads();
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
-        const int32_t t = qi[b].thr;
+        const int32_t t = b < PT ? own_thr : qi[b].thr;
         if (t < 0) continue;
         order[at[t] + atomicAdd(&bin[t], 1)] = b;
         if (!((coarse_mask >> t) & 1)) atomicAdd(&n_finer, 1);
@@ -311,15 +350,15 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
     __threadfence_block();
     __syncthreads();
     for (int32_t g = threadIdx.x; g < (n_slots + 3) / 4; g += PT) {
-        const int32_t c = qi[order[4 * g]].thr;
-        if (qi[order[min(4 * g + 3, n_slots - 1)]].thr == c) colg[g] = c;
+        const int32_t c = column_of(4 * g);
+        if (column_of(min(4 * g + 3, n_slots - 1)) == c) colg[g] = c;
     }
     // a thread per member of the mixed groups
     const int32_t g = threadIdx.x < 4 * GW ? mix[threadIdx.x >> 2] : -1;
     const int32_t slot = 4 * g + (int32_t)(threadIdx.x & 3);
     const bool member = g >= 0 && slot < n_slots;
     const int32_t b = member ? order[slot] : 0;
-    const int32_t own = member ? qi[b].thr : -1;
+    const int32_t own = member ? column_of(slot) : -1;
     // the group's columns: the largest, the next one below it, the smallest
     auto quad_max = [](int32_t x) {
         x = max(x, __shfl_xor(x, 1, 64));
@@ -360,7 +399,7 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
     if (member) {
         auto good = [&](int h) { return !over[h] && more[h] <= left / n_mix; };
         const int32_t c = !over[0] && added <= left ? c0 : good(0) ? c0 : good(1) ? c1 : least;
-        qi[b].thr = own <= c ? c : -1;
+        qi[b].thr = own <= c ? c : kNoRoom;
         if ((threadIdx.x & 3) == 0) colg[g] = c;
     }
     if (threadIdx.x == 0) {
@@ -378,6 +417,13 @@ __device__ __forceinline__ int64_t list_len(const ListCounters *ctr, int64_t cap
     return n <= cap ? n : 0;
 }
 
+// n places of the list, counted in 64 bits; past the list's capacity its end (32
+// bits hold it, cap <= INT32_MAX / 2), where nothing is written.
+__device__ __forceinline__ int32_t list_places(unsigned long long *list_n, int32_t n, int64_t cap) {
+    const unsigned long long first = atomicAdd(list_n, (unsigned long long)n);
+    return (int32_t)min(first, (unsigned long long)cap);
+}
+
 // Zeroes the list's counts per query and the scatter's cursors behind them.
 __device__ __forceinline__ void zero_counts(int32_t nq, uint32_t *__restrict__ g_cnt) {
     if (g_cnt && blockIdx.y == 0)
@@ -391,8 +437,7 @@ constexpr int kSlice = 512;
 
 struct ListQueue {
     uint2 e[QCAP];
-    int32_t n;
-    int64_t base;  // places are counted in 64 bits, also past the list's capacity
+    int32_t n, base;
 };
 
 // Appends each lane's pairs (bit 4 b + i of m: user u0 + 16 b, query slot_b[i])
@@ -415,10 +460,10 @@ __device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, 
     base = __shfl(base, 0, 64);
     int32_t p = base + x - c;
     // places at and past QCAP: the wavefront's share of the list
-    long long over = 0;
+    int32_t over = 0;
     if (base + tot > QCAP) {
         const int32_t first = max(base, QCAP);
-        if (lane == 0) over = (long long)atomicAdd(list_n, (unsigned long long)(base + tot - first));
+        if (lane == 0) over = list_places(list_n, base + tot - first, cap);
         over = __shfl(over, 0, 64) - first;
     }
     while (m) {
@@ -427,7 +472,7 @@ __device__ __forceinline__ void list_put(ListQueue &sq, uint32_t m, int32_t u0, 
         const int32_t u = u0 + (t >> 2) * 16, b = slot_b[t & 3];
         if (p < QCAP) {
             sq.e[p] = make_uint2((uint32_t)u, (uint32_t)b);
-        } else if (over + p < cap) {
+        } else if ((int64_t)over + p < cap) {
             cl_u[over + p] = u;
             cl_b[over + p] = b;
         }
@@ -441,7 +486,7 @@ __device__ __forceinline__ void list_flush(ListQueue &sq, int32_t *__restrict__ 
                                            int64_t cap, unsigned long long *__restrict__ list_n) {
     const int32_t n = min(sq.n, QCAP);
     if (n > 0) {  // uniform
-        if (threadIdx.x == 0) sq.base = (int64_t)atomicAdd(list_n, (unsigned long long)n);
+        if (threadIdx.x == 0) sq.base = list_places(list_n, n, cap);
         __syncthreads();
         const int64_t base = sq.base;
         for (int i = threadIdx.x; i < n; i += NT)
@@ -455,10 +500,10 @@ __device__ __forceinline__ void list_flush(ListQueue &sq, int32_t *__restrict__ 
 // their number in a register of every lane.
 constexpr int WQ = 256;
 
-__device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int64_t base, int32_t u0, const int32_t *ord,
+__device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int32_t base, int32_t u0, const int32_t *ord,
                                            int32_t *__restrict__ cl_u, int32_t *__restrict__ cl_b, int64_t cap) {
     for (int i = threadIdx.x & 63; i < n; i += 64)
-        if (base + i < cap) {
+        if ((int64_t)base + i < cap) {
             cl_u[base + i] = u0 + (int32_t)(q[i] & 0xFFu);
             cl_b[base + i] = ord[q[i] >> 8];
         }
@@ -490,8 +535,7 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
     __shared__ f32x4 sCs[kSlice / 4];
     __shared__ int32_t sCol[kSlice / 4 + QST / 4], sOrd[kSlice];
     __shared__ uint32_t sQ[NT / 64][WQ];
-    __shared__ int32_t sN[NT / 64];
-    __shared__ int64_t sBase;
+    __shared__ int32_t sN[NT / 64], sBase;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
     const int32_t n_slots = ctr->n_slots;
     zero_counts(P.nq, g_cnt);
@@ -590,8 +634,8 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
                             const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
                             if (m != 0) {
                                 if (n_q + 64 > WQ) {  // uniform: make room
-                                    long long base = 0;
-                                    if (lane == 0) base = (long long)atomicAdd(&ctr->n_list, (unsigned long long)n_q);
+                                    int32_t base = 0;
+                                    if (lane == 0) base = list_places(&ctr->n_list, n_q, list_cap);
                                     wave_flush(sQ[wave], n_q, __shfl(base, 0, 64), (int32_t)(rb * UB), sOrd, cl_u, cl_b,
                                                list_cap);
                                     n_q = 0;
@@ -621,7 +665,7 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
             tot += sN[w];
         }
         if (tot > 0) {  // uniform
-            if (threadIdx.x == 0) sBase = (int64_t)atomicAdd(&ctr->n_list, (unsigned long long)tot);
+            if (threadIdx.x == 0) sBase = list_places(&ctr->n_list, tot, list_cap);
             __syncthreads();
             wave_flush(sQ[wave], n_q, sBase + before, (int32_t)(rb * UB), sOrd, cl_u, cl_b, list_cap);
         }
@@ -973,8 +1017,8 @@ __device__ __forceinline__ void find_bin(const uint32_t *h, uint32_t before, uin
 // whole list of a few queries, skipping other queries' pairs): beta, the bucket
 // of the k-th smallest b_lo, then the candidates (b_hi <= beta) with their rank
 // when the bounds fix it, else ~(refine row).  A query with fewer than k buckets
-// up to its threshold, or a list that overflowed, gets thr = -1 and no
-// candidates: the full search answers it.
+// up to its threshold, or a list that overflowed, gets thr = -1 (a query that
+// found no room keeps kNoRoom) and no candidates: it is answered another way.
 //
 // Many candidates are users of bucket beta itself (an item that most of 100k
 // users rank first).  When that bucket fixes the rank, the answer takes the
@@ -1048,7 +1092,8 @@ __global__ void __launch_bounds__(FT) k_list_final(const int32_t *__restrict__ c
     }
     if (beta < 0) {  // uniform
         if (threadIdx.x == 0) {
-            qi[b].beta = qi[b].gamma = qi[b].thr = -1;
+            qi[b].beta = qi[b].gamma = -1;
+            if (q.thr != kNoRoom) qi[b].thr = -1;
             qi[b].n_cand = qi[b].n_dropped = qi[b].n_refine = qi[b].fill = qi[b].n_settled = 0;
             qi[b].cand_off = 0;
         }
@@ -1189,6 +1234,22 @@ __global__ void __launch_bounds__(NT) k_gather_guards(const float *__restrict__ 
     }
 }
 
+// Moves rows rows[0] < rows[1] < ... of x to rows 0, 1, ...: a thread per
+// column, eight rows read before any of their places is written (a later row's
+// source lies behind them, rows[i] >= i).
+__global__ void __launch_bounds__(NT) k_keep_rows(float *__restrict__ x, int64_t n_col, const int32_t *__restrict__ rows, int32_t n) {
+    const int64_t u = (int64_t)blockIdx.x * NT + threadIdx.x;
+    if (u >= n_col) return;
+    for (int32_t i = 0; i < n; i += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = x[(int64_t)rows[min(i + j, n - 1)] * n_col + u];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (i + j < n) x[(int64_t)(i + j) * n_col + u] = v[j];
+    }
+}
+
 bool fine_ok(const FineCols &fc, int64_t S) {
     if (fc.n < 1 || fc.n > kMaxFine) return false;
     for (int f = 0; f < fc.n; ++f)
@@ -1204,6 +1265,12 @@ hipError_t launch_gather_guards(hipStream_t s, const float *T, int64_t S, const 
     if ((fc.n > 0 && !fine_ok(fc, S)) || u0 + n_rows > pitch) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gather_guards, dim3((unsigned)((n_rows + 63) / 64)), dim3(NT), 0, s, T, S, fc, u0, n_rows, gv,
                        gc, pitch);
+    return hipGetLastError();
+}
+
+hipError_t launch_keep_rows(hipStream_t s, float *x, int64_t n_col, const int32_t *rows, int32_t n) {
+    if (n <= 0 || n_col <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_keep_rows, dim3((unsigned)((n_col + NT - 1) / NT)), dim3(NT), 0, s, x, n_col, rows, n);
     return hipGetLastError();
 }
 
@@ -1229,7 +1296,7 @@ hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L) {
     RKR_KS_SWITCH(L.Kp, RKR_SAMPLE_CASE)
 #undef RKR_SAMPLE_CASE
     hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
-                       L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
+                       L.room, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
     const int64_t ub = L.Kp <= 160 ? 256 : 128;
     const int64_t units = (L.n_user + ub - 1) / ub * ((L.nq + kSlice - 1) / kSlice);
     const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(units, (int64_t)L.n_cu * (L.Kp <= 160 ? 3 : 2))));
@@ -1252,7 +1319,7 @@ hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L) {
     hipLaunchKernelGGL(k_sample_scores, dim3(gx, qg), dim3(NT), 0, s, L.qip, L.n_user, L.nq, L.eps, L.gvals, L.fc.n,
                        n_s, L.stride, L.hist, L.t_bound);
     hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
-                       L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
+                       L.room, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
     hipLaunchKernelGGL(k_list_scores,
                        dim3((unsigned)((L.n_user + NT - 1) / NT), (unsigned)((L.nq + kScoreSlice - 1) / kScoreSlice)),
                        dim3(NT), 0, s, L.qip, L.n_user, L.eps, L.gcols, L.pitch, L.order, L.colg, L.nq, L.g_cnt, L.ctr,

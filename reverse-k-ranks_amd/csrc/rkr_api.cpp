@@ -1434,14 +1434,38 @@ int64_t list_entries(int64_t U, int64_t nq) {
     return std::min<int64_t>({std::max<int64_t>(nq * per, 2 * std::max<int64_t>(4096, U / 4)), nq * U, INT32_MAX / 2});
 }
 
-// Device batches of query_on_slot.  allow_list: exact batches take the
-// threshold lists (k_list.hip), or, with updates pending, the coarse bounds;
-// queries those cannot answer (no threshold, a list too long or too short) are
-// appended to *fallback (indices into queries) with their outputs left
-// unwritten.
+// How a set of queries is answered.
+struct Attempt {
+    bool lists = true;            // threshold lists (k_list.hip), or with updates pending the coarse bounds
+    int64_t entries = 0;          // list entries to make room for, beyond the usual
+    const int32_t *rows = nullptr;  // the queries' exact scores are these rows of the slot's scores (ascending)
+};
+// What run_batches left open.
+struct Outcome {
+    struct Open { int32_t query; bool room; };  // room: its list only found no room
+    std::vector<Open> open;       // outputs unwritten
+    int64_t need = 0;             // pairs of the lists that found no room, as estimated
+    int64_t entries = 0;          // list entries there were
+    bool lists = false;           // the queries went through lists or the coarse bounds
+    bool scores = false;          // the slot holds every query's exact scores, row i the i-th query's
+};
+
+// The longest list of a batch of n queries that is faster than its share of a
+// search over every user, which takes 4 ms and 20 us a query at 1M users; a
+// listed pair takes 0.25 ns from matrix-core scores, 0.5 from exact ones (they
+// are read twice), up to 1 in short lists.  So a quarter of all users for a few
+// queries (4 queries, 260k pairs: 0.41 ms, searched 4.6), a tenth or a twentieth
+// of them for many (1M users x 1000 queries, 8% of all pairs: 24 ms screened,
+// searched 29; 45 plain, searched 31).
+int64_t list_pairs_max(int64_t U, int64_t n, bool screened) {
+    return std::min(std::max<int64_t>(4096, U / 4), std::max<int64_t>(4096, 12 * U / n + U / (screened ? 12 : 24)));
+}
+
+// Device batches of query_on_slot.  Queries that the attempt cannot answer (no
+// threshold, a list too long or too short) go to out.open.
 int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int32_t n_query, const int32_t *topk,
                 int32_t max_k, int32_t *out_user, int32_t *out_rank, float *out_qip, rkr_query_stats *stats,
-                rkr_batch_timing &tm, bool allow_list, std::vector<int32_t> *fallback) {
+                rkr_batch_timing &tm, const Attempt &how, Outcome &out) {
     const int64_t U = dv.n_user, I = dv.n_item;
     const int32_t ld = c->ld, d = c->dim;
     const int mode = c->output;
@@ -1458,7 +1482,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // the QSRP screen (RKR_OPT_QSRP, built by rkr_qsrp_build) replaces the bound
     // stage of exact batches without pending updates
     const bool qsrp = c->qsrp && dv.qsrp_users && mode == RKR_OUTPUT_EXACT && !upd && U > 0;
-    const bool listable = !qsrp && allow_list && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
+    const bool listable = !qsrp && how.lists && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
                           dv.guards.n > 0 && U > 0;
     const bool mfma = screened && c->kp > 0 && dv.user_norm;
     const size_t pair_bytes = upd ? 12 : 8;  // <u,q> + buckets, or + two bound values
@@ -1479,6 +1503,10 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     const bool list = listable && !upd &&
                       (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
     const bool list_mfma = list && mfma;
+    // scores left by the last attempt, of this attempt's queries
+    const bool scored = how.rows && !list_mfma && !upd && !qsrp && n_query <= nqb;
+    out.lists = list || (listable && upd);
+    out.scores = list && !list_mfma && n_query <= nqb;
     // a few users: bounds to candidates in one kernel, its arrays sized for
     // every pair (6 MB at most)
     const bool small = !list && !upd && !qsrp && mode == RKR_OUTPUT_EXACT && U <= kSmallUsers && nqb * U <= (1 << 18);
@@ -1511,13 +1539,16 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     const std::vector<int32_t> &hrk = *dv.hrk;
     const GuardCols &gc = dv.guards;
     // an (estimated) list longer than list_max takes the full path instead
-    const int64_t list_max = std::max<int64_t>(4096, U / 4);
+    const int64_t list_max = list ? list_pairs_max(U, nqb, list_mfma) : std::max<int64_t>(4096, U / 4);
     int64_t list_cap = 0;
     if (list) {
         // what is held already, or what a quarter of the free budget allows
         const int64_t avail = (int64_t)((c->budget > c->held ? c->budget - c->held : 0) / 4);
-        const int64_t have = (int64_t)std::min({sl.list.bytes / 12, sl.cand.bytes / 8, sl.refine_idx.bytes / 16});
-        list_cap = std::min<int64_t>(list_entries(U, nqb), std::max<int64_t>({have, avail / kListBytes, 1}));
+        const int64_t have = std::min<int64_t>({(int64_t)sl.list.bytes / 12, (int64_t)sl.cand.bytes / 8,
+                                                (int64_t)sl.refine_idx.bytes / 16, nqb * U, INT32_MAX / 2});
+        const int64_t want = std::max(list_entries(U, nqb), std::min<int64_t>({how.entries, nqb * U, INT32_MAX / 2}));
+        list_cap = std::max<int64_t>({have, std::min(want, avail / kListBytes), 1});
+        out.entries = list_cap;
         if ((rc = ensure(c, sl.list, 12 * (size_t)list_cap, "listed pairs")) ||
             (rc = ensure(c, sl.list_info, sizeof(uint32_t) * (66 * (size_t)nqb + 64), "list thresholds")) ||
             (rc = ensure(c, sl.cand, sizeof(int32_t) * 2 * (size_t)list_cap, "candidates")) ||
@@ -1531,6 +1562,18 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     char *stg = reinterpret_cast<char *>(sl.stage.p);
     int32_t *hcq = reinterpret_cast<int32_t *>(stg + stage_io);
     int32_t *hhc = hcq + 4 * (size_t)nqb;
+    if (scored) {  // to the front, where a row is not already (the list of rows on its way through the histograms)
+        int32_t first = 0;
+        while (first < n_query && how.rows[first] == first) ++first;
+        const int32_t n = n_query - first;
+        if (n > 0) {
+            for (int32_t i = 0; i < n; ++i) hcq[i] = how.rows[first + i] - first;
+            RKR_HIP(c, hipMemcpyAsync(sl.hist.p, hcq, sizeof(int32_t) * n, hipMemcpyHostToDevice, sl.stream));
+            RKR_HIP(c, launch_keep_rows(sl.stream, reinterpret_cast<float *>(sl.qip.p) + (size_t)first * U, U,
+                                        reinterpret_cast<const int32_t *>(sl.hist.p), n));
+            RKR_HIP(c, hipStreamSynchronize(sl.stream));  // the staging is the batch's again
+        }
+    }
 
     for (int64_t q0 = 0; q0 < n_query; q0 += nqb) {
         const int32_t nq = (int32_t)std::min<int64_t>(nqb, n_query - q0);
@@ -1547,7 +1590,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         int32_t *refine_total = &ctr->n_refine;
         uint64_t *const t = use_ev ? nullptr : ctr->t;  // stage stamps
         // few users and queries: the scores' kernel also searches the table
-        uint32_t *const small_bk = small && nq <= 16 && eps == 0.0f ? reinterpret_cast<uint32_t *>(sl.bk.p) : nullptr;
+        uint32_t *const small_bk = small && nq <= 16 && eps == 0.0f && !scored ? reinterpret_cast<uint32_t *>(sl.bk.p) : nullptr;
         uint64_t *t_up = reinterpret_cast<uint64_t *>(hcq);  // when the direct upload began
         auto at = [t](int i) { return t ? t + i : nullptr; };
         auto event = [&](int i) { return use_ev ? hipEventRecord(sl.ev[i], sl.stream) : hipSuccess; };
@@ -1605,6 +1648,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             LL.user_hi = dv.user_hi; LL.user_norm = dv.user_norm; LL.gvals = dv.gvals; LL.gcols = dv.gcols; LL.pitch = dv.gpitch;
             LL.q_hi = q_hi; LL.q_cs = qcs; LL.fc = dv.fine; LL.C = est_C; LL.floor = est_floor; LL.eps = eps;
             LL.qip = qip; LL.stride = sample_stride(U); LL.cap = list_max; LL.list_cap = list_cap;
+            LL.room = list_cap / 2;  // the estimates may be half of what comes
             LL.hist = reinterpret_cast<uint32_t *>(sl.list_info.p);
             LL.order = reinterpret_cast<int32_t *>(LL.hist + 64 * (size_t)nq);
             LL.colg = LL.order + nq;
@@ -1686,8 +1730,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                     e[1] = (int32_t)std::min<int64_t>(n, INT32_MAX);
                 }
                 if (e[0] < 0 || e[1] > list_max) {
-                    if (fallback) fallback->push_back((int32_t)(q0 + i));
-                    tm.n_fallback += 1;
+                    out.open.push_back({(int32_t)(q0 + i), false});
                     e[0] = -1;
                     e[1] = 0;
                 }
@@ -1736,9 +1779,9 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             RKR_HIP(c, launch_hist_kth(sl.stream, bk, U, S, R, I, nq, mode, 0, cu, ghist, qi));
         } else {
             // <u, q> for every (query, user): qip[b * U + u]
-            if (nq <= 16)
+            if (!scored && nq <= 16)
                 RKR_HIP(c, launch_gemv_panels(sl.stream, dv.usersT, U, ld, d, q_in, nq, qip, T, S, small_bk, at(kTimeIp)));
-            else RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false, at(kTimeIp)));
+            else if (!scored) RKR_HIP(c, launch_scores_store(sl.stream, dv.users, U, ld, q_in, nq, ld, d, qip, U, false, at(kTimeIp)));
             RKR_HIP(c, event(2));
             if (list) {
                 if (!direct) RKR_HIP(c, hipMemsetAsync(LL.hist, 0, sizeof(uint32_t) * 64 * (size_t)nq, sl.stream));
@@ -1777,10 +1820,8 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             // L (QueryInfo.gamma of the value selection) is below that
             const int64_t floor_rank = (int64_t)hrk[gc.col[gc.n - 1]] + 1 - dv.n_del;
             for (int32_t i : deep_check)
-                if (hcq[(size_t)i * 4] >= 0 && (int64_t)hqi[i].gamma >= floor_rank) {
-                    if (fallback) fallback->push_back((int32_t)(q0 + i));
-                    tm.n_fallback += 1;
-                }
+                if (hcq[(size_t)i * 4] >= 0 && (int64_t)hqi[i].gamma >= floor_rank)
+                    out.open.push_back({(int32_t)(q0 + i), false});
         }
         if (total >= INT32_MAX) return set_err(c, RKR_ERR_NOMEM, "query: candidate count exceeds 2^31; lower the query batch");
         const size_t cap = (size_t)std::max<int64_t>(total, 1);
@@ -1872,10 +1913,8 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         }
         if (list) {
             for (int32_t i = 0; i < nq; ++i)
-                if (hqi[i].thr < 0) {
-                    if (fallback) fallback->push_back((int32_t)(q0 + i));
-                    tm.n_fallback += 1;
-                }
+                if (hqi[i].thr < 0) out.open.push_back({(int32_t)(q0 + i), hqi[i].thr == kNoRoom});
+            out.need += (int64_t)hctr->n_need;
             if ((int64_t)hctr->n_list <= list_cap) tm.n_listed += (int64_t)hctr->n_list;  // else no stage read the list
             tm.n_coarse_refined += hctr->n_finer;
         }
@@ -1925,7 +1964,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                 for (int32_t i = 0; i < nq; ++i) end = std::max(end, (uint32_t)hqi[i].pad - (uint32_t)ts[kTimeTopk]);
                 ts[kTimeEnd] = ts[kTimeTopk] + end;
             }
-            for (int i = kTimeEnd - 1; i > 0; --i)
+            for (int i = kTimeEnd - 1; i >= 0; --i)
                 if (ts[i] == 0) ts[i] = ts[i + 1];
             auto ms = [&](int i) { return ts[i + 1] > ts[i] ? (double)(ts[i + 1] - ts[i]) / c->clock_khz : 0.0; };
             tm.ip_ms += ms(kTimeIp);
@@ -1956,40 +1995,76 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
 
 }  // namespace
 
+namespace {
+
+// Answers n queries by one attempt, and what it leaves open by others: lists
+// that only found no room once more with more of it, the rest by a search over
+// every user.
+int answer(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int32_t n, const int32_t *topk, int32_t max_k,
+           int32_t *out_user, int32_t *out_rank, float *out_qip, rkr_query_stats *stats, rkr_batch_timing &tm,
+           const Attempt &how) {
+    Outcome o;
+    int rc = run_batches(c, sl, dv, queries, n, topk, max_k, out_user, out_rank, out_qip, stats, tm, how, o);
+    if (rc || o.open.empty()) return rc;
+    // n queries' lists get one more attempt, if they are not all of this one's
+    // or there can be more room
+    auto order = [](const Outcome::Open &x, const Outcome::Open &y) { return x.query < y.query; };
+    std::sort(o.open.begin(), o.open.end(), order);
+    const int64_t n_open = (int64_t)o.open.size();
+    int64_t n_room = 0;
+    for (const auto &x : o.open) n_room += x.room;
+    Attempt more = how;
+    more.entries = std::max<int64_t>(1, 2 * (o.need + o.need / 8));
+    const bool again = how.entries == 0 && n_room > 0 && (n_room < n || more.entries > o.entries);
+    Attempt search;
+    search.lists = false;
+    // the larger part first: it finds its scores where they are, and they are gone then
+    const bool lists_first = again && 2 * n_room >= n_open;
+    bool scores = o.scores;
+    for (const bool lists : {lists_first, !lists_first}) {
+        std::vector<int32_t> idx;
+        for (const auto &x : o.open)
+            if ((again && x.room) == lists) idx.push_back(x.query);
+        const int32_t m = (int32_t)idx.size(), d = c->dim;
+        if (m == 0) continue;
+        if (!lists) tm.n_fallback += m;
+        std::vector<float> q((size_t)m * d), qip((size_t)m * max_k);
+        std::vector<int32_t> k((size_t)m), u((size_t)m * max_k), r((size_t)m * max_k);
+        std::vector<rkr_query_stats> st(stats ? (size_t)m : 0);
+        for (int32_t i = 0; i < m; ++i) {
+            std::memcpy(&q[(size_t)i * d], queries + (size_t)idx[i] * d, sizeof(float) * d);
+            k[i] = topk[idx[i]];
+        }
+        Attempt next = lists ? more : search;
+        next.rows = scores ? idx.data() : nullptr;
+        scores = false;
+        rc = answer(c, sl, dv, q.data(), m, k.data(), max_k, u.data(), r.data(), qip.data(), stats ? st.data() : nullptr,
+                    tm, next);
+        if (rc) return rc;
+        for (int32_t i = 0; i < m; ++i) {
+            const size_t to = (size_t)idx[i] * max_k, from = (size_t)i * max_k;
+            std::memcpy(out_user + to, &u[from], sizeof(int32_t) * max_k);
+            std::memcpy(out_rank + to, &r[from], sizeof(int32_t) * max_k);
+            if (out_qip) std::memcpy(out_qip + to, &qip[from], sizeof(float) * max_k);
+            if (stats) {
+                stats[idx[i]] = st[i];
+                stats[idx[i]].query_id = idx[i];
+            }
+        }
+    }
+    return RKR_OK;
+}
+
+}  // namespace
+
 int query_on_slot(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int32_t n_query, const int32_t *topk,
                   int32_t max_k, int32_t *out_user, int32_t *out_rank, float *out_qip, rkr_query_stats *stats,
                   rkr_batch_timing *timing) {
     using clock = std::chrono::steady_clock;
     const auto t_start = clock::now();
     rkr_batch_timing tm{};
-    std::vector<int32_t> fb;
-    int rc = run_batches(c, sl, dv, queries, n_query, topk, max_k, out_user, out_rank, out_qip, stats, tm, true, &fb);
+    const int rc = answer(c, sl, dv, queries, n_query, topk, max_k, out_user, out_rank, out_qip, stats, tm, Attempt{});
     if (rc) return rc;
-    if (!fb.empty()) {
-        // queries the coarse bounds could not narrow enough: full path
-        const int32_t n = (int32_t)fb.size(), d = c->dim;
-        std::vector<float> fq((size_t)n * d);
-        std::vector<int32_t> fk(n), fu((size_t)n * max_k), fr((size_t)n * max_k);
-        std::vector<float> fqip((size_t)n * max_k);
-        std::vector<rkr_query_stats> fs(stats ? n : 0);
-        for (int32_t i = 0; i < n; ++i) {
-            std::memcpy(&fq[(size_t)i * d], queries + (size_t)fb[i] * d, sizeof(float) * d);
-            fk[i] = topk[fb[i]];
-        }
-        rc = run_batches(c, sl, dv, fq.data(), n, fk.data(), max_k, fu.data(), fr.data(), fqip.data(),
-                         stats ? fs.data() : nullptr, tm, false, nullptr);
-        if (rc) return rc;
-        for (int32_t i = 0; i < n; ++i) {
-            const size_t o = (size_t)fb[i] * max_k, f = (size_t)i * max_k;
-            std::memcpy(out_user + o, &fu[f], sizeof(int32_t) * max_k);
-            std::memcpy(out_rank + o, &fr[f], sizeof(int32_t) * max_k);
-            if (out_qip) std::memcpy(out_qip + o, &fqip[f], sizeof(float) * max_k);
-            if (stats) {
-                stats[fb[i]] = fs[i];
-                stats[fb[i]].query_id = fb[i];
-            }
-        }
-    }
     tm.total_ms = std::chrono::duration<double, std::milli>(clock::now() - t_start).count();
     if (timing) *timing = tm;
     return RKR_OK;

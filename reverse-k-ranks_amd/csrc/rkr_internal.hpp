@@ -474,9 +474,11 @@ struct QueryInfo {          // one per query of a device batch
     int32_t fill;           // candidates written so far (chunked compaction)
     int32_t n_screen;       // users a screen kept and scored exactly (QSRP)
     int64_t cand_off;       // offset of this query's candidates
-    int32_t thr;            // fine column of the query's list, -1: the full search answers it
+    int32_t thr;            // fine column of the query's list; -1: no list answers it, kNoRoom: its list did not fit
     int32_t n_dropped;      // candidates counted but not written: the answer cannot hold them
 };
+
+constexpr int32_t kNoRoom = -2;
 
 // Counters of a device batch, uploaded as zeros with the queries and read back
 // with the outputs.
@@ -490,6 +492,7 @@ struct alignas(64) ListCounters {
     int32_t pad[2];
     unsigned long long n_list;  // listed pairs, past the list's capacity when it overflowed: up to
                                 // every pair of the batch, which nothing keeps below 2^32
+    unsigned long long n_need;  // estimated pairs of the lists that found no room
     uint64_t t[8];          // device clock at the stages' starts (enum below)
 };
 // Stages of a batch timed by its kernels: the first kernel of a stage writes
@@ -555,6 +558,7 @@ struct ListLaunch {
     int64_t stride;          // one user of every stride is sampled
     int64_t cap;             // a longer estimated list takes the full search
     int64_t list_cap;        // entries of the lists
+    int64_t room;            // pairs that the estimated lists may hold
     uint32_t *hist;          // nq x 64, zeroed
     int32_t *order, *colg;   // nq slots, nq / 4 threshold columns
     QueryInfo *qi;
@@ -580,6 +584,9 @@ hipError_t launch_list_exact(hipStream_t s, const ListLaunch &L, const float *us
 hipError_t launch_list_final(hipStream_t s, const ListLaunch &L, const uint32_t *bk_c, const int32_t *ranks,
                              int64_t n_item, int32_t *cand_user, int32_t *cand_rank, int32_t *refine_user,
                              int32_t *refine_query, float *refine_thr, int32_t *cnt);
+
+// Rows rows[0] < rows[1] < ... (device) of x, of n_col floats each, to rows 0 .. n - 1.
+hipError_t launch_keep_rows(hipStream_t s, float *x, int64_t n_col, const int32_t *rows, int32_t n);
 
 // Table rows staged per workgroup by the batched bounds kernels: 16 rows of
 // S + 1 floats (<= 32 KB at S = 511), fewer for long rows; 0 when one row

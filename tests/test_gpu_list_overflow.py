@@ -33,7 +33,7 @@ def test_list_overflow(gpu_index_factory, form, nq):
     ordered by query, after a larger batch whose pairs the arrays still hold."""
     _case(f"list overflow {form} nq={nq}")
     rng = np.random.default_rng(nq)
-    U, I, d = 70_001, 800, 16
+    U, I, d = 200_001, 800, 16
     items = rng.standard_normal((I, d), dtype=np.float32)
     users = items[7] + np.float32(0.02) * rng.standard_normal((U, d), dtype=np.float32)
     at = _sampled(U)
@@ -41,7 +41,7 @@ def test_list_overflow(gpu_index_factory, form, nq):
     queries = items[7] + np.float32(1e-3) * rng.standard_normal((nq, d), dtype=np.float32)
     idx, _ = gpu_index_factory(users, items, 48)
     idx.set_form(form)
-    before = idx.query(rng.standard_normal((700, d), dtype=np.float32), 10)
+    before = idx.query(rng.standard_normal((280, d), dtype=np.float32), 10)  # leaves room for 1.1M pairs
     assert before.timing["n_listed"] > 0
     ks = [int(k) for k in rng.integers(1, 50, nq)]
     got = idx.query(queries, ks)
@@ -121,4 +121,34 @@ def test_one_deep_query_among_ordinary_ones(gpu_index_factory, form, scale):
     assert got.timing["n_listed"] > 0 and got.timing["n_fallback"] <= 1
     idx.set_option(9, 0)  # RKR_OPT_COARSE
     _same_answers(got, idx.query(queries, ks), ks)
+    idx.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+@pytest.mark.parametrize("deep,popular", [(5, 60), (60, 5), (0, 200), (200, 0), (70, 70)])
+def test_batches_that_do_not_fit_at_once(gpu_index_factory, form, deep, popular):
+    """Popular queries whose lists find no room at first, short ones that no
+    list answers and ordinary ones, in one batch: each is answered on its own
+    terms, also when the same batch comes again and finds the room there."""
+    _case(f"{deep} deep and {popular} popular queries of 200, {form}")
+    rng = np.random.default_rng(deep + popular)
+    U, I, d, nq = 70_001, 800, 16, 200
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal((I, d), dtype=np.float32)
+    queries = items[rng.choice(I, nq, replace=False)].copy()
+    at = rng.permutation(nq)
+    queries[at[:deep]] *= np.float32(0.003)
+    queries[at[deep:deep + popular]] *= np.float32(1.7)
+    ks = [int(k) for k in rng.integers(1, 60, nq)]
+    idx, _ = gpu_index_factory(users, items, 48)
+    idx.set_form(form)
+    got = [idx.query(queries, ks) for _ in range(2)]
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    want = idx.query(queries, ks)
+    for g in got:
+        print({f: g.timing[f] for f in ("n_batches", "n_listed", "n_fallback")}, flush=True)
+        _same_answers(g, want, ks)
+        for f in ("n_candidate", "n_refine_user", "n_prune_user", "n_result_user", "query_id"):
+            assert [s[f] for s in g.stats] == [s[f] for s in want.stats], f
+        assert g.timing["n_fallback"] <= deep + popular // 20  # a list can be too long for a batch of 200
     idx.close()
