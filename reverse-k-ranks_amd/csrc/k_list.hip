@@ -21,7 +21,12 @@
 //
 // Scores come either from the matrix cores (screened form: one BF16 product,
 // |s^ - s| <= e = ||u|| cs(q) + floor, see k_screen.hip) or from the exact
-// scores of the batch (plain form, e = eps of an installed table).
+// scores of the batch (plain form, e = eps of an installed table).  Where the
+// items' scores lie closer together than the one product's error tells apart
+// (items that share a large common part), a query is attempted again with three
+// products of the high and low halves, an error 33 times smaller, and then with
+// exact scores.  1M users x 1000 queries, items = mean + noise of 5%, 3% and 1% of
+// it: 29, 47 and 50 ms with one product for all, now 2.3 each.
 #include "rkr_internal.hpp"
 
 namespace rkr {
@@ -105,38 +110,48 @@ __device__ __forceinline__ int guard_pos_reg(const float (&hd)[7], const float *
 
 // ---- sample ----------------------------------------------------------------
 // hist[b * 64 + p] += #{sampled users with p fine columns above s - e}, p <
-// n_fine.  A workgroup takes one stage of 64 queries (blockIdx.y) and every
-// gridDim.x-th block of 128 sampled users, so its counts leave LDS once.
-// Queries are the A operand, users the B operand: lane (lr, lq) of a 16 x 16
-// block owns user lr and queries 4 lq .. 4 lq + 3.
-template <int KS>
-__global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScreen P, int64_t n_s, int64_t stride,
+// n_fine, and in the bits from kPossible up the same for s + e, from one pair in
+// kPossibleOf: the first says which column enough users reach for certain, both
+// together how many users the list at that column holds.  (With a search of its
+// own for s + e in every pair the sample takes twice as long.)  A workgroup takes
+// one stage of 64 queries (blockIdx.y) and every gridDim.x-th block of 128
+// sampled users, so its counts leave LDS once.  Queries are the A operand, users
+// the B operand: lane (lr, lq) of a 16 x 16 block owns user lr and queries
+// 4 lq .. 4 lq + 3.  PROD: one product u_hi q_hi, or three with the low halves.
+constexpr int kPossible = 18, kPossibleOf = 32;  // n_s < 2^17: 18 bits hold a certain count, 14 a possible one
+template <int KS, int PROD>
+__global__ void __launch_bounds__(NT, PROD == 1 && KS <= 7 ? 2 : 1) k_sample_screen(ListScreen P, int64_t n_s, int64_t stride,
                                                          int64_t n_user, uint32_t *__restrict__ hist) {
-    constexpr int ROWQ = (KS * 32 + KPAD_LDS) / 8, KQ = KS * 4;
-    __shared__ u32x4 sA[QST * ROWQ];
+    constexpr int ROWQ = (KS * 32 + KPAD_LDS) / 8, KQ = KS * 4, NH = PROD == 1 ? 1 : 2;
+    __shared__ u32x4 sA[NH][QST * ROWQ];
     __shared__ float sCs[QST];
     __shared__ float sG[128 * GP];
     __shared__ uint32_t sH[QST * GW];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
     const int32_t q0 = (int32_t)blockIdx.y * QST;
-    u32x4 pre[KS];
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-        const int c = (int)threadIdx.x + k * NT;
-        pre[k] = reinterpret_cast<const u32x4 *>(P.q_hi)[(int64_t)min(q0 + c / KQ, P.nq - 1) * KQ + c % KQ];
-    }
+    for (int h = 0; h < NH; ++h) {
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(h ? P.q_lo : P.q_hi);
+        u32x4 pre[KS];
 #pragma unroll
-    for (int k = 0; k < KS; ++k) {
-        const int c = (int)threadIdx.x + k * NT;
-        sA[(c / KQ) * ROWQ + c % KQ] = pre[k];
+        for (int k = 0; k < KS; ++k) {
+            const int c = (int)threadIdx.x + k * NT;
+            pre[k] = src[(int64_t)min(q0 + c / KQ, P.nq - 1) * KQ + c % KQ];
+        }
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            const int c = (int)threadIdx.x + k * NT;
+            sA[h][(c / KQ) * ROWQ + c % KQ] = pre[k];
+        }
     }
     if (threadIdx.x < QST) sCs[threadIdx.x] = P.q_cs[min(q0 + (int)threadIdx.x, P.nq - 1)];
     for (int i = threadIdx.x; i < QST * GW; i += NT) sH[i] = 0u;
     const int64_t n_rb = (n_s + 127) / 128;
-    for (int64_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x) {
+    uint32_t turn = blockIdx.x;  // which of a block's pairs are searched for s + e too
+    for (int64_t rb = blockIdx.x; rb < n_rb; rb += gridDim.x, turn += gridDim.x + 1) {
         __syncthreads();  // the previous block is done with sG
         stage_guards<128>(sG, P.gvals, rb * 128, n_s, stride, n_user);
-        Frag uh[2][KS];
+        Frag uh[2][KS], ul[PROD == 1 ? 1 : 2][PROD == 1 ? 1 : KS];
         float ar[2];
         bool live[2];
 #pragma unroll
@@ -146,6 +161,9 @@ __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScree
             const int64_t u = sample_user(min(r, n_s - 1), stride, n_user);
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) uh[b][ks].q = reinterpret_cast<const u32x4 *>(P.user_hi + u * P.Kp)[ks * 4 + lq];
+            if constexpr (PROD > 1)
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) ul[b][ks].q = reinterpret_cast<const u32x4 *>(P.user_lo + u * P.Kp)[ks * 4 + lq];
             ar[b] = P.C * P.user_norm[u];
         }
         __syncthreads();
@@ -160,9 +178,17 @@ __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScree
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 Frag qh;
-                qh.q = sA[(g * 16 + lr) * ROWQ + ks * 4 + lq];
+                qh.q = sA[0][(g * 16 + lr) * ROWQ + ks * 4 + lq];
+                [[maybe_unused]] Frag ql;
+                if constexpr (PROD > 1) ql.q = sA[NH - 1][(g * 16 + lr) * ROWQ + ks * 4 + lq];
 #pragma unroll
-                for (int b = 0; b < 2; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                for (int b = 0; b < 2; ++b) {
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                    if constexpr (PROD > 1) {
+                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, ul[b][ks].v, acc[b], 0, 0, 0);
+                    }
+                }
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -171,9 +197,21 @@ __global__ void __launch_bounds__(NT, KS <= 7 ? 2 : 1) k_sample_screen(ListScree
 #pragma unroll
                 for (int b = 0; b < 2; ++b) {
                     const float e = __fmaf_rn(ar[b], cs, P.floor);
-                    const int p = guard_pos_reg(hd[b], &sG[(wave * 32 + b * 16 + lr) * GP], acc[b][i] - e);
+                    const float *row = &sG[(wave * 32 + b * 16 + lr) * GP];
+                    const int p = guard_pos_reg(hd[b], row, acc[b][i] - e);
                     if (live[b] && p < P.n_fine) atomicAdd(&sH[ql * GW + p], 1u);
                 }
+            }
+            if (g == (int)(turn & 3)) {  // uniform, as is the next: one search a block, so no workgroup has more
+                static_assert(kPossibleOf == 4 * 8, "one of 8 pairs of one of 4 groups of queries");
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if ((int)(turn >> 2 & 7) == j) {
+                        const int b = j >> 2, ql = g * 16 + 4 * lq + (j & 3);
+                        const float e = __fmaf_rn(ar[b], sCs[ql], P.floor);
+                        const int p = guard_pos_reg(hd[b], &sG[(wave * 32 + b * 16 + lr) * GP], acc[b][j & 3] + e);
+                        if (live[b] && p < P.n_fine) atomicAdd(&sH[ql * GW + p], 1u << kPossible);
+                    }
             }
         }
     }
@@ -216,28 +254,41 @@ __global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ 
 // One workgroup.  Each query's threshold column, the queries ordered by it
 // (slot -> query), and for every four neighbouring slots the column they share,
 // the largest of theirs (a larger column lists more users, never fewer).  A
-// query with no such column or with an estimated list over cap gets thr = -1 (a
-// search over every user answers it) and no slot.  Lists are taken in order of
+// query with no such column, or with a list that the scores' error takes past
+// cap, gets thr = -1 (finer scores answer it) and no slot, one whose list is over
+// cap without the error kNoList (a search over every user answers it).  So
+// do the queries whose lists the scores' error makes more than `band` pairs
+// longer, and those whose lists are longer than `share`, if that is enough in all
+// to pay for what another attempt costs however few its queries: kBandMin pairs,
+// the 80 us of a pass from finer scores, or kSearchUsers pairs a user, the
+// search's 4 ms at 1M users (nothing if some query is searched anyway).  Lists are taken in order of
 // their length, up to `room` pairs; the longer ones get thr = kNoRoom and
 // ctr->n_need says how many pairs they hold.  (Taken in order of their column,
 // popular queries came first and one of them kept every other out.)
 // Four slots of different columns are estimated again at the shared one: a query
 // that few users rank high can make three others list most users.  Where such a
-// list is over cap, or what all of them add does not fit and the four take more
-// than an equal share of the room, they keep a smaller one of their columns and
-// the deeper queries get thr = kNoRoom.
+// list is over cap, or what all of them add does not fit the arrays and the four
+// take more than an equal share of what is left of them, they keep a smaller one
+// of their columns and the deeper queries get thr = kNoRoom.
 constexpr int PT = 1024;
+constexpr int64_t kBandMin = 400000, kSearchUsers = 12;
 
 __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ hist, int32_t nq, int32_t n_fine,
-                                                  int64_t stride, int64_t n_user, int64_t cap, int64_t room,
-                                                  uint64_t coarse_mask, QueryInfo *__restrict__ qi,
+                                                  int64_t stride, int64_t n_user, int64_t cap, int64_t share,
+                                                  int64_t band, int64_t room, int64_t list_cap, uint64_t coarse_mask, QueryInfo *__restrict__ qi,
                                                   int32_t *__restrict__ order, int32_t *__restrict__ colg,
                                                   ListCounters *__restrict__ ctr) {
     __shared__ int32_t bin[GW], at[GW], mix[GW];
     __shared__ int64_t load[GW];  // pairs of the lists of each length class
+    __shared__ int64_t longer[2];  // pairs that the scores' error adds to lists it makes `band` longer; past `share`
     __shared__ int64_t left, added;  // room beside the lists at their own columns, and what sharing adds
-    __shared__ int32_t n_finer, n_slots, n_mix, longest;
-    auto estimate = [&](int64_t sampled) { return min(sampled * stride, n_user); };
+    __shared__ int32_t n_finer, n_slots, n_mix, longest, searched;
+    // pairs of a list that `certain` sampled users reach for certain, and so many
+    // of the few searched for it possibly
+    constexpr uint32_t kCertain = (1u << kPossible) - 1;
+    auto estimate = [&](int64_t certain, int64_t possible) {
+        return min(max(certain, possible * kPossibleOf) * stride, n_user);
+    };
     // two length classes an octave
     auto length_class = [](int32_t n) {
         const int top = 31 - __clz(max(n, 1));
@@ -275,7 +326,7 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
         return t;
     };
     for (int i = threadIdx.x; i < GW; i += PT) { bin[i] = 0; load[i] = 0; }
-    if (threadIdx.x == 0) n_finer = n_slots = n_mix = longest = 0, left = added = 0;
+    if (threadIdx.x == 0) n_finer = n_slots = n_mix = longest = searched = 0, longer[0] = longer[1] = left = added = 0;
     __syncthreads();
     int32_t own_thr = -1;  // of the thread's first query, which then needs no reading back
     for (int32_t b = threadIdx.x; b < nq; b += PT) {
@@ -284,27 +335,60 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
         u32x4 v[GW / 4];
 #pragma unroll
         for (int j = 0; j < GW / 4; ++j) v[j] = reinterpret_cast<const u32x4 *>(hist + (int64_t)b * GW)[j];
-        const int64_t k = qi[b].topk;
+        const int32_t k = qi[b].topk;
         const double mean = (double)k / (double)stride;
-        const int64_t want = stride == 1 ? k : (int64_t)(mean + 3.0 * sqrt(mean) + 4.0) + 1;
-        int32_t t = -1;
-        int64_t cum = 0, n = 0;
+        const uint32_t want = stride == 1 ? (uint32_t)k : (uint32_t)(mean + 3.0 * sqrt(mean) + 4.0) + 1u;
+        // the sums grow with the column: the first one that reaches `want` is the
+        // smallest that does (there are none past the fine columns)
+        int32_t t = 0;
+        uint32_t cum = 0, pos = 0, certain = ~0u, possible = ~0u;
 #pragma unroll
         for (int f = 0; f < GW; ++f) {
-            cum += v[f / 4][f % 4];
-            if (t < 0 && f < n_fine && cum >= want) { t = f; n = cum; }
+            cum += v[f / 4][f % 4] & kCertain;
+            pos += v[f / 4][f % 4] >> kPossible;
+            t += cum < want ? 1 : 0;
+            certain = min(certain, cum < want ? ~0u : cum);
+            possible = min(possible, cum < want ? ~0u : pos);
         }
-        n = estimate(n);
-        if (n > cap) t = -1;
+        if (t >= n_fine) { t = -1; certain = possible = 0; }
+        const int64_t n = estimate(certain, possible);
+        const int64_t error = n - min(certain * stride, n_user);
+        if (n - error > cap) {
+            t = kNoList;
+            searched = 1;
+        } else if (n > cap && 4 * error > n) {
+            t = -1;
+        }
         if (b < PT) own_thr = t;
         qi[b].thr = t;
         qi[b].n_cand = (int32_t)n;  // until the candidates are counted
+        qi[b].n_dropped = (int32_t)error;
         if (t >= 0) {
+            if (error > band) atomicAdd(reinterpret_cast<unsigned long long *>(&longer[0]), (unsigned long long)error);
+            if (n > share) atomicAdd(reinterpret_cast<unsigned long long *>(&longer[1]), (unsigned long long)(n - share));
             atomicAdd(&bin[t], 1);
             atomicAdd(reinterpret_cast<unsigned long long *>(&load[length_class((int32_t)n)]), (unsigned long long)n);
         }
     }
     __syncthreads();
+    const bool by_band = longer[0] > kBandMin, by_length = longer[1] > (searched ? 0 : kSearchUsers * n_user);
+    if (by_band || by_length) {  // uniform
+        for (int i = threadIdx.x; i < GW; i += PT) { bin[i] = 0; load[i] = 0; }
+        __syncthreads();
+        for (int32_t b = threadIdx.x; b < nq; b += PT) {
+            const int32_t t = qi[b].thr;
+            if (t < 0) continue;
+            if ((by_band && qi[b].n_dropped > band) || (by_length && qi[b].n_cand > share)) {
+                const int32_t why = by_band && qi[b].n_dropped > band ? -1 : kNoList;
+                qi[b].thr = why;
+                if (b < PT) own_thr = why;
+                continue;
+            }
+            atomicAdd(&bin[t], 1);
+            atomicAdd(reinterpret_cast<unsigned long long *>(&load[length_class(qi[b].n_cand)]), (unsigned long long)qi[b].n_cand);
+        }
+        __syncthreads();
+    }
     static_assert(GW == 64, "one wavefront");
     if (threadIdx.x < 64) {
         const int t = threadIdx.x;
@@ -319,7 +403,7 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
         const int64_t all = __shfl(sum, 63, 64), in = last >= 0 ? __shfl(sum, max(last, 0), 64) : 0;
         if (t == 0) {
             longest = last;
-            left = room - in;
+            left = list_cap / 8 * 7 - in;
             ctr->n_need = (unsigned long long)(all - in);
         }
         if (last == 63) first_slots();
@@ -370,19 +454,22 @@ __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ h
     bool over[2] = {false, false};
     if (member && own < c0) {
         const u32x4 *row = reinterpret_cast<const u32x4 *>(hist + (int64_t)b * GW);
-        int64_t cum[2] = {0, 0};
+        uint32_t cum[2] = {0, 0}, pos[2] = {0, 0};
 #pragma unroll
         for (int j = 0; j < GW / 4; ++j) {
             const u32x4 v = row[j];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                cum[0] += 4 * j + i <= c0 ? v[i] : 0u;
-                cum[1] += 4 * j + i <= c1 ? v[i] : 0u;
+                const uint32_t x0 = 4 * j + i <= c0 ? v[i] : 0u, x1 = 4 * j + i <= c1 ? v[i] : 0u;
+                cum[0] += x0 & kCertain;
+                pos[0] += x0 >> kPossible;
+                cum[1] += x1 & kCertain;
+                pos[1] += x1 >> kPossible;
             }
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int64_t n = estimate(cum[h]);
+            const int64_t n = estimate(cum[h], pos[h]);
             more[h] = n - qi[b].n_cand;
             over[h] = n > cap;
         }
@@ -513,25 +600,27 @@ __device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int32_t bas
 // VGPRs) x a slice of the slots, 64 queries at a time through LDS (two buffers:
 // the next stage's rows go straight to LDS while one is computed, one barrier
 // per stage); a block's thresholds are loaded while the previous one is
-// computed.  A pair costs one fused multiply-add and one compare beside its
+// computed.  With PROD = 3 the stage is 32 queries' hi and lo rows.  A
+// workgroup whose pairs find the list full stops there (reading the counter at
+// the start of each unit instead took 140 of 705 us, 1M users x 1000 queries).  A pair costs one fused multiply-add and one compare beside its
 // share of the matrix products; listed pairs are queued per wavefront without
 // an atomic, and a unit takes its part of the list with one.  Bound: the
 // matrix cores' 16 cycles per 16x16x32 product and about 100 VALU instructions
 // per 16 queries x 16 NB users beside them.
-template <int KS, int NB>
-__global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen P, int64_t n_user,
+template <int KS, int NB, int PROD>
+__global__ void __launch_bounds__(NT, PROD == 1 && KS <= 5 ? 3 : 2) k_list_screen(ListScreen P, int64_t n_user,
                                                                      const int32_t *__restrict__ order,
                                                                      const int32_t *__restrict__ colg,
                                                                      uint32_t *__restrict__ g_cnt,
                                                                      ListCounters *__restrict__ ctr,
                                                                      int32_t *__restrict__ cl_u,
                                                                      int32_t *__restrict__ cl_b, int64_t list_cap) {
-    constexpr int KQ = KS * 4, UB = 64 * NB;
-    static_assert(QST * KQ == KS * NT, "KS 16-byte pieces per thread and stage");
+    constexpr int KQ = KS * 4, UB = 64 * NB, NH = PROD == 1 ? 1 : 2, QS = QST / NH;  // queries per stage
+    static_assert(NH * QS * KQ == KS * NT, "KS 16-byte pieces per thread and stage");
     static_assert(UB <= 256 && kSlice % QST == 0, "a queued pair's user takes 8 bits");
     // two variables, not one array: a read of one then does not wait for the
     // loads into the other
-    __shared__ u32x4 sA0[QST * KQ], sA1[QST * KQ];
+    __shared__ u32x4 sA0[NH * QS * KQ], sA1[NH * QS * KQ];
     __shared__ f32x4 sCs[kSlice / 4];
     __shared__ int32_t sCol[kSlice / 4 + QST / 4], sOrd[kSlice];
     __shared__ uint32_t sQ[NT / 64][WQ];
@@ -555,22 +644,28 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
         const int last = (int)min((int64_t)(UB - 1), n_user - 1 - rb * UB);
         const u32x4 *ubase = reinterpret_cast<const u32x4 *>(P.user_hi + rb * UB * P.Kp);
         const float *gbase = P.gcols + rb * UB, *nbase = P.user_norm + rb * UB;
-        Frag uh[NB][KS];
+        Frag uh[NB][KS], ul[PROD == 1 ? 1 : NB][PROD == 1 ? 1 : KS];
         float ar[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int ul = wave * 16 * NB + b * 16 + lr, uc = min(ul, last);
+            const int at = wave * 16 * NB + b * 16 + lr, uc = min(at, last);
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) uh[b][ks].q = ubase[uc * KQ + ks * 4 + lq];
+            if constexpr (PROD > 1) {
+                const u32x4 *lbase = reinterpret_cast<const u32x4 *>(P.user_lo + rb * UB * P.Kp);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) ul[b][ks].q = lbase[uc * KQ + ks * 4 + lq];
+            }
             // rows past the last user never reach a threshold
-            ar[b] = ul <= last ? P.C * nbase[uc] : -INFINITY;
+            ar[b] = at <= last ? P.C * nbase[uc] : -INFINITY;
         }
         int n_q = 0;  // queued pairs of the wavefront
         auto load_stage = [&](u32x4 *dst, int32_t q) __attribute__((always_inline)) {  // slots s0 + q ..
 #pragma unroll
             for (int k = 0; k < KS; ++k) {
-                const int c = (int)threadIdx.x + k * NT, r = c / KQ;
-                load_to_lds(reinterpret_cast<const u32x4 *>(P.q_hi) + ((uint32_t)sOrd[q + r] * KQ + swizzled<KS>(r, c % KQ)),
+                const int c = (int)threadIdx.x + k * NT, r = c / KQ % QS;
+                const uint16_t *src = NH > 1 && c >= QS * KQ ? P.q_lo : P.q_hi;  // the same in a wavefront
+                load_to_lds(reinterpret_cast<const u32x4 *>(src) + ((uint32_t)sOrd[q + r] * KQ + swizzled<KS>(r, c % KQ)),
                             dst + wave * 64 + k * NT);
             }
         };
@@ -587,8 +682,8 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's rows are in LDS
         __syncthreads();
         auto stage = [&](const u32x4 *rows, u32x4 *ahead, int32_t q0) __attribute__((always_inline)) {
-            if (q0 + QST < ns) load_stage(ahead, q0 + QST);
-            const int n_g = min(QST / 16, (ns - q0 + 15) / 16);
+            if (q0 + QS < ns) load_stage(ahead, q0 + QS);
+            const int n_g = min(QS / 16, (ns - q0 + 15) / 16);
 #pragma unroll 1
             for (int g = 0; g < n_g; ++g) {
                 const int t4 = (q0 >> 2) + g * 4 + lq;  // the lane's four slots: s0 + 4 t4 ..
@@ -614,6 +709,15 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
 #pragma unroll
                     for (int b = 0; b < NB; ++b)
                         acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                    if constexpr (PROD > 1) {
+                        Frag ql;
+                        ql.q = rows[QS * KQ + (g * 16 + lr) * KQ + swizzled<KS>(g * 16 + lr, ks * 4 + lq)];
+#pragma unroll
+                        for (int b = 0; b < NB; ++b) {
+                            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql.v, uh[b][ks].v, acc[b], 0, 0, 0);
+                            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh.v, ul[b][ks].v, acc[b], 0, 0, 0);
+                        }
+                    }
                 }
                 // D[4 lq + i][lr]: slot s0 + 4 t4 + i, user b * 16 + lr of the wave
                 const f32x4 cs = sCs[t4];
@@ -651,9 +755,9 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's rows of the next stage are in LDS
             __syncthreads();
         };
-        for (int32_t q0 = 0; q0 < ns; q0 += 2 * QST) {
+        for (int32_t q0 = 0; q0 < ns; q0 += 2 * QS) {
             stage(sA0, sA1, q0);
-            if (q0 + QST < ns) stage(sA1, sA0, q0 + QST);
+            if (q0 + QS < ns) stage(sA1, sA0, q0 + QS);
         }
         // the unit's pairs: one place in the list for the four wavefronts
         if (lane == 0) sN[wave] = n_q;
@@ -667,7 +771,9 @@ __global__ void __launch_bounds__(NT, KS <= 5 ? 3 : 2) k_list_screen(ListScreen 
         if (tot > 0) {  // uniform
             if (threadIdx.x == 0) sBase = list_places(&ctr->n_list, tot, list_cap);
             __syncthreads();
-            wave_flush(sQ[wave], n_q, sBase + before, (int32_t)(rb * UB), sOrd, cl_u, cl_b, list_cap);
+            const int32_t base = sBase;
+            if (base >= list_cap) return;  // uniform: the list has outgrown its arrays, no stage will read it
+            wave_flush(sQ[wave], n_q, base + before, (int32_t)(rb * UB), sOrd, cl_u, cl_b, list_cap);
         }
         __syncthreads();  // the next unit rewrites the slice, the queues and the stages
     }
@@ -1017,8 +1123,8 @@ __device__ __forceinline__ void find_bin(const uint32_t *h, uint32_t before, uin
 // whole list of a few queries, skipping other queries' pairs): beta, the bucket
 // of the k-th smallest b_lo, then the candidates (b_hi <= beta) with their rank
 // when the bounds fix it, else ~(refine row).  A query with fewer than k buckets
-// up to its threshold, or a list that overflowed, gets thr = -1 (a query that
-// found no room keeps kNoRoom) and no candidates: it is answered another way.
+// up to its threshold, or a list that overflowed, gets thr = -1 (the plan's own
+// reasons stay) and no candidates: it is answered another way.
 //
 // Many candidates are users of bucket beta itself (an item that most of 100k
 // users rank first).  When that bucket fixes the rank, the answer takes the
@@ -1093,7 +1199,7 @@ __global__ void __launch_bounds__(FT) k_list_final(const int32_t *__restrict__ c
     if (beta < 0) {  // uniform
         if (threadIdx.x == 0) {
             qi[b].beta = qi[b].gamma = -1;
-            if (q.thr != kNoRoom) qi[b].thr = -1;
+            if (q.thr >= 0) qi[b].thr = -1;
             qi[b].n_cand = qi[b].n_dropped = qi[b].n_refine = qi[b].fill = qi[b].n_settled = 0;
             qi[b].cand_off = 0;
         }
@@ -1284,26 +1390,37 @@ hipError_t launch_keep_rows(hipStream_t s, float *x, int64_t n_col, const int32_
 hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L) {
     if (L.nq <= 0 || L.n_user <= 0) return hipSuccess;
     if (!fine_ok(L.fc, L.S) || !L.gvals || !L.gcols || L.pitch < L.n_user || !L.user_hi || !L.q_hi) return hipErrorInvalidValue;
-    ListScreen P{L.user_hi, L.user_norm, L.gvals, L.gcols, L.pitch, L.q_hi, L.q_cs, L.nq, L.Kp, L.fc.n, L.C, L.floor};
+    if (L.products != 1 && (L.products != 3 || !L.user_lo || !L.q_lo)) return hipErrorInvalidValue;
+    ListScreen P{L.user_hi, L.user_lo, L.user_norm, L.gvals, L.gcols, L.pitch, L.q_hi, L.q_lo, L.q_cs, L.nq, L.Kp, L.fc.n,
+                 L.C, L.floor};
     const int64_t n_s = (L.n_user + L.stride - 1) / L.stride, n_sb = (n_s + 127) / 128;
     const unsigned qg = (unsigned)((L.nq + QST - 1) / QST);
     // two workgroups of the sample fit a CU
     const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>(n_sb, (2 * L.n_cu + qg - 1) / qg));
 #define RKR_SAMPLE_CASE(ks)                                                                                       \
     case ks:                                                                                                      \
-        hipLaunchKernelGGL(k_sample_screen<ks>, dim3(gx, qg), dim3(NT), 0, s, P, n_s, L.stride, L.n_user, L.hist);           \
+        if (L.products == 1)                                                                                      \
+            hipLaunchKernelGGL((k_sample_screen<ks, 1>), dim3(gx, qg), dim3(NT), 0, s, P, n_s, L.stride, L.n_user, L.hist); \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_sample_screen<ks, 3>), dim3(gx, qg), dim3(NT), 0, s, P, n_s, L.stride, L.n_user, L.hist); \
         break;
     RKR_KS_SWITCH(L.Kp, RKR_SAMPLE_CASE)
 #undef RKR_SAMPLE_CASE
-    hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
-                       L.room, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
-    const int64_t ub = L.Kp <= 160 ? 256 : 128;
+    hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap, L.share,
+                       L.band, L.room, L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
+    // users per unit and workgroups per CU
+    const bool wide = L.products == 1 && L.Kp <= 160;
+    const int64_t ub = wide ? 256 : 128;
     const int64_t units = (L.n_user + ub - 1) / ub * ((L.nq + kSlice - 1) / kSlice);
-    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(units, (int64_t)L.n_cu * (L.Kp <= 160 ? 3 : 2))));
+    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(units, (int64_t)L.n_cu * (wide ? 3 : 2))));
 #define RKR_LIST_CASE(ks)                                                                                          \
     case ks:                                                                                                       \
-        hipLaunchKernelGGL((k_list_screen<ks, ks <= 5 ? 4 : 2>), grid, dim3(NT), 0, s, P, L.n_user, L.order, \
-                           L.colg, L.g_cnt, L.ctr, L.raw_u, L.raw_b, L.list_cap);                                  \
+        if (L.products == 1)                                                                                       \
+            hipLaunchKernelGGL((k_list_screen<ks, ks <= 5 ? 4 : 2, 1>), grid, dim3(NT), 0, s, P, L.n_user, L.order, \
+                               L.colg, L.g_cnt, L.ctr, L.raw_u, L.raw_b, L.list_cap);                              \
+        else                                                                                                       \
+            hipLaunchKernelGGL((k_list_screen<ks, 2, 3>), grid, dim3(NT), 0, s, P, L.n_user, L.order, L.colg,      \
+                               L.g_cnt, L.ctr, L.raw_u, L.raw_b, L.list_cap);                                      \
         break;
     RKR_KS_SWITCH(L.Kp, RKR_LIST_CASE)
 #undef RKR_LIST_CASE
@@ -1318,8 +1435,8 @@ hipError_t launch_list_scores(hipStream_t s, const ListLaunch &L) {
     const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n_s + 63) / 64, (8 * L.n_cu + qg - 1) / qg));
     hipLaunchKernelGGL(k_sample_scores, dim3(gx, qg), dim3(NT), 0, s, L.qip, L.n_user, L.nq, L.eps, L.gvals, L.fc.n,
                        n_s, L.stride, L.hist, L.t_bound);
-    hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap,
-                       L.room, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
+    hipLaunchKernelGGL(k_list_plan, dim3(1), dim3(PT), 0, s, L.hist, L.nq, L.fc.n, L.stride, L.n_user, L.cap, L.share,
+                       L.band, L.room, L.list_cap, L.fc.coarse, L.qi, L.order, L.colg, L.ctr);
     hipLaunchKernelGGL(k_list_scores,
                        dim3((unsigned)((L.n_user + NT - 1) / NT), (unsigned)((L.nq + kScoreSlice - 1) / kScoreSlice)),
                        dim3(NT), 0, s, L.qip, L.n_user, L.eps, L.gcols, L.pitch, L.order, L.colg, L.nq, L.g_cnt, L.ctr,

@@ -1434,32 +1434,37 @@ int64_t list_entries(int64_t U, int64_t nq) {
     return std::min<int64_t>({std::max<int64_t>(nq * per, 2 * std::max<int64_t>(4096, U / 4)), nq * U, INT32_MAX / 2});
 }
 
-// How a set of queries is answered.
+// How a set of queries is answered: threshold lists (k_list.hip) from matrix-core
+// scores of one or three products or from exact scores, or a search over every
+// user.  With updates pending the coarse bounds stand for all lists; the plain
+// form, and rows too wide for the matrix cores, have lists from exact scores only.
+enum Level { kOneProduct, kThreeProducts, kScores, kSearch };  // in the order they are tried
 struct Attempt {
-    bool lists = true;            // threshold lists (k_list.hip), or with updates pending the coarse bounds
+    Level level = kOneProduct;
     int64_t entries = 0;          // list entries to make room for, beyond the usual
     const int32_t *rows = nullptr;  // the queries' exact scores are these rows of the slot's scores (ascending)
 };
+// Fewer users are searched rather than listed from finer scores.
+constexpr int64_t kFinerUsers = 16384;
+// So are a few queries beside others that are searched: 20 ps a pair.
+constexpr int64_t kJoinPairs = 5000000;
 // What run_batches left open.
 struct Outcome {
-    struct Open { int32_t query; bool room; };  // room: its list only found no room
+    struct Open { int32_t query, thr; };  // and QueryInfo::thr, the reason
     std::vector<Open> open;       // outputs unwritten
     int64_t need = 0;             // pairs of the lists that found no room, as estimated
     int64_t entries = 0;          // list entries there were
-    bool lists = false;           // the queries went through lists or the coarse bounds
+    Level level = kSearch;        // what the attempt came to
     bool scores = false;          // the slot holds every query's exact scores, row i the i-th query's
 };
 
-// The longest list of a batch of n queries that is faster than its share of a
-// search over every user, which takes 4 ms and 20 us a query at 1M users; a
-// listed pair takes 0.25 ns from matrix-core scores, 0.5 from exact ones (they
-// are read twice), up to 1 in short lists.  So a quarter of all users for a few
-// queries (4 queries, 260k pairs: 0.41 ms, searched 4.6), a tenth or a twentieth
-// of them for many (1M users x 1000 queries, 8% of all pairs: 24 ms screened,
-// searched 29; 45 plain, searched 31).
-int64_t list_pairs_max(int64_t U, int64_t n, bool screened) {
-    return std::min(std::max<int64_t>(4096, U / 4), std::max<int64_t>(4096, 12 * U / n + U / (screened ? 12 : 24)));
-}
+// Among many queries, the longest list that is faster than its query's part of a
+// search over every user: the search takes 4 ms and 20 us a query at 1M users, a
+// listed pair 0.25 ns from matrix-core scores and 0.5 from exact ones, which are
+// read twice.  1M users x 1000 queries, 8% of all pairs: 24 ms screened, searched
+// 29; 45 plain, searched 31.  (Few long lists are faster all the same, up to a
+// quarter of all users: 4 queries, 260k pairs 0.41 ms, searched 4.6.)
+int64_t list_share(int64_t U, bool screened) { return std::max<int64_t>(4096, U / (screened ? 12 : 24)); }
 
 // Device batches of query_on_slot.  Queries that the attempt cannot answer (no
 // threshold, a list too long or too short) go to out.open.
@@ -1482,7 +1487,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // the QSRP screen (RKR_OPT_QSRP, built by rkr_qsrp_build) replaces the bound
     // stage of exact batches without pending updates
     const bool qsrp = c->qsrp && dv.qsrp_users && mode == RKR_OUTPUT_EXACT && !upd && U > 0;
-    const bool listable = !qsrp && how.lists && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
+    const bool listable = !qsrp && how.level != kSearch && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
                           dv.guards.n > 0 && U > 0;
     const bool mfma = screened && c->kp > 0 && dv.user_norm;
     const size_t pair_bytes = upd ? 12 : 8;  // <u,q> + buckets, or + two bound values
@@ -1502,10 +1507,11 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // query is even, and batches of 8 at 4k users.
     const bool list = listable && !upd &&
                       (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
-    const bool list_mfma = list && mfma;
+    const bool list_mfma = list && mfma && how.level <= kThreeProducts;
+    const int products = how.level == kThreeProducts ? 3 : 1;
     // scores left by the last attempt, of this attempt's queries
     const bool scored = how.rows && !list_mfma && !upd && !qsrp && n_query <= nqb;
-    out.lists = list || (listable && upd);
+    out.level = list_mfma ? how.level : list ? kScores : listable && upd ? kOneProduct : kSearch;
     out.scores = list && !list_mfma && n_query <= nqb;
     // a few users: bounds to candidates in one kernel, its arrays sized for
     // every pair (6 MB at most)
@@ -1539,7 +1545,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     const std::vector<int32_t> &hrk = *dv.hrk;
     const GuardCols &gc = dv.guards;
     // an (estimated) list longer than list_max takes the full path instead
-    const int64_t list_max = list ? list_pairs_max(U, nqb, list_mfma) : std::max<int64_t>(4096, U / 4);
+    const int64_t list_max = std::max<int64_t>(4096, U / 4);
     int64_t list_cap = 0;
     if (list) {
         // what is held already, or what a quarter of the free budget allows
@@ -1646,9 +1652,17 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         if (list) {
             LL.n_user = U; LL.nq = nq; LL.S = S; LL.Kp = c->kp; LL.n_cu = c->n_cu;
             LL.user_hi = dv.user_hi; LL.user_norm = dv.user_norm; LL.gvals = dv.gvals; LL.gcols = dv.gcols; LL.pitch = dv.gpitch;
-            LL.q_hi = q_hi; LL.q_cs = qcs; LL.fc = dv.fine; LL.C = est_C; LL.floor = est_floor; LL.eps = eps;
-            LL.qip = qip; LL.stride = sample_stride(U); LL.cap = list_max; LL.list_cap = list_cap;
-            LL.room = list_cap / 2;  // the estimates may be half of what comes
+            LL.q_hi = q_hi; LL.q_cs = products == 1 ? qcs : qn; LL.C = products == 1 ? est_C : c->screen_C;
+            LL.fc = dv.fine; LL.floor = est_floor; LL.eps = eps;
+            LL.qip = qip; LL.stride = sample_stride(U); LL.cap = list_max; LL.share = list_share(U, list_mfma); LL.list_cap = list_cap;
+            // An estimate is off by what the sample is; without the pairs that the
+            // scores' error adds it would be half of what comes.
+            LL.room = list_mfma ? list_cap / 4 * 3 : list_cap / 2;
+            // A list that one product's error makes longer than this is cheaper
+            // from three (1.3 us a query at 1M users, 0.25 ns a pair).
+            LL.band = list_mfma && products == 1 && U >= kFinerUsers ? std::max<int64_t>(4096, U / 64) : U;
+            LL.products = products;
+            LL.user_lo = dv.user_lo; LL.q_lo = q_lo;
             LL.hist = reinterpret_cast<uint32_t *>(sl.list_info.p);
             LL.order = reinterpret_cast<int32_t *>(LL.hist + 64 * (size_t)nq);
             LL.colg = LL.order + nq;
@@ -1730,7 +1744,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
                     e[1] = (int32_t)std::min<int64_t>(n, INT32_MAX);
                 }
                 if (e[0] < 0 || e[1] > list_max) {
-                    out.open.push_back({(int32_t)(q0 + i), false});
+                    out.open.push_back({(int32_t)(q0 + i), kNoList});
                     e[0] = -1;
                     e[1] = 0;
                 }
@@ -1821,7 +1835,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             const int64_t floor_rank = (int64_t)hrk[gc.col[gc.n - 1]] + 1 - dv.n_del;
             for (int32_t i : deep_check)
                 if (hcq[(size_t)i * 4] >= 0 && (int64_t)hqi[i].gamma >= floor_rank)
-                    out.open.push_back({(int32_t)(q0 + i), false});
+                    out.open.push_back({(int32_t)(q0 + i), kNoList});
         }
         if (total >= INT32_MAX) return set_err(c, RKR_ERR_NOMEM, "query: candidate count exceeds 2^31; lower the query batch");
         const size_t cap = (size_t)std::max<int64_t>(total, 1);
@@ -1913,7 +1927,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
         }
         if (list) {
             for (int32_t i = 0; i < nq; ++i)
-                if (hqi[i].thr < 0) out.open.push_back({(int32_t)(q0 + i), hqi[i].thr == kNoRoom});
+                if (hqi[i].thr < 0) out.open.push_back({(int32_t)(q0 + i), hqi[i].thr});
             out.need += (int64_t)hctr->n_need;
             if ((int64_t)hctr->n_list <= list_cap) tm.n_listed += (int64_t)hctr->n_list;  // else no stage read the list
             tm.n_coarse_refined += hctr->n_finer;
@@ -1997,60 +2011,100 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
 
 namespace {
 
-// Answers n queries by one attempt, and what it leaves open by others: lists
-// that only found no room once more with more of it, the rest by a search over
-// every user.
+// Queries that wait for an attempt.
+struct Group {
+    Attempt how;
+    std::vector<int32_t> idx;  // ascending
+};
+
+// Answers n queries: every attempt's open queries join the group of their next
+// one -- lists that only found no room once more with more of it, the others
+// finer scores or the search -- and the groups are taken in the order of their
+// levels, so that the search runs once.
 int answer(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int32_t n, const int32_t *topk, int32_t max_k,
-           int32_t *out_user, int32_t *out_rank, float *out_qip, rkr_query_stats *stats, rkr_batch_timing &tm,
-           const Attempt &how) {
+           int32_t *out_user, int32_t *out_rank, float *out_qip, rkr_query_stats *stats, rkr_batch_timing &tm) {
     Outcome o;
-    int rc = run_batches(c, sl, dv, queries, n, topk, max_k, out_user, out_rank, out_qip, stats, tm, how, o);
+    int rc = run_batches(c, sl, dv, queries, n, topk, max_k, out_user, out_rank, out_qip, stats, tm, Attempt{}, o);
     if (rc || o.open.empty()) return rc;
-    // n queries' lists get one more attempt, if they are not all of this one's
-    // or there can be more room
-    auto order = [](const Outcome::Open &x, const Outcome::Open &y) { return x.query < y.query; };
-    std::sort(o.open.begin(), o.open.end(), order);
-    const int64_t n_open = (int64_t)o.open.size();
-    int64_t n_room = 0;
-    for (const auto &x : o.open) n_room += x.room;
-    Attempt more = how;
-    more.entries = std::max<int64_t>(1, 2 * (o.need + o.need / 8));
-    const bool again = how.entries == 0 && n_room > 0 && (n_room < n || more.entries > o.entries);
-    Attempt search;
-    search.lists = false;
-    // the larger part first: it finds its scores where they are, and they are gone then
-    const bool lists_first = again && 2 * n_room >= n_open;
-    bool scores = o.scores;
-    for (const bool lists : {lists_first, !lists_first}) {
-        std::vector<int32_t> idx;
-        for (const auto &x : o.open)
-            if ((again && x.room) == lists) idx.push_back(x.query);
-        const int32_t m = (int32_t)idx.size(), d = c->dim;
-        if (m == 0) continue;
-        if (!lists) tm.n_fallback += m;
+    const int32_t d = c->dim;
+    const bool upd = dv.n_ins > 0 || dv.n_del > 0;
+    std::vector<Group> todo;
+    std::vector<int32_t> scored;  // queries whose scores the slot holds, row by row
+    auto put = [&](Level level, int64_t entries, int32_t q) {
+        for (Group &g : todo)
+            if (g.how.level == level && (g.how.entries > 0) == (entries > 0)) {
+                g.how.entries = std::max(g.how.entries, entries);
+                g.idx.push_back(q);
+                return;
+            }
+        todo.emplace_back();
+        todo.back().how.level = level;
+        todo.back().how.entries = entries;
+        todo.back().idx.push_back(q);
+    };
+    // the open queries of an attempt on `idx` (null: all queries in order)
+    auto sort_out = [&](const Attempt &how, const std::vector<int32_t> *idx, int32_t m) {
+        int64_t n_room = 0, n_search = 0;
+        for (const auto &x : o.open) {
+            n_room += x.thr == kNoRoom;
+            n_search += x.thr == kNoList;
+        }
+        // an attempt of their own (100 us) costs these more than joining the others' search
+        const bool join = n_search > 0 && ((int64_t)o.open.size() - n_search) * dv.n_user < kJoinPairs;
+        const int64_t entries = std::max<int64_t>(1, 2 * (o.need + o.need / 8));
+        const bool again = how.entries == 0 && n_room > 0 && (n_room < m || entries > o.entries);
+        const Level finer = upd || o.level == kScores || dv.n_user < kFinerUsers ? kSearch
+                            : o.level == kOneProduct                            ? kThreeProducts
+                                                                                : kScores;
+        for (const auto &x : o.open) {
+            const int32_t q = idx ? (*idx)[x.query] : x.query;
+            if (join) put(kSearch, 0, q);
+            else if (again && x.thr == kNoRoom) put(o.level, entries, q);
+            else put(x.thr == kNoList ? kSearch : finer, 0, q);
+        }
+        scored.clear();
+        if (o.scores)
+            for (int32_t i = 0; i < m; ++i) scored.push_back(idx ? (*idx)[i] : i);
+    };
+    sort_out(Attempt{}, nullptr, n);
+    while (!todo.empty()) {
+        const auto first = std::min_element(todo.begin(), todo.end(), [](const Group &x, const Group &y) {
+            return x.how.level != y.how.level ? x.how.level < y.how.level : x.how.entries < y.how.entries;
+        });
+        Group g = std::move(*first);
+        todo.erase(first);
+        std::sort(g.idx.begin(), g.idx.end());
+        const int32_t m = (int32_t)g.idx.size();
+        // the scores of the last attempt, if it held them all
+        std::vector<int32_t> rows;
+        if (g.how.level >= kScores)
+            for (size_t i = 0; i < scored.size() && rows.size() < g.idx.size(); ++i)
+                if (scored[i] == g.idx[rows.size()]) rows.push_back((int32_t)i);
+        if (rows.size() == g.idx.size()) g.how.rows = rows.data();
         std::vector<float> q((size_t)m * d), qip((size_t)m * max_k);
         std::vector<int32_t> k((size_t)m), u((size_t)m * max_k), r((size_t)m * max_k);
         std::vector<rkr_query_stats> st(stats ? (size_t)m : 0);
         for (int32_t i = 0; i < m; ++i) {
-            std::memcpy(&q[(size_t)i * d], queries + (size_t)idx[i] * d, sizeof(float) * d);
-            k[i] = topk[idx[i]];
+            std::memcpy(&q[(size_t)i * d], queries + (size_t)g.idx[i] * d, sizeof(float) * d);
+            k[i] = topk[g.idx[i]];
         }
-        Attempt next = lists ? more : search;
-        next.rows = scores ? idx.data() : nullptr;
-        scores = false;
-        rc = answer(c, sl, dv, q.data(), m, k.data(), max_k, u.data(), r.data(), qip.data(), stats ? st.data() : nullptr,
-                    tm, next);
+        o = Outcome{};
+        rc = run_batches(c, sl, dv, q.data(), m, k.data(), max_k, u.data(), r.data(), qip.data(), stats ? st.data() : nullptr,
+                         tm, g.how, o);
         if (rc) return rc;
+        if (o.level == kSearch) tm.n_fallback += m;
+        // rows of a query that is still open are written again
         for (int32_t i = 0; i < m; ++i) {
-            const size_t to = (size_t)idx[i] * max_k, from = (size_t)i * max_k;
+            const size_t to = (size_t)g.idx[i] * max_k, from = (size_t)i * max_k;
             std::memcpy(out_user + to, &u[from], sizeof(int32_t) * max_k);
             std::memcpy(out_rank + to, &r[from], sizeof(int32_t) * max_k);
             if (out_qip) std::memcpy(out_qip + to, &qip[from], sizeof(float) * max_k);
             if (stats) {
-                stats[idx[i]] = st[i];
-                stats[idx[i]].query_id = idx[i];
+                stats[g.idx[i]] = st[i];
+                stats[g.idx[i]].query_id = g.idx[i];
             }
         }
+        sort_out(g.how, &g.idx, m);
     }
     return RKR_OK;
 }
@@ -2063,7 +2117,7 @@ int query_on_slot(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, in
     using clock = std::chrono::steady_clock;
     const auto t_start = clock::now();
     rkr_batch_timing tm{};
-    const int rc = answer(c, sl, dv, queries, n_query, topk, max_k, out_user, out_rank, out_qip, stats, tm, Attempt{});
+    const int rc = answer(c, sl, dv, queries, n_query, topk, max_k, out_user, out_rank, out_qip, stats, tm);
     if (rc) return rc;
     tm.total_ms = std::chrono::duration<double, std::milli>(clock::now() - t_start).count();
     if (timing) *timing = tm;

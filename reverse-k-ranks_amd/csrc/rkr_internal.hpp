@@ -474,11 +474,11 @@ struct QueryInfo {          // one per query of a device batch
     int32_t fill;           // candidates written so far (chunked compaction)
     int32_t n_screen;       // users a screen kept and scored exactly (QSRP)
     int64_t cand_off;       // offset of this query's candidates
-    int32_t thr;            // fine column of the query's list; -1: no list answers it, kNoRoom: its list did not fit
+    int32_t thr;            // fine column of the query's list; -1: none from these scores answers it, or kNoRoom, kNoList
     int32_t n_dropped;      // candidates counted but not written: the answer cannot hold them
 };
 
-constexpr int32_t kNoRoom = -2;
+constexpr int32_t kNoRoom = -2, kNoList = -3;  // its list found no room; too long from finer scores, too
 
 // Counters of a device batch, uploaded as zeros with the queries and read back
 // with the outputs.
@@ -538,10 +538,10 @@ struct HostResult {         // where the top-k puts what the host reads (qi null
 
 // ---- threshold lists of exact output (k_list.hip) ----------------------------
 struct ListScreen {          // the screened scores of a batch
-    const uint16_t *user_hi; // n_user x Kp BF16 hi halves
+    const uint16_t *user_hi, *user_lo;  // n_user x Kp BF16 halves (lo: three products)
     const float *user_norm, *gvals, *gcols;
     int64_t pitch;           // of gcols
-    const uint16_t *q_hi;    // nq x Kp
+    const uint16_t *q_hi, *q_lo;  // nq x Kp
     const float *q_cs;       // error scales: |s^ - s| <= C ||u|| cs + floor
     int32_t nq, Kp, n_fine;
     float C, floor;
@@ -549,14 +549,17 @@ struct ListScreen {          // the screened scores of a batch
 struct ListLaunch {
     int64_t n_user;
     int32_t nq, S, Kp, n_cu;
-    const uint16_t *user_hi, *q_hi;
+    int products;            // of the matrix-core scores: 1 or 3
+    const uint16_t *user_hi, *user_lo, *q_hi, *q_lo;
     const float *user_norm, *gvals, *gcols, *q_cs;
     int64_t pitch;           // of gcols
     FineCols fc;
     float C, floor, eps;
     float *qip;              // exact scores (read with scores, else written for listed pairs)
     int64_t stride;          // one user of every stride is sampled
-    int64_t cap;             // a longer estimated list takes the full search
+    int64_t cap;             // a longer estimated list is not made
+    int64_t share;           // nor ones longer than this, if they are many
+    int64_t band;            // nor ones that the scores' error makes so many pairs longer, if they are many
     int64_t list_cap;        // entries of the lists
     int64_t room;            // pairs that the estimated lists may hold
     uint32_t *hist;          // nq x 64, zeroed

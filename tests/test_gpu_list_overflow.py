@@ -71,7 +71,9 @@ def test_more_listed_pairs_than_31_bits_count(gpu_index_factory, form):
     idx.set_form(form)
     ks = [10] * nq
     got = idx.query(queries, ks)
-    assert got.timing["n_batches"] == 2 and got.timing["n_fallback"] == nq and got.timing["n_listed"] == 0
+    # lists from exact scores and the search, before them from one and three products
+    assert got.timing["n_batches"] == {"plain": 2, "screened": 4}[form]
+    assert got.timing["n_fallback"] == nq and got.timing["n_listed"] == 0
     idx.set_option(9, 0)  # RKR_OPT_COARSE
     _same_answers(got, idx.query(queries, ks), ks)
     idx.close()
@@ -150,5 +152,34 @@ def test_batches_that_do_not_fit_at_once(gpu_index_factory, form, deep, popular)
         _same_answers(g, want, ks)
         for f in ("n_candidate", "n_refine_user", "n_prune_user", "n_result_user", "query_id"):
             assert [s[f] for s in g.stats] == [s[f] for s in want.stats], f
-        assert g.timing["n_fallback"] <= deep + popular // 20  # a list can be too long for a batch of 200
+        # long lists join a search that other queries need
+        assert g.timing["n_listed"] > 0 and g.timing["n_fallback"] <= deep + popular // 2
+    idx.close()
+
+
+@pytest.mark.parametrize("U,nq", [(17_000, 8), (40_001, 37), (90_000, 600)])
+@pytest.mark.parametrize("d,noise", [(40, 1.0), (40, 0.3), (40, 0.1), (40, 0.03), (40, 0.01), (20, 0.02), (90, 0.02), (120, 0.02),
+                                     (150, 0.02), (190, 0.02), (220, 0.02), (256, 0.02)])
+def test_items_that_share_a_common_part(gpu_index_factory, U, nq, d, noise):
+    """Items = mean + noise: the less noise, the more users one BF16 product
+    cannot tell apart.  Every row width of the three-product scores."""
+    _case(f"items = mean + {noise} noise, U={U} nq={nq} d={d}")
+    rng = np.random.default_rng(d + nq)
+    I = 900
+    users = rng.standard_normal((U, d), dtype=np.float32)
+    items = rng.standard_normal(d, dtype=np.float32) + np.float32(noise) * rng.standard_normal((I, d), dtype=np.float32)
+    queries = items[rng.choice(I, nq, replace=False)]
+    ks = [int(k) for k in rng.integers(1, 60, nq)]
+    idx, _ = gpu_index_factory(users, items, 64)
+    idx.set_form("screened")
+    got = idx.query(queries, ks)
+    print({f: got.timing[f] for f in ("n_batches", "n_listed", "n_fallback")}, flush=True)
+    assert got.timing["n_listed"] > 0 and got.timing["n_fallback"] <= nq // 8
+    if noise <= 0.02 and d >= 90:
+        assert got.timing["n_batches"] > 1
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    want = idx.query(queries, ks)
+    _same_answers(got, want, ks)
+    for f in ("n_candidate", "n_refine_user", "n_prune_user", "n_result_user", "query_id"):
+        assert [s[f] for s in got.stats] == [s[f] for s in want.stats], f
     idx.close()
