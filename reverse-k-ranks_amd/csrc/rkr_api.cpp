@@ -1974,9 +1974,10 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             uint64_t ts[kTimeEnd + 1];
             for (int i = 0; i <= kTimeEnd; ++i) ts[i] = hctr->t[i];
             if (direct) {  // the last workgroup's end, from the low words
-                uint32_t end = 0;
-                for (int32_t i = 0; i < nq; ++i) end = std::max(end, (uint32_t)hqi[i].pad - (uint32_t)ts[kTimeTopk]);
-                ts[kTimeEnd] = ts[kTimeTopk] + end;
+                // (a query without candidates can be done before the first workgroup stamps the start)
+                int32_t end = 0;
+                for (int32_t i = 0; i < nq; ++i) end = std::max(end, (int32_t)((uint32_t)hqi[i].pad - (uint32_t)ts[kTimeTopk]));
+                ts[kTimeEnd] = ts[kTimeTopk] + (uint32_t)end;
             }
             for (int i = kTimeEnd - 1; i >= 0; --i)
                 if (ts[i] == 0) ts[i] = ts[i + 1];

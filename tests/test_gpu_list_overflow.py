@@ -183,3 +183,20 @@ def test_items_that_share_a_common_part(gpu_index_factory, U, nq, d, noise):
     for f in ("n_candidate", "n_refine_user", "n_prune_user", "n_result_user", "query_id"):
         assert [s[f] for s in got.stats] == [s[f] for s in want.stats], f
     idx.close()
+
+
+def test_stage_times(gpu_index_factory):
+    """Stage times of batches on two streams at once: a query's top-k workgroup
+    can end before the batch's first one has stamped the start."""
+    _case("stage times")
+    rng = np.random.default_rng(2)
+    users = rng.standard_normal((300_001, 32), dtype=np.float32)
+    items = rng.standard_normal((3000, 32), dtype=np.float32) * np.exp(0.5 * rng.standard_normal((3000, 1), dtype=np.float32))
+    idx, _ = gpu_index_factory(users, items, 48)
+    for form in ("screened", "plain"):
+        idx.set_form(form)
+        for _ in range(40):
+            t = idx.query(items[:2600], 20).timing
+            for f in ("ip_ms", "bound_ms", "prune_ms", "refine_ms", "recheck_ms", "topk_ms", "h2d_ms", "d2h_ms"):
+                assert 0 <= t[f] <= 3 * t["total_ms"], f  # of three batches
+    idx.close()
