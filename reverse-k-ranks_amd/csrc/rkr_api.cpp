@@ -572,6 +572,10 @@ int rkr_set_option(rkr_ctx *c, int option, int64_t value) {
             if (value != 0 && value != 1) return set_err(c, RKR_ERR_INVALID, "qsrp must be 0 or 1");
             c->qsrp = (int)value;
             return RKR_OK;
+        case kOptDpSpin:
+            if (value < 0 || value > (1 << 20)) return set_err(c, RKR_ERR_INVALID, "DP looks must be in [0, 2^20]");
+            c->dp_spin = (int32_t)value;
+            return RKR_OK;
         default:
             return set_err(c, RKR_ERR_INVALID, "unknown option");
     }

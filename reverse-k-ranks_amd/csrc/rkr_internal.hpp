@@ -166,6 +166,7 @@ struct Ctx {
     float *rho = nullptr;
     int n_cu = 256;
     double clock_khz = 1e5;  // rate of the device clock (stamp())
+    int32_t dp_spin = 1 << 20;  // looks at a value that another workgroup of the sample-rank DP writes (kOptDpSpin)
 
     // QSRP screen (rkr_qsrp_build): users rotated into the SVD basis, the query
     // rotation, and per-user norms and regression parameters (kQsrp* rows of
@@ -297,6 +298,8 @@ struct DataSnap {
     float qsrp_gcd = 0.0f, qsrp_crot = 0.0f;
 };
 DataSnap snap_of(const Ctx *c);
+// Option of rkr_set_option for tests: Ctx::dp_spin.
+constexpr int kOptDpSpin = 1001;
 // Sets Ctx::fine, guards and hrk for the searched table's ranks.
 void set_table_columns(Ctx *c);
 // The table over the current items at sampled ranks S (build_table), and the

@@ -224,23 +224,31 @@ int rkr_find_optimal_sample(rkr_ctx *c, int64_t n_user, int64_t n_item, int32_t 
     RKR_HIP(c, hipMemcpyAsync(dDp.p, dp0.data(), sizeof(int64_t) * R, hipMemcpyHostToDevice, s));
     RKR_HIP(c, hipMemcpyAsync(dPath.p, pos0.data(), sizeof(int32_t) * R, hipMemcpyHostToDevice, s));
     RKR_HIP(c, launch_transit(s, dC.p, (int32_t)Q, dPos.p, dPos.p + R, dEnd.p, (int32_t)R, dT.p));
+    std::vector<int64_t> last((size_t)R);
+    std::vector<int32_t> path((size_t)n_sample * R);
+    auto read_back = [&](int64_t last_row) {
+        RKR_HIP(c, hipMemcpyAsync(last.data(), dDp.p + last_row * R, sizeof(int64_t) * R, hipMemcpyDeviceToHost, s));
+        RKR_HIP(c, hipMemcpyAsync(path.data(), dPath.p, sizeof(int32_t) * path.size(), hipMemcpyDeviceToHost, s));
+        RKR_HIP(c, hipStreamSynchronize(s));
+        return (int)RKR_OK;
+    };
+    int32_t err = 0;
     if (one) {
         RKR_HIP(c, hipMemsetAsync(dErr.p, 0, sizeof(int32_t), s));
         if (n_sample > 1) RKR_HIP(c, hipMemsetAsync(dDp.p + R, 0x80, sizeof(int64_t) * (size_t)((n_sample - 1) * R), s));
-        RKR_HIP(c, launch_dp_layers(s, dT.p, (int32_t)R, n_sample, dDp.p, dPath.p, 1 << 20, dErr.p));
+        RKR_HIP(c, launch_dp_layers(s, dT.p, (int32_t)R, n_sample, dDp.p, dPath.p, c->dp_spin, dErr.p));
+        RKR_HIP(c, hipMemcpyAsync(&err, dErr.p, sizeof(err), hipMemcpyDeviceToHost, s));
+        if ((rc = read_back(n_sample - 1))) return rc;
     }
-    for (int32_t l = 1; !one && l < n_sample; ++l)
-        RKR_HIP(c, launch_dp_layer(s, dT.p, dDp.p + ((l - 1) & 1) * R, dPath.p + (int64_t)(l - 1) * R, (int32_t)R,
-                                   dDp.p + (l & 1) * R, dPath.p + (int64_t)l * R));
-    std::vector<int64_t> last((size_t)R);
-    std::vector<int32_t> path((size_t)n_sample * R);
-    int32_t err = 0;
-    if (one) RKR_HIP(c, hipMemcpyAsync(&err, dErr.p, sizeof(err), hipMemcpyDeviceToHost, s));
-    RKR_HIP(c, hipMemcpyAsync(last.data(), dDp.p + (one ? n_sample - 1 : (n_sample - 1) & 1) * R, sizeof(int64_t) * R,
-                              hipMemcpyDeviceToHost, s));
-    RKR_HIP(c, hipMemcpyAsync(path.data(), dPath.p, sizeof(int32_t) * path.size(), hipMemcpyDeviceToHost, s));
-    RKR_HIP(c, hipStreamSynchronize(s));
-    if (err) return set_err(c, RKR_ERR_HIP, "find_optimal_sample: the DP's workgroups waited too long for each other");
+    if (!one || err) {
+        // a launch per layer, which waits for nothing: the ranks are too many for
+        // one launch, or its workgroups waited too long for each other (the
+        // device was busy with other work).  Row 0 is as it was put there.
+        for (int32_t l = 1; l < n_sample; ++l)
+            RKR_HIP(c, launch_dp_layer(s, dT.p, dDp.p + ((l - 1) & 1) * R, dPath.p + (int64_t)(l - 1) * R, (int32_t)R,
+                                       dDp.p + (l & 1) * R, dPath.p + (int64_t)l * R));
+        if ((rc = read_back((n_sample - 1) & 1))) return rc;
+    }
 
     // smallest final cost, first index on ties (unsigned compare as the reference's)
     uint64_t min_cost = UINT64_MAX;
