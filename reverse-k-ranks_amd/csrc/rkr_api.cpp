@@ -227,17 +227,20 @@ int refresh_guard_values(Ctx *c, int64_t u0, int64_t n) {
 
 // Guard rows and columns, one allocation.
 static size_t guard_bytes(int64_t cap) { return sizeof(float) * 2 * (size_t)cap * kGuardRow; }
-static void place_guards(Ctx *c, int64_t cap) {
-    c->gcols = c->gvals + (size_t)cap * kGuardRow;
+
+int new_guards(Ctx *c, int64_t cap, float **gv) { return dev_alloc_t(c, gv, guard_bytes(cap) / sizeof(float), "guard values"); }
+
+void place_guards(Ctx *c, float *gv, int64_t cap) {
+    if (gv != c->gvals) dev_free(c, c->gvals, 0);
+    c->gvals = gv;
+    c->gcols = gv + (size_t)cap * kGuardRow;
     c->gpitch = cap;
 }
 
 int alloc_guards(Ctx *c, int64_t cap) {
     float *gv = nullptr;
-    if (int rc = dev_alloc_t(c, &gv, guard_bytes(cap) / sizeof(float), "guard values")) return rc;
-    dev_free(c, c->gvals, 0);
-    c->gvals = gv;
-    place_guards(c, cap);
+    if (int rc = new_guards(c, cap, &gv)) return rc;
+    place_guards(c, gv, cap);
     return RKR_OK;
 }
 
@@ -756,8 +759,7 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
     c->qcol = k_qcol;
     c->table = k_table;
     c->qtable = k_qtable;
-    c->gvals = k_guards;
-    if (k_guards) place_guards(c, cap);
+    if (k_guards) place_guards(c, k_guards, cap);
     int rc = RKR_OK;
     if ((!c->ranks && (rc = dev_alloc_t(c, &c->ranks, (size_t)S, "ranks"))) ||
         (!c->table && (rc = dev_alloc_t(c, &c->table, (size_t)cap * S, "table"))) || (!c->gvals && (rc = alloc_guards(c, cap))) ||

@@ -312,6 +312,9 @@ int rebuild_table(Ctx *c);
 int refresh_guard_values(Ctx *c, int64_t u0, int64_t n);
 // New (unfilled) guard arrays for `cap` users; the old ones go through dev_free.
 int alloc_guards(Ctx *c, int64_t cap);
+// The same in two steps, for a caller that replaces other arrays with them.
+int new_guards(Ctx *c, int64_t cap, float **gv);
+void place_guards(Ctx *c, float *gv, int64_t cap);
 // Recomputes Ctx::ins_gmax after inserted items changed (u0 = 0), or raises it
 // for the new users u0 and up.
 int refresh_ins_guard_max(Ctx *c, int64_t u0);

@@ -78,22 +78,23 @@ int reserve_users(Ctx *c, int64_t need) {
     const int32_t ld = c->ld, S = c->n_sample;
     const int32_t QS = c->n_qs;
     float *users = nullptr, *panels = nullptr, *unorm = nullptr, *table = nullptr, *qtable = nullptr, *si = nullptr,
-          *sd = nullptr;
+          *sd = nullptr, *gv = nullptr;
     int rc = RKR_OK;
-    if ((rc = dev_alloc_t(c, &users, (size_t)cap * ld, "users")) ||
+    // everything that can be refused for memory comes before the first array is replaced
+    if ((c->gvals && (rc = new_guards(c, cap, &gv))) || (rc = dev_alloc_t(c, &users, (size_t)cap * ld, "users")) ||
         (rc = dev_alloc_t(c, &panels, (size_t)((cap + 63) / 64) * 64 * ld, "user panels")) ||
         (c->kp && (rc = dev_alloc_t(c, &unorm, (size_t)cap, "user norms"))) ||
         (rc = dev_alloc_t(c, &table, (size_t)cap * S, "table")) ||
         (QS && (rc = dev_alloc_t(c, &qtable, (size_t)cap * QS, "query table"))) ||
         (c->ld_ins && (rc = dev_alloc_t(c, &si, (size_t)cap * c->ld_ins, "side array"))) ||
         (c->ld_del && (rc = dev_alloc_t(c, &sd, (size_t)cap * c->ld_del, "side array")))) {
-        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
+        for (float *p : {users, panels, unorm, table, qtable, si, sd, gv}) dev_free(c, p, 0);
         return rc;
     }
     uint16_t *uhi = nullptr, *ulo = nullptr;
     if (c->kp && ((rc = dev_alloc_t(c, &uhi, (size_t)cap * c->kp, "user hi")) ||
                   (rc = dev_alloc_t(c, &ulo, (size_t)cap * c->kp, "user lo")))) {
-        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
+        for (float *p : {users, panels, unorm, table, qtable, si, sd, gv}) dev_free(c, p, 0);
         dev_free(c, uhi, 0);
         dev_free(c, ulo, 0);
         return rc;
@@ -129,7 +130,10 @@ int reserve_users(Ctx *c, int64_t need) {
     c->side_del = sd;
     c->side_ins_spare = c->side_del_spare = nullptr;
     c->u_cap = cap;
-    if (c->gvals && ((rc = alloc_guards(c, cap)) || (rc = refresh_guard_values(c, 0, U)))) return rc;
+    if (gv) {
+        place_guards(c, gv, cap);
+        if ((rc = refresh_guard_values(c, 0, U))) return rc;
+    }
     RKR_HIP(c, hipStreamSynchronize(c->stream));
     return RKR_OK;
 }

@@ -28,3 +28,71 @@ def test_sample_rank_dp_without_waiting(I, Q, n_sample):
             ranks, cost = train.find_optimal_sample(idx, 40, I, kth, accu[order], n_sample, "OptimalPart")
             got.append((ranks.tolist(), cost))
     assert got[1:] == got[:1] * 3
+
+
+def _smallest_budget(works, lo=1 << 10, hi=1 << 28, step=1 << 10):
+    """The smallest memory budget (to `step` bytes) that works(budget) accepts."""
+    from rkr import _lib
+    while hi - lo > step:
+        mid = (lo + hi) // 2
+        try:
+            works(mid)
+            hi = mid
+        except _lib.RkrError as e:
+            assert e.status == _lib.RKR_ERR_NOMEM, e
+            lo = mid
+    return hi
+
+
+def test_users_that_do_not_fit():
+    """Inserts of users refused for memory, with every budget between one that
+    holds the index and one that holds the larger one beside it: the index still
+    answers, and the next insert is answered or refused for memory again."""
+    _case("insert users without memory")
+    import rkr
+    from rkr import _lib
+    rng = np.random.default_rng(1)
+    users = rng.standard_normal((20_000, 8), dtype=np.float32)
+    more = rng.standard_normal((9000, 8), dtype=np.float32)
+    items = rng.standard_normal((500, 8), dtype=np.float32)
+    ranks = rkr.Index.uniform_sample_ranks(500, 16)
+    with rkr.Index(0) as idx:
+        idx.set_data(users, items)
+        idx.build_table(ranks)
+        want = idx.query(items[:9], 12)
+
+    def index(budget):
+        idx = rkr.Index(0, budget)
+        idx.set_option(8, 0)  # RKR_OPT_DENSE_TOP: the sampled table alone
+        idx.set_data(users, items)
+        idx.set_option(4, 64)  # RKR_OPT_BUILD_BATCH
+        idx.build_table(ranks)
+        return idx
+
+    def built(budget):
+        index(budget).close()
+
+    def grown(budget):
+        idx = index(budget)
+        try:
+            idx.insert_users(more)
+        finally:
+            idx.close()
+
+    low, high = _smallest_budget(built), _smallest_budget(grown)
+    assert high > low
+    refused = 0
+    for budget in range(low, high, max(1 << 18, (high - low) // 24)):
+        idx = index(budget)
+        for n in (9000, 1, 1):
+            try:
+                idx.insert_users(more[:n])
+            except _lib.RkrError as e:
+                assert e.status == _lib.RKR_ERR_NOMEM, e
+                refused += 1
+        n_user = idx.counts()["n_user"]
+        if n_user == 20_000 and budget > low + (4 << 20):  # room for a query
+            got = idx.query(items[:9], 12)
+            assert np.array_equal(got.users, want.users) and np.array_equal(got.ranks, want.ranks)
+        idx.close()
+    assert refused > 0
