@@ -390,6 +390,7 @@ void free_data(Ctx *c) {
     c->item_norm = c->user_norm = nullptr;
     c->kp = 0;
     c->users = c->usersT = c->items = nullptr;
+    c->items_base = nullptr;  // it was c->items by now
     c->n_user = c->n_item = 0;
     c->dim = c->ld = 0;
 }

@@ -96,3 +96,27 @@ def test_users_that_do_not_fit():
             assert np.array_equal(got.users, want.users) and np.array_equal(got.ranks, want.ranks)
         idx.close()
     assert refused > 0
+
+
+def test_data_that_does_not_fit():
+    """set_data refused for memory at each of its allocations: nothing is freed
+    twice, other indexes are not disturbed."""
+    _case("set_data without memory")
+    import rkr
+    from rkr import _lib
+    rng = np.random.default_rng(1)
+    users = rng.standard_normal((3000, 20), dtype=np.float32)
+    items = rng.standard_normal((900, 20), dtype=np.float32)
+    ranks = rkr.Index.uniform_sample_ranks(900, 16)
+    answers = []
+    for budget in list(range(0, 2_000_000, 50_000)) + [0]:
+        with rkr.Index(0, budget) as idx, rkr.Index(0) as other:
+            try:
+                idx.set_data(users, items)
+            except _lib.RkrError as e:
+                assert e.status == _lib.RKR_ERR_NOMEM, e
+            other.set_data(users, items)
+            other.build_table(ranks)
+            answers.append(other.query(items[:5], 7))
+    for a in answers[1:]:
+        assert np.array_equal(a.users, answers[0].users) and np.array_equal(a.ranks, answers[0].ranks)
