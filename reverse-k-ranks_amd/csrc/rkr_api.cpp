@@ -972,14 +972,16 @@ struct Staging {
 };
 }  // namespace
 
-// Calls sink(rows, user, m, more) for users [u0, u0 + n) in batches of m rows:
-// rows (device memory, stride n_item) holds each user's scores against the
-// current items, sorted in descending order, and more is scratch of `extra`
-// floats per row.  The block size follows the memory budget
-// as the table build's does.
+// Calls sink(rows, user, m, more, spare) for users [u0, u0 + n) in batches of m
+// rows: rows (device memory, stride n_item) holds each user's scores against the
+// current items, sorted in descending order, more is scratch of `extra` floats
+// per row, and spare of `wish` floats per row behind it, null where they do not
+// fit beside one row.  The block size follows the memory budget as the table
+// build's does.
 template <class Sink>
 static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *what, Sink &&sink,
-                                double *gemm_ms = nullptr, double *sort_ms = nullptr, int64_t extra = 0) {
+                                double *gemm_ms = nullptr, double *sort_ms = nullptr, int64_t extra = 0,
+                                int64_t wish = 0) {
     const int64_t I = c->n_item;
     const size_t row_bytes = sizeof(float) * (size_t)I;
     // the scratch kept from an earlier call is there to be used
@@ -987,17 +989,23 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
     int64_t nb = (int64_t)std::min<size_t>(avail / 3 / row_bytes, (size_t)(2ull << 30) / row_bytes);
     if (c->build_batch > 0) nb = std::min<int64_t>(nb, c->build_batch);
     nb = std::min<int64_t>(nb, n);
+    // a third of the budget for the block; its sort scratch and the caller's floats
+    // are as much again for each of nb rows, but not more than all of it
+    const auto need = [&](int64_t rows, int64_t per_row) { return (size_t)rows * (2 * row_bytes + sizeof(float) * (size_t)per_row) + 512; };
+    if (wish > 0 && need(1, extra + wish) > avail) wish = 0;
+    while (nb > 1 && need(nb, extra + wish) > avail) nb -= std::max<int64_t>(1, nb / 16);
     if (nb <= 0) return set_err(c, RKR_ERR_NOMEM, std::string(what) + ": no memory for a score block");
     // the build scratch, kept between calls (allocating and freeing the block
     // took 1 ms of a call over 13k users)
     const int64_t tmp_rows = std::min<int64_t>(nb, sort_rows_in_flight(I, c->n_cu));
     const size_t blk_bytes = ((size_t)nb * row_bytes + 255) & ~(size_t)255;
     const size_t tmp_bytes = ((size_t)tmp_rows * row_bytes + 255) & ~(size_t)255;
-    int rc = ensure(c, c->misc, blk_bytes + tmp_bytes + sizeof(float) * (size_t)(nb * extra), "score block");
+    int rc = ensure(c, c->misc, blk_bytes + tmp_bytes + sizeof(float) * (size_t)(nb * (extra + wish)), "score block");
     if (rc) return rc;
     char *buf = reinterpret_cast<char *>(c->misc.p);
     float *blk = reinterpret_cast<float *>(buf), *tmp = reinterpret_cast<float *>(buf + blk_bytes);
     float *more = reinterpret_cast<float *>(buf + blk_bytes + tmp_bytes);
+    float *spare = wish > 0 ? more + nb * extra : nullptr;
     for (int64_t b0 = 0; b0 < n; b0 += nb) {
         const int64_t m = std::min<int64_t>(nb, n - b0);
         RKR_HIP(c, hipEventRecord(c->ev[0], c->stream));
@@ -1006,7 +1014,7 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
         RKR_HIP(c, hipEventRecord(c->ev[1], c->stream));
         RKR_HIP(c, launch_sort_rows(c->stream, blk, I, m, I, blk, tmp, tmp_rows, I, c->n_cu));
         RKR_HIP(c, hipEventRecord(c->ev[2], c->stream));
-        if ((rc = sink(blk, u0 + b0, m, more))) return rc;  // the sink synchronises the stream
+        if ((rc = sink(blk, u0 + b0, m, more, spare))) return rc;  // the sink synchronises the stream
         if (gemm_ms) *gemm_ms += ev_ms(c->ev, 0, 1);
         if (sort_ms) *sort_ms += ev_ms(c->ev, 1, 2);
     }
@@ -1041,7 +1049,7 @@ int rkr_sorted_scores(rkr_ctx *c, int64_t user_begin, int64_t n_rows, float *out
     const int64_t I = c->n_item;
     Staging stg{c->stream};
     RKR_HIP(c, stg.init(std::min(kStageBytes, sizeof(float) * (size_t)(n_rows * I))));
-    return sorted_score_batches(c, user_begin, n_rows, "sorted_scores", [&](const float *rows, int64_t u, int64_t m, float *) {
+    return sorted_score_batches(c, user_begin, n_rows, "sorted_scores", [&](const float *rows, int64_t u, int64_t m, float *, float *) {
         RKR_HIP(c, stg.to_host(out + (u - user_begin) * I, rows, sizeof(float) * (size_t)(m * I)));
         return (int)RKR_OK;
     });
@@ -1066,7 +1074,7 @@ int rkr_save_score_table(rkr_ctx *c, const char *path, int64_t n_rows, double *t
     const double t0 = rkr_now();
     int rc = n_rows == 0 ? (int)RKR_OK
                          : sorted_score_batches(c, 0, n_rows, "save_score_table",
-                                                [&](const float *rows, int64_t, int64_t m, float *) {
+                                                [&](const float *rows, int64_t, int64_t m, float *, float *) {
         const size_t bytes = sizeof(float) * (size_t)(m * I);
         bool ok = true;
         RKR_HIP(c, stg.run(
@@ -1125,17 +1133,16 @@ int rkr_query_rank_distribution(rkr_ctx *c, const int32_t *item_ids, int32_t n_s
     RKR_HIP(c, launch_gather_rows(c->stream, c->items, c->ld, dids.as<const int64_t>(), ns, c->ld, smat.as<float>(),
                                   c->ld));
     double ms = 0;
-    rc = sorted_score_batches(c, 0, c->n_user, "query_rank_distribution", [&](const float *rows, int64_t u, int64_t m, float *qbuf) {
+    rc = sorted_score_batches(c, 0, c->n_user, "query_rank_distribution", [&](const float *rows, int64_t u, int64_t m, float *qbuf, float *rbuf) {
         RKR_HIP(c, hipEventRecord(c->ev[3], c->stream));
         RKR_HIP(c, launch_scores_store(c->stream, c->users + u * c->ld, m, c->ld, smat.as<float>(), ns, c->ld,
                                        c->dim, qbuf, ns, true));
-        RKR_HIP(c, launch_rank_hist(c->stream, rows, I, m, I, qbuf, ns, (int32_t)ns, h,
-                                    reinterpret_cast<uint16_t *>(qbuf + m * ns + (m * ns & 1))));
+        RKR_HIP(c, launch_rank_hist(c->stream, rows, I, m, I, qbuf, ns, (int32_t)ns, h, reinterpret_cast<uint16_t *>(rbuf)));
         RKR_HIP(c, hipEventRecord(c->ev[4], c->stream));
         RKR_HIP(c, hipEventSynchronize(c->ev[4]));
         ms += ev_ms(c->ev, 0, 2) + ev_ms(c->ev, 3, 4);
         return (int)RKR_OK;
-    }, nullptr, nullptr, ns + rank_row(ns) / 2 + 1);  // a batch's scores (rounded to 8 bytes) and 16-bit ranks
+    }, nullptr, nullptr, ns + (ns & 1), rank_row(ns) / 2);  // a batch's scores (8-byte aligned ends) and, if they fit, 16-bit ranks
     if (rc) return rc;
     // The counts leave through the pinned staging buffers in chunks of whole
     // rows; host threads turn each chunk's counts per rank into users with

@@ -120,3 +120,28 @@ def test_data_that_does_not_fit():
             answers.append(other.query(items[:5], 7))
     for a in answers[1:]:
         assert np.array_equal(a.users, answers[0].users) and np.array_equal(a.ranks, answers[0].ranks)
+@pytest.mark.parametrize("I,ns", [(4000, 4000), (4001, 3999), (3000, 700)])
+def test_rank_distribution_in_little_memory(orc, I, ns):
+    """The distribution is answered wherever its inputs, its counts, one row of
+    scores, one of sort scratch and one of sample scores fit the budget."""
+    _case(f"rank distribution in little memory I={I} ns={ns}")
+    import rkr
+    from rkr import train
+    rng = np.random.default_rng(I)
+    users = rng.standard_normal((30, 6), dtype=np.float32)
+    items = rng.standard_normal((I, 6), dtype=np.float32)
+    ids = rng.choice(I, ns, replace=False).astype(np.int32)
+
+    def loaded(budget):
+        with rkr.Index(0, budget) as idx:
+            idx.set_data(users, items)
+
+    base = _smallest_budget(loaded, step=256)
+    ld = 8
+    need = base + 4 * ns * ld + 8 * ns + 4 * ns * (I + 1) + 3 * 4 * I
+    want = orc.query_rank_distribution(orc.normalize_users(users), items, ids)
+    for spare in (1 << 10, 1 << 13, 1 << 16, 1 << 20):
+        with rkr.Index(0, need + spare) as idx:
+            idx.set_data(users, items)
+            accu, _ = train.query_rank_distribution(idx, ids)
+        assert np.array_equal(accu, want)
