@@ -30,16 +30,38 @@ int set_err(Ctx *c, int code, const std::string &msg) {
 
 const char *kVersion = "rkr 0.1 (gfx950)";
 
+// Frees the build scratch if no call is using it (mem_mu is held).
+static bool drop_misc(Ctx *c) {
+    if (c->misc_busy || !c->misc.p) return false;
+    const auto it = c->alloc_bytes.find(c->misc.p);
+    (void)hipFree(c->misc.p);
+    c->held -= std::min(c->held, it->second);
+    c->alloc_bytes.erase(it);
+    c->misc = DeviceBuf{};
+    return true;
+}
+
+size_t free_bytes(Ctx *c) {
+    std::lock_guard<std::mutex> g(c->mem_mu);
+    return (c->budget > c->held ? c->budget - c->held : 0) + (c->misc_busy ? 0 : c->misc.bytes);
+}
+
 int dev_alloc(Ctx *c, void **p, size_t bytes, const char *what) {
     *p = nullptr;
     if (bytes == 0) return RKR_OK;
     std::lock_guard<std::mutex> g(c->mem_mu);
+    if (c->held + bytes > c->budget) (void)drop_misc(c);
     if (c->held + bytes > c->budget)
         return set_err(c, RKR_ERR_NOMEM, std::string("device memory budget exceeded allocating ") + what + " (" +
                                              std::to_string(bytes) + " bytes, budget " + std::to_string(c->budget) +
                                              ", held " + std::to_string(c->held) + ")");
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && drop_misc(c)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         *p = nullptr;
         return set_err(c, RKR_ERR_NOMEM, std::string("hipMalloc ") + what + ": " + hipGetErrorString(e));
     }
@@ -405,7 +427,7 @@ void free_bufs(Ctx *c, std::initializer_list<DeviceBuf *> bufs) {
 
 void free_scratch(Ctx *c) {
     Slot &s = c->main;
-    free_bufs(c, {&s.io, &s.qip, &s.bk, &s.cand, &s.refine_idx, &s.recheck, &c->misc});
+    free_bufs(c, {&s.io, &s.qip, &s.bk, &s.cand, &s.refine_idx, &s.recheck, &s.hist, &s.q_split, &s.list_info, &s.list, &c->misc});
 }
 
 }  // namespace
@@ -795,7 +817,8 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
     // reference sizes its batch from free memory the same way,
     // GPUComputeSort.hpp:112-135).
     const size_t row_bytes = sizeof(float) * (size_t)c->n_item;
-    size_t avail = c->budget > c->held ? c->budget - c->held : 0;
+    const size_t avail = free_bytes(c);
+    const MiscUse use(c);
     int64_t nb = (int64_t)std::min<size_t>(avail / 2 / row_bytes, (size_t)(8ull << 30) / row_bytes);
     if (c->build_batch > 0) nb = std::min<int64_t>(nb, c->build_batch);
     nb = std::min<int64_t>(nb, c->n_user);
@@ -985,7 +1008,8 @@ static int sorted_score_batches(rkr_ctx *c, int64_t u0, int64_t n, const char *w
     const int64_t I = c->n_item;
     const size_t row_bytes = sizeof(float) * (size_t)I;
     // the scratch kept from an earlier call is there to be used
-    const size_t free_b = c->budget > c->held ? c->budget - c->held : 0, avail = free_b + c->misc.bytes;
+    const size_t avail = free_bytes(c);
+    const MiscUse use(c);
     int64_t nb = (int64_t)std::min<size_t>(avail / 3 / row_bytes, (size_t)(2ull << 30) / row_bytes);
     if (c->build_batch > 0) nb = std::min<int64_t>(nb, c->build_batch);
     nb = std::min<int64_t>(nb, n);
@@ -1509,7 +1533,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // queries per device batch
     int64_t nqb = c->query_batch > 0 ? c->query_batch : 1024;
     {
-        size_t avail = c->budget > c->held ? c->budget - c->held : 0;
+        const size_t avail = free_bytes(c);
         const int64_t by_mem = (int64_t)(avail / 4 / ((size_t)U * pair_bytes + 1));
         nqb = std::max<int64_t>(1, std::min<int64_t>(nqb, by_mem));
         nqb = std::min<int64_t>(nqb, n_query);
@@ -1563,7 +1587,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     int64_t list_cap = 0;
     if (list) {
         // what is held already, or what a quarter of the free budget allows
-        const int64_t avail = (int64_t)((c->budget > c->held ? c->budget - c->held : 0) / 4);
+        const int64_t avail = (int64_t)(free_bytes(c) / 4);
         const int64_t have = std::min<int64_t>({(int64_t)sl.list.bytes / 12, (int64_t)sl.cand.bytes / 8,
                                                 (int64_t)sl.refine_idx.bytes / 16, nqb * U, INT32_MAX / 2});
         const int64_t want = std::max(list_entries(U, nqb), std::min<int64_t>({how.entries, nqb * U, INT32_MAX / 2}));

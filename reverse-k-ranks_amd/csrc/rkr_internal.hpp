@@ -184,7 +184,8 @@ struct Ctx {
     Slot main;
     Slot aux;                   // second stream of split rkr_query calls, made on first use
     bool aux_ready = false;
-    DeviceBuf misc;
+    DeviceBuf misc;             // build scratch, kept between calls and given back when memory is short
+    bool misc_busy = false;     // a call is using it (mem_mu)
 
     // buffers an update thread freed while batches may still read them
     // (snapshot-mode server): released once every batch that started before
@@ -210,6 +211,24 @@ enum {
 constexpr double kQsrpPhiDevErr = 2e-6;
 // Frees the QSRP screen's buffers (the table or the users changed).
 void free_qsrp(Ctx *c);
+
+// Bytes that the context may still allocate: what is left of the budget and the
+// build scratch that no call is using (an allocation that needs it takes it).
+size_t free_bytes(Ctx *c);
+// The build scratch is this call's while one of these lives.
+struct MiscUse {
+    Ctx *c;
+    explicit MiscUse(Ctx *ctx) : c(ctx) { set(true); }
+    ~MiscUse() { set(false); }
+    MiscUse(const MiscUse &) = delete;
+    MiscUse &operator=(const MiscUse &) = delete;
+
+private:
+    void set(bool on) {
+        std::lock_guard<std::mutex> g(c->mem_mu);
+        c->misc_busy = on;
+    }
+};
 
 // Frees made by this thread go to Ctx::retired instead of hipFree: batches may be
 // reading what an update of this thread replaces, so nothing is moved in place.

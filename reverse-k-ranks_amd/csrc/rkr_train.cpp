@@ -208,7 +208,7 @@ int rkr_find_optimal_sample(rkr_ctx *c, int64_t n_user, int64_t n_item, int32_t 
     // one launch keeps every layer's row, if the budget has room beside the rest
     const size_t dp_need = sizeof(int64_t) * (C.size() + (size_t)R + (size_t)(R * (R - 1) / 2) + (size_t)n_sample * R) +
                            sizeof(int32_t) * ((size_t)(2 * R) + (size_t)n_sample * R + 64);
-    const bool one = dp_in_one_launch(R) && c->held + dp_need <= c->budget;
+    const bool one = dp_in_one_launch(R) && dp_need <= free_bytes(c);
     const int64_t dp_rows = one ? n_sample : 2;
     int rc;
     if ((rc = dC.alloc(C.size(), "training prefix sums")) || (rc = dEnd.alloc((size_t)R, "training costs")) ||

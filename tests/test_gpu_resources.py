@@ -145,3 +145,41 @@ def test_rank_distribution_in_little_memory(orc, I, ns):
             idx.set_data(users, items)
             accu, _ = train.query_rank_distribution(idx, ids)
         assert np.array_equal(accu, want)
+
+
+@pytest.mark.parametrize("call", ["insert_users", "query", "find_optimal_sample"])
+def test_scratch_is_given_back(call):
+    """A call in a budget that just holds it is answered whether or not sorted
+    scores, whose scratch takes two thirds of what is free, came before."""
+    _case(f"{call} after sorted scores")
+    import rkr
+    from rkr import train
+    from test_gpu_train import _synthetic_distribution
+    rng = np.random.default_rng(3)
+    users = rng.standard_normal((4000, 8), dtype=np.float32)
+    more = rng.standard_normal((5000, 8), dtype=np.float32)
+    items = rng.standard_normal((600, 8), dtype=np.float32)
+    accu = _synthetic_distribution(rng, 40, 6000, 700, 3000)
+    kth, order = train.sort_kth_rank(accu, 5)
+    queries = items[:1]
+
+    def run(budget, sorted_before):
+        with rkr.Index(0, budget) as idx:
+            idx.set_option(8, 0)  # RKR_OPT_DENSE_TOP: the sampled table alone
+            idx.set_option(9, 0)  # RKR_OPT_COARSE
+            idx.set_data(users, items)
+            if call != "find_optimal_sample":
+                idx.build_table(rkr.Index.uniform_sample_ranks(600, 16))
+            if sorted_before:
+                idx.sorted_scores(0, 100)
+                idx.sorted_scores()
+            if call == "insert_users":
+                idx.insert_users(more)
+            elif call == "query":
+                return idx.query(queries, 10).users.tolist()
+            else:
+                return train.find_optimal_sample(idx, 40, 6000, kth, accu[order], 300, "OptimalPart")[0].tolist()
+
+    budget = _smallest_budget(lambda b: run(b, False))
+    for spare in (1 << 12, 1 << 18, 1 << 20):
+        assert run(budget + spare, True) == run(0, False)
