@@ -1318,7 +1318,7 @@ __global__ void __launch_bounds__(FT) k_list_final(const int32_t *__restrict__ c
 
 // gv[u * kGuardRow + f] = gc[f * pitch + u] = T[u][col_f], -inf past the fine
 // columns, rows [u0, u0 + n_rows): by rows for the searches of one user, by
-// columns for the lists, which read one column of many users.
+// columns (if gc) for the lists, which read one column of many users.
 __global__ void __launch_bounds__(NT) k_gather_guards(const float *__restrict__ T, int64_t S, FineCols fc, int64_t u0,
                                                       int64_t n_rows, float *__restrict__ gv, float *__restrict__ gc,
                                                       int64_t pitch) {
@@ -1333,6 +1333,7 @@ __global__ void __launch_bounds__(NT) k_gather_guards(const float *__restrict__ 
         gv[u * GW + f] = v;
         tile[r][f] = v;
     }
+    if (!gc) return;
     __syncthreads();
     for (int i = threadIdx.x; i < 64 * GW; i += NT) {
         const int f = i / 64, r = i % 64;

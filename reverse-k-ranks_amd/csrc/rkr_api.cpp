@@ -247,22 +247,28 @@ int refresh_guard_values(Ctx *c, int64_t u0, int64_t n) {
     return RKR_OK;
 }
 
-// Guard rows and columns, one allocation.
-static size_t guard_bytes(int64_t cap) { return sizeof(float) * 2 * (size_t)cap * kGuardRow; }
+// Guard rows and columns, one allocation.  The columns only spare the lists a
+// stride of 64 floats; where they would take what a query needs there are rows
+// only, and queries are searched.
+static size_t guard_bytes(int64_t cap, bool cols) { return sizeof(float) * (cols ? 2 : 1) * (size_t)cap * kGuardRow; }
 
-int new_guards(Ctx *c, int64_t cap, float **gv) { return dev_alloc_t(c, gv, guard_bytes(cap) / sizeof(float), "guard values"); }
-
-void place_guards(Ctx *c, float *gv, int64_t cap) {
-    if (gv != c->gvals) dev_free(c, c->gvals, 0);
-    c->gvals = gv;
-    c->gcols = gv + (size_t)cap * kGuardRow;
-    c->gpitch = cap;
+int new_guards(Ctx *c, int64_t cap, size_t spare, Guards *g) {
+    g->cap = cap;
+    g->cols = free_bytes(c) >= 3 * guard_bytes(cap, false) + spare;
+    return dev_alloc_t(c, &g->p, guard_bytes(cap, g->cols) / sizeof(float), "guard values");
 }
 
-int alloc_guards(Ctx *c, int64_t cap) {
-    float *gv = nullptr;
-    if (int rc = new_guards(c, cap, &gv)) return rc;
-    place_guards(c, gv, cap);
+void place_guards(Ctx *c, const Guards &g) {
+    if (g.p != c->gvals) dev_free(c, c->gvals, 0);
+    c->gvals = g.p;
+    c->gcols = g.cols ? g.p + (size_t)g.cap * kGuardRow : nullptr;
+    c->gpitch = g.cap;
+}
+
+int alloc_guards(Ctx *c, int64_t cap, size_t spare) {
+    Guards g;
+    if (int rc = new_guards(c, cap, spare, &g)) return rc;
+    place_guards(c, g);
     return RKR_OK;
 }
 
@@ -774,7 +780,7 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
     int32_t *k_ranks = keep_buffer(c, c->ranks, n_ranks), *k_qranks = keep_buffer(c, c->qranks, n_qr);
     int32_t *k_qcol = nqs ? keep_buffer(c, c->qcol, n_ranks) : nullptr;
     float *k_table = keep_buffer(c, c->table, row * S), *k_qtable = keep_buffer(c, c->qtable, row * nqs);
-    float *k_guards = keep_buffer(c, c->gvals, guard_bytes(cap));
+    float *k_guards = keep_buffer(c, c->gvals, guard_bytes(cap, true));
     free_table(c);
     free_update_state(c, keep_update_buffers);  // the new table describes the current item set
     c->ranks = k_ranks;
@@ -782,13 +788,15 @@ int build_table(Ctx *c, const int32_t *ranks, int32_t S, double *build_ms, bool 
     c->qcol = k_qcol;
     c->table = k_table;
     c->qtable = k_qtable;
-    if (k_guards) place_guards(c, k_guards, cap);
+    if (k_guards) place_guards(c, Guards{k_guards, cap, true});
     int rc = RKR_OK;
     if ((!c->ranks && (rc = dev_alloc_t(c, &c->ranks, (size_t)S, "ranks"))) ||
-        (!c->table && (rc = dev_alloc_t(c, &c->table, (size_t)cap * S, "table"))) || (!c->gvals && (rc = alloc_guards(c, cap))) ||
+        (!c->table && (rc = dev_alloc_t(c, &c->table, (size_t)cap * S, "table"))) ||
         (nqs && !c->qranks && (rc = dev_alloc_t(c, &c->qranks, (size_t)nqs, "query table ranks"))) ||
         (nqs && !c->qcol && (rc = dev_alloc_t(c, &c->qcol, (size_t)S, "query table columns"))) ||
-        (nqs && !c->qtable && (rc = dev_alloc_t(c, &c->qtable, (size_t)cap * nqs, "query table")))) {
+        (nqs && !c->qtable && (rc = dev_alloc_t(c, &c->qtable, (size_t)cap * nqs, "query table"))) ||
+        // beside them the smallest score block fits: two rows of the free budget
+        (!c->gvals && (rc = alloc_guards(c, cap, 2 * sizeof(float) * (size_t)c->n_item)))) {
         free_table(c);
         return rc;
     }
@@ -866,7 +874,7 @@ int rkr_set_table(rkr_ctx *c, const int32_t *ranks, int32_t S, const float *tabl
     int rc = dev_alloc_t(c, &c->ranks, (size_t)S, "ranks");
     if (rc) return rc;
     rc = dev_alloc_t(c, &c->table, (size_t)std::max(c->u_cap, c->n_user) * S, "table");
-    if (!rc) rc = alloc_guards(c, std::max(c->u_cap, c->n_user));
+    if (!rc) rc = alloc_guards(c, std::max(c->u_cap, c->n_user), 0);
     if (rc) { free_table(c); return rc; }
     c->n_sample = S;
     c->h_ranks.assign(ranks, ranks + S);
@@ -1543,7 +1551,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // they spare (one user's table row per query, or per batch of 4 and more)
     // outweighs their three launches of about 5 us: at 64k users one plain
     // query is even, and batches of 8 at 4k users.
-    const bool list = listable && !upd &&
+    const bool list = listable && !upd && dv.gcols &&
                       (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
     const bool list_mfma = list && mfma && how.level <= kThreeProducts;
     const int products = how.level == kThreeProducts ? 3 : 1;

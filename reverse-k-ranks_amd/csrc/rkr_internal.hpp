@@ -143,7 +143,7 @@ struct Ctx {
     // guard rows: [u_cap][kGuardRow], the values of the searched table at its
     // fine columns, -inf past them; kept with the table
     float *gvals = nullptr;
-    float *gcols = nullptr;     // the same values by column behind them: [kGuardRow][u_cap at allocation]
+    float *gcols = nullptr;     // the same values by column behind them: [kGuardRow][u_cap at allocation], or null
     int64_t gpitch = 0;
     // columns of the guard rows, the guard columns among them and the searched
     // table's ranks, set with the table
@@ -297,7 +297,7 @@ struct DataSnap {
     GuardCols guards{};              // guard columns of the coarse bounds
     FineCols fine{};                 // columns of the guard rows
     const float *gvals = nullptr;    // guard values per user (kGuardRow floats)
-    const float *gcols = nullptr;    // and by column, rows of gpitch users
+    const float *gcols = nullptr;    // and by column, rows of gpitch users, or null
     int64_t gpitch = 0;
     // the sampled table's ranks (device), count and eps, the query table's
     // column of each sampled column, and the searched table's ranks on the
@@ -330,10 +330,16 @@ int rebuild_table(Ctx *c);
 // Fills Ctx::gvals and gcols of users [u0, u0 + n) from the searched table.
 int refresh_guard_values(Ctx *c, int64_t u0, int64_t n);
 // New (unfilled) guard arrays for `cap` users; the old ones go through dev_free.
-int alloc_guards(Ctx *c, int64_t cap);
+// Columns only where `spare` bytes and as much again as they take stay free.
+int alloc_guards(Ctx *c, int64_t cap, size_t spare);
 // The same in two steps, for a caller that replaces other arrays with them.
-int new_guards(Ctx *c, int64_t cap, float **gv);
-void place_guards(Ctx *c, float *gv, int64_t cap);
+struct Guards {
+    float *p = nullptr;
+    int64_t cap = 0;
+    bool cols = false;
+};
+int new_guards(Ctx *c, int64_t cap, size_t spare, Guards *g);
+void place_guards(Ctx *c, const Guards &g);
 // Recomputes Ctx::ins_gmax after inserted items changed (u0 = 0), or raises it
 // for the new users u0 and up.
 int refresh_ins_guard_max(Ctx *c, int64_t u0);

@@ -78,23 +78,30 @@ int reserve_users(Ctx *c, int64_t need) {
     const int32_t ld = c->ld, S = c->n_sample;
     const int32_t QS = c->n_qs;
     float *users = nullptr, *panels = nullptr, *unorm = nullptr, *table = nullptr, *qtable = nullptr, *si = nullptr,
-          *sd = nullptr, *gv = nullptr;
+          *sd = nullptr;
+    Guards gv;
     int rc = RKR_OK;
     // everything that can be refused for memory comes before the first array is replaced
-    if ((c->gvals && (rc = new_guards(c, cap, &gv))) || (rc = dev_alloc_t(c, &users, (size_t)cap * ld, "users")) ||
+    if ((rc = dev_alloc_t(c, &users, (size_t)cap * ld, "users")) ||
         (rc = dev_alloc_t(c, &panels, (size_t)((cap + 63) / 64) * 64 * ld, "user panels")) ||
         (c->kp && (rc = dev_alloc_t(c, &unorm, (size_t)cap, "user norms"))) ||
         (rc = dev_alloc_t(c, &table, (size_t)cap * S, "table")) ||
         (QS && (rc = dev_alloc_t(c, &qtable, (size_t)cap * QS, "query table"))) ||
         (c->ld_ins && (rc = dev_alloc_t(c, &si, (size_t)cap * c->ld_ins, "side array"))) ||
         (c->ld_del && (rc = dev_alloc_t(c, &sd, (size_t)cap * c->ld_del, "side array")))) {
-        for (float *p : {users, panels, unorm, table, qtable, si, sd, gv}) dev_free(c, p, 0);
+        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
         return rc;
     }
     uint16_t *uhi = nullptr, *ulo = nullptr;
     if (c->kp && ((rc = dev_alloc_t(c, &uhi, (size_t)cap * c->kp, "user hi")) ||
                   (rc = dev_alloc_t(c, &ulo, (size_t)cap * c->kp, "user lo")))) {
-        for (float *p : {users, panels, unorm, table, qtable, si, sd, gv}) dev_free(c, p, 0);
+        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
+        dev_free(c, uhi, 0);
+        dev_free(c, ulo, 0);
+        return rc;
+    }
+    if (c->gvals && (rc = new_guards(c, cap, 0, &gv))) {
+        for (float *p : {users, panels, unorm, table, qtable, si, sd}) dev_free(c, p, 0);
         dev_free(c, uhi, 0);
         dev_free(c, ulo, 0);
         return rc;
@@ -130,8 +137,8 @@ int reserve_users(Ctx *c, int64_t need) {
     c->side_del = sd;
     c->side_ins_spare = c->side_del_spare = nullptr;
     c->u_cap = cap;
-    if (gv) {
-        place_guards(c, gv, cap);
+    if (gv.p) {
+        place_guards(c, gv);
         if ((rc = refresh_guard_values(c, 0, U))) return rc;
     }
     RKR_HIP(c, hipStreamSynchronize(c->stream));
@@ -648,7 +655,7 @@ int rkr_delete_users(rkr_ctx *c, const int64_t *ids, int64_t n) {
     rc = keep_user_rows(c, &c->users, ld, ld, d_keep, nk, "users");
     if (!rc) rc = keep_user_rows(c, &c->table, c->n_sample, c->n_sample, d_keep, nk, "table");
     if (!rc) rc = keep_user_rows(c, &c->qtable, c->n_qs, c->n_qs, d_keep, nk, "query table");
-    if (!rc && c->gvals && !(rc = alloc_guards(c, c->u_cap))) rc = refresh_guard_values(c, 0, nk);
+    if (!rc && c->gvals && !(rc = alloc_guards(c, c->u_cap, 0))) rc = refresh_guard_values(c, 0, nk);
     if (!rc) rc = keep_user_rows(c, &c->side_ins, c->n_ins, c->ld_ins, d_keep, nk, "side array");
     if (!rc) rc = keep_user_rows(c, &c->side_del, c->n_del, c->ld_del, d_keep, nk, "side array");
     dev_free(c, d_keep, 0);

@@ -183,3 +183,54 @@ def test_scratch_is_given_back(call):
     budget = _smallest_budget(lambda b: run(b, False))
     for spare in (1 << 12, 1 << 18, 1 << 20):
         assert run(budget + spare, True) == run(0, False)
+
+
+@pytest.mark.parametrize("dense", [0, 2])
+def test_table_without_room_for_guard_columns(dense):
+    """A table is built, and its queries are answered, wherever it fits with 64
+    guard values a user and two rows of scores, whatever else would be faster."""
+    _case(f"table in little memory, dense={dense}")
+    import rkr
+    rng = np.random.default_rng(5)
+    U, I, S = 30_000, 700, 20
+    users = rng.standard_normal((U, 12), dtype=np.float32)
+    items = rng.standard_normal((I, 12), dtype=np.float32)
+    ranks = rkr.Index.uniform_sample_ranks(I, S)
+    more = rng.standard_normal((500, 12), dtype=np.float32)
+    with rkr.Index(0) as idx:
+        idx.set_option(8, dense)  # RKR_OPT_DENSE_TOP
+        idx.set_data(users, items)
+        idx.build_table(ranks)
+        want = idx.query(items[:20], 9)
+        table = idx.get_table()
+        idx.insert_users(more)
+        later = idx.query(items[:20], 9)
+
+    def loaded(budget):
+        with rkr.Index(0, budget) as idx:
+            idx.set_data(users, items)
+
+    base = _smallest_budget(loaded)
+    cols = S + (I if dense else 0)
+    need = base + 4 * U * cols + 4 * (3 * S + I) + 256 * U + 2 * 4 * I
+    for spare in (1 << 12, 4 << 20, 8 << 20, 16 << 20, 32 << 20):
+        with rkr.Index(0, need + spare) as idx:
+            idx.set_option(8, dense)
+            idx.set_data(users, items)
+            idx.build_table(ranks)
+            assert np.array_equal(idx.get_table(), table)
+            if spare < 4 << 20:
+                continue
+            for form in ("plain", "screened"):
+                if form == "screened" and spare < 32 << 20:
+                    continue  # its recheck list alone takes 16 MB
+                idx.set_form(form)
+                got = idx.query(items[:20], 9)
+                assert np.array_equal(got.users, want.users) and np.array_equal(got.ranks, want.ranks)
+    with rkr.Index(0, need + 4 * U * (cols + 100) + (40 << 20)) as idx:  # grown, perhaps without columns
+        idx.set_option(8, dense)
+        idx.set_data(users, items)
+        idx.build_table(ranks)
+        idx.insert_users(more)
+        got = idx.query(items[:20], 9)
+        assert np.array_equal(got.users, later.users) and np.array_equal(got.ranks, later.ranks)
