@@ -200,3 +200,23 @@ def test_stage_times(gpu_index_factory):
             for f in ("ip_ms", "bound_ms", "prune_ms", "refine_ms", "recheck_ms", "topk_ms", "h2d_ms", "d2h_ms"):
                 assert 0 <= t[f] <= 3 * t["total_ms"], f  # of three batches
     idx.close()
+
+
+@pytest.mark.parametrize("form", ["plain", "screened"])
+@pytest.mark.parametrize("U,nq", [(64, 300), (1000, 64), (1000, 400), (5000, 20)])
+def test_k_on_either_side_of_a_quarter_of_the_users(gpu_index_factory, form, U, nq):
+    """Batches that want less and more than a quarter of all users on average."""
+    _case(f"k about U / 4, {form} U={U} nq={nq}")
+    rng = np.random.default_rng(U)
+    users = rng.standard_normal((U, 14), dtype=np.float32)
+    items = rng.standard_normal((700, 14), dtype=np.float32)
+    queries = items[rng.choice(700, nq, replace=False)]
+    idx, _ = gpu_index_factory(users, items, 30)
+    idx.set_form(form)
+    for k in (U // 4 - 1, U // 4, U // 4 + 1, U // 2, U):
+        ks = [min(k, 4096)] * nq
+        idx.set_option(9, 1)  # RKR_OPT_COARSE
+        got = idx.query(queries, ks)
+        idx.set_option(9, 0)
+        _same_answers(got, idx.query(queries, ks), ks)
+    idx.close()
