@@ -1533,12 +1533,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // the QSRP screen (RKR_OPT_QSRP, built by rkr_qsrp_build) replaces the bound
     // stage of exact batches without pending updates
     const bool qsrp = c->qsrp && dv.qsrp_users && mode == RKR_OUTPUT_EXACT && !upd && U > 0;
-    // a list holds k users at least: with a quarter of all users wanted there is
-    // nothing to leave out (64 queries, 1000 users, k = 500: 0.33 ms with lists
-    // tried first, 0.09 now)
-    int64_t k_sum = 0;
-    for (int32_t i = 0; i < n_query; ++i) k_sum += topk[i];
-    const bool listable = (upd || 4 * k_sum <= (int64_t)n_query * U) && !qsrp && how.level != kSearch && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
+    const bool listable = !qsrp && how.level != kSearch && c->coarse && mode == RKR_OUTPUT_EXACT && dv.fine.n > 0 && dv.gvals &&
                           dv.guards.n > 0 && U > 0;
     const bool mfma = screened && c->kp > 0 && dv.user_norm;
     const size_t pair_bytes = upd ? 12 : 8;  // <u,q> + buckets, or + two bound values
@@ -1556,8 +1551,15 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     // they spare (one user's table row per query, or per batch of 4 and more)
     // outweighs their three launches of about 5 us: at 64k users one plain
     // query is even, and batches of 8 at 4k users.
-    const bool list = listable && !upd && dv.gcols &&
-                      (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
+    const bool list_size = listable && !upd && dv.gcols &&
+                           (nqb >= kCoarseMinBatch ? screened || U >= 4096 : U >= (nqb >= 4 ? 8192 : 65536));
+    // A list holds k users at least: with a quarter of all users wanted there is
+    // nothing to leave out (64 queries, 1000 users, k = 500: 0.33 ms with lists
+    // tried first, 0.09 now).
+    int64_t k_sum = 0;
+    for (int32_t i = 0; i < n_query; ++i) k_sum += topk[i];
+    const bool list = list_size && 4 * k_sum <= (int64_t)n_query * U;
+    if (list_size && !list && how.level == kOneProduct) tm.n_fallback += n_query;
     const bool list_mfma = list && mfma && how.level <= kThreeProducts;
     const int products = how.level == kThreeProducts ? 3 : 1;
     // scores left by the last attempt, of this attempt's queries
