@@ -1877,9 +1877,12 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
             RKR_HIP(c, launch_offsets(sl.stream, qi, nq, refine_total));
             RKR_HIP(c, hipMemcpyAsync(hqi, qi, sizeof(QueryInfo) * nq, hipMemcpyDeviceToHost, sl.stream));
             RKR_HIP(c, hipStreamSynchronize(sl.stream));
-            total = hqi[nq - 1].cand_off + hqi[nq - 1].n_settled + hqi[nq - 1].n_cand;
-            total_cand = 0;
-            for (int32_t i = 0; i < nq; ++i) total_cand += hqi[i].n_cand;
+            // (the device's offsets are 32-bit sums: past that the check below is on these)
+            total = total_cand = 0;
+            for (int32_t i = 0; i < nq; ++i) {
+                total += (int64_t)hqi[i].n_settled + hqi[i].n_cand;
+                total_cand += hqi[i].n_cand;
+            }
         }
         if (!deep_check.empty()) {
             // a user below the deepest guard has rank >= r[j_last] + 1 - n_del:

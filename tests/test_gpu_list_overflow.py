@@ -220,3 +220,25 @@ def test_k_on_either_side_of_a_quarter_of_the_users(gpu_index_factory, form, U, 
         idx.set_option(9, 0)
         _same_answers(got, idx.query(queries, ks), ks)
     idx.close()
+
+
+def test_more_candidates_than_32_bits_count(gpu_index_factory):
+    """2000 queries that each of 2.2 million users ranks first, 4.4e9 candidates
+    in one batch: refused, as from 2^31 candidates on, whatever a 32-bit sum says."""
+    _case("4.4e9 candidates")
+    from rkr import _lib
+    rng = np.random.default_rng(1)
+    U, nq, d = 2_200_000, 2000, 4
+    users = np.abs(rng.standard_normal((U, d), dtype=np.float32)) + np.float32(0.1)
+    items = -np.abs(rng.standard_normal((60, d), dtype=np.float32))
+    queries = np.abs(rng.standard_normal((nq, d), dtype=np.float32)) + np.float32(0.1)
+    idx, _ = gpu_index_factory(users, items, 16, dense_top=0)
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    idx.set_option(3, 2000)  # RKR_OPT_QUERY_BATCH
+    with pytest.raises(_lib.RkrError) as e:
+        idx.query(queries, 5)
+    assert e.value.status == _lib.RKR_ERR_NOMEM and "lower the query batch" in str(e.value)
+    idx.set_option(3, 200)
+    idx.set_option(9, 1)
+    assert np.array_equal(idx.query(queries[:300], 5).users, np.tile(np.arange(5), (300, 1)))
+    idx.close()
