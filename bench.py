@@ -488,14 +488,14 @@ def cpu_baseline(wl, table, ranks, users_norm, gpu_users, k, n_max, seconds):
 # plain 1 GiB device copy gives, bench.py --copy-calibration).  Keyed by
 # (workload, form); other configurations report null.
 PROFILED_TRAFFIC = {
-    ("precision", "screened"): {"kernel": "k_list_screen", "bytes": 1.042e9, "fetch_kib": 484924.0,
-                                "write_kib": 48115.0, "profile": "profiles/query_batch_1M_x_50k_d150_k50.md"},
+    ("precision", "screened"): {"kernel": "k_list_screen", "bytes": 1.053e9, "fetch_kib": 489397.0,
+                                "write_kib": 49337.0, "profile": "profiles/query_batch_1M_x_50k_d150_k50.md"},
 }
 
 
-# k_sort_rows, 100k x 20k: FETCH_SIZE 1,054,886.2 KiB (x2.0) + WRITE_SIZE 2,115,848.5 KiB (x1.0) per
+# k_sort_rows, 100k x 20k: FETCH_SIZE 1,054,946 KiB (x2.0) + WRITE_SIZE 2,099,157 KiB (x1.0) per
 # full-batch launch (26,843 rows)
-SORT_TRAFFIC_BYTES = 4.327e9
+SORT_TRAFFIC_BYTES = 4.310e9
 
 
 def copy_calibration():

@@ -76,9 +76,13 @@ typedef struct rkr_ctx rkr_ctx;
                                    users whose score can reach a threshold column
                                    of their table row, and only those are searched;
                                    the screened form takes the scores for this from
-                                   BF16 matrix cores and scores the listed users
-                                   exactly, the plain form scores every user
-                                   exactly.  0: every user is scored and searched.
+                                   BF16 matrix cores (one product, or three where
+                                   one cannot tell the users apart) and scores the
+                                   listed users exactly, the plain form scores
+                                   every user exactly.  Queries whose lists hold
+                                   too much of the users, and batches that want a
+                                   quarter of all of them, are searched.  0: every
+                                   user is scored and searched.
                                    Answers are unchanged.                        */
 #define RKR_OPT_QSRP 11         /* 0 (default); 1: exact queries without pending
                                    updates screen users with the QSRP bounds that
@@ -120,7 +124,8 @@ typedef struct rkr_batch_timing {
     int64_t n_rechecked;
     int64_t n_screened;
     double max_screen_err;  /* screened form: max |screen - FP64| observed     */
-    int64_t n_listed;       /* RKR_OPT_COARSE: (query, user) pairs listed      */
+    int64_t n_listed;       /* RKR_OPT_COARSE: (query, user) pairs listed, in
+                               the lists that were used                        */
     int64_t n_fallback;     /* RKR_OPT_COARSE: queries that took the full path */
     int64_t n_coarse_refined; /* RKR_OPT_COARSE: queries listed against a column
                                  finer than the 7 guard columns                */

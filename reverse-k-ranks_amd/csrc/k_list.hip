@@ -65,8 +65,9 @@ __device__ __forceinline__ int64_t sample_user(int64_t r, int64_t stride, int64_
     return min((uint32_t)r * (uint32_t)stride + __umulhi(h, (uint32_t)stride), (uint32_t)n_user - 1u);
 }
 
-// Guard rows of NU sampled users (r0 + i, i < NU, clamped to the last) to LDS rows of stride GW + 1: an odd stride, so the lanes' searches
-// fall in different banks.  Every load is in flight before the first write.
+// Guard rows of NU sampled users (r0 + i, i < NU, clamped to the last) to LDS rows
+// of stride GW + 1: an odd stride, so the lanes' searches fall in different banks.
+// Every load is in flight before the first write.
 constexpr int GP = GW + 1;
 template <int NU>
 __device__ __forceinline__ void stage_guards(float *dst, const float *__restrict__ gvals, int64_t r0, int64_t n_s,
@@ -256,12 +257,12 @@ __global__ void __launch_bounds__(NT) k_sample_scores(const float *__restrict__ 
 // the largest of theirs (a larger column lists more users, never fewer).  A
 // query with no such column, or with a list that the scores' error takes past
 // cap, gets thr = -1 (finer scores answer it) and no slot, one whose list is over
-// cap without the error kNoList (a search over every user answers it).  So
-// do the queries whose lists the scores' error makes more than `band` pairs
-// longer, and those whose lists are longer than `share`, if that is enough in all
-// to pay for what another attempt costs however few its queries: kBandMin pairs,
-// the 80 us of a pass from finer scores, or kSearchUsers pairs a user, the
-// search's 4 ms at 1M users (nothing if some query is searched anyway).  Lists are taken in order of
+// cap without the error kNoList (a search over every user answers it).  So do the
+// queries whose lists the scores' error makes more than `band` pairs longer, and
+// those whose lists are longer than `share`, if that is enough in all to pay for
+// what another attempt costs however few its queries: kBandMin pairs, the 80 us
+// of a pass from finer scores, or kSearchUsers pairs a user, the search's 4 ms at
+// 1M users (nothing if some query is searched anyway).  Lists are taken in order of
 // their length, up to `room` pairs; the longer ones get thr = kNoRoom and
 // ctr->n_need says how many pairs they hold.  (Taken in order of their column,
 // popular queries came first and one of them kept every other out.)
@@ -275,7 +276,8 @@ constexpr int64_t kBandMin = 400000, kSearchUsers = 12;
 
 __global__ void __launch_bounds__(PT) k_list_plan(const uint32_t *__restrict__ hist, int32_t nq, int32_t n_fine,
                                                   int64_t stride, int64_t n_user, int64_t cap, int64_t share,
-                                                  int64_t band, int64_t room, int64_t list_cap, uint64_t coarse_mask, QueryInfo *__restrict__ qi,
+                                                  int64_t band, int64_t room, int64_t list_cap,
+                                                  uint64_t coarse_mask, QueryInfo *__restrict__ qi,
                                                   int32_t *__restrict__ order, int32_t *__restrict__ colg,
                                                   ListCounters *__restrict__ ctr) {
     __shared__ int32_t bin[GW], at[GW], mix[GW];
@@ -602,11 +604,13 @@ __device__ __forceinline__ void wave_flush(const uint32_t *q, int n, int32_t bas
 // per stage); a block's thresholds are loaded while the previous one is
 // computed.  With PROD = 3 the stage is 32 queries' hi and lo rows.  A
 // workgroup whose pairs find the list full stops there (reading the counter at
-// the start of each unit instead took 140 of 705 us, 1M users x 1000 queries).  A pair costs one fused multiply-add and one compare beside its
-// share of the matrix products; listed pairs are queued per wavefront without
-// an atomic, and a unit takes its part of the list with one.  Bound: the
-// matrix cores' 16 cycles per 16x16x32 product and about 100 VALU instructions
-// per 16 queries x 16 NB users beside them.
+// the start of each unit instead took 140 of 705 us, 1M users x 1000 queries).
+// A pair costs one fused multiply-add and one compare beside its share of the
+// matrix products; listed pairs are queued per wavefront without an atomic, and
+// a unit takes its part of the list with one.  Bound: the matrix cores' 16
+// cycles per 16x16x32 product and about 100 VALU instructions per 16 queries x
+// 16 NB users beside them: 573 us at 1M users x 150 dims x 1000 queries, 560
+// TFLOP/s (80 bytes a thread spilled).
 template <int KS, int NB, int PROD>
 __global__ void __launch_bounds__(NT, PROD == 1 && KS <= 5 ? 3 : 2) k_list_screen(ListScreen P, int64_t n_user,
                                                                      const int32_t *__restrict__ order,

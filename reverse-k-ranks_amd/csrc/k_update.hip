@@ -607,7 +607,8 @@ hipError_t launch_subtract_rows(hipStream_t s, const float *a, int64_t lda, int3
 // Queries up to which the guard rows' path is taken.  100k users, 20k items, 500
 // pending: 16 queries 0.33 ms against 0.65 with rows staged, 32 0.63 against
 // 0.55; 60k users, 8k items, 40 pending: 32 0.18 against 0.32, 64 0.35 against
-// 0.34 (the staged rows serve any number of queries).
+// 0.34 (the staged rows serve any number of queries).  The crossing moves with the
+// columns and the pending items; 24 lies between the sides of the nearer one.
 constexpr int kGuardBounds = 24;
 
 hipError_t launch_bounds_upd(hipStream_t s, const float *qip, const float *table, const float *gvals,

@@ -606,7 +606,9 @@ struct ListLaunch {
 // which spares the two launches that order it.  Without the order and with it,
 // ms: 16 queries over 1M users 0.31 and 0.35, 6 over 30k 0.13 and 0.14.  Each
 // query reads all of the list, so popular queries pay for it: 16 of them over
-// 1M users 0.59 and 0.42, 8 over 250k 0.22 and 0.19.
+// 1M users 0.59 and 0.42, 8 over 250k 0.22 and 0.19.  A count of queries it stays,
+// since how long their lists are is known on the device only when the launches
+// are already made; ordinary queries are the more frequent.
 constexpr int kFilterQueries = 16;
 // Threshold per query and the listed pairs, from the matrix cores or from qip.
 hipError_t launch_list_screen(hipStream_t s, const ListLaunch &L);
