@@ -1559,7 +1559,7 @@ int run_batches(Ctx *c, Slot &sl, const DataSnap &dv, const float *queries, int3
     int64_t k_sum = 0;
     for (int32_t i = 0; i < n_query; ++i) k_sum += topk[i];
     const bool list = list_size && 4 * k_sum <= (int64_t)n_query * U;
-    if (list_size && !list && how.level == kOneProduct) tm.n_fallback += n_query;
+    if (list_size && !list && how.level == kOneProduct && how.entries == 0) tm.n_fallback += n_query;
     const bool list_mfma = list && mfma && how.level <= kThreeProducts;
     const int products = how.level == kThreeProducts ? 3 : 1;
     // scores left by the last attempt, of this attempt's queries

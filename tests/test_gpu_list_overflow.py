@@ -222,6 +222,26 @@ def test_k_on_either_side_of_a_quarter_of_the_users(gpu_index_factory, form, U, 
     idx.close()
 
 
+def test_queries_left_without_room_are_counted_once(gpu_index_factory):
+    """Lists of a little more than a quarter of all users in a batch that wants less on
+    average: the ones without room are searched, and are one query each of n_fallback."""
+    _case("long lists without room")
+    rng = np.random.default_rng(5)
+    U, I, nq = 12_000, 3000, 64
+    users = rng.standard_normal((U, 24), dtype=np.float32)
+    items = rng.standard_normal((I, 24), dtype=np.float32)
+    items /= np.linalg.norm(items, axis=1, keepdims=True)
+    queries = items[rng.choice(I, nq, replace=False)]
+    ks = [10] * 4 + [3010] * 60
+    idx, _ = gpu_index_factory(users, items, 64)
+    idx.set_form("screened")
+    got = idx.query(queries, ks)
+    assert 0 < got.timing["n_fallback"] <= nq
+    idx.set_option(9, 0)  # RKR_OPT_COARSE
+    _same_answers(got, idx.query(queries, ks), ks)
+    idx.close()
+
+
 def test_more_candidates_than_32_bits_count(gpu_index_factory):
     """2000 queries that each of 2.2 million users ranks first, 4.4e9 candidates
     in one batch: refused, as from 2^31 candidates on, whatever a 32-bit sum says."""
